@@ -101,15 +101,29 @@ __global__ __launch_bounds__(256) void kb_absmax_kernel(const float *__restrict_
     if (threadIdx.x < 64)
         m[threadIdx.x] = 0.0;
     __syncthreads();
-    // Thread t takes feature t % d of samples t / d, t / d + spp, ... (d <= 64).
+    // Thread t takes feature t % d of samples t / d, t / d + spp, ... (d <= 64), eight loads in
+    // flight (one at a time left the pass latency-bound).
     const int spp = 256 / d, sub = (int)threadIdx.x / d, l = (int)threadIdx.x - sub * d;
     if (sub < spp) {
-        double mx = 0.0;
-        for (int i = sub; i < ch.count; i += spp) {
-            const double v = fabs((double)x[(int64_t)i * d + l]);
-            if (v == v && v < __builtin_huge_val())
-                mx = fmax(mx, v);
+        float mf = 0.0f;
+        auto take = [&](float v) {
+            const float a = fabsf(v);
+            if (a < __builtin_huge_valf()) // false for NaN too
+                mf = fmaxf(mf, a);
+        };
+        int i = sub;
+        for (; i + 7 * spp < ch.count; i += 8 * spp) {
+            float v[8];
+#pragma unroll
+            for (int u = 0; u < 8; u++)
+                v[u] = x[(int64_t)(i + u * spp) * d + l];
+#pragma unroll
+            for (int u = 0; u < 8; u++)
+                take(v[u]);
         }
+        for (; i < ch.count; i += spp)
+            take(x[(int64_t)i * d + l]);
+        const double mx = (double)mf;
         atomicMax(reinterpret_cast<unsigned long long *>(&m[l]),
                   (unsigned long long)__double_as_longlong(mx));
     }
@@ -147,7 +161,8 @@ __global__ void kb_escale_kernel(KBatchDesc b, int n_inst,
     escale[inst * 65 + 64] = 61 - l2n;
 }
 
-// Copy of each instance's rows in the operand type, padded to kp features.
+// Copy of each instance's rows in the operand type, padded to kp features. Instances whose
+// rows already are operand rows (xboff < 0, see kb_operand_rows) are left out.
 template <class Op>
 __global__ __launch_bounds__(256) void kb_to_op_kernel(const float *__restrict__ X, KBatchDesc b,
                                                        const KChunk *__restrict__ chunks,
@@ -155,17 +170,44 @@ __global__ __launch_bounds__(256) void kb_to_op_kernel(const float *__restrict__
     using T = typename Op::T;
     const KChunk ch = chunks[blockIdx.x];
     const int inst = ch.inst, d = b.d[inst], kp = b.kp[inst];
+    if (b.xboff[inst] < 0)
+        return;
     const float *x = X + b.xoff[inst] + (int64_t)ch.start * d;
     const int rs = kp * Op::NS;
     T *y = Xo + b.xboff[inst] + (int64_t)ch.start * rs;
     const int spp = 256 / kp, sub = (int)threadIdx.x / kp, l = (int)threadIdx.x - sub * kp;
-    for (int i = sub; i < ch.count; i += spp) {
-        const float v = l < d ? x[(int64_t)i * d + l] : 0.0f;
+    auto put = [&](int i, float v) {
         const T hi = (T)v;
         y[(int64_t)i * rs + l] = hi;
         if constexpr (Op::NS == 2)
             y[(int64_t)i * rs + kp + l] = (T)(v - (float)hi);
+    };
+    int i = sub;
+    for (; i + 7 * spp < ch.count; i += 8 * spp) {
+        float v[8];
+#pragma unroll
+        for (int u = 0; u < 8; u++)
+            v[u] = l < d ? x[(int64_t)(i + u * spp) * d + l] : 0.0f;
+#pragma unroll
+        for (int u = 0; u < 8; u++)
+            put(i + u * spp, v[u]);
     }
+    for (; i < ch.count; i += spp)
+        put(i, l < d ? x[(int64_t)i * d + l] : 0.0f);
+}
+
+// Operand rows of an instance: its padded copy, or, in the fp32 form, the caller's rows
+// themselves where they already have a padded width and 16-byte alignment (the host marks these
+// with xboff < 0): the copy would only cost its write and a second read.
+template <class Op>
+__device__ __forceinline__ const typename Op::T *kb_operand_rows(const typename Op::T *Xo,
+                                                                 const float *X,
+                                                                 const KBatchDesc &b, int inst) {
+    const int64_t o = b.xboff[inst];
+    if constexpr (Op::E == 1)
+        if (o < 0)
+            return X + b.xoff[inst];
+    return Xo + o;
 }
 
 // Initial centres (fp32, packed k x d per instance) into the double master copy.
@@ -399,8 +441,8 @@ __device__ __forceinline__ void kb_assign_tile(const typename Op::T *__restrict_
 constexpr int KB_RUN = 4;
 template <class Op, int PT>
 __global__ __launch_bounds__(256) void kb_assign_kernel(
-    const typename Op::T *__restrict__ Xo, KBatchDesc b, const KTile *__restrict__ tiles,
-    int ntiles, const int *__restrict__ state, const int *__restrict__ fpar, int mode, int par,
+    const typename Op::T *__restrict__ Xo, const float *__restrict__ X, KBatchDesc b,
+    const KTile *__restrict__ tiles, int ntiles, const int *__restrict__ state, const int *__restrict__ fpar, int mode, int par,
     const typename Op::T *__restrict__ Cb, const float *__restrict__ chalf,
     const double *__restrict__ cmax2, int *__restrict__ L0, int *__restrict__ L1,
     int *__restrict__ changed, int *__restrict__ list_count, KTile *__restrict__ list) {
@@ -433,7 +475,7 @@ __global__ __launch_bounds__(256) void kb_assign_kernel(
         int *lab_new = (p ? L1 : L0) + b.loff[inst];
         const int *lab_old = mode == 0 ? (p ? L0 : L1) + b.loff[inst] : nullptr;
         const double cmax = sqrt(cmax2[inst]);
-        const T *xo = Xo + b.xboff[inst];
+        const T *xo = kb_operand_rows<Op>(Xo, X, b, inst);
         const int n = b.n[inst];
 #define KB_TILE(NFV)                                                                             \
     kb_assign_tile<Op, NFV, PT>(xo, n, kp, tl.start, Cs, Hs, k, cmax, lab_new, lab_old,        \
@@ -566,20 +608,28 @@ __global__ __launch_bounds__(1024) void kb_partial_kernel(
     // R-th sample of the cluster from the r-th on.
     const int P = k * d;
     const int R = P >= 1024 ? 1 : 1024 / P;
+    // A value x becomes h = rint(x 2^e_l) and, where that leaves a remainder, a low word. The
+    // scale is a double of its own (|e_l| < 210 for float data), so h takes a product and a
+    // rounding; |h| < 2^(60 - l2n), so eight of them add up exactly in a double once l2n >= 10
+    // (1,023 samples or more), and only their sum is converted to an integer. Non-finite values
+    // are left out. Against ldexp and one conversion per value this cut the pass from 851 us to
+    // 190 us (256 instances, 3.2 M samples of 8-64 features, together with smaller chunks).
+    const bool exact8 = lshift <= 51;
+    const double lscale = ldexp(1.0, lshift);
     auto pair_sum = [&](int p, int r, long long &H, long long &Lw) {
         const int c = p / d, l = p - c * d;
         const int j1 = off[c + 1];
-        const int el = es[l];
+        const double scale = ldexp(1.0, es[l]);
         H = 0;
         Lw = 0;
-        auto add = [&](float xv) {
-            const double v = (double)xv;
-            if (v == v && v - v == 0.0) {
-                const double sv = ldexp(v, el);
-                const double h = rint(sv);
-                H += (long long)h;
-                Lw += (long long)rint(ldexp(sv - h, lshift));
-            }
+        auto high = [&](float xv) {
+            const double sv = (double)xv * scale;
+            const bool ok = fabs(sv) < 0x1p60;
+            const double h = ok ? rint(sv) : 0.0;
+            const double rem = ok ? sv - h : 0.0;
+            if (rem != 0.0)
+                Lw += (long long)rint(rem * lscale);
+            return h;
         };
         const float *xs = x + l;
         int j = off[c] + r;
@@ -589,12 +639,20 @@ __global__ __launch_bounds__(1024) void kb_partial_kernel(
 #pragma unroll
             for (int u = 0; u < 8; u++)
                 v[u] = xs[(int64_t)list[j + u * R] * d];
+            if (exact8) {
+                double hs = 0.0;
 #pragma unroll
-            for (int u = 0; u < 8; u++)
-                add(v[u]);
+                for (int u = 0; u < 8; u++)
+                    hs += high(v[u]);
+                H += (long long)hs;
+            } else {
+#pragma unroll
+                for (int u = 0; u < 8; u++)
+                    H += (long long)high(v[u]);
+            }
         }
         for (; j < j1; j += R)
-            add(xs[(int64_t)list[j] * d]);
+            H += (long long)high(xs[(int64_t)list[j] * d]);
     };
     if (R == 1) {
         for (int p = threadIdx.x; p < P; p += 1024) {
@@ -631,7 +689,7 @@ __global__ __launch_bounds__(1024) void kb_partial_kernel(
 // Per instance: new centres from its chunks' partials (fixed order), the centre shift and
 // norm, and the convergence test of kmeans.cpp:1359-1397 (iteration j > 1 with no label
 // change: stop with labels unchanged; shift below tol * norm: stop on the shift).
-__global__ __launch_bounds__(256) void kb_reduce_kernel(
+__global__ __launch_bounds__(1024) void kb_reduce_kernel(
     KBatchDesc b, const int *__restrict__ cbeg, const int *__restrict__ cend,
     const int64_t *__restrict__ poff, const long long *__restrict__ part,
     const int *__restrict__ pcnt, const int *__restrict__ escale, int par, int iter,
@@ -645,17 +703,38 @@ __global__ __launch_bounds__(256) void kb_reduce_kernel(
     double *Cout = (par ? C0 : C1) + b.coff[inst];
     const int *es = escale + inst * 65;
     const int lshift = es[64];
-    __shared__ double s0[256], s1[256];
+    __shared__ double s0[1024], s1[1024];
+    __shared__ int cnt[64];
+    const int q0 = cbeg[inst], nq = cend[inst] - q0;
+    // Cluster sizes: 16 threads per cluster (k <= 64).
+    {
+        const int c = threadIdx.x >> 4, u = threadIdx.x & 15;
+        int v = 0;
+        if (c < k)
+            for (int q = u; q < nq; q += 16)
+                v += pcnt[(int64_t)(q0 + q) * 64 + c];
+#pragma unroll
+        for (int o = 8; o > 0; o >>= 1)
+            v += __shfl_xor(v, o, 16);
+        if (u == 0)
+            cnt[c] = v;
+    }
+    __syncthreads();
+    // The partials of an instance's chunks lie one after another.
+    const int64_t ps = (int64_t)k * d * 2;
+    const long long *p0 = part + (nq > 0 ? poff[q0] : 0);
     double x0 = 0.0, x1 = 0.0;
-    for (int e = threadIdx.x; e < k * d; e += 256) {
+    for (int e = threadIdx.x; e < k * d; e += 1024) {
         const int c = e / d, l = e - c * d;
         long long H = 0, Lw = 0;
-        int count = 0;
-        for (int q = cbeg[inst]; q < cend[inst]; q++) {
-            H += part[poff[q] + 2 * e];
-            Lw += part[poff[q] + 2 * e + 1];
-            count += pcnt[(int64_t)q * 64 + c];
+        const longlong2 *pe = reinterpret_cast<const longlong2 *>(p0 + 2 * e);
+#pragma unroll 8
+        for (int q = 0; q < nq; q++) {
+            const longlong2 v = pe[q * (ps / 2)];
+            H += v.x;
+            Lw += v.y;
         }
+        const int count = cnt[c];
         const double sum = ldexp((double)H, -es[l]) + ldexp((double)Lw, -(es[l] + lshift));
         // An empty cluster keeps count 1 and a zero sum: the origin
         // (scale_current_cluster_centres, kmeans_lloyd.hpp:363-373).
@@ -668,7 +747,7 @@ __global__ __launch_bounds__(256) void kb_reduce_kernel(
     s0[threadIdx.x] = x0;
     s1[threadIdx.x] = x1;
     __syncthreads();
-    for (int w = 128; w > 0; w >>= 1) {
+    for (int w = 512; w > 0; w >>= 1) {
         if ((int)threadIdx.x < w) {
             s0[threadIdx.x] += s0[threadIdx.x + w];
             s1[threadIdx.x] += s1[threadIdx.x + w];
@@ -705,24 +784,46 @@ __device__ __forceinline__ const int *kb_final_labels(const int *L0, const int *
     return p ? L1 : L0;
 }
 
-// Inertia per chunk: sum of exact squared distances to the final centres in a fixed order.
+// Inertia per chunk: sum of exact squared distances to the final centres in a fixed order; and
+// the chunk's final labels into the caller's array.
 __global__ __launch_bounds__(256) void kb_inertia_kernel(
     const float *__restrict__ X, KBatchDesc b, const KChunk *__restrict__ chunks,
     const double *C0, const double *C1, const int *__restrict__ state,
     const int *__restrict__ fpar, const int *__restrict__ L0, const int *__restrict__ L1,
-    double *__restrict__ cin) {
+    double *__restrict__ cin, int *__restrict__ labels) {
     const KChunk ch = chunks[blockIdx.x];
     const int inst = ch.inst, d = b.d[inst];
     const double *C = (1 - fpar[inst] ? C1 : C0) + b.coff[inst];
     const int *lab = kb_final_labels(L0, L1, state, fpar, inst) + b.loff[inst];
+    int *out = labels + b.loff[inst];
     const float *x = X + b.xoff[inst];
+    // Rows of whole 16-byte pieces are read in them (the same sums in the same order).
+    const bool vec = (d & 3) == 0 && (reinterpret_cast<uintptr_t>(x) & 15) == 0;
     double s = 0.0;
     for (int i = ch.start + threadIdx.x; i < ch.start + ch.count; i += 256) {
         const int c = lab[i];
+        out[i] = c;
+        const double *cc = C + (int64_t)c * d;
         double acc = 0.0;
-        for (int l = 0; l < d; l++) {
-            const double v = (double)x[(int64_t)i * d + l] - C[(int64_t)c * d + l];
-            acc = fma(v, v, acc);
+        if (vec) {
+            const float4 *x4 = reinterpret_cast<const float4 *>(x + (int64_t)i * d);
+#pragma unroll 4
+            for (int l4 = 0; l4 < d / 4; l4++) {
+                const float4 f = x4[l4];
+                double v = (double)f.x - cc[4 * l4];
+                acc = fma(v, v, acc);
+                v = (double)f.y - cc[4 * l4 + 1];
+                acc = fma(v, v, acc);
+                v = (double)f.z - cc[4 * l4 + 2];
+                acc = fma(v, v, acc);
+                v = (double)f.w - cc[4 * l4 + 3];
+                acc = fma(v, v, acc);
+            }
+        } else {
+            for (int l = 0; l < d; l++) {
+                const double v = (double)x[(int64_t)i * d + l] - cc[l];
+                acc = fma(v, v, acc);
+            }
         }
         s += acc;
     }
@@ -738,21 +839,17 @@ __global__ __launch_bounds__(256) void kb_inertia_kernel(
         cin[blockIdx.x] = sh[0];
 }
 
-// Outputs: final centres (fp32) and labels in the caller's packed arrays, inertia per
-// instance (its chunks summed in order).
+// Outputs: final centres (fp32) in the caller's packed array, inertia per instance (its chunks
+// summed in order).
 __global__ __launch_bounds__(256) void kb_output_kernel(
-    KBatchDesc b, const double *C0, const double *C1, const int *__restrict__ state,
-    const int *__restrict__ fpar, const int *__restrict__ L0, const int *__restrict__ L1,
+    KBatchDesc b, const double *C0, const double *C1, const int *__restrict__ fpar,
     const int *__restrict__ cbeg, const int *__restrict__ cend, const double *__restrict__ cin,
-    float *__restrict__ Cout, int *__restrict__ labels, double *__restrict__ inertia) {
+    float *__restrict__ Cout, double *__restrict__ inertia) {
     const int inst = blockIdx.x;
-    const int d = b.d[inst], k = b.k[inst], n = b.n[inst];
+    const int d = b.d[inst], k = b.k[inst];
     const double *C = (1 - fpar[inst] ? C1 : C0) + b.coff[inst];
     for (int e = threadIdx.x; e < k * d; e += 256)
         Cout[b.coff[inst] + e] = (float)C[e];
-    const int *lab = kb_final_labels(L0, L1, state, fpar, inst) + b.loff[inst];
-    for (int i = threadIdx.x; i < n; i += 256)
-        labels[b.loff[inst] + i] = lab[i];
     if (threadIdx.x == 0) {
         double s = 0.0;
         for (int q = cbeg[inst]; q < cend[inst]; q++)
@@ -815,11 +912,11 @@ static void kb_assign_op(const KBatchBuffers &w, const KBatchDesc &b, int n_inst
     hipLaunchKernelGGL(kb_centre_prep_kernel<Op>, dim3(n_inst), dim3(64), 0, s, b, w.C0, w.C1,
                        w.state, w.fpar, mode, par, Cb, w.chalf, w.cmax2);
     if (pt == 2)
-        hipLaunchKernelGGL((kb_assign_kernel<Op, 2>), dim3(grid), dim3(256), 0, s, Xo, b, w.tiles,
+        hipLaunchKernelGGL((kb_assign_kernel<Op, 2>), dim3(grid), dim3(256), 0, s, Xo, w.X, b, w.tiles,
                            w.ntiles, w.state, w.fpar, mode, par, Cb, w.chalf, w.cmax2, w.L0, w.L1,
                            w.changed, w.list_count, w.list);
     else
-        hipLaunchKernelGGL((kb_assign_kernel<Op, 4>), dim3(grid), dim3(256), 0, s, Xo, b, w.tiles,
+        hipLaunchKernelGGL((kb_assign_kernel<Op, 4>), dim3(grid), dim3(256), 0, s, Xo, w.X, b, w.tiles,
                            w.ntiles, w.state, w.fpar, mode, par, Cb, w.chalf, w.cmax2, w.L0, w.L1,
                            w.changed, w.list_count, w.list);
 }
@@ -843,7 +940,7 @@ hipError_t kb_launch_update(const KBatchBuffers &w, const KBatchDesc &b, int n_i
                             int iter, double tol, size_t lds, hipStream_t s) {
     hipLaunchKernelGGL(kb_partial_kernel, dim3(w.nchunks), dim3(1024), lds, s, w.X, b, w.chunks,
                        w.poff, w.state, par, w.L0, w.L1, w.escale, w.part, w.pcnt);
-    hipLaunchKernelGGL(kb_reduce_kernel, dim3(n_inst), dim3(256), 0, s, b, w.cbeg, w.cend, w.poff,
+    hipLaunchKernelGGL(kb_reduce_kernel, dim3(n_inst), dim3(1024), 0, s, b, w.cbeg, w.cend, w.poff,
                        w.part, w.pcnt, w.escale, par, iter, tol, w.C0, w.C1, w.changed,
                        w.state, w.fpar, w.n_iter);
     return hipGetLastError();
@@ -857,9 +954,9 @@ hipError_t kb_launch_finish(const KBatchBuffers &w, const KBatchDesc &b, int n_i
     if (e != hipSuccess)
         return e;
     hipLaunchKernelGGL(kb_inertia_kernel, dim3(w.nchunks), dim3(256), 0, s, w.X, b, w.chunks, w.C0,
-                       w.C1, w.state, w.fpar, w.L0, w.L1, w.cin);
-    hipLaunchKernelGGL(kb_output_kernel, dim3(n_inst), dim3(256), 0, s, b, w.C0, w.C1, w.state,
-                       w.fpar, w.L0, w.L1, w.cbeg, w.cend, w.cin, Cout, labels, inertia);
+                       w.C1, w.state, w.fpar, w.L0, w.L1, w.cin, labels);
+    hipLaunchKernelGGL(kb_output_kernel, dim3(n_inst), dim3(256), 0, s, b, w.C0, w.C1, w.fpar,
+                       w.cbeg, w.cend, w.cin, Cout, inertia);
     return hipGetLastError();
 }
 

@@ -83,7 +83,7 @@ int op_width(int prec, int d) {
 }
 
 da_status build(BatchRun &r, da_int n_inst, const da_int *n, const da_int *d, const da_int *k,
-                const float *X, int chunk_hint, int prec) {
+                const float *X, int prec) {
     hipStream_t st = r.gpu.stream();
     r.n_inst = n_inst;
     std::vector<int> hn(n, n + n_inst), hd(d, d + n_inst), hk(k, k + n_inst), hkp(n_inst);
@@ -93,25 +93,45 @@ da_status build(BatchRun &r, da_int n_inst, const da_int *n, const da_int *d, co
     for (int i = 0; i < n_inst; i++) {
         hkp[i] = op_width(prec, hd[i]);
         xoff[i] = xo;
-        xboff[i] = xbo;
+        // fp32 rows of a padded width and 16-byte alignment are their own operand rows.
+        const bool direct = prec == 0 && hkp[i] == hd[i] &&
+                            (reinterpret_cast<uintptr_t>(X + xo) & 15) == 0;
+        xboff[i] = direct ? -1 : xbo;
         coff[i] = co;
         cboff[i] = cbo;
         loff[i] = lo;
         xo += (int64_t)hn[i] * hd[i];
-        xbo += (int64_t)hn[i] * hkp[i] * parts;
+        if (!direct)
+            xbo += (int64_t)hn[i] * hkp[i] * parts;
         co += (int64_t)hk[i] * hd[i];
         cbo += (int64_t)((hk[i] + 15) / 16 * 16) * hkp[i] * parts;
         lo += hn[i];
     }
     r.ctotal = co;
-    // Sample chunks for sums, maxima and inertia.
-    const int cs = chunk_hint;
+    // Sample chunks for sums, maxima and inertia: about eight per CU over the whole batch, of
+    // equal work (samples x features), so that a small batch fills the chip too and no chunk of a
+    // wide instance ends last. At least 16 k samples, so that a chunk's partial sums (16 k d
+    // bytes written, then read) stay below a quarter of its rows; at most 16,384 (the sorted
+    // sample list in LDS). With 16,384-sample chunks throughout, 256 instances of 1,000-50,000
+    // samples gave some 400 workgroups and 18.6 ms a run; now 2,000 and 5.5 ms.
+    int dev = 0, cus = 0;
+    if (hipGetDevice(&dev) != hipSuccess ||
+        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
+        cus < 1)
+        cus = 256;
+    const int64_t chunk_work = std::max<int64_t>(1, xo / (8 * cus));
+    auto chunk_samples = [&](int i) {
+        const int64_t want = (chunk_work + hd[i] - 1) / hd[i];
+        const int64_t lo = std::max(512, 16 * hk[i]);
+        return (int)(std::max<int64_t>(lo, std::min<int64_t>(16384, want)) + 63) / 64 * 64;
+    };
     std::vector<KChunk> chunks;
     std::vector<int> cbeg(n_inst), cend(n_inst);
     std::vector<int64_t> poff;
     int64_t po = 0;
     for (int i = 0; i < n_inst; i++) {
         cbeg[i] = (int)chunks.size();
+        const int cs = chunk_samples(i);
         for (int s0 = 0; s0 < hn[i]; s0 += cs) {
             chunks.push_back({i, s0, std::min(cs, hn[i] - s0), 0});
             poff.push_back(po);
@@ -324,8 +344,7 @@ da_status da_kmeans_batch_device_s(da_int n_inst, const da_int *n, const da_int 
         da_status s = run->gpu.init(&g_err);
         if (s != da_status_success)
             return s;
-        // Chunks of about 16 K samples (the centroid partials of a chunk are k*d*16 bytes).
-        s = build(*run, n_inst, n, d, k, X, 16384, (int)cross_term);
+        s = build(*run, n_inst, n, d, k, X, (int)cross_term);
         if (s != da_status_success)
             return s;
         s = tune(*run, n, d, k, C);
