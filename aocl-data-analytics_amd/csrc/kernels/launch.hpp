@@ -141,30 +141,51 @@ template <typename T>
 hipError_t launch_gather_rows(const T *X, int d, const int *idx, int m, double *C,
                               hipStream_t s);
 
-// k-means++ helpers. w[i] = squared distance of X_i to row `ci` of X (exact, double), with
+// AFK-MC2 helpers. w[i] = squared distance of X_i to row `ci` of X (exact, double), with
 // negative or non-finite values set to 0 and w[ci] = 0. sph: the cosine distance
 // max(0, 1 - X_i.X_ci inv[i] inv[ci]) instead (inv null: rows taken as unit rows); the same
-// choice for launch_candidate_cost and launch_min_update.
+// choice for launch_min_update.
 template <typename T>
 hipError_t launch_dist_to_row(const T *X, int n, int d, int ci, double *w, hipStream_t s,
                               int sph = 0, const double *inv = nullptr);
 // cp[i] = inclusive prefix sum of w[i]/sum (sum = *total), cp[n-1] = 1. tmp: >= 2*1024 doubles.
 hipError_t launch_normalised_scan(const double *w, int n, const double *total, double *cp,
                                   double *tmp, hipStream_t s);
-// out[t] = first i with cp[i] >= u[t] (lower_bound), t < nt.
-hipError_t launch_lower_bound(const double *cp, int n, const double *u, int nt, int *out,
-                              hipStream_t s);
-// For each candidate row cand[t]: part[t*nb + b] = partial of sum_i max(0, min(w[i], d_i(t))).
-template <typename T>
-hipError_t launch_candidate_cost(const T *X, int n, int d, const double *w, const int *cand,
-                                 int nt, double *part, int nb, hipStream_t s, int sph = 0,
-                                 const double *inv = nullptr);
 // w[i] = max(0, min(w[i], d_i(ci))), w[ci] = 0.
 template <typename T>
 hipError_t launch_min_update(const T *X, int n, int d, int ci, double *w, hipStream_t s,
                              int sph = 0, const double *inv = nullptr);
-// Reduces part[t*nb + b] over b for each t into out[t] (fixed order).
-hipError_t launch_reduce_rows(const double *part, int nt, int nb, double *out, hipStream_t s);
+// ---- k-means++ (kmeans_pp.hip) ----
+// Device state of one initialisation: the centre chosen last and the candidates of the current
+// and of the previous round (by the parity of the round); same: every sample coincides with the
+// first centre.
+constexpr int KPP_TRIALS_MAX = 23; // 2 + ln k for any 32-bit k
+struct KppState {
+    int best, same;
+    int cand[2][KPP_TRIALS_MAX];
+};
+// Sample chunks of the passes (nb <= 1,024 of `chunk` rows) and the width of a row of crow.
+struct KppPlan {
+    int chunk, nb, slots;
+};
+KppPlan kpp_plan(int n, int nt);
+// State and crow (d x p.slots doubles) for the first centre, row `first` of X.
+template <typename T>
+hipError_t launch_kpp_begin(const T *X, int d, int first, double *crow, const KppPlan &p,
+                            KppState *st, hipStream_t s);
+// The pass over the data of round c: the weights w (n doubles) take in the centre st->best,
+// part[t*p.nb + b] = the sums of min(w, d(candidate t)). c = 0: the weights are set from the
+// first centre, part[b] = their sums.
+template <typename T>
+hipError_t launch_kpp_cost(const T *X, int n, int d, double *w, const double *crow,
+                           const KppState *st, int c, int nt, const KppPlan &p, double *part,
+                           hipStream_t s, int sph, const double *inv);
+// Round c: chosen[c - 1] from the costs in part (c = 1: the first centre), then, for c < k, the
+// nt candidates of centre c from the draws u[0..nt) and their rows in crow. c = k ends it.
+template <typename T>
+hipError_t launch_kpp_draw(const T *X, int n, int d, const double *w, const double *part, int nt,
+                           int c, int k, const double *u, double *crow, const KppPlan &p,
+                           KppState *st, int *chosen, hipStream_t s, int sph, const double *inv);
 // Direct distances of rows of X to centres (double), sqrt applied: D[i*ldd + c]. sph: the
 // cosine distance 1 - clamp(X_i.C_c inv[i], -1, 1) (inv null: 1 - clamp(X_i.C_c)).
 template <typename T>

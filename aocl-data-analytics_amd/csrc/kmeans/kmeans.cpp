@@ -652,76 +652,50 @@ da_status KMeansHandle<T>::run_lloyd(const U *dX, double tol, da_int max_iter, R
 }
 
 // k-means++ (kmeans.cpp:1524-1664): the random draws are made on the host with the same
-// libstdc++ engine and distributions in the same order; the distance passes, the weight
-// normalisation and the inverse-CDF lookup of std::discrete_distribution run on the GPU.
+// libstdc++ engine and distributions in the same order (their number does not depend on the
+// data), everything else, the choice of each centre included, runs on the device
+// (kmeans_pp.hip): two launches per centre and one synchronisation at the end.
 template <typename T> da_status KMeansHandle<T>::kmeans_plusplus() {
     hipStream_t st = gpu->stream();
     const int n = n_samples_, d = n_features_, k = n_clusters_;
     const T *dX = X_.as<T>();
-    std::vector<int> chosen(k, 0);
     const da_int n_trials = 2 + (da_int)std::log((double)k);
     std::uniform_int_distribution<> dis_int(0, n - 1);
     const int first = dis_int(mt_);
-    chosen[0] = first;
+    const std::mt19937_64 after_first = mt_;
+    const size_t draws = n >= 2 ? (size_t)(k - 1) * n_trials : 0;
+    std::vector<double> u(draws);
+    for (auto &v : u)
+        v = std::generate_canonical<double, std::numeric_limits<double>::digits>(mt_);
+    const KppPlan plan = kpp_plan(n, n_trials);
+    // One block of scratch: the rows of the candidates, the partial sums, the draws, the state.
+    const size_t nrow = (size_t)d * plan.slots, npart = (size_t)n_trials * plan.nb;
+    DA_HIP(err, w_.reserve((size_t)n * sizeof(double)));
+    DA_HIP(err, kpp_.reserve((nrow + npart + draws) * sizeof(double) + sizeof(KppState)));
     double *w = w_.as<double>();
-    DA_HIP(err, launch_dist_to_row<T>(dX, n, d, first, w, st, sph_, winv()));
-    double *total = small_.as<double>() + 3;
-    DA_HIP(err, launch_sum_double(w, n, tmp_.as<double>(), total, st));
-    double htot = 0;
-    DA_HIP(err, hipMemcpyAsync(&htot, total, sizeof(double), hipMemcpyDeviceToHost, st));
-    DA_HIP(err, hipStreamSynchronize(st));
-    if (!(htot > 0.0)) {
-        // All points coincide with the first centre: take the first k points.
-        for (int c = 0; c < k; c++)
-            chosen[c] = c;
-    } else {
-        // Partial sums of the candidate costs: one per workgroup, about 1,024 samples each, at
-        // most 2,048 (their n_trials * nb partials fit the n doubles of cp_, n_trials <= 32).
-        const int nb = (int)std::max<int64_t>(1, std::min<int64_t>(2048, (int64_t)n / 1024));
-        std::vector<double> u(n_trials), cost(n_trials);
-        std::vector<int> cand(n_trials);
-        double *du = tmp_.as<double>() + 1024;
-        int *dcand = idx_.as<int>();
-        double *dcost = tmp_.as<double>() + 1024 + 64;
-        double *part = cp_.as<double>(); // reused after the lookup
-        for (int c = 1; c < k; c++) {
-            if (n >= 2) {
-                DA_HIP(err, launch_sum_double(w, n, tmp_.as<double>(), total, st));
-                DA_HIP(err, launch_normalised_scan(w, n, total, cp_.as<double>(), tmp_.as<double>(), st));
-                for (int t = 0; t < n_trials; t++)
-                    u[t] = std::generate_canonical<double, std::numeric_limits<double>::digits>(mt_);
-                DA_HIP(err, hipMemcpyAsync(du, u.data(), n_trials * sizeof(double), hipMemcpyHostToDevice, st));
-                DA_HIP(err, launch_lower_bound(cp_.as<double>(), n, du, n_trials, dcand, st));
-                DA_HIP(err, hipMemcpyAsync(cand.data(), dcand, n_trials * sizeof(int), hipMemcpyDeviceToHost, st));
-                DA_HIP(err, hipStreamSynchronize(st));
-            } else {
-                std::fill(cand.begin(), cand.end(), 0);
-            }
-            DA_HIP(err, launch_candidate_cost<T>(dX, n, d, w, dcand, n_trials, part, nb, st, sph_,
-                                                 winv()));
-            DA_HIP(err, launch_reduce_rows(part, n_trials, nb, dcost, st));
-            DA_HIP(err, hipMemcpyAsync(cost.data(), dcost, n_trials * sizeof(double), hipMemcpyDeviceToHost, st));
-            DA_HIP(err, hipStreamSynchronize(st));
-            int best = 0;
-            double best_cost = std::numeric_limits<double>::infinity();
-            for (int t = 0; t < n_trials; t++) {
-                bool repeat = false;
-                for (int j = 0; j < t; j++)
-                    repeat |= cand[j] == cand[t];
-                if (repeat)
-                    continue;
-                if (std::isfinite(cost[t]) && cost[t] < best_cost) {
-                    best_cost = cost[t];
-                    best = cand[t];
-                }
-            }
-            chosen[c] = best;
-            DA_HIP(err, launch_min_update<T>(dX, n, d, best, w, st, sph_, winv()));
-        }
+    double *crow = kpp_.as<double>(), *part = crow + nrow, *du = part + npart;
+    KppState *state = reinterpret_cast<KppState *>(du + draws);
+    if (draws > 0)
+        DA_HIP(err, hipMemcpyAsync(du, u.data(), draws * sizeof(double), hipMemcpyHostToDevice, st));
+    DA_HIP(err, launch_kpp_begin<T>(dX, d, first, crow, plan, state, st));
+    DA_HIP(err, launch_kpp_cost<T>(dX, n, d, w, crow, state, 0, 0, plan, part, st, sph_, winv()));
+    for (int c = 1; c < k; c++) {
+        DA_HIP(err, launch_kpp_draw<T>(dX, n, d, w, part, n_trials, c, k,
+                                       du + (size_t)(c - 1) * n_trials, crow, plan, state,
+                                       idx_.as<int>(), st, sph_, winv()));
+        DA_HIP(err, launch_kpp_cost<T>(dX, n, d, w, crow, state, c, n_trials, plan, part, st,
+                                       sph_, winv()));
     }
-    DA_HIP(err, hipMemcpyAsync(idx_.ptr(), chosen.data(), k * sizeof(int), hipMemcpyHostToDevice, st));
+    DA_HIP(err, launch_kpp_draw<T>(dX, n, d, w, part, n_trials, k, k, du, crow, plan, state,
+                                   idx_.as<int>(), st, sph_, winv()));
     DA_HIP(err, launch_gather_rows<T>(dX, d, idx_.as<int>(), k, Ccur_, st));
+    int same = 0;
+    DA_HIP(err, hipMemcpyAsync(&same, &state->same, sizeof(int), hipMemcpyDeviceToHost, st));
     DA_HIP(err, hipStreamSynchronize(st));
+    // When every sample coincides with the first centre, the first k samples are taken and no
+    // draw is made.
+    if (same)
+        mt_ = after_first;
     return da_status_success;
 }
 
@@ -807,12 +781,14 @@ template <typename T> da_status KMeansHandle<T>::afk_mc2() {
     std::uniform_int_distribution<> dis_int(0, n - 1);
     chosen[0] = dis_int(mt_);
     // w: squared distance of each sample to its nearest chosen centre.
+    DA_HIP(err, w_.reserve((size_t)n * sizeof(double)));
     double *w = w_.as<double>();
     DA_HIP(err, launch_dist_to_row<T>(dX, n, d, chosen[0], w, st, sph_, winv()));
     if (k > 1) {
         double *total = small_.as<double>() + 3;
         int *dout = reinterpret_cast<int *>(small_.as<double>() + 10);
         DA_HIP(err, aq_.reserve((size_t)n * sizeof(double)));
+        DA_HIP(err, cp_.reserve((size_t)n * sizeof(double)));
         DA_HIP(err, au_.reserve((size_t)(2 * m + 1) * sizeof(double)));
         double *q = aq_.as<double>(), *cp = cp_.as<double>();
         DA_HIP(err, launch_sum_double(w, n, tmp_.as<double>(), total, st));
@@ -921,8 +897,6 @@ template <typename T> da_status KMeansHandle<T>::compute() {
     DA_HIP(err, small_.reserve(16 * sizeof(double)));
     DA_HIP(err, tmp_.reserve(4096 * sizeof(double)));
     DA_HIP(err, idx_.reserve((size_t)std::max(k, 64) * sizeof(int)));
-    DA_HIP(err, w_.reserve((size_t)n * sizeof(double)));
-    DA_HIP(err, cp_.reserve((size_t)std::max(n, 256 * 64) * sizeof(double)));
     // Centroid sums: chunks of up to 8,192 points (sorted by label in LDS), about two per
     // workgroup, one workgroup per CU; passes of at most KMEANS_PASS_PAIRS (cluster, feature)
     // pairs summed in registers (all of them for k = 256 at d = 32), at most 12,288 clusters

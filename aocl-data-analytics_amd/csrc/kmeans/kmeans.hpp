@@ -88,7 +88,7 @@ template <typename T> class KMeansHandle : public AlgHandle {
     std::mt19937_64 mt_;
     // Device state.
     DeviceBuffer X_, Xlp_, escale_, Ca_, Cb_, lab_a_, lab_b_, counts_, part_, pcnt_, mind_,
-        small_, w_, cp_, tmp_, idx_, Cbest_, q_, q_stage_, out_;
+        small_, w_, cp_, tmp_, idx_, kpp_, Cbest_, q_, q_stage_, out_;
     // Spherical k-means (the "distance" option "cosine"): sph_ set by compute, sph_norm_ when
     // the data are normalised; inv_ the inverse sample norms; escale_unit_ the exponents of
     // sums of unit rows; qinv_ the inverse norms of transformed samples.
