@@ -8,6 +8,9 @@
 
 namespace dagpu {
 
+// Smallest set served by hit bits: below it the general path's few launches are as fast.
+constexpr int BITS_MIN_ROWS = 2048;
+
 // Algorithm codes of the "algorithm" option (da_neighbors_types::nn_algorithm).
 enum { DB_BRUTE = 0, DB_KD_TREE = 1, DB_BALL_TREE = 2, DB_AUTO = 3 };
 
@@ -89,8 +92,112 @@ da_status DBSCANHandle<T>::set_data(da_int n_samples, da_int n_features, const T
     return da_status_success;
 }
 
+template <typename T>
+da_status DBSCANHandle<T>::reserve_edges(long long total, long long used) {
+    const size_t cap = ind_.size() / sizeof(int);
+    if ((size_t)total <= cap)
+        return da_status_success;
+    hipStream_t st = gpu->stream();
+    const size_t ncap = std::max<size_t>({(size_t)total, 2 * cap, (size_t)1 << 20});
+    DA_HIP(err, ind_spare_.reserve(ncap * sizeof(int)));
+    if (used > 0)
+        DA_HIP(err, hipMemcpyAsync(ind_spare_.ptr(), ind_.ptr(), (size_t)used * sizeof(int),
+                                   hipMemcpyDeviceToDevice, st));
+    DA_HIP(err, hipStreamSynchronize(st));
+    ind_.swap(ind_spare_);
+    ind_spare_.release();
+    return da_status_success;
+}
+
+// Hit bits (radius_mfma.hip) for row blocks of up to 128 MiB of bits (which stay in the last
+// level cache between the sweep, the verification and the fill), counts, offsets and a fill of
+// the set bits. Measured at 100,000 x 16 fp32 against the key tiles of the general path (40 GB
+// of keys written and read): PERF_DBSCAN.
+template <typename T>
+da_status DBSCANHandle<T>::neighbour_graph_bits(int km, T thr, const double *nrm, bool &done) {
+    done = false;
+    hipStream_t st = gpu->stream();
+    const int n = n_samples_, d = n_features_;
+    const RadiusPlan plan = radius_plan(d);
+    const int n_pad = (n + 511) / 512 * 512;
+    const size_t range_bytes = (size_t)(2 * d + 1) * sizeof(unsigned long long);
+    DA_HIP(err, rsc_.reserve(sizeof(RadiusScale) + range_bytes + sizeof(unsigned long long)));
+    DA_HIP(err, rop_.reserve(radius_operand_elems(plan, n_pad) * 2));
+    DA_HIP(err, rthr_.reserve((size_t)2 * n_pad * sizeof(float)));
+    RadiusScale *sc = rsc_.as<RadiusScale>();
+    unsigned long long *range = reinterpret_cast<unsigned long long *>(sc + 1);
+    unsigned long long *total = range + 2 * d + 1;
+    float *A = rthr_.as<float>(), *B = A + n_pad;
+    const T *X = X_.as<T>();
+    const double thr2 = km == KM_EUCLIDEAN ? (double)thr * (double)thr : (double)thr;
+    const int chunk = (int)std::max<size_t>(
+        512, std::min<size_t>((size_t)n_pad, ((size_t)128 << 20) / ((size_t)n_pad / 8) / 512 * 512));
+    DA_HIP(err, rbits_.reserve((size_t)chunk * n_pad / 8));
+    DA_HIP(err, cnt_.reserve((size_t)n_pad * sizeof(int)));
+    DA_HIP(err, offs_.reserve((size_t)(n + 1) * sizeof(long long)));
+    size_t scan_bytes = 0;
+    DA_HIP(err, dbscan_offs_bytes(std::min(chunk, n), &scan_bytes));
+    DA_HIP(err, tmp_.reserve(std::max<size_t>(scan_bytes, 1)));
+    count_.assign(n, 0);
+    long long E = 0;
+    {
+        KernelScope ks(*gpu, "radius_pack");
+        DA_HIP(err, launch_radius_scale<T>(X, n, (const T *)nullptr, 0, d, km, range, sc, st));
+        DA_HIP(err, launch_radius_pack<T>(X, n, n_pad, d, plan, sc, thr2, rop_.ptr(), A, B, st));
+    }
+    for (int r0 = 0; r0 < n; r0 += chunk) {
+        const int rows = std::min(chunk, n - r0);
+        const int rows_pad = (rows + plan.row_block - 1) / plan.row_block * plan.row_block;
+        int *cnt = cnt_.as<int>() + r0;
+        unsigned *bits = rbits_.as<unsigned>();
+        DA_HIP(err, hipMemsetAsync(total, 0, sizeof(*total), st));
+        {
+            KernelScope ks(*gpu, "radius_sweep");
+            DA_HIP(err, launch_radius_sweep(plan, rop_.as<char>() + radius_operand_elems(plan, r0) * 2,
+                                            rows_pad, rop_.ptr(), n_pad, A + r0, B, bits, total, st));
+        }
+        struct {
+            unsigned long long set;
+            int bad;
+        } h = {0, 0};
+        DA_HIP(err, hipMemcpyAsync(&h.set, total, sizeof(h.set), hipMemcpyDeviceToHost, st));
+        if (r0 == 0)
+            DA_HIP(err, hipMemcpyAsync(&h.bad, &sc->bad, sizeof(int), hipMemcpyDeviceToHost, st));
+        DA_HIP(err, hipStreamSynchronize(st));
+        if (h.bad || !radius_bits_sparse(h.set, rows, n))
+            return da_status_success;
+        {
+            KernelScope ks(*gpu, "radius_verify");
+            DA_HIP(err, launch_radius_verify<T>(km, X + (size_t)r0 * d, X, rows, d,
+                                                nrm ? nrm + r0 : nullptr, nrm, thr, r0, n_pad, bits,
+                                                cnt, st));
+        }
+        // Room for every bit of the sweep; the verified ones are at most as many.
+        da_status s = reserve_edges(E + (long long)h.set, E);
+        if (s != da_status_success)
+            return s;
+        KernelScope ks(*gpu, "radius_fill");
+        DA_HIP(err, launch_dbscan_offs(tmp_.ptr(), scan_bytes, cnt, E, offs_.as<long long>() + r0,
+                                       rows, st));
+        DA_HIP(err, launch_radius_bits_fill<long long>(bits, rows, n_pad,
+                                                       offs_.as<long long>() + r0, cnt,
+                                                       ind_.as<int>(), st));
+        DA_HIP(err, hipMemcpyAsync(count_.data() + r0, cnt, (size_t)rows * sizeof(int),
+                                   hipMemcpyDeviceToHost, st));
+        DA_HIP(err, hipStreamSynchronize(st));
+        for (int r = 0; r < rows; r++)
+            E += count_[r0 + r];
+    }
+    edges_ = E;
+    DA_HIP(err, hipMemcpyAsync(offs_.as<long long>() + n, &edges_, sizeof(long long),
+                               hipMemcpyHostToDevice, st));
+    done = true;
+    return da_status_success;
+}
+
 // The eps-neighbour graph in CSR form (radius_neighbors.cpp:47-200 builds the same lists):
-// per block of rows, the exact key tile against all samples (double accumulation, rounded
+// hit bits from the matrix cores where the metric is a function of the squared distance and the
+// set is large enough; else, per block of rows, the exact key tile against all samples (double accumulation, rounded
 // to T) with the count of the keys <= thr other than the point itself taken as the tile is
 // written, then a fill of the neighbour indices in ascending order. Leaves count_ (host), offs_ (n + 1 int64) and ind_.
 template <typename T> da_status DBSCANHandle<T>::neighbour_graph(int km, T thr) {
@@ -104,6 +211,17 @@ template <typename T> da_status DBSCANHandle<T>::neighbour_graph(int km, T thr) 
                                         st));
         nrm = norms_.as<double>();
     }
+    if (radius_bits_metric(km) && d <= 128 && n >= BITS_MIN_ROWS && thr >= (T)0) {
+        if (km == KM_SQEUCLIDEAN_GEMM) {
+            DA_HIP(err, norms_.reserve((size_t)n * sizeof(double)));
+            DA_HIP(err, launch_row_sqnorms<T>(X_.as<T>(), d, n, d, norms_.as<double>(), st));
+            nrm = norms_.as<double>();
+        }
+        bool done = false;
+        da_status s = neighbour_graph_bits(km, thr, nrm, done);
+        if (s != da_status_success || done)
+            return s;
+    }
     // Row blocks whose key tile stays within 1 GiB (and 2^28 entries): each block costs a
     // host round trip for its counts, so blocks are made large.
     const size_t max_keys = std::min<size_t>(((size_t)1 << 30) / sizeof(T), (size_t)1 << 28);
@@ -116,7 +234,6 @@ template <typename T> da_status DBSCANHandle<T>::neighbour_graph(int km, T thr) 
     count_.assign(n, 0);
     std::vector<int> scnt((size_t)chunk * nseg), boff((size_t)chunk * nseg);
     long long E = 0;
-    size_t cap = ind_.size() / sizeof(int);
     const T *X = X_.as<T>();
     for (int r0 = 0; r0 < n; r0 += chunk) {
         const int rows = std::min(chunk, n - r0);
@@ -124,8 +241,8 @@ template <typename T> da_status DBSCANHandle<T>::neighbour_graph(int km, T thr) 
             KernelScope ks(*gpu, "pairwise_direct");
             DA_HIP(err, (launch_pairwise_direct_count<T, T>(
                             km, X + (size_t)r0 * d, X, rows, n, d, keys_.as<T>(), n,
-                            nrm ? nrm + r0 : nullptr, nrm, (double)p_, thr, r0, tile_.as<int>(),
-                            st)));
+                            km == KM_COSINE ? nrm + r0 : nullptr, km == KM_COSINE ? nrm : nullptr,
+                            (double)p_, thr, r0, tile_.as<int>(), st)));
         }
         {
             KernelScope ks(*gpu, "radius_segsum");
@@ -147,18 +264,9 @@ template <typename T> da_status DBSCANHandle<T>::neighbour_graph(int km, T thr) 
         }
         if (tb == 0)
             continue;
-        if ((size_t)(E + tb) > cap) {
-            // Grow the neighbour list, keeping what is filled.
-            const size_t ncap = std::max<size_t>({(size_t)(E + tb), 2 * cap, (size_t)1 << 20});
-            DA_HIP(err, ind_spare_.reserve(ncap * sizeof(int)));
-            if (E > 0)
-                DA_HIP(err, hipMemcpyAsync(ind_spare_.ptr(), ind_.ptr(), (size_t)E * sizeof(int),
-                                           hipMemcpyDeviceToDevice, st));
-            DA_HIP(err, hipStreamSynchronize(st));
-            ind_.swap(ind_spare_);
-            ind_spare_.release();
-            cap = ncap;
-        }
+        da_status s = reserve_edges(E + tb, E);
+        if (s != da_status_success)
+            return s;
         DA_HIP(err, hipMemcpyAsync(boff_.ptr(), boff.data(), (size_t)rows * nseg * sizeof(int),
                                    hipMemcpyHostToDevice, st));
         KernelScope ks(*gpu, "radius_fill");
@@ -173,6 +281,9 @@ template <typename T> da_status DBSCANHandle<T>::neighbour_graph(int km, T thr) 
         offs[i + 1] = offs[i] + count_[i];
     DA_HIP(err, offs_.reserve((size_t)(n + 1) * sizeof(long long)));
     DA_HIP(err, hipMemcpyAsync(offs_.ptr(), offs.data(), (n + 1) * sizeof(long long),
+                               hipMemcpyHostToDevice, st));
+    DA_HIP(err, cnt_.reserve((size_t)n * sizeof(int)));
+    DA_HIP(err, hipMemcpyAsync(cnt_.ptr(), count_.data(), (size_t)n * sizeof(int),
                                hipMemcpyHostToDevice, st));
     DA_HIP(err, hipStreamSynchronize(st));
     return da_status_success;
@@ -245,13 +356,6 @@ template <typename T> da_status DBSCANHandle<T>::compute() {
     // (dbscan.cpp:459-468).
     const int n = n_samples_;
     hipStream_t st = gpu->stream();
-    core_.assign(n, 0);
-    n_core_ = 0;
-    for (int i = 0; i < n; i++)
-        if (count_[i] >= min_samples_ - 1) {
-            core_[i] = 1;
-            n_core_++;
-        }
     DA_HIP(err, core_d_.reserve((size_t)n));
     DA_HIP(err, parent_.reserve((size_t)n * sizeof(int)));
     DA_HIP(err, is_root_.reserve((size_t)n * sizeof(int)));
@@ -260,7 +364,8 @@ template <typename T> da_status DBSCANHandle<T>::compute() {
     size_t scan_bytes = 0;
     DA_HIP(err, dbscan_scan_bytes(n, &scan_bytes));
     DA_HIP(err, tmp_.reserve(std::max<size_t>(scan_bytes, 1)));
-    DA_HIP(err, hipMemcpyAsync(core_d_.ptr(), core_.data(), n, hipMemcpyHostToDevice, st));
+    DA_HIP(err, launch_dbscan_core(cnt_.as<int>(), min_samples_ - 1,
+                                   core_d_.as<unsigned char>(), n, st));
     const long long *offs = offs_.as<long long>();
     const int *ind = ind_.as<int>();
     const unsigned char *core = core_d_.as<unsigned char>();
@@ -277,6 +382,13 @@ template <typename T> da_status DBSCANHandle<T>::compute() {
         DA_HIP(err, launch_dbscan_label(offs, ind, core, parent_.as<int>(), rid_.as<int>(),
                                         labels_d_.as<int>(), n, st));
     }
+    core_.assign(n, 0);
+    n_core_ = 0;
+    for (int i = 0; i < n; i++)
+        if (count_[i] >= min_samples_ - 1) {
+            core_[i] = 1;
+            n_core_++;
+        }
     labels_.assign(n, -1);
     DA_HIP(err, hipMemcpyAsync(labels_.data(), labels_d_.ptr(), (size_t)n * sizeof(int),
                                hipMemcpyDeviceToHost, st));

@@ -23,6 +23,11 @@ template <typename T> class DBSCANHandle : public AlgHandle {
 
   private:
     da_status neighbour_graph(int km, T thr);
+    // The graph through hit bits from the matrix cores; done = false when the general path has
+    // to build it.
+    da_status neighbour_graph_bits(int km, T thr, const double *nrm, bool &done);
+    // Room for `total` neighbour indices, the first `used` kept.
+    da_status reserve_edges(long long total, long long used);
 
     bool initdone_ = false;
     da_int n_samples_ = 0, n_features_ = 0, lda_in_ = 0;
@@ -39,6 +44,8 @@ template <typename T> class DBSCANHandle : public AlgHandle {
     // union-find links and the cluster numbering.
     DeviceBuffer X_, norms_, keys_, tile_, cnt_, boff_, ind_, ind_spare_, offs_, core_d_, parent_,
         is_root_, rid_, labels_d_, tmp_;
+    // Hit bits: scale and column ranges, operand rows, thresholds, bits.
+    DeviceBuffer rsc_, rop_, rthr_, rbits_;
 };
 
 } // namespace dagpu

@@ -149,6 +149,12 @@ __global__ __launch_bounds__(256) void dbscan_label_kernel(const long long *__re
         labels[row] = best == INT_MAX ? -1 : best;
 }
 
+__global__ void dbscan_core_kernel(const int *__restrict__ cnt, int need,
+                                   unsigned char *__restrict__ core, int n) {
+    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x)
+        core[i] = cnt[i] >= need;
+}
+
 inline unsigned grid_for(int n, int per_block) {
     return (unsigned)std::max(1, std::min((n + per_block - 1) / per_block, 1 << 20));
 }
@@ -190,6 +196,27 @@ hipError_t launch_dbscan_scan(void *temp, size_t bytes, const int *in, int *out,
     if (n <= 0)
         return hipSuccess;
     return hipcub::DeviceScan::ExclusiveSum(temp, bytes, in, out, n, s);
+}
+
+hipError_t launch_dbscan_core(const int *cnt, int need, unsigned char *core, int n,
+                              hipStream_t s) {
+    if (n <= 0)
+        return hipSuccess;
+    hipLaunchKernelGGL(dbscan_core_kernel, dim3(grid_for(n, 256)), dim3(256), 0, s, cnt, need,
+                       core, n);
+    return hipGetLastError();
+}
+
+hipError_t dbscan_offs_bytes(int n, size_t *bytes) {
+    return hipcub::DeviceScan::ExclusiveScan(nullptr, *bytes, (const int *)nullptr,
+                                             (long long *)nullptr, hipcub::Sum(), 0ll, n);
+}
+
+hipError_t launch_dbscan_offs(void *temp, size_t bytes, const int *cnt, long long base,
+                              long long *offs, int n, hipStream_t s) {
+    if (n <= 0)
+        return hipSuccess;
+    return hipcub::DeviceScan::ExclusiveScan(temp, bytes, cnt, offs, hipcub::Sum(), base, n, s);
 }
 
 hipError_t launch_dbscan_label(const long long *offs, const int *ind, const unsigned char *core,

@@ -311,9 +311,75 @@ hipError_t launch_dbscan_scan(void *temp, size_t bytes, const int *in, int *out,
                               hipStream_t s);
 // labels[i]: for a core point, the cluster number of its root (rid = scan of is_root); for a
 // non-core point, the smallest cluster number among its core neighbours, or -1 (noise).
+// core[i] = cnt[i] >= need, i < n.
+hipError_t launch_dbscan_core(const int *cnt, int need, unsigned char *core, int n,
+                              hipStream_t s);
+// offs[i] = base + cnt[0] + ... + cnt[i - 1], i < n.
+hipError_t dbscan_offs_bytes(int n, size_t *bytes);
+hipError_t launch_dbscan_offs(void *temp, size_t bytes, const int *cnt, long long base,
+                              long long *offs, int n, hipStream_t s);
 hipError_t launch_dbscan_label(const long long *offs, const int *ind, const unsigned char *core,
                                const int *parent, const int *rid, int *labels, int n,
                                hipStream_t s);
+// ---- Radius search on the matrix cores (radius_mfma.hip): a hit bit per pair ----
+// Metrics whose key is a function of the squared euclidean distance.
+bool radius_bits_metric(int metric);
+// Centre per column and the power-of-two scale of the operand rows, the constant part of the
+// error bound, and whether a value is not finite (the general path then serves the search).
+struct RadiusScale {
+    double scale, ca;
+    double mu[128];
+    int bad;
+};
+// Operand shape for d <= 128 features: ks steps of 32; row_block query rows per workgroup (the
+// query operand is padded to a multiple of it, the training operand to a multiple of 512 rows);
+// ce: the relative part of the error bound.
+struct RadiusPlan {
+    int ks, row_block;
+    double ce;
+};
+RadiusPlan radius_plan(int d);
+// Elements (fp16) of `rows_pad` operand rows.
+inline size_t radius_operand_elems(const RadiusPlan &p, int64_t rows_pad) {
+    return (size_t)rows_pad * p.ks * 64;
+}
+// *sc from the ranges of the columns of X (nx x d) and Y (may be null); range: 2 d + 1 words of
+// scratch.
+template <typename T>
+hipError_t launch_radius_scale(const T *X, int64_t nx, const T *Y, int64_t ny, int d, int metric,
+                               unsigned long long *range, RadiusScale *sc, hipStream_t s);
+// Operand rows P (rows_pad, a multiple of 16) and their thresholds: A for query rows, B for
+// training rows (either may be null). thr2: the threshold on the squared distance.
+template <typename T>
+hipError_t launch_radius_pack(const T *X, int rows, int rows_pad, int d, const RadiusPlan &p,
+                              const RadiusScale *sc, double thr2, void *P, float *A, float *B,
+                              hipStream_t s);
+// bits: n_pad bits per row (all written; in the order of radius_mfma.hip), set where the pair may
+// be within the threshold; *total (zeroed before) counts them. n_pad: a multiple of 512.
+hipError_t launch_radius_sweep(const RadiusPlan &p, const void *PA, int rows_pad, const void *PB,
+                               int n_pad, const float *A, const float *B, unsigned *bits,
+                               unsigned long long *total, hipStream_t s);
+// Clears the bits of pairs whose key (double, features in order, rounded to T) is above thr, and
+// of column self0 + row when self0 >= 0; cnt[row]: the bits left. nx, ny: squared norms
+// (KM_SQEUCLIDEAN_GEMM).
+template <typename T>
+hipError_t launch_radius_verify(int metric, const T *X, const T *Y, int rows, int d,
+                                const double *nx, const double *ny, T thr, int self0, int n_pad,
+                                unsigned *bits, int *cnt, hipStream_t s);
+// The set bits of each row as ascending indices from offs[row] (O: int or long long).
+template <typename O>
+hipError_t launch_radius_bits_fill(const unsigned *bits, int rows, int n_pad, const O *offs,
+                                   const int *cnt, int *ind, hipStream_t s);
+// Whether `set` of rows x n pairs are few enough to be verified one by one: up to one in 32. A
+// pair verified costs a gather of its row, some ten times a pair of the general path's tiles.
+inline bool radius_bits_sparse(unsigned long long set, int64_t rows, int64_t n) {
+    return set <= (unsigned long long)(rows * n / 32 + 65536);
+}
+// key[p] for the listed neighbours p in [offs[row], offs[row + 1]) of each row.
+template <typename T>
+hipError_t launch_radius_hit_keys(int metric, const T *X, const T *Y, int rows, int d,
+                                  const double *nx, const double *ny, const int *offs,
+                                  const int *ind, T *key, hipStream_t s);
 template <typename U> hipError_t radius_sort_bytes(int total, int rows, size_t *bytes);
 template <typename U>
 hipError_t launch_radius_sort(void *temp, size_t bytes, const U *key_in, U *key_out,

@@ -1160,56 +1160,150 @@ da_status NNHandle<T>::radius_core(const T *dQ, da_int n_queries, T radius, bool
         }
         nq_norm = main_ctx.q_norm.as<double>();
     }
-    // Query blocks whose key tile stays within 256 MB (and 2^28 entries).
+    // Hit bits from the matrix cores (radius_mfma.hip) where the metric is a function of the
+    // squared distance and the search is large enough for their preparation (2^22 pairs: below
+    // it the general path's few launches are as fast); the general path takes over for values
+    // that are not finite and for radii that hold too many rows to verify one by one.
+    bool use_bits = radius_bits_metric(km) && d <= 128 && n >= 2048 && n <= (1 << 23) &&
+                    (int64_t)n_queries * n >= ((int64_t)1 << 22) && thr >= (T)0;
+    const RadiusPlan plan = radius_plan(std::min<int>(d, 128));
+    const int nw = (n + 63) / 64;
+    const int n_pad = (n + 511) / 512 * 512, q_pad = (n_queries + 511) / 512 * 512;
+    RadiusScale *rsc = nullptr;
+    unsigned long long *set_total = nullptr;
+    float *A = nullptr, *B = nullptr;
+    const size_t opb = use_bits ? radius_operand_elems(plan, n_pad) * 2 : 0;
+    if (use_bits) {
+        const size_t range_words = (size_t)2 * d + 1;
+        DA_HIP(err, rnn_scale_.reserve(sizeof(RadiusScale) +
+                                       (range_words + 1) * sizeof(unsigned long long)));
+        DA_HIP(err, rnn_op_.reserve(opb + radius_operand_elems(plan, q_pad) * 2));
+        DA_HIP(err, rnn_thr_.reserve(((size_t)q_pad + n_pad) * sizeof(float)));
+        rsc = rnn_scale_.as<RadiusScale>();
+        unsigned long long *range = reinterpret_cast<unsigned long long *>(rsc + 1);
+        set_total = range + range_words;
+        A = rnn_thr_.as<float>();
+        B = A + q_pad;
+        KernelScope ks(*gpu, "radius_pack");
+        DA_HIP(err, launch_radius_scale<T>(train_.as<T>(), n, dQ, n_queries, d, km, range, rsc, st));
+        DA_HIP(err, launch_radius_pack<T>(train_.as<T>(), n, n_pad, d, plan, rsc, (double)thr,
+                                          rnn_op_.ptr(), nullptr, B, st));
+        DA_HIP(err, launch_radius_pack<T>(dQ, n_queries, q_pad, d, plan, rsc, (double)thr,
+                                          rnn_op_.as<char>() + opb, A, nullptr, st));
+    }
+    // Query blocks whose key tile stays within 256 MB (and 2^28 entries), or whose bits stay
+    // within 128 MiB and whose neighbours fit 32-bit offsets.
     const size_t max_keys = ((size_t)256 << 20) / sizeof(T);
-    const da_int chunk = (da_int)std::max<size_t>(
+    const da_int tile_chunk = (da_int)std::max<size_t>(
         1, std::min<size_t>(n_queries, std::min<size_t>(max_keys, (size_t)1 << 28) / (size_t)n));
+    const da_int bits_chunk = (da_int)std::max<int64_t>(
+        256, std::min<int64_t>({(int64_t)q_pad, ((int64_t)128 << 20) / (n_pad / 8) / 256 * 256,
+                                (int64_t)std::numeric_limits<int>::max() / n / 256 * 256}));
     const int seg = radius_segment_len(n), nseg = (n + seg - 1) / seg;
-    DA_HIP(err, rnn_keys_.reserve((size_t)chunk * n * sizeof(T)));
-    DA_HIP(err, rnn_cnt_.reserve((size_t)chunk * nseg * sizeof(int)));
-    DA_HIP(err, rnn_tile_.reserve((size_t)chunk * ((n + 63) / 64) * sizeof(int)));
-    DA_HIP(err, rnn_segoff_.reserve((size_t)chunk * nseg * sizeof(int)));
-    DA_HIP(err, rnn_off_.reserve((size_t)(chunk + 1) * sizeof(int)));
-    std::vector<int> scnt((size_t)chunk * nseg), soff((size_t)chunk * nseg), off(chunk + 1);
-    for (da_int q0 = 0; q0 < n_queries; q0 += chunk) {
-        const da_int rows = std::min(chunk, n_queries - q0);
-        {
-            KernelScope ks(*gpu, "pairwise_direct");
-            DA_HIP(err, (launch_pairwise_direct_count<T, T>(
-                            km, dQ + (size_t)q0 * d, train_.as<T>(), rows, n, d, rnn_keys_.as<T>(),
-                            n, nq_norm ? nq_norm + q0 : nullptr, nt_norm, p_, thr, -1,
-                            rnn_tile_.as<int>(), st)));
-        }
-        KernelScope ks(*gpu, "radius_select");
-        DA_HIP(err, launch_radius_segsum(rnn_tile_.as<int>(), rows, n, rnn_cnt_.as<int>(), st));
-        DA_HIP(err, hipMemcpyAsync(scnt.data(), rnn_cnt_.ptr(), (size_t)rows * nseg * sizeof(int),
-                                   hipMemcpyDeviceToHost, st));
-        DA_HIP(err, hipStreamSynchronize(st));
-        // Offsets per row (for the sort) and per row segment (for the fill).
+    std::vector<int> scnt, soff, off(std::max(tile_chunk, use_bits ? bits_chunk : 0) + 1);
+    for (da_int q0 = 0; q0 < n_queries;) {
+        const da_int rows = std::min(use_bits ? bits_chunk : tile_chunk, n_queries - q0);
+        const double *qn = nq_norm ? nq_norm + q0 : nullptr;
         off[0] = 0;
-        for (da_int r = 0; r < rows; r++) {
-            int c = 0;
-            for (int g = 0; g < nseg; g++) {
-                soff[(size_t)r * nseg + g] = off[r] + c;
-                c += scnt[(size_t)r * nseg + g];
+        if (use_bits) {
+            const int rows_pad = (rows + plan.row_block - 1) / plan.row_block * plan.row_block;
+            DA_HIP(err, rnn_bits_.reserve((size_t)rows_pad * n_pad / 8));
+            DA_HIP(err, rnn_cnt_.reserve((size_t)rows_pad * sizeof(int)));
+            unsigned *bits = rnn_bits_.as<unsigned>();
+            unsigned long long set = 0;
+            int bad = 0;
+            scnt.resize(rows);
+            {
+                KernelScope ks(*gpu, "radius_sweep");
+                DA_HIP(err, hipMemsetAsync(set_total, 0, sizeof(*set_total), st));
+                DA_HIP(err, launch_radius_sweep(
+                                plan,
+                                rnn_op_.as<char>() + opb + radius_operand_elems(plan, q0) * 2,
+                                rows_pad, rnn_op_.ptr(), n_pad, A + q0, B, bits, set_total, st));
             }
-            off[r + 1] = off[r] + c;
-            if (!sink)
-                rnn_count_[q0 + r] = c;
+            DA_HIP(err, hipMemcpyAsync(&set, set_total, sizeof(set), hipMemcpyDeviceToHost, st));
+            if (q0 == 0)
+                DA_HIP(err, hipMemcpyAsync(&bad, &rsc->bad, sizeof(int), hipMemcpyDeviceToHost, st));
+            DA_HIP(err, hipStreamSynchronize(st));
+            if (bad || !radius_bits_sparse(set, rows, n)) {
+                use_bits = false; // this block and the rest through the key tiles
+                continue;
+            }
+            {
+                KernelScope ks(*gpu, "radius_verify");
+                DA_HIP(err, launch_radius_verify<T>(km, dQ + (size_t)q0 * d, train_.as<T>(), rows,
+                                                    d, qn, nt_norm, thr, -1, n_pad, bits,
+                                                    rnn_cnt_.as<int>(), st));
+            }
+            DA_HIP(err, hipMemcpyAsync(scnt.data(), rnn_cnt_.ptr(), (size_t)rows * sizeof(int),
+                                       hipMemcpyDeviceToHost, st));
+            DA_HIP(err, hipStreamSynchronize(st));
+            for (da_int r = 0; r < rows; r++) {
+                off[r + 1] = off[r] + scnt[r];
+                if (!sink)
+                    rnn_count_[q0 + r] = scnt[r];
+            }
+        } else {
+            DA_HIP(err, rnn_keys_.reserve((size_t)tile_chunk * n * sizeof(T)));
+            DA_HIP(err, rnn_cnt_.reserve((size_t)tile_chunk * nseg * sizeof(int)));
+            DA_HIP(err, rnn_tile_.reserve((size_t)tile_chunk * nw * sizeof(int)));
+            DA_HIP(err, rnn_segoff_.reserve((size_t)tile_chunk * nseg * sizeof(int)));
+            scnt.resize((size_t)rows * nseg);
+            soff.resize((size_t)rows * nseg);
+            {
+                KernelScope ks(*gpu, "pairwise_direct");
+                DA_HIP(err, (launch_pairwise_direct_count<T, T>(
+                                km, dQ + (size_t)q0 * d, train_.as<T>(), rows, n, d,
+                                rnn_keys_.as<T>(), n, qn, nt_norm, p_, thr, -1,
+                                rnn_tile_.as<int>(), st)));
+            }
+            KernelScope ks(*gpu, "radius_select");
+            DA_HIP(err, launch_radius_segsum(rnn_tile_.as<int>(), rows, n, rnn_cnt_.as<int>(), st));
+            DA_HIP(err, hipMemcpyAsync(scnt.data(), rnn_cnt_.ptr(),
+                                       (size_t)rows * nseg * sizeof(int), hipMemcpyDeviceToHost,
+                                       st));
+            DA_HIP(err, hipStreamSynchronize(st));
+            // Offsets per row (for the sort) and per row segment (for the fill).
+            for (da_int r = 0; r < rows; r++) {
+                int c = 0;
+                for (int g = 0; g < nseg; g++) {
+                    soff[(size_t)r * nseg + g] = off[r] + c;
+                    c += scnt[(size_t)r * nseg + g];
+                }
+                off[r + 1] = off[r] + c;
+                if (!sink)
+                    rnn_count_[q0 + r] = c;
+            }
         }
         const int total = off[rows];
-        if (total == 0 && !sink)
+        if (total == 0 && !sink) {
+            q0 += rows;
             continue;
+        }
+        DA_HIP(err, rnn_off_.reserve((size_t)(rows + 1) * sizeof(int)));
         DA_HIP(err, hipMemcpyAsync(rnn_off_.ptr(), off.data(), (rows + 1) * sizeof(int),
                                    hipMemcpyHostToDevice, st));
-        DA_HIP(err, hipMemcpyAsync(rnn_segoff_.ptr(), soff.data(),
-                                   (size_t)rows * nseg * sizeof(int), hipMemcpyHostToDevice, st));
         DA_HIP(err, rnn_ind_buf_.reserve((size_t)std::max(total, 1) * sizeof(int)));
         DA_HIP(err, rnn_key_buf_.reserve((size_t)std::max(total, 1) * sizeof(T)));
-        DA_HIP(err, launch_radius_fill<T>(rnn_keys_.as<T>(), n, rows, n, thr, -1,
-                                          rnn_segoff_.as<int>(),
-                                          rnn_ind_buf_.as<int>(),
-                                          want_dist ? rnn_key_buf_.as<T>() : nullptr, st));
+        if (use_bits) {
+            KernelScope ks(*gpu, "radius_select");
+            DA_HIP(err, launch_radius_bits_fill<int>(rnn_bits_.as<unsigned>(), rows, n_pad,
+                                                     rnn_off_.as<int>(), rnn_cnt_.as<int>(),
+                                                     rnn_ind_buf_.as<int>(), st));
+            if (want_dist)
+                DA_HIP(err, launch_radius_hit_keys<T>(km, dQ + (size_t)q0 * d, train_.as<T>(), rows,
+                                                      d, qn, nt_norm, rnn_off_.as<int>(),
+                                                      rnn_ind_buf_.as<int>(), rnn_key_buf_.as<T>(),
+                                                      st));
+        } else {
+            KernelScope ks(*gpu, "radius_select");
+            DA_HIP(err, hipMemcpyAsync(rnn_segoff_.ptr(), soff.data(),
+                                       (size_t)rows * nseg * sizeof(int), hipMemcpyHostToDevice,
+                                       st));
+            DA_HIP(err, launch_radius_fill<T>(rnn_keys_.as<T>(), n, rows, n, thr, -1,
+                                              rnn_segoff_.as<int>(), rnn_ind_buf_.as<int>(),
+                                              want_dist ? rnn_key_buf_.as<T>() : nullptr, st));
+        }
         int *ind = rnn_ind_buf_.as<int>();
         T *key = rnn_key_buf_.as<T>();
         if (sort_results && total > 0) {
@@ -1230,6 +1324,7 @@ da_status NNHandle<T>::radius_core(const T *dQ, da_int n_queries, T radius, bool
             da_status ss = (*sink)(q0, rows, rnn_off_.as<int>(), ind, key);
             if (ss != da_status_success)
                 return ss;
+            q0 += rows;
             continue;
         }
         const size_t base = rnn_ind_.size();
@@ -1242,6 +1337,7 @@ da_status NNHandle<T>::radius_core(const T *dQ, da_int n_queries, T radius, bool
                                        hipMemcpyDeviceToHost, st));
         }
         DA_HIP(err, hipStreamSynchronize(st));
+        q0 += rows;
     }
     return da_status_success;
 }

@@ -139,6 +139,8 @@ template <typename T> class NNHandle : public AlgHandle {
     std::vector<T> rnn_d_;
     DeviceBuffer rnn_keys_, rnn_tile_, rnn_cnt_, rnn_off_, rnn_segoff_, rnn_ind_buf_, rnn_key_buf_, rnn_ind2_, rnn_key2_,
         rnn_tmp_;
+    // Hit bits: scale and column ranges, operand rows, thresholds, bits.
+    DeviceBuffer rnn_scale_, rnn_op_, rnn_thr_, rnn_bits_;
     // Options as read at set_data (nearest_neighbors.cpp:295-352).
     da_int n_neighbors_ = 5, algo_ = 3, metric_ = 0;
     double p_ = 2.0;

@@ -1,0 +1,94 @@
+"""Radius search and DBSCAN through the matrix-core hit bits (squared-euclidean metrics, up to
+128 features, 2,048 rows or more) against the oracle: tile edges, padded widths, rows that need
+the exact re-check, and the data that send the search to the general path."""
+import numpy as np
+import pytest
+
+import aoclda
+
+pytestmark = pytest.mark.gpu
+
+
+def blobs(rng, n, d, dtype, sigma=0.5, offset=0.0):
+    means = rng.uniform(-10, 10, (8, d)) + offset
+    return (means[rng.integers(0, 8, n)] + sigma * rng.standard_normal((n, d))).astype(dtype)
+
+
+def radius_of(X, Q, share):
+    """A radius that keeps about this share of the training rows."""
+    s = np.sqrt(((X[None, :400].astype(np.float64) - Q[:50, None].astype(np.float64)) ** 2).sum(-1))
+    return float(np.quantile(s, share))
+
+
+# Edges: 64-row words, 128- and 256-row blocks, every k-step count, the smallest width.
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+@pytest.mark.parametrize("n,nq,d", [(2048, 2048, 1), (2049, 2050, 3), (2111, 2300, 16),
+                                    (2113, 2047, 32), (2500, 1700, 33), (3000, 1500, 65),
+                                    (2100, 2100, 97), (2304, 1900, 128)])
+@pytest.mark.parametrize("metric", ["euclidean", "sqeuclidean", "euclidean_gemm"])
+def test_radius(oracle, dtype, n, nq, d, metric):
+    rng = np.random.default_rng(n + d)
+    X, Q = blobs(rng, n, d, dtype), blobs(rng, nq, d, dtype)
+    Q[:7] = X[:7]
+    r = radius_of(X, Q, 0.03)
+    r = float(dtype(r * r if metric == "sqeuclidean" else r))
+    nn = aoclda.neighbors.nearest_neighbors(metric=metric, radius=r).fit(X)
+    dist, ind = nn.radius_neighbors(Q)
+    cnt, ei, ed = oracle.radius(X, Q, r, metric, single=dtype == np.float32)
+    # The GEMM-form metric may differ where the key equals the threshold up to its rounding
+    # (absolute, about 1e-12 of the squared norms); none of these data has such a pair.
+    assert [len(v) for v in ind] == list(cnt)
+    np.testing.assert_array_equal(np.concatenate(list(ind)), ei)
+    # fp32: one rounding (2^-24). The GEMM form's squared key |x|^2 + |y|^2 - 2 x.y is off by up
+    # to 2 (d + 2) 2^-53 (|x|^2 + |y|^2), its root by up to the root of that (at distance 0).
+    tol = 1e-6 if dtype == np.float32 else 1e-12
+    big = max((X.astype(np.float64) ** 2).sum(1).max(), (Q.astype(np.float64) ** 2).sum(1).max())
+    atol = np.sqrt(2 * (d + 2) * 2.0 ** -53 * 2 * big) if metric == "euclidean_gemm" else tol
+    np.testing.assert_allclose(np.concatenate(list(dist)), ed, rtol=tol, atol=atol)
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+@pytest.mark.parametrize("case", ["offset", "duplicates", "all", "outlier", "boundary", "tiny",
+                                  "nonfinite"])
+def test_dbscan_data(oracle, dtype, case):
+    """Data far from the origin, exact duplicates with eps = 0, every pair a neighbour, an
+    outlier that makes every pair of a blob borderline, distances equal to eps, subnormal scales,
+    and values that are not finite."""
+    rng = np.random.default_rng(5)
+    n, d, eps = 2300, 6, 0.9
+    X = blobs(rng, n, d, dtype)
+    if case == "offset":
+        X = blobs(rng, n, d, dtype, offset=3e4 if dtype == np.float32 else 1e8)
+    elif case == "duplicates":
+        X, eps = X[rng.integers(0, 300, n)], 0.0
+    elif case == "all":
+        eps = 1e4
+    elif case == "outlier":
+        X[17] = 1e9
+    elif case == "boundary":
+        X = rng.integers(0, 12, (n, d)).astype(dtype)
+        eps = 3.0  # integer squared distances: many equal 9
+    elif case == "tiny":
+        scale = dtype(1e-18 if dtype == np.float32 else 1e-140)
+        X, eps = X * scale, float(dtype(0.9) * scale)
+    elif case == "nonfinite":
+        X[3, 2], X[100, 0], X[101, 5] = np.nan, np.inf, -np.inf
+    db = aoclda.clustering.DBSCAN(eps=eps, min_samples=6, algorithm="brute").fit(X)
+    with np.errstate(all="ignore"):
+        labels, core, nc = oracle.dbscan(X, eps, 6, single=dtype == np.float32)
+    np.testing.assert_array_equal(db.labels, labels)
+    np.testing.assert_array_equal(db.core_sample_indices, np.flatnonzero(core))
+    assert db.n_clusters == nc
+
+
+@pytest.mark.parametrize("metric", ["euclidean", "l2", "sqeuclidean"])
+@pytest.mark.parametrize("d", [2, 40, 128])
+def test_dbscan_metrics(oracle, metric, d):
+    rng = np.random.default_rng(d)
+    X = blobs(rng, 2600, d, np.float32)
+    eps = radius_of(X, X, 0.02)
+    eps = float(np.float32(eps * eps if metric == "sqeuclidean" else eps))
+    db = aoclda.clustering.DBSCAN(eps=eps, min_samples=5, metric=metric, algorithm="brute").fit(X)
+    labels, core, _ = oracle.dbscan(X, eps, 5, metric, single=True)
+    np.testing.assert_array_equal(db.labels, labels)
+    np.testing.assert_array_equal(db.core_sample_indices, np.flatnonzero(core))
