@@ -366,15 +366,12 @@ __device__ __forceinline__ void kb_assign_tile(const typename Op::T *__restrict_
             }
 #pragma unroll
             for (int i = 0; i < 4; i++) {
+                // Best, second best (the median of the three) and the code of the best, which
+                // is the same for all lanes: four instructions per score.
                 const float v = acc[i];
-                const int c = c0 + 4 * g + i;
-                if (v > best1[pt]) {
-                    best2[pt] = best1[pt];
-                    best1[pt] = v;
-                    bidx[pt] = c;
-                } else if (v > best2[pt]) {
-                    best2[pt] = v;
-                }
+                bidx[pt] = v > best1[pt] ? c0 / 4 + i : bidx[pt];
+                best2[pt] = __builtin_amdgcn_fmed3f(best1[pt], best2[pt], v);
+                best1[pt] = fmaxf(best1[pt], v);
             }
         }
     }
@@ -382,6 +379,8 @@ __device__ __forceinline__ void kb_assign_tile(const typename Op::T *__restrict_
 #pragma unroll
     for (int pt = 0; pt < PT; pt++) {
         float xs = xn[pt];
+        if (bidx[pt] != INT_MAX)
+            bidx[pt] = (bidx[pt] >> 2) * 16 + 4 * g + (bidx[pt] & 3);
 #pragma unroll
         for (int off = 16; off <= 32; off <<= 1) {
             const float o1 = __shfl_xor(best1[pt], off, 64);
@@ -440,7 +439,8 @@ __device__ __forceinline__ void kb_assign_tile(const typename Op::T *__restrict_
 // centres of an instance are staged once per run.
 constexpr int KB_RUN = 4;
 template <class Op, int PT>
-__global__ __launch_bounds__(256) void kb_assign_kernel(
+__global__ __launch_bounds__(256)
+__attribute__((amdgpu_waves_per_eu(2))) void kb_assign_kernel(
     const typename Op::T *__restrict__ Xo, const float *__restrict__ X, KBatchDesc b,
     const KTile *__restrict__ tiles, int ntiles, const int *__restrict__ state, const int *__restrict__ fpar, int mode, int par,
     const typename Op::T *__restrict__ Cb, const float *__restrict__ chalf,

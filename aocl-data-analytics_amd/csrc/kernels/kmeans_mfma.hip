@@ -50,6 +50,32 @@ template <> struct AssignOp<double> {
     }
 };
 
+// Takes score v into a lane's best and second-best: the second is the median of the three (best1
+// >= best2), so it costs one instruction, the whole step four (compare, select, median, maximum).
+// code names the score within the lane (uniform over the wave, so that the select takes it from a
+// scalar register); the first of equal scores keeps its code. A NaN score changes nothing (fp32)
+// or raises the second best to the best (fp64), which only lists the sample for the re-check.
+__device__ __forceinline__ void take_score(float v, int code, float &best1, float &best2,
+                                           int &bcode) {
+    bcode = v > best1 ? code : bcode;
+    best2 = __builtin_amdgcn_fmed3f(best1, best2, v);
+    best1 = fmaxf(best1, v);
+}
+__device__ __forceinline__ void take_score(double v, int code, double &best1, double &best2,
+                                           int &bcode) {
+    bcode = v > best1 ? code : bcode;
+    best2 = fmax(best2, fmin(best1, v));
+    best1 = fmax(best1, v);
+}
+// Code of element i of the 16-centre block blk, and the centre it names for lane group g.
+__device__ __forceinline__ int score_code(int blk, int i) { return blk * 4 + i; }
+__device__ __forceinline__ int code_centre(int code, int g, bool strided) {
+    if (code == INT_MAX)
+        return code;
+    const int i = code & 3;
+    return (code >> 2) * 16 + (strided ? g + 4 * i : 4 * g + i);
+}
+
 // KCH consecutive elements (16-byte aligned) into registers as 16-byte loads.
 template <typename E, int KCH> __device__ __forceinline__ void load_row(const E *p, E (&v)[KCH]) {
     constexpr int PER = 16 / (int)sizeof(E);
@@ -82,8 +108,11 @@ template <typename E> int assign_chunk(int k, int Kp) {
 // tiles of 16 samples in registers as B operands; the centres, A operands, are staged in LDS
 // kch at a time (one chunk: staged once per workgroup; more: each chunk staged in turn for
 // every tile, with the best and second-best scores carried across chunks).
+// Two waves per SIMD asked for: left alone the compiler keeps the accumulators in accumulation
+// registers and copies each score out before the bookkeeping reads it.
 template <typename E, int KCH, int PTT>
-__global__ __launch_bounds__(256) void kmeans_assign_mfma_kernel(
+__global__ __launch_bounds__(256)
+__attribute__((amdgpu_waves_per_eu(2))) void kmeans_assign_mfma_kernel(
     const E *__restrict__ X, int n, int Kp, const E *__restrict__ CP,
     const E *__restrict__ chalf, int k, int kch, double cmax, int *__restrict__ labels,
     const int *__restrict__ prev, int *__restrict__ changed, int *__restrict__ list_count,
@@ -157,17 +186,9 @@ __global__ __launch_bounds__(256) void kmeans_assign_mfma_kernel(
                     for (int f = 0; f < KCH; f++)
                         acc = Op::mfma(a[f], b[pt][f], acc);
 #pragma unroll
-                    for (int i = 0; i < 4; i++) {
-                        const E v = acc[i];
-                        const int c = cb + c0 + (Op::strided ? g + 4 * i : 4 * g + i);
-                        if (v > best1[pt]) {
-                            best2[pt] = best1[pt];
-                            best1[pt] = v;
-                            bidx[pt] = c;
-                        } else if (v > best2[pt]) {
-                            best2[pt] = v;
-                        }
-                    }
+                    for (int i = 0; i < 4; i++)
+                        take_score(acc[i], score_code((cb + c0) / 16, i), best1[pt], best2[pt],
+                                   bidx[pt]);
                 }
             }
         }
@@ -175,6 +196,7 @@ __global__ __launch_bounds__(256) void kmeans_assign_mfma_kernel(
 #pragma unroll
         for (int pt = 0; pt < PTT; pt++) {
             E xs = xn[pt];
+            bidx[pt] = code_centre(bidx[pt], g, Op::strided);
 #pragma unroll
             for (int off = 16; off <= 32; off <<= 1) {
                 const E o1 = __shfl_xor(best1[pt], off, 64);
@@ -230,7 +252,8 @@ typedef __bf16 v8bf __attribute__((ext_vector_type(8)));
 // contiguous), KCH / 8 MFMA steps per 16 x 16 tile. The near-tie bound adds the bf16
 // rounding of both operands to the fp32 bound.
 template <int KCH>
-__global__ __launch_bounds__(256) void kmeans_assign_bf16_kernel(
+__global__ __launch_bounds__(256)
+__attribute__((amdgpu_waves_per_eu(2))) void kmeans_assign_bf16_kernel(
     const __bf16 *__restrict__ X, int n, int Kp, const __bf16 *__restrict__ C16,
     const float *__restrict__ chalf, int k, double cmax, int *__restrict__ labels,
     const int *__restrict__ prev, int *__restrict__ changed, int *__restrict__ list_count,
@@ -303,23 +326,15 @@ __global__ __launch_bounds__(256) void kmeans_assign_bf16_kernel(
                 for (int f = 0; f < NF; f++)
                     acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[f], b[pt][f], acc, 0, 0, 0);
 #pragma unroll
-                for (int i = 0; i < 4; i++) {
-                    const float v = acc[i];
-                    const int c = c0 + 4 * g + i;
-                    if (v > best1[pt]) {
-                        best2[pt] = best1[pt];
-                        best1[pt] = v;
-                        bidx[pt] = c;
-                    } else if (v > best2[pt]) {
-                        best2[pt] = v;
-                    }
-                }
+                for (int i = 0; i < 4; i++)
+                    take_score(acc[i], score_code(c0 / 16, i), best1[pt], best2[pt], bidx[pt]);
             }
         }
         const double u = 1.0 / 256.0, u32 = 1.0 / 16777216.0;
 #pragma unroll
         for (int pt = 0; pt < PT; pt++) {
             float xs = xn[pt];
+            bidx[pt] = code_centre(bidx[pt], g, false);
 #pragma unroll
             for (int off = 16; off <= 32; off <<= 1) {
                 const float o1 = __shfl_xor(best1[pt], off, 64);

@@ -672,10 +672,11 @@ __device__ __forceinline__ void knn_tile_body(
 }
 
 // The sweep as a kernel: K2 asks the compiler for registers that leave room for WPE waves
-// per SIMD (as many workgroups as fit a CU's LDS); the fp64 operands need more registers
-// and run one wave per SIMD without spilling.
+// per SIMD (as many workgroups as fit a CU's LDS); the fp64 operands of more than 64 features
+// need more registers and run one wave per SIMD without spilling.
 template <class Op, int KCH, int KC, bool SPLIT, int PF>
-__global__ __launch_bounds__(64 * TileShape<KC>::WV) void knn_tile_kernel(
+__global__ __launch_bounds__(64 * TileShape<KC>::WV)
+__attribute__((amdgpu_waves_per_eu(KCH <= 16 ? 2 : 1))) void knn_tile_kernel(
     const typename Op::in_t *__restrict__ Q, int nq, const typename Op::in_t *__restrict__ Y,
     const typename Op::acc_e *__restrict__ nyh, int n, int Kp, int split_len, int nsplit,
     float *__restrict__ part_key, int *__restrict__ part_idx, float *__restrict__ part_tau,
@@ -705,7 +706,8 @@ knn_tile_kernel_k2(const typename Op::in_t *__restrict__ Q, int nq,
 // part_tau[q * nsplit + split] for launch_knn_seed. Fixed shape: four waves of 32 queries,
 // two 16-row training tiles per step, loads then products.
 template <class Op, int KCH, bool SPLIT>
-__global__ __launch_bounds__(256) void knn_seed_min_kernel(
+__global__ __launch_bounds__(256)
+__attribute__((amdgpu_waves_per_eu(2))) void knn_seed_min_kernel(
     const typename Op::in_t *__restrict__ Q, int nq, const typename Op::in_t *__restrict__ Y,
     const typename Op::acc_e *__restrict__ nyh, int n, int Kp, int split_len, int nsplit, int k,
     float *__restrict__ part_tau) {

@@ -202,23 +202,29 @@ __device__ __forceinline__ void copy_to_lds(const _Float16 *g, _Float16 *l) {
                                      (__attribute__((address_space(3))) void *)l, 16, 0, 0);
 }
 
+// Row tiles per wave by k steps (registers), 16-row training tiles per stage.
+constexpr int CTS = 4;
+constexpr int rt_of(int ks) { return ks <= 2 ? 4 : 2; }
 // The sweep. A wave holds RT tiles of 16 query rows in registers and takes the training rows of
-// its segment 64 at a time; the 64 rows' fragments are copied to LDS once for the workgroup's
+// its segment 16 CTS at a time; their fragments are copied to LDS once for the workgroup's
 // four waves, straight from memory, a step ahead (two buffers, one barrier a step). A tile's
 // accumulators start at -A_x - B_y, so the sign of the result is the outcome, and one
 // v_alignbit shifts it into the lane's word of the row: two vector operations per pair beside
 // the products, no compare, no branch, no matter how many pairs hit. (With a branch per 64 x 64
 // step that assembled words from ballots the kernel took 7.75 ms at 100,000 x 16, where nine
-// steps in ten hold a hit; this form: PERF_RADIUS.)
+// steps in ten hold a hit; this form takes 1.8 ms, 0.55 PFLOP/s of products issued.)
 //
 // Bit order: a lane (r, g) sees columns 16 k + r of a row, so word [row][j / 512][j % 16] holds
 // column j at bit 31 - (j % 512) / 16.
+// Two waves per SIMD are asked for explicitly: with the whole register file to itself the
+// compiler keeps the accumulators in accumulation registers and copies every element in and out.
 template <int KS, int RT>
-__global__ __launch_bounds__(256) void radius_sweep_kernel(
+__global__ __launch_bounds__(256)
+__attribute__((amdgpu_waves_per_eu(2))) void radius_sweep_kernel(
     const _Float16 *__restrict__ PA, const _Float16 *__restrict__ PB,
     const float *__restrict__ A, const float *__restrict__ B, int nrb, int nblk, int segblk,
     unsigned *__restrict__ bits, unsigned long long *__restrict__ total) {
-    constexpr int STAGE = 4 * KS * 1024; // fp16 elements of 64 training rows
+    constexpr int STAGE = CTS * KS * 1024; // fp16 elements of 16 CTS training rows
     __shared__ __attribute__((aligned(16))) _Float16 s0[STAGE];
     __shared__ __attribute__((aligned(16))) _Float16 s1[STAGE];
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
@@ -246,21 +252,21 @@ __global__ __launch_bounds__(256) void radius_sweep_kernel(
             word[rt][i] = 0;
         }
     }
-    float hv[4];
+    float hv[CTS];
     auto stage = [&](int j0, _Float16 *dst) {
         const _Float16 *src = PB + (int64_t)(j0 / 16) * KS * 1024;
 #pragma unroll
-        for (int b = 0; b < 2 * KS; b++) {
-            const int blk = w * 2 * KS + b;
+        for (int b = 0; b < CTS / 2 * KS; b++) {
+            const int blk = w * (CTS / 2 * KS) + b;
             copy_to_lds(src + blk * 512 + lane * 8, dst + blk * 512);
         }
 #pragma unroll
-        for (int ct = 0; ct < 4; ct++)
+        for (int ct = 0; ct < CTS; ct++)
             hv[ct] = B[j0 + ct * 16 + r];
     };
-    auto compute = [&](const _Float16 *sb, const float (&bv)[4]) {
+    auto compute = [&](const _Float16 *sb, const float (&bv)[CTS]) {
 #pragma unroll
-        for (int ct = 0; ct < 4; ct++) {
+        for (int ct = 0; ct < CTS; ct++) {
             v4f acc[RT];
 #pragma unroll
             for (int rt = 0; rt < RT; rt++)
@@ -294,23 +300,24 @@ __global__ __launch_bounds__(256) void radius_sweep_kernel(
     const int j1 = b1 * 512;
     stage(b0 * 512, s0);
     for (int blk = b0; blk < b1; blk++) {
-        for (int j0 = blk * 512; j0 < blk * 512 + 512; j0 += 128) {
-            // Rows j0 from s0, the next 64 into s1; then the other way round.
+        constexpr int ST = 16 * CTS;
+        for (int j0 = blk * 512; j0 < blk * 512 + 512; j0 += 2 * ST) {
+            // Rows j0 from s0, the next ST into s1; then the other way round.
             __builtin_amdgcn_s_waitcnt(0x0F70); // vmcnt(0): this wave's copies have landed
             __syncthreads();
-            float bv[4];
+            float bv[CTS];
 #pragma unroll
-            for (int ct = 0; ct < 4; ct++)
+            for (int ct = 0; ct < CTS; ct++)
                 bv[ct] = hv[ct];
-            stage(j0 + 64, s1);
+            stage(j0 + ST, s1);
             compute(s0, bv);
             __builtin_amdgcn_s_waitcnt(0x0F70);
             __syncthreads();
 #pragma unroll
-            for (int ct = 0; ct < 4; ct++)
+            for (int ct = 0; ct < CTS; ct++)
                 bv[ct] = hv[ct];
-            if (j0 + 128 < j1)
-                stage(j0 + 128, s0);
+            if (j0 + 2 * ST < j1)
+                stage(j0 + 2 * ST, s0);
             compute(s1, bv);
         }
         // 32 sign bits per row and lane: set means miss.
@@ -522,7 +529,6 @@ __global__ __launch_bounds__(256) void radius_hit_keys_kernel(
     }
 }
 
-constexpr int rt_of(int ks) { return ks <= 2 ? 4 : 2; }
 
 } // namespace
 
@@ -578,9 +584,10 @@ hipError_t launch_radius_sweep(const RadiusPlan &p, const void *PA, int rows_pad
         return hipErrorInvalidValue;
     const int nblk = n_pad / 512;
     const int nrb = rows_pad / p.row_block;
-    // Column segments: about 4,096 workgroups, each of at least 1,024 training rows (a segment's
-    // operands also stay in an XCD's 4 MB L2 while the row blocks pass over them).
-    int nseg = std::max(1, std::min((nblk + 1) / 2, (4096 + nrb - 1) / nrb));
+    // Column segments: about 1,024 workgroups (two run on a CU at a time), each of at least 1,024
+    // training rows: a workgroup's start (its query rows) and end cost a few steps. 10,000 x
+    // 100,000 pairs of 16 features: 222 us with 4,096 workgroups, 177 us with 512 to 2,048.
+    int nseg = std::max(1, std::min((nblk + 1) / 2, (1024 + nrb - 1) / nrb));
     const int segblk = (nblk + nseg - 1) / nseg;
     nseg = (nblk + segblk - 1) / segblk;
     const _Float16 *pa = static_cast<const _Float16 *>(PA), *pb = static_cast<const _Float16 *>(PB);
