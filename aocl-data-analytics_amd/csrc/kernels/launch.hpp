@@ -70,10 +70,14 @@ hipError_t launch_pairwise_mfma(int metric, const T *X, const T *Y, int m, int n
 
 // Per-row top-k of a row-major key matrix (rows x n, leading dimension ld) by
 // (key, column index), ascending (descending when `largest`). Writes the k best keys and
-// indices per row, sorted, to out_key[row*k + j] / out_idx[row*k + j]. k <= 3840.
+// indices per row, sorted, to out_key[row*k + j] / out_idx[row*k + j]. k <= 3840. With tmp_key
+// and tmp_idx (rows * row_topk_segments(rows, n, k) * k entries each), few long rows are cut
+// into segments that are selected from in parallel.
 template <typename K>
 hipError_t launch_row_topk(const K *keys, int64_t ld, int rows, int n, int k, int largest,
-                           K *out_key, int *out_idx, hipStream_t s);
+                           K *out_key, int *out_idx, hipStream_t s, K *tmp_key = nullptr,
+                           int *tmp_idx = nullptr);
+int row_topk_segments(int rows, int n, int k);
 
 } // namespace dagpu
 

@@ -8,6 +8,7 @@
 // bitonic-sorts it, keeps the k best and tightens the threshold. Elements are ordered by
 // (key, column index), so the result is deterministic, including at equal keys.
 #include "launch.hpp"
+#include <algorithm>
 #include <climits>
 #include <hip/hip_runtime.h>
 
@@ -47,14 +48,19 @@ template <typename K, int CAP>
 __global__ __launch_bounds__(256) void row_topk_kernel(const K *__restrict__ keys, int64_t ld,
                                                        int rows, int n, int k, int largest,
                                                        K *__restrict__ out_key,
-                                                       int *__restrict__ out_idx) {
+                                                       int *__restrict__ out_idx, int listed,
+                                                       int seg) {
     __shared__ K bkey[CAP];
     __shared__ int bidx[CAP];
     __shared__ int count;
     __shared__ K thr_k;
     __shared__ int thr_i;
-    const int row = blockIdx.x;
-    if (row >= rows)
+    // Segment blockIdx.y of `seg` columns (the whole row when there is one); the results of
+    // (row, segment) pairs lie one after another.
+    const int64_t o = ((int64_t)blockIdx.x * gridDim.y + blockIdx.y) * k;
+    const int c0 = (int)blockIdx.y * seg;
+    // listed: only those that the bounded selection has left (marked -2).
+    if ((int)blockIdx.x >= rows || (listed && out_idx[o] != -2))
         return;
     const K inf = (K)__builtin_huge_val();
     if (threadIdx.x == 0) {
@@ -63,7 +69,8 @@ __global__ __launch_bounds__(256) void row_topk_kernel(const K *__restrict__ key
         thr_i = INT_MAX;
     }
     __syncthreads();
-    const K *rk = keys + (int64_t)row * ld;
+    const K *rk = keys + (int64_t)blockIdx.x * ld + c0;
+    n = n - c0 < seg ? n - c0 : seg;
     for (int base = 0; base < n; base += 256) {
         const int j = base + threadIdx.x;
         if (j < n) {
@@ -108,38 +115,202 @@ __global__ __launch_bounds__(256) void row_topk_kernel(const K *__restrict__ key
     block_bitonic_sort<K, CAP>(bkey, bidx);
     for (int t = threadIdx.x; t < k; t += blockDim.x) {
         K v = bkey[t];
-        out_key[(int64_t)row * k + t] = largest ? -v : v;
-        out_idx[(int64_t)row * k + t] = bidx[t];
+        out_key[o + t] = largest ? -v : v;
+        out_idx[o + t] = bidx[t] == INT_MAX ? INT_MAX : c0 + bidx[t];
     }
 }
 
 } // namespace
 
+namespace {
+
+// The same selection for k <= 128: thread t keeps the smallest of elements t, t + 256, ..., and
+// the k-th smallest of the 256 group minima, attained by k elements of the row, bounds the k-th
+// key from above. A second pass collects the elements at or below it, -256 ln(1 - k / 256) on
+// average (5 for k = 5, 127 for k = 100), and one sort of those ends the row: two barriers-free
+// sweeps instead of two barriers per 256 elements and a 512-entry sort whenever the buffer fills.
+// Rows with more than SEL_CAP elements at or below the bound (ties) are left to the general
+// kernel: their out_idx[0] is set to -2.
+constexpr int SEL_CAP = 1024;
+template <typename K>
+__global__ __launch_bounds__(256) void row_topk_bound_kernel(const K *__restrict__ keys,
+                                                             int64_t ld, int n, int k,
+                                                             int largest, K *__restrict__ out_key,
+                                                             int *__restrict__ out_idx, int seg) {
+    __shared__ K bkey[SEL_CAP];
+    __shared__ int bidx[SEL_CAP];
+    __shared__ int count;
+    __shared__ K bound;
+    const K inf = (K)__builtin_huge_val();
+    const int tid = threadIdx.x;
+    const int64_t o = ((int64_t)blockIdx.x * gridDim.y + blockIdx.y) * k;
+    const int c0 = (int)blockIdx.y * seg;
+    const K *rk = keys + (int64_t)blockIdx.x * ld + c0;
+    n = n - c0 < seg ? n - c0 : seg;
+    auto value = [&](K v) {
+        v = largest ? -v : v;
+        return v != v ? inf : v;
+    };
+    K mn = inf;
+    int j = tid;
+    for (; j + 7 * 256 < n; j += 8 * 256) {
+        K v[8];
+#pragma unroll
+        for (int u = 0; u < 8; u++)
+            v[u] = rk[j + u * 256];
+#pragma unroll
+        for (int u = 0; u < 8; u++) {
+            const K x = value(v[u]);
+            mn = x < mn ? x : mn;
+        }
+    }
+    for (; j < n; j += 256) {
+        const K x = value(rk[j]);
+        mn = x < mn ? x : mn;
+    }
+    // The k-th smallest minimum: the one with rank k - 1 (ties by thread).
+    bkey[tid] = mn;
+    if (tid == 0)
+        count = 0;
+    __syncthreads();
+    int rank = 0;
+#pragma unroll 8
+    for (int t = 0; t < 256; t++) {
+        const K o = bkey[t];
+        rank += o < mn || (o == mn && t < tid);
+    }
+    if (rank == k - 1)
+        bound = mn;
+    __syncthreads();
+    const K bd = bound;
+    __syncthreads();
+    auto take = [&](K x, int jj) {
+        if (x <= bd) {
+            const int p = atomicAdd(&count, 1);
+            if (p < SEL_CAP) {
+                bkey[p] = x;
+                bidx[p] = jj;
+            }
+        }
+    };
+    j = tid;
+    for (; j + 7 * 256 < n; j += 8 * 256) {
+        K v[8];
+#pragma unroll
+        for (int u = 0; u < 8; u++)
+            v[u] = rk[j + u * 256];
+#pragma unroll
+        for (int u = 0; u < 8; u++)
+            take(value(v[u]), j + u * 256);
+    }
+    for (; j < n; j += 256)
+        take(value(rk[j]), j);
+    __syncthreads();
+    const int c = count;
+    if (c > SEL_CAP) {
+        if (tid == 0)
+            out_idx[o] = -2;
+        return;
+    }
+    int cap = 2;
+    while (cap < c || cap < k)
+        cap <<= 1;
+    for (int t = c + tid; t < cap; t += 256) {
+        bkey[t] = inf;
+        bidx[t] = INT_MAX;
+    }
+    __syncthreads();
+    for (int size = 2; size <= cap; size <<= 1) {
+        for (int stride = size >> 1; stride > 0; stride >>= 1) {
+            for (int t = tid; t < cap / 2; t += 256) {
+                const int a = 2 * t - (t & (stride - 1));
+                const int b = a + stride;
+                const bool asc = (a & size) == 0;
+                const K ka = bkey[a], kb = bkey[b];
+                const int ia = bidx[a], ib = bidx[b];
+                if (pair_less(kb, ib, ka, ia) == asc) {
+                    bkey[a] = kb;
+                    bkey[b] = ka;
+                    bidx[a] = ib;
+                    bidx[b] = ia;
+                }
+            }
+            __syncthreads();
+        }
+    }
+    for (int t = tid; t < k; t += 256) {
+        const K v = bkey[t];
+        out_key[o + t] = largest ? -v : v;
+        out_idx[o + t] = bidx[t] == INT_MAX ? INT_MAX : c0 + bidx[t];
+    }
+}
+
+// idx[e] = cols[row of e][idx[e]]: the columns behind the positions of a second selection.
+__global__ void row_topk_map_kernel(int *__restrict__ idx, const int *__restrict__ cols, int rows,
+                                    int k, int width) {
+    const int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (e >= (int64_t)rows * k)
+        return;
+    const int p = idx[e];
+    if (p != INT_MAX)
+        idx[e] = cols[e / k * width + p];
+}
+
+} // namespace
+
+// The selection over (row, segment) pairs: rows x nseg results of k.
+template <typename K>
+static hipError_t topk_level(const K *keys, int64_t ld, int rows, int n, int k, int largest,
+                             K *out_key, int *out_idx, int seg, int nseg, hipStream_t s) {
+    dim3 grid(rows, nseg), block(256);
+    if (k <= 128)
+        hipLaunchKernelGGL(row_topk_bound_kernel<K>, grid, block, 0, s, keys, ld, n, k, largest,
+                           out_key, out_idx, seg);
+    auto kern = k + 256 <= 512    ? row_topk_kernel<K, 512>
+                : k + 256 <= 1024 ? row_topk_kernel<K, 1024>
+                : k + 256 <= 2048 ? row_topk_kernel<K, 2048>
+                                  : row_topk_kernel<K, 4096>;
+    hipLaunchKernelGGL(kern, grid, block, 0, s, keys, ld, rows, n, k, largest, out_key, out_idx,
+                       k <= 128 ? 1 : 0, seg);
+    return hipGetLastError();
+}
+
+// Few long rows (one workgroup each would leave the chip idle: a row of 2,000,000 keys takes one
+// workgroup some 2 ms) are cut into segments of 8,192 columns or more, about 1,024 workgroups in
+// all, each segment's k best selected, then the best of those.
+int row_topk_segments(int rows, int n, int k) {
+    if (k > 128 || rows >= 512 || n < 32768)
+        return 1;
+    return std::max(1, std::min({n / 8192, 1024 / rows, 256}));
+}
+
 template <typename K>
 hipError_t launch_row_topk(const K *keys, int64_t ld, int rows, int n, int k, int largest,
-                           K *out_key, int *out_idx, hipStream_t s) {
+                           K *out_key, int *out_idx, hipStream_t s, K *tmp_key, int *tmp_idx) {
     if (k < 1 || k > 3840 || rows < 1)
         return hipErrorInvalidValue;
-    dim3 grid(rows), block(256);
-    if (k + 256 <= 512)
-        hipLaunchKernelGGL((row_topk_kernel<K, 512>), grid, block, 0, s, keys, ld, rows, n, k,
-                           largest, out_key, out_idx);
-    else if (k + 256 <= 1024)
-        hipLaunchKernelGGL((row_topk_kernel<K, 1024>), grid, block, 0, s, keys, ld, rows, n, k,
-                           largest, out_key, out_idx);
-    else if (k + 256 <= 2048)
-        hipLaunchKernelGGL((row_topk_kernel<K, 2048>), grid, block, 0, s, keys, ld, rows, n, k,
-                           largest, out_key, out_idx);
-    else
-        hipLaunchKernelGGL((row_topk_kernel<K, 4096>), grid, block, 0, s, keys, ld, rows, n, k,
-                           largest, out_key, out_idx);
+    const int want = tmp_key && tmp_idx ? row_topk_segments(rows, n, k) : 1;
+    if (want <= 1)
+        return topk_level<K>(keys, ld, rows, n, k, largest, out_key, out_idx, n, 1, s);
+    const int seg = (n + want - 1) / want, nseg = (n + seg - 1) / seg;
+    hipError_t e = topk_level<K>(keys, ld, rows, n, k, largest, tmp_key, tmp_idx, seg, nseg, s);
+    if (e != hipSuccess)
+        return e;
+    // Among equal keys the earlier segment and, within it, the earlier column come first, so the
+    // order of the positions is that of the columns.
+    e = topk_level<K>(tmp_key, (int64_t)nseg * k, rows, nseg * k, k, largest, out_key, out_idx,
+                      nseg * k, 1, s);
+    if (e != hipSuccess)
+        return e;
+    hipLaunchKernelGGL(row_topk_map_kernel, dim3((unsigned)(((int64_t)rows * k + 255) / 256)),
+                       dim3(256), 0, s, out_idx, tmp_idx, rows, k, nseg * k);
     return hipGetLastError();
 }
 
 template hipError_t launch_row_topk<float>(const float *, int64_t, int, int, int, int, float *,
-                                           int *, hipStream_t);
+                                           int *, hipStream_t, float *, int *);
 template hipError_t launch_row_topk<double>(const double *, int64_t, int, int, int, int,
-                                            double *, int *, hipStream_t);
+                                            double *, int *, hipStream_t, double *, int *);
 
 } // namespace dagpu
 

@@ -16,6 +16,7 @@ struct SearchParams {
     int prec = 0;     // operand precision of the fused tile (KP_*)
     int variant = -1; // fused tile kernel variant (-1: tuning table)
     int kc_min = 0;   // minimum candidates kept per (query, split) on the fused tile
+    bool automatic = false; // operand form and tile options as the library chooses
     bool seed = false; // seed the fused tile's thresholds (group minima over a row sample)
     // Candidate-list length of the fused tile for k neighbours.
     int tile_kc(int k) const;
@@ -31,7 +32,7 @@ struct SearchContext {
     // When set, the tuned maps above are read and written in this context instead: contexts
     // that search the same handle from one thread share their tuning.
     SearchContext *tuning = nullptr;
-    DeviceBuffer q_norm, keys, sel_key, sel_idx, qpad, part_key, part_idx, part_tau, fb, fb_q,
+    DeviceBuffer q_norm, keys, sel_key, sel_idx, seg_key, seg_idx, qpad, part_key, part_idx, part_tau, fb, fb_q,
         fb_ind, fb_dist, fb_bound, tau0, qc;
     // Pinned host word receiving the fallback count of the last fused launch.
     int *h_fb = nullptr;
@@ -118,6 +119,7 @@ template <typename T> class NNHandle : public AlgHandle {
     da_status search_tiles(SearchContext &ctx, const T *dQ, da_int nq, da_int k,
                            bool return_distance, da_int *d_ind, T *d_dist);
     bool fused_eligible(da_int k) const;
+    bool tiles_faster(da_int nq) const;
     int split_cap(int kc) const;
     int tile_splits(SearchContext &ctx, int prec, int kc, int variant, da_int nq,
                     const void *qpad, const float *seed, hipStream_t st,
