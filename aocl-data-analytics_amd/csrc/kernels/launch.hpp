@@ -325,6 +325,41 @@ hipError_t launch_dbscan_offs(void *temp, size_t bytes, const int *cnt, long lon
 hipError_t launch_dbscan_label(const long long *offs, const int *ind, const unsigned char *core,
                                const int *parent, const int *rid, int *labels, int n,
                                hipStream_t s);
+// ---- kNN of wide rows and of the cosine metric (knn_wide.hip) ----
+// Scale of the operand rows, the largest training value as given, the bits of the largest
+// squared operand norm, and whether a training value is not finite or out of range (the general
+// path then serves the search).
+struct WideScale {
+    double scale, big;
+    unsigned long long ymax2;
+    int bad;
+};
+// Operand rows come in blocks of 128, k steps of 32 features.
+inline int wide_rows(int n) { return (n + 127) / 128 * 128; }
+inline int wide_ksteps(int d) { return (d + 31) / 32; }
+inline size_t wide_operand_bytes(int n, int d) {
+    return (size_t)wide_rows(n) * wide_ksteps(d) * 128;
+}
+// Training operand P (wide_operand_bytes), h (wide_rows(n) floats), centre mu (d doubles) and
+// *sc. ycos: the rows' cosine norms (cosine metric) or null. range: 2 d words of scratch.
+template <typename T>
+hipError_t launch_wide_prepare(const T *Y, int n, int d, const double *ycos,
+                               unsigned long long *range, double *mu, WideScale *sc, void *P,
+                               float *h, hipStream_t s);
+// Query operand and the error bound of each query's scores (wide_rows(nq) floats).
+template <typename T>
+hipError_t launch_wide_queries(const T *Q, int nq, int d, const double *qcos, const double *mu,
+                               WideScale *sc, void *P, float *err, hipStream_t s);
+// out[q * wide_rows(n) + j] = score of the pair, all wide_rows(nq) rows written.
+hipError_t launch_wide_scores(const void *PA, int nq, const void *PB, int n, int d, const float *h,
+                              float *out, hipStream_t s);
+// Exact keys of the selected rows (kc <= 128 per query, ascending by (score, row)) within twice
+// the bound of the k-th; queries that cannot be certified are appended to fb_list (as q0 + q).
+template <typename T>
+hipError_t launch_wide_merge(const float *skey, const int *sidx, int nq, int kc, int k, int all,
+                             const T *Q, const T *Y, int d, const float *err, const double *qcos,
+                             const double *ycos, int post, int q0, T *out_dist, int *out_idx,
+                             int *fb_count, int *fb_list, hipStream_t s);
 // ---- Radius search on the matrix cores (radius_mfma.hip): a hit bit per pair ----
 // Metrics whose key is a function of the squared euclidean distance.
 bool radius_bits_metric(int metric);

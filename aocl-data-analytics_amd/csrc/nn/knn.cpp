@@ -218,6 +218,7 @@ da_status NNHandle<T>::set_data(da_int n_samples, da_int n_features, const T *X,
     trained_ = true;
     fused_ready_ = false;
     ypad_prec_ = -1;
+    wide_state_ = 0;
     return prepare_fused(tile_prec());
 }
 
@@ -655,8 +656,18 @@ da_status NNHandle<T>::search_launch(SearchContext &ctx, const SearchParams &sp,
         fused = false;
         ctx.last_candidates = n_samples_; // every row has its exact key
     }
-    if (!fused)
+    if (!fused) {
+        if (!ctx.second_pass && wide_eligible(nq, k)) {
+            da_status s = prepare_wide();
+            if (s != da_status_success)
+                return s;
+            if (wide_state_ == 1) {
+                fused = true;
+                return search_wide(ctx, dQ, nq, k, return_distance, d_ind, d_dist);
+            }
+        }
         return search_tiles(ctx, dQ, nq, k, return_distance, d_ind, d_dist);
+    }
     hipStream_t st = ctx.gpu->stream();
     const int n = n_samples_, d = n_features_;
     const int prec = sp.prec;
@@ -738,6 +749,107 @@ da_status NNHandle<T>::search_launch(SearchContext &ctx, const SearchParams &sp,
     }
     DA_HIP(err, hipMemcpyAsync(ctx.h_fb, fbc, sizeof(int), hipMemcpyDeviceToHost, st));
     ctx.last_candidates = nsplit * kc;
+    return da_status_success;
+}
+
+// Searches served by approximate scores on the matrix cores, a margin and exact keys
+// (knn_wide.hip): squared-euclidean rows too wide for the fused tile, and the cosine metric, up
+// to k = 96 (the selection holds 128) and 4,096 features (a query row in LDS). Below 2^31
+// products its preparation and extra launches cost more than the exact key tiles (85 fs per
+// product: 0.18 ms).
+template <typename T> bool NNHandle<T>::wide_eligible(da_int nq, da_int k) const {
+    const bool sq = metric_ == da_euclidean || metric_ == da_sqeuclidean ||
+                    (metric_ == da_minkowski && p_ == 2.0);
+    return ((sq && n_features_ > 128) || metric_ == da_cosine) && n_features_ <= 4096 && k <= 96 &&
+           n_samples_ >= 1024 &&
+           (double)nq * n_samples_ * n_features_ >= (double)((int64_t)1 << 31);
+}
+
+template <typename T> da_status NNHandle<T>::prepare_wide() {
+    const int cos = metric_ == da_cosine;
+    if (wide_state_ != 0 && wide_cos_ == cos)
+        return da_status_success;
+    hipStream_t st = gpu->stream();
+    const int n = n_samples_, d = n_features_;
+    DA_HIP(err, wide_op_.reserve(wide_operand_bytes(n, d)));
+    DA_HIP(err, wide_h_.reserve((size_t)wide_rows(n) * sizeof(float)));
+    DA_HIP(err, wide_mu_.reserve((size_t)3 * d * sizeof(double)));
+    DA_HIP(err, wide_sc_.reserve(sizeof(WideScale)));
+    WideScale *sc = wide_sc_.as<WideScale>();
+    double *mu = wide_mu_.as<double>();
+    DA_HIP(err, launch_wide_prepare<T>(train_.as<T>(), n, d, cos ? train_cos_.as<double>() : nullptr,
+                                       reinterpret_cast<unsigned long long *>(mu + d), mu, sc,
+                                       wide_op_.ptr(), wide_h_.as<float>(), st));
+    int bad = 0;
+    DA_HIP(err, hipMemcpyAsync(&bad, &sc->bad, sizeof(int), hipMemcpyDeviceToHost, st));
+    DA_HIP(err, hipStreamSynchronize(st));
+    wide_state_ = bad ? 2 : 1;
+    wide_cos_ = cos;
+    return da_status_success;
+}
+
+// Query blocks of up to 256 MB of scores. The selection keeps 64 candidates for k <= 32 and 128
+// beyond: the margin between the k-th and the last of them certifies a query.
+template <typename T>
+da_status NNHandle<T>::search_wide(SearchContext &ctx, const T *dQ, da_int nq, da_int k,
+                                   bool return_distance, da_int *d_ind, T *d_dist) {
+    hipStream_t st = ctx.gpu->stream();
+    const int n = n_samples_, d = n_features_;
+    const bool cos = metric_ == da_cosine;
+    const int kc = std::min(n, k <= 32 ? 64 : 128);
+    const int post = cos || metric_ == da_sqeuclidean ? 0 : 1;
+    if (!ctx.h_fb)
+        DA_HIP(err, hipHostMalloc((void **)&ctx.h_fb, sizeof(int)));
+    const double *qcos = nullptr;
+    if (cos) {
+        DA_HIP(err, ctx.q_norm.reserve((size_t)nq * sizeof(double)));
+        DA_HIP(err, launch_row_sqnorms<T>(dQ, d, nq, d, ctx.q_norm.as<double>(), st));
+        DA_HIP(err, launch_cosine_norms(ctx.q_norm.as<double>(), nq,
+                                        std::numeric_limits<T>::epsilon(), st));
+        qcos = ctx.q_norm.as<double>();
+    }
+    const int64_t ld = wide_rows(n);
+    const int chunk = (int)std::max<int64_t>(
+        128, std::min<int64_t>(wide_rows(nq), ((int64_t)64 << 20) / ld / 128 * 128));
+    DA_HIP(err, ctx.wide_q.reserve(wide_operand_bytes(chunk, d)));
+    DA_HIP(err, ctx.wide_err.reserve((size_t)chunk * sizeof(float)));
+    DA_HIP(err, ctx.keys.reserve((size_t)chunk * ld * sizeof(float)));
+    DA_HIP(err, ctx.sel_key.reserve((size_t)chunk * kc * sizeof(float)));
+    DA_HIP(err, ctx.sel_idx.reserve((size_t)chunk * kc * sizeof(int)));
+    DA_HIP(err, ctx.seg_key.reserve((size_t)1024 * kc * sizeof(double)));
+    DA_HIP(err, ctx.seg_idx.reserve((size_t)1024 * kc * sizeof(int)));
+    DA_HIP(err, ctx.fb.reserve((size_t)(nq + 1) * sizeof(int)));
+    DA_HIP(err, ctx.fb_bound.reserve((size_t)nq * sizeof(float)));
+    int *fbc = ctx.fb.as<int>();
+    DA_HIP(err, hipMemsetAsync(fbc, 0, sizeof(int), st));
+    WideScale *sc = wide_sc_.as<WideScale>();
+    for (da_int q0 = 0; q0 < nq; q0 += chunk) {
+        const da_int rows = std::min<da_int>(chunk, nq - q0);
+        const T *q = dQ + (size_t)q0 * d;
+        {
+            KernelScope ks(*ctx.gpu, "knn_wide_scores");
+            DA_HIP(err, launch_wide_queries<T>(q, rows, d, qcos ? qcos + q0 : nullptr,
+                                               wide_mu_.as<double>(), sc, ctx.wide_q.ptr(),
+                                               ctx.wide_err.as<float>(), st));
+            DA_HIP(err, launch_wide_scores(ctx.wide_q.ptr(), rows, wide_op_.ptr(), n, d,
+                                           wide_h_.as<float>(), ctx.keys.as<float>(), st));
+        }
+        {
+            KernelScope ks(*ctx.gpu, "row_topk");
+            DA_HIP(err, launch_row_topk<float>(ctx.keys.as<float>(), ld, rows, n, kc, 0,
+                                               ctx.sel_key.as<float>(), ctx.sel_idx.as<int>(), st,
+                                               ctx.seg_key.as<float>(), ctx.seg_idx.as<int>()));
+        }
+        KernelScope ks(*ctx.gpu, "knn_merge");
+        DA_HIP(err, launch_wide_merge<T>(
+                        ctx.sel_key.as<float>(), ctx.sel_idx.as<int>(), rows, kc, k, kc == n, q,
+                        train_.as<T>(), d, ctx.wide_err.as<float>(), qcos ? qcos + q0 : nullptr,
+                        cos ? train_cos_.as<double>() : nullptr, post, q0,
+                        return_distance ? d_dist + (size_t)q0 * k : nullptr,
+                        d_ind + (size_t)q0 * k, fbc, fbc + 1, st));
+    }
+    DA_HIP(err, hipMemcpyAsync(ctx.h_fb, fbc, sizeof(int), hipMemcpyDeviceToHost, st));
+    ctx.last_candidates = kc;
     return da_status_success;
 }
 

@@ -32,7 +32,7 @@ struct SearchContext {
     // When set, the tuned maps above are read and written in this context instead: contexts
     // that search the same handle from one thread share their tuning.
     SearchContext *tuning = nullptr;
-    DeviceBuffer q_norm, keys, sel_key, sel_idx, seg_key, seg_idx, qpad, part_key, part_idx, part_tau, fb, fb_q,
+    DeviceBuffer q_norm, keys, sel_key, sel_idx, seg_key, seg_idx, wide_q, wide_err, qpad, part_key, part_idx, part_tau, fb, fb_q,
         fb_ind, fb_dist, fb_bound, tau0, qc;
     // Pinned host word receiving the fallback count of the last fused launch.
     int *h_fb = nullptr;
@@ -125,6 +125,15 @@ template <typename T> class NNHandle : public AlgHandle {
                     const void *qpad, const float *seed, hipStream_t st,
                     const KnnCentring *cen = nullptr);
     da_status prepare_fused(int prec);
+    // Wide rows and the cosine metric (knn_wide.hip): the training operand is laid out at the
+    // first search that uses it.
+    bool wide_eligible(da_int nq, da_int k) const;
+    da_status prepare_wide();
+    da_status search_wide(SearchContext &ctx, const T *dQ, da_int nq, da_int k,
+                          bool return_distance, da_int *d_ind, T *d_dist);
+    int wide_state_ = 0; // 0: not laid out, 1: ready, 2: the data need the general path
+    int wide_cos_ = -1;  // metric of the layout: cosine or euclidean
+    DeviceBuffer wide_op_, wide_h_, wide_mu_, wide_sc_;
 
     bool trained_ = false;
     // Training rows (column-major) read back from a stored model, until restore() uploads them.
