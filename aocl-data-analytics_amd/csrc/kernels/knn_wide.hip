@@ -130,24 +130,26 @@ __global__ __launch_bounds__(256) void wide_scale_kernel(const unsigned long lon
 }
 
 // Operand rows, 16 a tile: [k step of 32][hi, lo][lane][8], lane 16 g + r holding features
-// 32 ks + 8 g .. + 7 of row r (a fragment is 1 KB of contiguous memory). One wave per tile.
+// 32 ks + 8 g .. + 7 of row r (a fragment is 1 KB of contiguous memory). One workgroup per tile,
+// its waves taking every blockDim / 64-th k step (1,066 queries of 784 features are 67 tiles: with
+// one wave each the pass took 74 us).
 // Training rows: h[row] = |y'|^2/2 (0 for cosine) and the largest |y'|^2; query rows: the error
 // bound err[row] of their scores, +inf where a value is not finite or exceeds fp16's range.
 template <typename T>
-__global__ __launch_bounds__(256) void wide_pack_kernel(
-    const T *__restrict__ X, int rows, int tiles, int d, int KS, const double *__restrict__ mu,
+__global__ __launch_bounds__(1024) void wide_pack_kernel(
+    const T *__restrict__ X, int rows, int d, int KS, const double *__restrict__ mu,
     WideScale *sc, const double *__restrict__ cosn, double ce, _Float16 *__restrict__ P,
     float *__restrict__ h, float *__restrict__ err) {
-    const int t = blockIdx.x * 4 + (int)(threadIdx.x >> 6);
-    if (t >= tiles)
-        return;
+    __shared__ double rn[16][16], rb[16][16], rt[16][16];
+    __shared__ int rf[16][16];
+    const int t = blockIdx.x, w = threadIdx.x >> 6, nw = blockDim.x >> 6;
     const int lane = threadIdx.x & 63, r = lane & 15, g = lane >> 4;
     const int row = t * 16 + r;
     const double s = sc->scale;
     const double inv = (cosn && row < rows) ? 1.0 / cosn[row] : 1.0;
     double nn = 0.0, big = 0.0, top = 0.0;
     bool nf = false;
-    for (int ks = 0; ks < KS; ks++) {
+    for (int ks = w; ks < KS; ks += nw) {
         v8h hi, lo;
 #pragma unroll
         for (int e = 0; e < 8; e++) {
@@ -176,8 +178,21 @@ __global__ __launch_bounds__(256) void wide_pack_kernel(
         top = fmax(top, __shfl_xor(top, o, 64));
         nf |= __shfl_xor((int)nf, o, 64) != 0;
     }
-    if (g != 0)
+    if (g == 0) {
+        rn[w][r] = nn;
+        rb[w][r] = big;
+        rt[w][r] = top;
+        rf[w][r] = nf;
+    }
+    __syncthreads();
+    if (w != 0 || g != 0)
         return;
+    for (int q = 1; q < nw; q++) {
+        nn += rn[q][r];
+        big = fmax(big, rb[q][r]);
+        top = fmax(top, rt[q][r]);
+        nf |= rf[q][r] != 0;
+    }
     const bool fits = !nf && top < 60000.0;
     if (h) {
         h[row] = cosn ? 0.0f : (float)(0.5 * nn);
@@ -352,7 +367,7 @@ __global__ __launch_bounds__(64) void wide_merge_kernel(
             }
         };
         if (vec) {
-#pragma unroll 4
+#pragma unroll 16
             for (int l = 0; l < d; l += VE) {
                 const uint4 u = *reinterpret_cast<const uint4 *>(y + l);
                 T v[VE];
@@ -401,7 +416,7 @@ hipError_t launch_wide_prepare(const T *Y, int n, int d, const double *ycos,
                            dim3((d + 63) / 64, std::min(128, (n + 63) / 64)), dim3(256), 0, s, Y, n,
                            d, range, sc);
     hipLaunchKernelGGL(wide_scale_kernel, dim3(1), dim3(256), 0, s, range, d, ycos ? 1 : 0, mu, sc);
-    hipLaunchKernelGGL(wide_pack_kernel<T>, dim3((tiles + 3) / 4), dim3(256), 0, s, Y, n, tiles, d,
+    hipLaunchKernelGGL(wide_pack_kernel<T>, dim3(tiles), dim3(64 * std::min(16, KS)), 0, s, Y, n, d,
                        KS, mu, sc, ycos, 0.0, static_cast<_Float16 *>(P), h, nullptr);
     return hipGetLastError();
 }
@@ -410,7 +425,7 @@ template <typename T>
 hipError_t launch_wide_queries(const T *Q, int nq, int d, const double *qcos, const double *mu,
                                WideScale *sc, void *P, float *err, hipStream_t s) {
     const int KS = wide_ksteps(d), tiles = wide_rows(nq) / 16;
-    hipLaunchKernelGGL(wide_pack_kernel<T>, dim3((tiles + 3) / 4), dim3(256), 0, s, Q, nq, tiles, d,
+    hipLaunchKernelGGL(wide_pack_kernel<T>, dim3(tiles), dim3(64 * std::min(16, KS)), 0, s, Q, nq, d,
                        KS, mu, sc, qcos, wide_relative_bound(), static_cast<_Float16 *>(P),
                        nullptr, err);
     return hipGetLastError();
