@@ -5,6 +5,7 @@
 #include <algorithm>
 #include <climits>
 #include <cmath>
+#include <functional>
 #include <limits>
 
 namespace dagpu {
@@ -201,6 +202,7 @@ template <typename T> da_status ApproxNNHandle<T>::train() {
     DA_HIP(err, hipStreamSynchronize(st));
     list_sizes_.assign(n_list_, 0);
     lists_.assign(n_list_, {});
+    tiles_state_ = 0;
     err->clear();
     model_trained = true;
     return da_status_success;
@@ -328,6 +330,7 @@ da_status ApproxNNHandle<T>::add(da_int n_add, da_int n_features, const T *X, da
     DA_HIP(err, hipMemcpyAsync(off_d_.ptr(), off.data(), off.size() * sizeof(int),
                                hipMemcpyHostToDevice, st));
     DA_HIP(err, hipStreamSynchronize(st));
+    tiles_state_ = 0;
     data_added_ = true;
     return da_status_success;
 }
@@ -337,6 +340,211 @@ template <typename T> da_status ApproxNNHandle<T>::train_and_add() {
     if (s != da_status_success)
         return s;
     return add(n_samples_, n_features_, X_train_, ldx_train_);
+}
+
+// Coarse step: the n_probe nearest centroids of each query, by (distance, index); for the
+// inner-product and cosine metrics the largest q.c (:1093-1127). Probes go to probe_d_.
+template <typename T>
+da_status ApproxNNHandle<T>::coarse(const T *Q, int rows, da_int n_probe) {
+    hipStream_t st = gpu->stream();
+    const bool ip = metric_ == ANN_INNER || metric_ == ANN_COSINE;
+    const int d = n_features_;
+    DA_HIP(err, ckeys_.reserve((size_t)rows * n_list_ * sizeof(T)));
+    DA_HIP(err, probe_key_.reserve((size_t)rows * n_probe * sizeof(T)));
+    DA_HIP(err, probe_d_.reserve((size_t)rows * n_probe * sizeof(int)));
+    KernelScope ks(*gpu, "ivf_coarse");
+    DA_HIP(err, (launch_pairwise_direct<T, T>(ip ? KM_INNER : KM_SQEUCLIDEAN, Q, C_d_.as<T>(), rows,
+                                              n_list_, d, ckeys_.as<T>(), n_list_, nullptr,
+                                              nullptr, 2.0, 0, 0, st)));
+    DA_HIP(err, launch_row_topk<T>(ckeys_.as<T>(), n_list_, rows, n_list_, n_probe, ip ? 1 : 0,
+                                   probe_key_.as<T>(), probe_d_.as<int>(), st));
+    return da_status_success;
+}
+
+template <typename T>
+da_status ApproxNNHandle<T>::search_scan(const T *Q, da_int n_queries, da_int k, da_int n_probe,
+                                         T *dist, int *ind) {
+    hipStream_t st = gpu->stream();
+    const int d = n_features_;
+    const bool ip = metric_ == ANN_INNER || metric_ == ANN_COSINE;
+    const da_int max_list = *std::max_element(list_sizes_.begin(), list_sizes_.end());
+    // Query blocks whose candidate rows (n_probe lists of at most max_list vectors) and
+    // coarse keys stay within 2^26 entries.
+    const int64_t row_cap = std::max<int64_t>({(int64_t)n_probe * max_list, (int64_t)k,
+                                               (int64_t)n_list_});
+    const da_int qb = (da_int)std::max<int64_t>(
+        1, std::min<int64_t>(n_queries, ((int64_t)1 << 26) / row_cap));
+    DA_HIP(err, seg_d_.reserve((size_t)qb * n_probe * sizeof(int)));
+    DA_HIP(err, sel_key_.reserve((size_t)qb * k * sizeof(T)));
+    DA_HIP(err, sel_idx_.reserve((size_t)qb * k * sizeof(int)));
+    std::vector<int> probes((size_t)qb * n_probe), seg((size_t)qb * n_probe);
+    for (da_int q0 = 0; q0 < n_queries; q0 += qb) {
+        const int rows = (int)std::min<da_int>(qb, n_queries - q0);
+        da_status s = coarse(Q + (size_t)q0 * d, rows, n_probe);
+        if (s != da_status_success)
+            return s;
+        DA_HIP(err, hipMemcpyAsync(probes.data(), probe_d_.ptr(),
+                                   (size_t)rows * n_probe * sizeof(int), hipMemcpyDeviceToHost,
+                                   st));
+        DA_HIP(err, hipStreamSynchronize(st));
+        // Candidate columns of each probed list within its query's row, the lists in
+        // ascending list number: selection by (key, column) then keeps, among equal keys,
+        // the vector of the lower list and the earlier position in it, the vector the
+        // reference's search (lists in number order, strict < on its heap) keeps.
+        int64_t ld = k;
+        std::vector<int> by_list(n_probe);
+        for (int r = 0; r < rows; r++) {
+            const int *pr = probes.data() + (size_t)r * n_probe;
+            for (da_int p = 0; p < n_probe; p++)
+                by_list[p] = p;
+            std::sort(by_list.begin(), by_list.end(),
+                      [&](int a, int b) { return pr[a] < pr[b]; });
+            int64_t pos = 0;
+            for (da_int p = 0; p < n_probe; p++) {
+                seg[(size_t)r * n_probe + by_list[p]] = (int)pos;
+                pos += list_sizes_[pr[by_list[p]]];
+            }
+            ld = std::max(ld, pos);
+        }
+        DA_HIP(err, hipMemcpyAsync(seg_d_.ptr(), seg.data(), (size_t)rows * n_probe * sizeof(int),
+                                   hipMemcpyHostToDevice, st));
+        DA_HIP(err, cand_key_.reserve((size_t)rows * ld * sizeof(T)));
+        DA_HIP(err, cand_idx_.reserve((size_t)rows * ld * sizeof(int)));
+        {
+            KernelScope ks(*gpu, "ivf_scan");
+            DA_HIP(err, launch_ivf_pad<T>(cand_key_.as<T>(), cand_idx_.as<int>(),
+                                          (int64_t)rows * ld, st));
+            DA_HIP(err, launch_ivf_scan<T>(Q + (size_t)q0 * d, rows, n_probe, d, X_d_.as<T>(),
+                                           perm_d_.as<int>(), off_d_.as<int>(), probe_d_.as<int>(),
+                                           seg_d_.as<int>(), ld, cand_key_.as<T>(),
+                                           cand_idx_.as<int>(), st, ip ? 1 : 0));
+        }
+        {
+            KernelScope ks(*gpu, "ivf_select");
+            DA_HIP(err, launch_row_topk<T>(cand_key_.as<T>(), ld, rows, (int)ld, k, 0,
+                                           sel_key_.as<T>(), sel_idx_.as<int>(), st));
+            const int post = metric_ == ANN_EUCLIDEAN ? 1
+                             : metric_ == ANN_COSINE  ? 2
+                             : metric_ == ANN_INNER   ? 3
+                                                      : 0;
+            DA_HIP(err, launch_ivf_finish<T>(sel_key_.as<T>(), sel_idx_.as<int>(),
+                                             cand_idx_.as<int>(), ld, k, (int64_t)rows * k, post,
+                                             dist + (size_t)q0 * k,
+                                             ind + (size_t)q0 * k, st));
+        }
+    }
+    return da_status_success;
+}
+
+// Operand rows of the lists, each padded to whole tiles of 16. ready: the data fit the fp16 range
+// and the memory sufficed.
+template <typename T> da_status ApproxNNHandle<T>::prepare_tiles(bool &ready) {
+    hipStream_t st = gpu->stream();
+    const int d = n_features_;
+    if (tiles_state_ == 0) {
+        tile_off_.assign(n_list_ + 1, 0);
+        int64_t rows = 0;
+        for (da_int c = 0; c < n_list_; c++) {
+            rows += ((int64_t)list_sizes_[c] + 15) / 16 * 16;
+            tile_off_[c + 1] = (int)(rows / 16);
+        }
+        // Without the memory the scans serve this search, and the next one tries again.
+        if (rows + 16 > INT_MAX ||
+            tile_op_.reserve((size_t)rows * wide_ksteps(d) * 128) != hipSuccess ||
+            tile_map_.reserve((size_t)rows * sizeof(int)) != hipSuccess ||
+            tile_h_.reserve((size_t)rows * sizeof(float)) != hipSuccess) {
+            (void)hipGetLastError();
+            ready = false;
+            return da_status_success;
+        }
+        DA_HIP(err, tile_off_d_.reserve(tile_off_.size() * sizeof(int)));
+        DA_HIP(err, tile_mu_.reserve((size_t)3 * d * sizeof(double)));
+        DA_HIP(err, tile_sc_.reserve(sizeof(WideScale)));
+        DA_HIP(err, hipMemcpyAsync(tile_off_d_.ptr(), tile_off_.data(),
+                                   tile_off_.size() * sizeof(int), hipMemcpyHostToDevice, st));
+        DA_HIP(err, launch_ivf_map(perm_d_.as<int>(), off_d_.as<int>(), tile_off_d_.as<int>(),
+                                   n_list_, tile_map_.as<int>(), st));
+        WideScale *sc = tile_sc_.as<WideScale>();
+        double *mu = tile_mu_.as<double>();
+        const int ip = metric_ == ANN_INNER || metric_ == ANN_COSINE;
+        DA_HIP(err, launch_ivf_lists<T>(X_d_.as<T>(), n_index_, d, ip, tile_map_.as<int>(),
+                                        (int)rows, reinterpret_cast<unsigned long long *>(mu + d),
+                                        mu, sc, tile_op_.ptr(), tile_h_.as<float>(), st));
+        int bad = 0;
+        DA_HIP(err, hipMemcpyAsync(&bad, &sc->bad, sizeof(int), hipMemcpyDeviceToHost, st));
+        DA_HIP(err, hipStreamSynchronize(st));
+        tiles_state_ = bad ? 2 : 1;
+    }
+    ready = tiles_state_ == 1;
+    return da_status_success;
+}
+
+// Query blocks of up to 2^28 scores (1 GB) and 2^26 coarse keys.
+template <typename T>
+da_status ApproxNNHandle<T>::search_tiles(const T *Q, da_int n_queries, da_int k, da_int n_probe,
+                                          int64_t ld, T *dist, int *ind) {
+    hipStream_t st = gpu->stream();
+    const int d = n_features_;
+    const int ip = metric_ == ANN_INNER || metric_ == ANN_COSINE;
+    const int64_t most = std::max<int64_t>(
+        1, std::min<int64_t>({(int64_t)n_queries, ((int64_t)1 << 28) / ld,
+                              ((int64_t)1 << 26) / n_list_, ((int64_t)1 << 30) / n_probe}));
+    const da_int blocks = (da_int)((n_queries + most - 1) / most);
+    const da_int qb = (n_queries + blocks - 1) / blocks;
+    const int64_t pairs = (int64_t)qb * n_probe, items = ivf_items(pairs, n_list_);
+    DA_HIP(err, tile_q_.reserve((size_t)(qb + 15) / 16 * 16 * wide_ksteps(d) * 128));
+    DA_HIP(err, tile_err_.reserve((size_t)(qb + 15) / 16 * 16 * sizeof(float)));
+    DA_HIP(err, tile_work_.reserve(((size_t)items * 2 + 4 * pairs + qb + 2 * n_list_ + 1) *
+                                   sizeof(int)));
+    DA_HIP(err, fb_.reserve((size_t)(n_queries + 1) * sizeof(int)));
+    DA_HIP(err, hipMemsetAsync(fb_.ptr(), 0, sizeof(int), st));
+    if (tile_scores_.reserve((size_t)qb * ld * sizeof(float)) != hipSuccess) {
+        (void)hipGetLastError();
+        return search_scan(Q, n_queries, k, n_probe, dist, ind);
+    }
+    IvfTiles p;
+    p.tile_off = tile_off_d_.as<int>();
+    p.map = tile_map_.as<int>();
+    p.op = tile_op_.ptr();
+    p.h = tile_h_.as<float>();
+    p.n_list = n_list_;
+    p.n_probe = n_probe;
+    p.max_tiles = (*std::max_element(list_sizes_.begin(), list_sizes_.end()) + 15) / 16;
+    p.items = tile_work_.as<int2>();
+    p.slist = tile_work_.as<int>() + items * 2;
+    p.sseg = p.slist + pairs;
+    p.place = p.sseg + pairs;
+    p.group = p.place + pairs;
+    p.rowlen = p.group + pairs;
+    p.cnt = p.rowlen + qb;
+    p.qoff = p.cnt + n_list_;
+    p.n_items = p.qoff + n_list_;
+    const int post = metric_ == ANN_EUCLIDEAN ? 1
+                     : metric_ == ANN_COSINE  ? 2
+                     : metric_ == ANN_INNER   ? 3
+                                              : 0;
+    for (da_int q0 = 0; q0 < n_queries; q0 += qb) {
+        const int rows = (int)std::min<da_int>(qb, n_queries - q0);
+        const T *q = Q + (size_t)q0 * d;
+        da_status s = coarse(q, rows, n_probe);
+        if (s != da_status_success)
+            return s;
+        {
+            KernelScope ks(*gpu, "ivf_tile_scores");
+            DA_HIP(err, launch_ivf_queries<T>(q, rows, d, ip, tile_mu_.as<double>(),
+                                              tile_sc_.as<WideScale>(), tile_q_.ptr(),
+                                              tile_err_.as<float>(), st));
+            DA_HIP(err, launch_ivf_tile_scores(p, probe_d_.as<int>(), tile_q_.ptr(), rows, d,
+                                               tile_scores_.as<float>(), ld, st));
+        }
+        KernelScope ks(*gpu, "ivf_tile_select");
+        DA_HIP(err, launch_ivf_tile_select<T>(p, tile_scores_.as<float>(), ld,
+                                              tile_err_.as<float>(), q, X_d_.as<T>(), rows, d, k,
+                                              ip, post, q0, dist + (size_t)q0 * k,
+                                              ind + (size_t)q0 * k, fb_.as<int>(),
+                                              fb_.as<int>() + 1, st));
+    }
+    return da_status_success;
 }
 
 template <typename T>
@@ -386,92 +594,57 @@ da_status ApproxNNHandle<T>::kneighbors(da_int n_queries, da_int n_features, con
     if (s != da_status_success)
         return s;
     const int d = n_features_;
-    const bool ip = metric_ == ANN_INNER || metric_ == ANN_COSINE;
     // Cosine: queries normalised like the stored vectors (:1068-1081).
     if (metric_ == ANN_COSINE)
         DA_HIP(err, launch_ivf_normalize<T>(q_d_.as<T>(), n_queries, d, st));
-    const da_int max_list = *std::max_element(list_sizes_.begin(), list_sizes_.end());
-    // Query blocks whose candidate rows (n_probe lists of at most max_list vectors) and
-    // coarse keys stay within 2^26 entries.
-    const int64_t row_cap = std::max<int64_t>({(int64_t)n_probe * max_list, (int64_t)k,
-                                               (int64_t)n_list_});
-    const da_int qb = (da_int)std::max<int64_t>(
-        1, std::min<int64_t>(n_queries, ((int64_t)1 << 26) / row_cap));
     const size_t ob = (size_t)n_queries * k;
     DA_HIP(err, out_ind_.reserve(ob * sizeof(int)));
     DA_HIP(err, out_dist_.reserve(ob * sizeof(T)));
-    DA_HIP(err, ckeys_.reserve((size_t)qb * n_list_ * sizeof(T)));
-    DA_HIP(err, probe_key_.reserve((size_t)qb * n_probe * sizeof(T)));
-    DA_HIP(err, probe_d_.reserve((size_t)qb * n_probe * sizeof(int)));
-    DA_HIP(err, seg_d_.reserve((size_t)qb * n_probe * sizeof(int)));
-    DA_HIP(err, sel_key_.reserve((size_t)qb * k * sizeof(T)));
-    DA_HIP(err, sel_idx_.reserve((size_t)qb * k * sizeof(int)));
-    std::vector<int> probes((size_t)qb * n_probe), seg((size_t)qb * n_probe);
     const T *Q = q_d_.as<T>();
-    for (da_int q0 = 0; q0 < n_queries; q0 += qb) {
-        const int rows = (int)std::min<da_int>(qb, n_queries - q0);
-        // Coarse step: the n_probe nearest centroids of each query, by (distance, index);
-        // for the inner-product and cosine metrics the largest q.c (:1093-1127).
-        {
-            KernelScope ks(*gpu, "ivf_coarse");
-            DA_HIP(err, (launch_pairwise_direct<T, T>(ip ? KM_INNER : KM_SQEUCLIDEAN,
-                                                      Q + (size_t)q0 * d, C_d_.as<T>(), rows,
-                                                      n_list_, d, ckeys_.as<T>(), n_list_,
-                                                      nullptr, nullptr, 2.0, 0, 0, st)));
-            DA_HIP(err, launch_row_topk<T>(ckeys_.as<T>(), n_list_, rows, n_list_, n_probe,
-                                           ip ? 1 : 0, probe_key_.as<T>(), probe_d_.as<int>(),
-                                           st));
-        }
-        DA_HIP(err, hipMemcpyAsync(probes.data(), probe_d_.ptr(),
-                                   (size_t)rows * n_probe * sizeof(int), hipMemcpyDeviceToHost,
-                                   st));
-        DA_HIP(err, hipStreamSynchronize(st));
-        // Candidate columns of each probed list within its query's row, the lists in
-        // ascending list number: selection by (key, column) then keeps, among equal keys,
-        // the vector of the lower list and the earlier position in it, the vector the
-        // reference's search (lists in number order, strict < on its heap) keeps.
-        int64_t ld = k;
-        std::vector<int> by_list(n_probe);
-        for (int r = 0; r < rows; r++) {
-            const int *pr = probes.data() + (size_t)r * n_probe;
-            for (da_int p = 0; p < n_probe; p++)
-                by_list[p] = p;
-            std::sort(by_list.begin(), by_list.end(),
-                      [&](int a, int b) { return pr[a] < pr[b]; });
-            int64_t pos = 0;
-            for (da_int p = 0; p < n_probe; p++) {
-                seg[(size_t)r * n_probe + by_list[p]] = (int)pos;
-                pos += list_sizes_[pr[by_list[p]]];
-            }
-            ld = std::max(ld, pos);
-        }
-        DA_HIP(err, hipMemcpyAsync(seg_d_.ptr(), seg.data(), (size_t)rows * n_probe * sizeof(int),
-                                   hipMemcpyHostToDevice, st));
-        DA_HIP(err, cand_key_.reserve((size_t)rows * ld * sizeof(T)));
-        DA_HIP(err, cand_idx_.reserve((size_t)rows * ld * sizeof(int)));
-        {
-            KernelScope ks(*gpu, "ivf_scan");
-            DA_HIP(err, launch_ivf_pad<T>(cand_key_.as<T>(), cand_idx_.as<int>(),
-                                          (int64_t)rows * ld, st));
-            DA_HIP(err, launch_ivf_scan<T>(Q + (size_t)q0 * d, rows, n_probe, d, X_d_.as<T>(),
-                                           perm_d_.as<int>(), off_d_.as<int>(), probe_d_.as<int>(),
-                                           seg_d_.as<int>(), ld, cand_key_.as<T>(),
-                                           cand_idx_.as<int>(), st, ip ? 1 : 0));
-        }
-        {
-            KernelScope ks(*gpu, "ivf_select");
-            DA_HIP(err, launch_row_topk<T>(cand_key_.as<T>(), ld, rows, (int)ld, k, 0,
-                                           sel_key_.as<T>(), sel_idx_.as<int>(), st));
-            const int post = metric_ == ANN_EUCLIDEAN ? 1
-                             : metric_ == ANN_COSINE  ? 2
-                             : metric_ == ANN_INNER   ? 3
-                                                      : 0;
-            DA_HIP(err, launch_ivf_finish<T>(sel_key_.as<T>(), sel_idx_.as<int>(),
-                                             cand_idx_.as<int>(), ld, k, (int64_t)rows * k, post,
-                                             out_dist_.as<T>() + (size_t)q0 * k,
-                                             out_ind_.as<int>() + (size_t)q0 * k, st));
-        }
+    // Rows, neighbours and probes within the matrix-core kernels' limits and a query's longest
+    // possible score row within 2^26 columns take the list-major search, everything else the
+    // scans: 10,000 queries, 16 of 1,024 lists of 1,000,000 x 96 fp32: 1.4 ms against 28.
+    std::vector<int64_t> longest;
+    for (da_int n : list_sizes_)
+        longest.push_back((n + 15) / 16 * 16);
+    std::partial_sort(longest.begin(), longest.begin() + n_probe, longest.end(),
+                      std::greater<int64_t>());
+    int64_t ld = 16;
+    for (da_int p = 0; p < n_probe; p++)
+        ld += longest[p];
+    bool tiles = d <= IVF_TILE_D && k <= IVF_TILE_K && n_probe <= IVF_TILE_PROBE &&
+                 ld <= ((int64_t)1 << 26);
+    if (tiles) {
+        s = prepare_tiles(tiles);
+        if (s != da_status_success)
+            return s;
     }
+    if (tiles) {
+        s = search_tiles(Q, n_queries, k, n_probe, ld, out_dist_.as<T>(), out_ind_.as<int>());
+        int nfb = 0;
+        if (s == da_status_success) {
+            DA_HIP(err, hipMemcpyAsync(&nfb, fb_.ptr(), sizeof(int), hipMemcpyDeviceToHost, st));
+            DA_HIP(err, hipStreamSynchronize(st));
+        }
+        if (s == da_status_success && nfb > 0) {
+            const int *list = fb_.as<int>() + 1;
+            DA_HIP(err, fb_q_.reserve((size_t)nfb * d * sizeof(T)));
+            DA_HIP(err, fb_ind_.reserve((size_t)nfb * k * sizeof(int)));
+            DA_HIP(err, fb_dist_.reserve((size_t)nfb * k * sizeof(T)));
+            DA_HIP(err, launch_gather_scatter(Q, fb_q_.ptr(), list, nfb, d, sizeof(T), 0, st));
+            s = search_scan(fb_q_.as<T>(), nfb, k, n_probe, fb_dist_.as<T>(), fb_ind_.as<int>());
+            if (s != da_status_success)
+                return s;
+            DA_HIP(err, launch_gather_scatter(fb_ind_.ptr(), out_ind_.ptr(), list, nfb, k,
+                                              sizeof(int), 1, st));
+            DA_HIP(err, launch_gather_scatter(fb_dist_.ptr(), out_dist_.ptr(), list, nfb, k,
+                                              sizeof(T), 1, st));
+        }
+    } else {
+        s = search_scan(Q, n_queries, k, n_probe, out_dist_.as<T>(), out_ind_.as<int>());
+    }
+    if (s != da_status_success)
+        return s;
     // n_queries x k in the handle's storage order (kneighbors_compute_ivfflat, :1317-1344).
     if (order_ == row_major) {
         DA_HIP(err, hipMemcpyAsync(n_ind, out_ind_.ptr(), ob * sizeof(int), hipMemcpyDeviceToHost,
@@ -699,6 +872,7 @@ template <typename T> da_status ApproxNNHandle<T>::restore() {
                                    hipMemcpyHostToDevice, st));
     }
     DA_HIP(err, hipStreamSynchronize(st));
+    tiles_state_ = 0;
     stored_rows_.clear();
     stored_rows_.shrink_to_fit();
     return da_status_success;

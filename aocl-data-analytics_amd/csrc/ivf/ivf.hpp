@@ -27,6 +27,14 @@ template <typename T> class ApproxNNHandle : public AlgHandle {
 
   private:
     da_status check_options_update();
+    // The n_queries x k neighbours of device queries Q into dist and ind (device): by scans of the
+    // probed lists, or (tiles) by matrix-core scores with queries it could not certify listed in
+    // fb_ (count first).
+    da_status search_scan(const T *Q, da_int n_queries, da_int k, da_int n_probe, T *dist, int *ind);
+    da_status prepare_tiles(bool &ready);
+    da_status search_tiles(const T *Q, da_int n_queries, da_int k, da_int n_probe, int64_t ld,
+                           T *dist, int *ind);
+    da_status coarse(const T *Q, int rows, da_int n_probe);
     da_status upload_rows(const T *X, da_int n, da_int ld, DeviceBuffer &dst, size_t offset_rows);
 
     // Training data (the caller's pointer, as the reference keeps it; a loaded model points
@@ -50,6 +58,12 @@ template <typename T> class ApproxNNHandle : public AlgHandle {
     // Buffers of the MFMA assignment of added vectors: padded rows, padded centroids and
     // their -|c|^2/2, counters, the re-check list and the transposed centroids.
     DeviceBuffer as_x_, as_c_, as_h_, as_small_, as_list_, as_ct_;
+    // Matrix-core search: operand rows of the lists, rebuilt by the first search after a change of
+    // the index (0 none, 1 usable, 2 the data do not fit), and the workspaces of a query block.
+    int tiles_state_ = 0;
+    std::vector<int> tile_off_;
+    DeviceBuffer tile_off_d_, tile_map_, tile_op_, tile_h_, tile_mu_, tile_sc_, tile_q_, tile_err_,
+        tile_scores_, tile_work_, fb_, fb_q_, fb_ind_, fb_dist_;
     DeviceBuffer C_d_, X_d_, X_spare_, perm_d_, off_d_, q_d_, q_stage_, ckeys_, probe_key_,
         probe_d_, seg_d_, cand_key_, cand_idx_, sel_key_, sel_idx_, out_ind_, out_dist_, lab_d_,
         cdouble_d_;

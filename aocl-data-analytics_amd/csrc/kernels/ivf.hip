@@ -11,6 +11,7 @@
 // Keys: the squared euclidean distance, or for the inner-product and cosine metrics (IP)
 // the negated dot product -q.x (the reference's GEMM with alpha = -1, approximate_neighbors.cpp
 // :1145-1151), so that the smallest key is the nearest vector for every metric.
+#include "ivf_keys.hpp"
 #include "launch.hpp"
 #include <climits>
 #include <type_traits>
@@ -67,41 +68,6 @@ __global__ __launch_bounds__(256) void ivf_scan_kernel(
         }
     }
 }
-
-// 16-byte chunks of a row: four floats or two doubles. acc adds the squared differences of
-// a chunk's elements in element order, dot their products.
-template <typename T> struct Chunk16;
-template <> struct Chunk16<float> {
-    using type = float4;
-    __device__ static type zero() { return make_float4(0.f, 0.f, 0.f, 0.f); }
-    __device__ static void acc(double &a, const type &q, const type &x) {
-        const double t0 = (double)q.x - (double)x.x, t1 = (double)q.y - (double)x.y;
-        const double t2 = (double)q.z - (double)x.z, t3 = (double)q.w - (double)x.w;
-        a += t0 * t0;
-        a += t1 * t1;
-        a += t2 * t2;
-        a += t3 * t3;
-    }
-    __device__ static void dot(double &a, const type &q, const type &x) {
-        a += (double)q.x * (double)x.x;
-        a += (double)q.y * (double)x.y;
-        a += (double)q.z * (double)x.z;
-        a += (double)q.w * (double)x.w;
-    }
-};
-template <> struct Chunk16<double> {
-    using type = double2;
-    __device__ static type zero() { return make_double2(0.0, 0.0); }
-    __device__ static void acc(double &a, const type &q, const type &x) {
-        const double t0 = q.x - x.x, t1 = q.y - x.y;
-        a += t0 * t0;
-        a += t1 * t1;
-    }
-    __device__ static void dot(double &a, const type &q, const type &x) {
-        a += q.x * x.x;
-        a += q.y * x.y;
-    }
-};
 
 // The same scan for rows of whole 16-byte chunks (dc chunks, at most 8 * NJ): eight lanes
 // share a vector and read it chunk by chunk (lane s takes chunks s, s + 8, ...), so a wave
@@ -235,11 +201,9 @@ static hipError_t ivf_scan_dispatch(const T *Q, int nq, int n_probe, int d, cons
     if (pairs <= 0)
         return hipSuccess;
     const dim3 grid((unsigned)((pairs + 3) / 4));
-    // Rows of whole 16-byte chunks (d a multiple of 4 for fp32, of 2 for fp64; the buffers
-    // are allocated 256-byte aligned), at most 128 elements, take the chunked scan.
     constexpr int per = 16 / (int)sizeof(T);
     const int dc = d / per;
-    if (d % per == 0 && d <= 128) {
+    if (ivf_chunked<T>(d)) {
         auto run = [&](auto kern) {
             hipLaunchKernelGGL(kern, grid, dim3(256), 0, s, Q, nq, n_probe, dc, X, perm,
                                list_off, probes, seg, ld, keys, idx);

@@ -22,6 +22,8 @@
 #include "launch.hpp"
 #include <algorithm>
 #include <climits>
+#include <cmath>
+#include <limits>
 #include <hip/hip_runtime.h>
 
 namespace dagpu {
@@ -86,17 +88,20 @@ __global__ __launch_bounds__(256) void wide_range_kernel(const T *__restrict__ X
     }
 }
 
-// Centre and scale (one workgroup). Cosine: no centre, unit rows scaled to 2^14.
+// Centre and scale (one workgroup). Cosine: no centre, unit rows scaled to 2^14; inner product: no
+// centre, the scale from the largest magnitude. kmax > 0: the largest value of the type that keys
+// are rounded to; data whose keys could exceed it are marked bad.
 __global__ __launch_bounds__(256) void wide_scale_kernel(const unsigned long long *range, int d,
-                                                         int cosine, double *mu, WideScale *sc) {
+                                                         int mode, double kmax, double *mu,
+                                                         WideScale *sc) {
     __shared__ double half[256], big[256];
     const int t = threadIdx.x;
     double h = 0.0, a = 0.0;
     for (int l = t; l < d; l += 256) {
         double m = 0.0;
-        if (!cosine && range[2 * l] <= range[2 * l + 1]) {
+        if (mode != WIDE_COSINE && range[2 * l] <= range[2 * l + 1]) {
             const double lo = wide_value(range[2 * l]), hi = wide_value(range[2 * l + 1]);
-            m = lo + 0.5 * (hi - lo);
+            m = mode == WIDE_INNER ? 0.0 : lo + 0.5 * (hi - lo);
             h = fmax(h, fmax(hi - m, m - lo));
             a = fmax(a, fmax(fabs(lo), fabs(hi)));
         }
@@ -114,14 +119,15 @@ __global__ __launch_bounds__(256) void wide_scale_kernel(const unsigned long lon
     }
     if (t == 0) {
         double s = 16384.0, b = 0.0;
-        if (!cosine) {
+        if (mode != WIDE_COSINE) {
             int E = 15;
             if (half[0] > 0.0)
                 (void)frexp(half[0], &E);
             E = E < -200 ? -200 : (E > 200 ? 200 : E);
             s = ldexp(1.0, 15 - E); // training values stay below 2^15 (for E <= 200)
             b = big[0];
-            if (!(b < 1e60))
+            // Queries reach twice the training range, so keys stay below 9 d half^2.
+            if (!(b < 1e60) || (kmax > 0.0 && !(16.0 * d * half[0] * half[0] < kmax)))
                 sc->bad = 1;
         }
         sc->scale = s;
@@ -135,18 +141,23 @@ __global__ __launch_bounds__(256) void wide_scale_kernel(const unsigned long lon
 // one wave each the pass took 74 us).
 // Training rows: h[row] = |y'|^2/2 (0 for cosine) and the largest |y'|^2; query rows: the error
 // bound err[row] of their scores, +inf where a value is not finite or exceeds fp16's range.
-template <typename T>
+// map: row i is row map[i] of X, -1 for padding (h = +inf). ROWWISE: [row][k step][hi, lo][32]
+// instead of tiles, for kernels that gather rows. quantum: the rounding of keys below the normal
+// range of the type they are rounded to.
+template <typename T, bool ROWWISE>
 __global__ __launch_bounds__(1024) void wide_pack_kernel(
     const T *__restrict__ X, int rows, int d, int KS, const double *__restrict__ mu,
-    WideScale *sc, const double *__restrict__ cosn, double ce, _Float16 *__restrict__ P,
+    WideScale *sc, const double *__restrict__ cosn, const int *__restrict__ map, int mode,
+    double ce, double quantum, _Float16 *__restrict__ P,
     float *__restrict__ h, float *__restrict__ err) {
     __shared__ double rn[16][16], rb[16][16], rt[16][16];
     __shared__ int rf[16][16];
     const int t = blockIdx.x, w = threadIdx.x >> 6, nw = blockDim.x >> 6;
     const int lane = threadIdx.x & 63, r = lane & 15, g = lane >> 4;
     const int row = t * 16 + r;
+    const int src = row < rows ? (map ? map[row] : row) : -1;
     const double s = sc->scale;
-    const double inv = (cosn && row < rows) ? 1.0 / cosn[row] : 1.0;
+    const double inv = (cosn && src >= 0) ? 1.0 / cosn[src] : 1.0;
     double nn = 0.0, big = 0.0, top = 0.0;
     bool nf = false;
     for (int ks = w; ks < KS; ks += nw) {
@@ -155,8 +166,8 @@ __global__ __launch_bounds__(1024) void wide_pack_kernel(
         for (int e = 0; e < 8; e++) {
             const int l = ks * 32 + g * 8 + e;
             double v = 0.0;
-            if (row < rows && l < d) {
-                const double x = (double)X[(int64_t)row * d + l];
+            if (src >= 0 && l < d) {
+                const double x = (double)X[(int64_t)src * d + l];
                 v = (x - mu[l]) * inv * s;
                 big = fmax(big, fabs(x));
             }
@@ -167,9 +178,10 @@ __global__ __launch_bounds__(1024) void wide_pack_kernel(
             lo[e] = (_Float16)(float)(v - (double)(float)hv);
             nn = fma(v, v, nn);
         }
-        _Float16 *dst = P + ((int64_t)t * KS + ks) * 1024 + lane * 8;
+        _Float16 *dst = ROWWISE ? P + ((int64_t)row * KS + ks) * 64 + g * 8
+                                : P + ((int64_t)t * KS + ks) * 1024 + lane * 8;
         *reinterpret_cast<v8h *>(dst) = hi;
-        *reinterpret_cast<v8h *>(dst + 512) = lo;
+        *reinterpret_cast<v8h *>(dst + (ROWWISE ? 32 : 512)) = lo;
     }
 #pragma unroll
     for (int o = 16; o <= 32; o <<= 1) {
@@ -195,19 +207,27 @@ __global__ __launch_bounds__(1024) void wide_pack_kernel(
     }
     const bool fits = !nf && top < 60000.0;
     if (h) {
-        h[row] = cosn ? 0.0f : (float)(0.5 * nn);
-        if (row < rows) {
-            atomicMax(&sc->ymax2, (unsigned long long)__double_as_longlong(fits ? nn : 0.0));
-            if (!fits)
-                atomicOr(&sc->bad, 1);
-        }
+        h[row] = map && src < 0          ? __builtin_huge_valf()
+                 : mode == WIDE_EUCLIDEAN ? (float)(0.5 * nn)
+                                          : 0.0f;
+        double top2 = fits ? nn : 0.0;
+#pragma unroll
+        for (int o = 1; o < 16; o <<= 1)
+            top2 = fmax(top2, __shfl_xor(top2, o, 16));
+        if (r == 0)
+            atomicMax(&sc->ymax2, (unsigned long long)__double_as_longlong(top2));
+        if (!fits)
+            atomicOr(&sc->bad, 1);
     }
     if (err) {
         const double y2 = __longlong_as_double((long long)sc->ymax2);
         // Centring: the double rounding of x - mu, relative to the larger of the two.
         const double alpha = ldexp(1.0, -24) +
                              (cosn ? ldexp(1.0, -50) * s : s * ldexp(1.0, -51) * (big + sc->big));
-        const double E = 0.5 * ce * (nn + y2) + 2.0 * alpha * sqrt((double)d) * (sqrt(nn) + sqrt(y2));
+        // Inner product: queries and rows may differ in magnitude, so the product of the norms.
+        const double p2 = mode == WIDE_INNER ? sqrt(nn) * sqrt(y2) : 0.5 * (nn + y2);
+        const double E = ce * p2 + 2.0 * alpha * sqrt((double)d) * (sqrt(nn) + sqrt(y2)) +
+                         s * s * quantum;
         err[row] = fits ? (float)(E * (1.0 + 1e-6)) : __builtin_huge_valf();
     }
 }
@@ -400,24 +420,34 @@ __global__ __launch_bounds__(64) void wide_merge_kernel(
 
 } // namespace
 
-double wide_relative_bound() {
-    const double terms = 3.0 * 256 + 16, u = 1.0 / 16777216.0;
+double wide_relative_bound(int products) {
+    const double terms = products + 16.0, u = 1.0 / 16777216.0;
     return 1.05 * terms * u / (1.0 - terms * u) + 1.0 / 262144.0;
+}
+
+template <typename T>
+static void wide_prepare(const T *Y, int n, int d, int mode, const double *ycos, const int *map,
+                         int rows, int tiles, double kmax, unsigned long long *range, double *mu,
+                         WideScale *sc, void *P, float *h, hipStream_t s) {
+    const int KS = wide_ksteps(d);
+    hipLaunchKernelGGL(wide_range_init_kernel, dim3((d + 255) / 256), dim3(256), 0, s, range, d, sc);
+    if (mode != WIDE_COSINE) {
+        const int by = std::min(d > 512 ? 128 : 512, (n + 63) / 64);
+        hipLaunchKernelGGL(wide_range_kernel<T>, dim3((d + 63) / 64, by), dim3(256), 0, s, Y, n, d,
+                           range, sc);
+    }
+    hipLaunchKernelGGL(wide_scale_kernel, dim3(1), dim3(256), 0, s, range, d, mode, kmax, mu, sc);
+    hipLaunchKernelGGL((wide_pack_kernel<T, false>), dim3(tiles), dim3(64 * std::min(16, KS)), 0, s,
+                       Y, rows, d, KS, mu, sc, ycos, map, mode, 0.0, 0.0,
+                       static_cast<_Float16 *>(P), h, (float *)nullptr);
 }
 
 template <typename T>
 hipError_t launch_wide_prepare(const T *Y, int n, int d, const double *ycos,
                                unsigned long long *range, double *mu, WideScale *sc, void *P,
                                float *h, hipStream_t s) {
-    const int KS = wide_ksteps(d), tiles = wide_rows(n) / 16;
-    hipLaunchKernelGGL(wide_range_init_kernel, dim3((d + 255) / 256), dim3(256), 0, s, range, d, sc);
-    if (!ycos)
-        hipLaunchKernelGGL(wide_range_kernel<T>,
-                           dim3((d + 63) / 64, std::min(128, (n + 63) / 64)), dim3(256), 0, s, Y, n,
-                           d, range, sc);
-    hipLaunchKernelGGL(wide_scale_kernel, dim3(1), dim3(256), 0, s, range, d, ycos ? 1 : 0, mu, sc);
-    hipLaunchKernelGGL(wide_pack_kernel<T>, dim3(tiles), dim3(64 * std::min(16, KS)), 0, s, Y, n, d,
-                       KS, mu, sc, ycos, 0.0, static_cast<_Float16 *>(P), h, nullptr);
+    wide_prepare<T>(Y, n, d, ycos ? WIDE_COSINE : WIDE_EUCLIDEAN, ycos, nullptr, n,
+                    wide_rows(n) / 16, 0.0, range, mu, sc, P, h, s);
     return hipGetLastError();
 }
 
@@ -425,9 +455,35 @@ template <typename T>
 hipError_t launch_wide_queries(const T *Q, int nq, int d, const double *qcos, const double *mu,
                                WideScale *sc, void *P, float *err, hipStream_t s) {
     const int KS = wide_ksteps(d), tiles = wide_rows(nq) / 16;
-    hipLaunchKernelGGL(wide_pack_kernel<T>, dim3(tiles), dim3(64 * std::min(16, KS)), 0, s, Q, nq, d,
-                       KS, mu, sc, qcos, wide_relative_bound(), static_cast<_Float16 *>(P),
-                       nullptr, err);
+    hipLaunchKernelGGL((wide_pack_kernel<T, false>), dim3(tiles), dim3(64 * std::min(16, KS)), 0, s,
+                       Q, nq, d, KS, mu, sc, qcos, (const int *)nullptr,
+                       qcos ? WIDE_COSINE : WIDE_EUCLIDEAN, wide_relative_bound(3 * 256), 0.0,
+                       static_cast<_Float16 *>(P), (float *)nullptr, err);
+    return hipGetLastError();
+}
+
+template <typename T>
+hipError_t launch_ivf_lists(const T *X, int n, int d, int ip, const int *map, int rows,
+                            unsigned long long *range, double *mu, WideScale *sc, void *P, float *h,
+                            hipStream_t s) {
+    wide_prepare<T>(X, n, d, ip ? WIDE_INNER : WIDE_EUCLIDEAN, nullptr, map, rows, rows / 16,
+                    (double)std::numeric_limits<T>::max(), range, mu, sc, P, h, s);
+    return hipGetLastError();
+}
+
+template <typename T>
+hipError_t launch_ivf_queries(const T *Q, int nq, int d, int ip, const double *mu, WideScale *sc,
+                              void *P, float *err, hipStream_t s) {
+    const int KS = wide_ksteps(d);
+    // Keys are rounded to T: relative 2^-24 (fp32) of at most 2 (|x'|^2 + |y'|^2), covered by the
+    // 2^-22 added to the relative bound, and the quantum below the normal range.
+    const double quantum = sizeof(T) == 4 ? std::ldexp(1.0, -149) : 0.0;
+    hipLaunchKernelGGL((wide_pack_kernel<T, true>), dim3((nq + 15) / 16),
+                       dim3(64 * std::min(16, KS)), 0, s, Q, nq, d, KS, mu, sc,
+                       (const double *)nullptr, (const int *)nullptr,
+                       ip ? WIDE_INNER : WIDE_EUCLIDEAN,
+                       wide_relative_bound(3 * 32 * KS) + 1.0 / 4194304.0, quantum,
+                       static_cast<_Float16 *>(P), (float *)nullptr, err);
     return hipGetLastError();
 }
 
@@ -461,6 +517,11 @@ hipError_t launch_wide_merge(const float *skey, const int *sidx, int nq, int kc,
     template hipError_t launch_wide_queries<T>(const T *, int, int, const double *,              \
                                                const double *, WideScale *, void *, float *,     \
                                                hipStream_t);                                     \
+    template hipError_t launch_ivf_lists<T>(const T *, int, int, int, const int *, int,          \
+                                            unsigned long long *, double *, WideScale *, void *, \
+                                            float *, hipStream_t);                               \
+    template hipError_t launch_ivf_queries<T>(const T *, int, int, int, const double *,          \
+                                              WideScale *, void *, float *, hipStream_t);        \
     template hipError_t launch_wide_merge<T>(const float *, const int *, int, int, int, int,     \
                                              const T *, const T *, int, const float *,           \
                                              const double *, const double *, int, int, T *,      \

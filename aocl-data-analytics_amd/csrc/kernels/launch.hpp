@@ -329,6 +329,7 @@ hipError_t launch_dbscan_label(const long long *offs, const int *ind, const unsi
 // Scale of the operand rows, the largest training value as given, the bits of the largest
 // squared operand norm, and whether a training value is not finite or out of range (the general
 // path then serves the search).
+enum { WIDE_EUCLIDEAN = 0, WIDE_COSINE = 1, WIDE_INNER = 2 };
 struct WideScale {
     double scale, big;
     unsigned long long ymax2;
@@ -360,6 +361,45 @@ hipError_t launch_wide_merge(const float *skey, const int *sidx, int nq, int kc,
                              const T *Q, const T *Y, int d, const float *err, const double *qcos,
                              const double *ycos, int post, int q0, T *out_dist, int *out_idx,
                              int *fb_count, int *fb_list, hipStream_t s);
+// ---- IVF-Flat search on the matrix cores (operands knn_wide.hip, search ivf_mfma.hip) ----
+// Largest row width, neighbours and probes of that path.
+constexpr int IVF_TILE_D = 128, IVF_TILE_K = 128, IVF_TILE_PROBE = 1024;
+// List rows in tiles of 16: row i of the operand is X[map[i]], -1 for padding; rows is a multiple
+// of 16, h has rows floats. ip: inner product instead of the squared distance.
+template <typename T>
+hipError_t launch_ivf_lists(const T *X, int n, int d, int ip, const int *map, int rows,
+                            unsigned long long *range, double *mu, WideScale *sc, void *P, float *h,
+                            hipStream_t s);
+hipError_t launch_ivf_map(const int *perm, const int *list_off, const int *tile_off, int n_list,
+                          int *map, hipStream_t s);
+// Query rows (nq rounded up to 16) and the error bounds of their scores.
+template <typename T>
+hipError_t launch_ivf_queries(const T *Q, int nq, int d, int ip, const double *mu, WideScale *sc,
+                              void *P, float *err, hipStream_t s);
+struct IvfTiles {
+    const int *tile_off;  // n_list + 1: first tile of each list
+    const int *map;       // operand row -> vector
+    const void *op;       // list operand
+    const float *h;       // its constants
+    int n_list, n_probe, max_tiles;
+    // Per query block: probed lists in ascending order and their first columns (nq x n_probe),
+    // their places in their lists' groups, row lengths; per list counts, group offsets; the
+    // queries of each list (nq x n_probe), work items (ivf_items) and their number.
+    int *slist, *sseg, *place, *rowlen, *cnt, *qoff, *group;
+    int2 *items;
+    int *n_items;
+};
+inline int64_t ivf_items(int64_t pairs, int n_list) { return pairs / 128 + n_list; }
+// Scores of nq queries (operand QP) against their probed lists (probes: nq x n_probe, distinct) into
+// rows of ld floats (a multiple of 16, at least the n_probe longest padded lists).
+hipError_t launch_ivf_tile_scores(const IvfTiles &p, const int *probes, const void *QP, int nq,
+                                  int d, float *out, int64_t ld, hipStream_t s);
+// The k best of each row by their exact keys, (key in T, column); uncertified queries are listed.
+template <typename T>
+hipError_t launch_ivf_tile_select(const IvfTiles &p, const float *scores, int64_t ld,
+                                  const float *err, const T *Q, const T *X, int nq, int d, int k,
+                                  int ip, int post, int q0, T *dist, int *ind, int *fb_count,
+                                  int *fb_list, hipStream_t s);
 // ---- Radius search on the matrix cores (radius_mfma.hip): a hit bit per pair ----
 // Metrics whose key is a function of the squared euclidean distance.
 bool radius_bits_metric(int metric);

@@ -1,0 +1,78 @@
+"""IVF-Flat search by matrix-core scores against the list scans, which serve k > 128: the scans'
+first k neighbours of a k = 129 search are the answer, bit for bit (both sum and round exact keys
+alike, ties by list and position)."""
+import numpy as np
+import pytest
+
+import aoclda
+
+pytestmark = pytest.mark.gpu
+
+
+def _check(ann, Q, ks, k_scan=129):
+    de, ie = ann.kneighbors(Q, n_neighbors=k_scan)
+    for k in ks:
+        dist, ind = ann.kneighbors(Q, n_neighbors=k)
+        np.testing.assert_array_equal(ind, ie[:, :k], err_msg=f"k {k}")
+        np.testing.assert_array_equal(dist, de[:, :k], err_msg=f"k {k}")
+
+
+@pytest.mark.parametrize("metric", ["sqeuclidean", "euclidean", "inner product", "cosine"])
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+@pytest.mark.parametrize("d", [1, 31, 32, 33, 64, 65, 96, 97, 127, 128])
+def test_same_as_scan(metric, dtype, d):
+    """One to four k steps and their edges; lists of one to several runs of tiles."""
+    rng = np.random.default_rng(d)
+    means = rng.uniform(-3, 3, (12, d))
+    X = (means[rng.integers(0, 12, 5003)] + rng.standard_normal((5003, d))).astype(dtype)
+    Q = (means[rng.integers(0, 12, 333)] + rng.standard_normal((333, d))).astype(dtype)
+    ann = aoclda.neighbors.approximate_neighbors(n_list=17, n_probe=5, metric=metric,
+                                                 kmeans_iter=3, seed=1).train_and_add(X)
+    _check(ann, Q, (1, 10, 128))
+
+
+@pytest.mark.parametrize("nq", [1, 15, 16, 17, 128, 129, 700])
+@pytest.mark.parametrize("n,n_list,n_probe", [(300, 200, 200), (300, 200, 3), (4096, 1, 1),
+                                              (9000, 3, 2)])
+def test_groups(nq, n, n_list, n_probe):
+    """Groups of one to several hundred queries; lists shorter than a tile, empty, longer than a
+    run; fewer vectors than k in the probed lists (index -1)."""
+    rng = np.random.default_rng(nq)
+    X = rng.standard_normal((n, 20)).astype(np.float32)
+    Q = rng.standard_normal((nq, 20)).astype(np.float32)
+    ann = aoclda.neighbors.approximate_neighbors(n_list=n_list, n_probe=n_probe, kmeans_iter=2,
+                                                 seed=1).train_and_add(X)
+    _check(ann, Q, (1, 33, 128))
+
+
+@pytest.mark.parametrize("metric", ["sqeuclidean", "inner product"])
+def test_ties_and_added_copies(metric):
+    """Equal keys keep list and position order: integer rows, each added three times, so that up
+    to hundreds of keys tie; more than 1,024 equal rows go to the scan."""
+    rng = np.random.default_rng(5)
+    X = rng.integers(0, 3, (2000, 6)).astype(np.float32)
+    ann = aoclda.neighbors.approximate_neighbors(n_list=8, n_probe=4, metric=metric, kmeans_iter=3,
+                                                 seed=2).train_and_add(X)
+    Q = rng.integers(0, 3, (90, 6)).astype(np.float32)
+    _check(ann, Q, (1, 50, 128))
+    ann.add(X)
+    ann.add(np.repeat(X[:1], 1500, axis=0))
+    _check(ann, np.concatenate([Q, X[:1]]), (1, 50, 128))
+
+
+@pytest.mark.parametrize("dtype,scale", [(np.float32, 1e-25), (np.float32, 1e18),
+                                         (np.float64, 1e-150), (np.float64, 1e70),
+                                         (np.float32, 1e-3)])
+@pytest.mark.parametrize("metric", ["sqeuclidean", "inner product"])
+def test_ranges(dtype, scale, metric):
+    """Keys that round to zero or overflow in the type, and queries far outside the data's range
+    beside ordinary ones."""
+    rng = np.random.default_rng(9)
+    X = (rng.standard_normal((3000, 24)) * scale).astype(dtype)
+    Q = (rng.standard_normal((40, 24)) * scale).astype(dtype)
+    Q[3] *= dtype(100)
+    Q[7] *= dtype(1e-6)
+    Q[11] = 0
+    ann = aoclda.neighbors.approximate_neighbors(n_list=10, n_probe=4, metric=metric, kmeans_iter=2,
+                                                 seed=1).train_and_add(X)
+    _check(ann, Q, (1, 10, 128))
