@@ -11,6 +11,7 @@
 // fp16's range is listed for the scan.
 #include "ivf_keys.hpp"
 #include "launch.hpp"
+#include "wave_rank.hpp"
 #include <algorithm>
 #include <climits>
 #include <hip/hip_runtime.h>
@@ -225,7 +226,7 @@ __global__ __launch_bounds__(256) void ivf_tile_select_kernel(
     const T *__restrict__ Q, const T *__restrict__ X, int d, int k, int post, int q0,
     T *__restrict__ dist, int *__restrict__ ind, int *__restrict__ fb_count,
     int *__restrict__ fb_list) {
-    __shared__ float mins[256];
+    __shared__ __attribute__((aligned(16))) float mins[256];
     __shared__ float bound;
     __shared__ int kept;
     __shared__ T xk[IVF_KEEP];
@@ -249,14 +250,13 @@ __global__ __launch_bounds__(256) void ivf_tile_select_kernel(
     if (t == 0)
         kept = 0;
     __syncthreads();
-    int rank = 0;
-#pragma unroll 8
-    for (int o = 0; o < 256; o++) {
-        const float mo = mins[o];
-        rank += mo < m || (mo == m && o < t);
+    if (t < 64) {
+        const float4 m4 = reinterpret_cast<const float4 *>(mins)[t];
+        const float v[4] = {m4.x, m4.y, m4.z, m4.w};
+        const float kth = wave_rank_256(v, k);
+        if (t == 0)
+            bound = __double2float_ru((double)kth + 2.0 * (double)E);
     }
-    if (rank == k - 1)
-        bound = __double2float_ru((double)m + 2.0 * (double)E);
     __syncthreads();
     const float lim = bound;
     auto take = [&](float v, int c) {

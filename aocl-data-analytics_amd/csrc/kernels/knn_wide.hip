@@ -141,15 +141,17 @@ __global__ __launch_bounds__(256) void wide_scale_kernel(const unsigned long lon
 // one wave each the pass took 74 us).
 // Training rows: h[row] = |y'|^2/2 (0 for cosine) and the largest |y'|^2; query rows: the error
 // bound err[row] of their scores, +inf where a value is not finite or exceeds fp16's range.
-// map: row i is row map[i] of X, -1 for padding (h = +inf). ROWWISE: [row][k step][hi, lo][32]
-// instead of tiles, for kernels that gather rows. quantum: the rounding of keys below the normal
-// range of the type they are rounded to.
-template <typename T, bool ROWWISE>
+// map: row i is row map[i] of X, -1 for padding (h = +inf). quantum: the rounding of keys below the
+// normal range of the type they are rounded to. FORM PACK_ROWS: [row][k step][hi, lo][32] instead of
+// tiles, for kernels that gather rows; PACK_HI: tiles of hi only, h = |y'|^2/2 (1 - ce), +inf for
+// padding. nrm: |x'|^2 of query rows, +inf where they do not fit.
+enum { PACK_TILES = 0, PACK_ROWS = 1, PACK_HI = 2 };
+template <typename T, int FORM>
 __global__ __launch_bounds__(1024) void wide_pack_kernel(
     const T *__restrict__ X, int rows, int d, int KS, const double *__restrict__ mu,
     WideScale *sc, const double *__restrict__ cosn, const int *__restrict__ map, int mode,
     double ce, double quantum, _Float16 *__restrict__ P,
-    float *__restrict__ h, float *__restrict__ err) {
+    float *__restrict__ h, float *__restrict__ err, double *__restrict__ nrm) {
     __shared__ double rn[16][16], rb[16][16], rt[16][16];
     __shared__ int rf[16][16];
     const int t = blockIdx.x, w = threadIdx.x >> 6, nw = blockDim.x >> 6;
@@ -178,10 +180,14 @@ __global__ __launch_bounds__(1024) void wide_pack_kernel(
             lo[e] = (_Float16)(float)(v - (double)(float)hv);
             nn = fma(v, v, nn);
         }
-        _Float16 *dst = ROWWISE ? P + ((int64_t)row * KS + ks) * 64 + g * 8
-                                : P + ((int64_t)t * KS + ks) * 1024 + lane * 8;
-        *reinterpret_cast<v8h *>(dst) = hi;
-        *reinterpret_cast<v8h *>(dst + (ROWWISE ? 32 : 512)) = lo;
+        if constexpr (FORM == PACK_HI) {
+            *reinterpret_cast<v8h *>(P + ((int64_t)t * KS + ks) * 512 + lane * 8) = hi;
+        } else {
+            _Float16 *dst = FORM == PACK_ROWS ? P + ((int64_t)row * KS + ks) * 64 + g * 8
+                                              : P + ((int64_t)t * KS + ks) * 1024 + lane * 8;
+            *reinterpret_cast<v8h *>(dst) = hi;
+            *reinterpret_cast<v8h *>(dst + (FORM == PACK_ROWS ? 32 : 512)) = lo;
+        }
     }
 #pragma unroll
     for (int o = 16; o <= 32; o <<= 1) {
@@ -207,7 +213,8 @@ __global__ __launch_bounds__(1024) void wide_pack_kernel(
     }
     const bool fits = !nf && top < 60000.0;
     if (h) {
-        h[row] = map && src < 0          ? __builtin_huge_valf()
+        h[row] = (map || FORM == PACK_HI) && src < 0 ? __builtin_huge_valf()
+                 : FORM == PACK_HI                   ? (float)(0.5 * nn * (1.0 - ce))
                  : mode == WIDE_EUCLIDEAN ? (float)(0.5 * nn)
                                           : 0.0f;
         double top2 = fits ? nn : 0.0;
@@ -219,6 +226,8 @@ __global__ __launch_bounds__(1024) void wide_pack_kernel(
         if (!fits)
             atomicOr(&sc->bad, 1);
     }
+    if (nrm)
+        nrm[row] = src >= 0 && fits ? nn : __builtin_huge_val();
     if (err) {
         const double y2 = __longlong_as_double((long long)sc->ymax2);
         // Centring: the double rounding of x - mu, relative to the larger of the two.
@@ -425,7 +434,7 @@ double wide_relative_bound(int products) {
     return 1.05 * terms * u / (1.0 - terms * u) + 1.0 / 262144.0;
 }
 
-template <typename T>
+template <typename T, int FORM = PACK_TILES>
 static void wide_prepare(const T *Y, int n, int d, int mode, const double *ycos, const int *map,
                          int rows, int tiles, double kmax, unsigned long long *range, double *mu,
                          WideScale *sc, void *P, float *h, hipStream_t s) {
@@ -437,9 +446,9 @@ static void wide_prepare(const T *Y, int n, int d, int mode, const double *ycos,
                            range, sc);
     }
     hipLaunchKernelGGL(wide_scale_kernel, dim3(1), dim3(256), 0, s, range, d, mode, kmax, mu, sc);
-    hipLaunchKernelGGL((wide_pack_kernel<T, false>), dim3(tiles), dim3(64 * std::min(16, KS)), 0, s,
+    hipLaunchKernelGGL((wide_pack_kernel<T, FORM>), dim3(tiles), dim3(64 * std::min(16, KS)), 0, s,
                        Y, rows, d, KS, mu, sc, ycos, map, mode, 0.0, 0.0,
-                       static_cast<_Float16 *>(P), h, (float *)nullptr);
+                       static_cast<_Float16 *>(P), h, (float *)nullptr, (double *)nullptr);
 }
 
 template <typename T>
@@ -455,10 +464,37 @@ template <typename T>
 hipError_t launch_wide_queries(const T *Q, int nq, int d, const double *qcos, const double *mu,
                                WideScale *sc, void *P, float *err, hipStream_t s) {
     const int KS = wide_ksteps(d), tiles = wide_rows(nq) / 16;
-    hipLaunchKernelGGL((wide_pack_kernel<T, false>), dim3(tiles), dim3(64 * std::min(16, KS)), 0, s,
+    hipLaunchKernelGGL((wide_pack_kernel<T, PACK_TILES>), dim3(tiles), dim3(64 * std::min(16, KS)), 0, s,
                        Q, nq, d, KS, mu, sc, qcos, (const int *)nullptr,
                        qcos ? WIDE_COSINE : WIDE_EUCLIDEAN, wide_relative_bound(3 * 256), 0.0,
-                       static_cast<_Float16 *>(P), (float *)nullptr, err);
+                       static_cast<_Float16 *>(P), (float *)nullptr, err, (double *)nullptr);
+    return hipGetLastError();
+}
+
+template <typename T>
+hipError_t launch_bits_prepare(const T *Y, int n, int d, double ce, const int *smap, int ns,
+                               unsigned long long *range, double *mu, WideScale *sc, void *PS,
+                               float *hS, void *P, float *B, hipStream_t s) {
+    const int KS = wide_ksteps(d);
+    // The sample's operand first: it leaves the centre and scale; the whole set's pass leaves the
+    // largest norm.
+    wide_prepare<T, PACK_HI>(Y, n, d, WIDE_EUCLIDEAN, nullptr, smap, ns, ns / 16, 0.0, range, mu, sc, PS, hS,
+                    s);
+    hipLaunchKernelGGL((wide_pack_kernel<T, PACK_HI>), dim3(bits_rows(n) / 16), dim3(64 * KS), 0, s,
+                       Y, n, d, KS, mu, sc, (const double *)nullptr, (const int *)nullptr,
+                       WIDE_EUCLIDEAN, ce, 0.0, static_cast<_Float16 *>(P), B, (float *)nullptr,
+                       (double *)nullptr);
+    return hipGetLastError();
+}
+
+template <typename T>
+hipError_t launch_bits_queries(const T *Q, int nq, int d, const double *mu, WideScale *sc, void *P,
+                               double *nrm, hipStream_t s) {
+    const int KS = wide_ksteps(d);
+    hipLaunchKernelGGL((wide_pack_kernel<T, PACK_HI>), dim3((nq + 255) / 256 * 16),
+                       dim3(64 * KS), 0, s, Q, nq, d, KS, mu, sc, (const double *)nullptr,
+                       (const int *)nullptr, WIDE_EUCLIDEAN, 0.0, 0.0, static_cast<_Float16 *>(P),
+                       (float *)nullptr, (float *)nullptr, nrm);
     return hipGetLastError();
 }
 
@@ -478,12 +514,12 @@ hipError_t launch_ivf_queries(const T *Q, int nq, int d, int ip, const double *m
     // Keys are rounded to T: relative 2^-24 (fp32) of at most 2 (|x'|^2 + |y'|^2), covered by the
     // 2^-22 added to the relative bound, and the quantum below the normal range.
     const double quantum = sizeof(T) == 4 ? std::ldexp(1.0, -149) : 0.0;
-    hipLaunchKernelGGL((wide_pack_kernel<T, true>), dim3((nq + 15) / 16),
+    hipLaunchKernelGGL((wide_pack_kernel<T, PACK_ROWS>), dim3((nq + 15) / 16),
                        dim3(64 * std::min(16, KS)), 0, s, Q, nq, d, KS, mu, sc,
                        (const double *)nullptr, (const int *)nullptr,
                        ip ? WIDE_INNER : WIDE_EUCLIDEAN,
                        wide_relative_bound(3 * 32 * KS) + 1.0 / 4194304.0, quantum,
-                       static_cast<_Float16 *>(P), (float *)nullptr, err);
+                       static_cast<_Float16 *>(P), (float *)nullptr, err, (double *)nullptr);
     return hipGetLastError();
 }
 
@@ -517,6 +553,11 @@ hipError_t launch_wide_merge(const float *skey, const int *sidx, int nq, int kc,
     template hipError_t launch_wide_queries<T>(const T *, int, int, const double *,              \
                                                const double *, WideScale *, void *, float *,     \
                                                hipStream_t);                                     \
+    template hipError_t launch_bits_prepare<T>(const T *, int, int, double, const int *, int,    \
+                                               unsigned long long *, double *, WideScale *,      \
+                                               void *, float *, void *, float *, hipStream_t);   \
+    template hipError_t launch_bits_queries<T>(const T *, int, int, const double *, WideScale *, \
+                                               void *, double *, hipStream_t);                   \
     template hipError_t launch_ivf_lists<T>(const T *, int, int, int, const int *, int,          \
                                             unsigned long long *, double *, WideScale *, void *, \
                                             float *, hipStream_t);                               \

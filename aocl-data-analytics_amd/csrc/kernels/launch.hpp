@@ -361,6 +361,43 @@ hipError_t launch_wide_merge(const float *skey, const int *sidx, int nq, int kc,
                              const T *Q, const T *Y, int d, const float *err, const double *qcos,
                              const double *ycos, int post, int q0, T *out_dist, int *out_idx,
                              int *fb_count, int *fb_list, hipStream_t s);
+// ---- kNN by hit bits (operands knn_wide.hip, search knn_bits.hip) ----
+constexpr int BITS_D = 128, BITS_K = 128, BITS_KEEP = 2048;
+inline int bits_rows(int n) { return (n + 511) / 512 * 512; }
+// Relative part of the error bound of the sweep's products.
+double bits_relative_bound(int d);
+// Rank taken in the sample of ns of n rows for k neighbours.
+int bits_rank(int k, int64_t n, int ns);
+// Sample operand PS, hS (row i is Y[smap[i]]; ns a multiple of BITS_SAMPLE), sweep operand P
+// (bits_rows(n) rows of 64 wide_ksteps(d) bytes, as PS) and thresholds B.
+constexpr int BITS_SAMPLE = 1024;
+template <typename T>
+hipError_t launch_bits_prepare(const T *Y, int n, int d, double ce, const int *smap, int ns,
+                               unsigned long long *range, double *mu, WideScale *sc, void *PS,
+                               float *hS, void *P, float *B, hipStream_t s);
+// Query operand (nq rounded up to 256 rows) and squared norms.
+template <typename T>
+hipError_t launch_bits_queries(const T *Q, int nq, int d, const double *mu, WideScale *sc, void *P,
+                               double *nrm, hipStream_t s);
+// mins: 256 minima per query of its scores against groups of ns / 256 sample rows.
+hipError_t launch_bits_sample(const void *PA, int nq, const void *PS, const float *hS, int ns, int d,
+                              float *mins, hipStream_t s);
+// Per query (nq rounded up to 256): threshold A of the sweep and the squared distance lim (scaled)
+// up to which it finds every row; hopeless queries are counted in *bad. Clears count[nq].
+hipError_t launch_bits_guess(const float *mins, int nq, int ns, int64_t n, int d, int rank,
+                             double ce, const double *nrm, const WideScale *sc, float *A,
+                             double *lim, int *bad, int *count, hipStream_t s);
+// bits: bits_rows(n) bits per query. Nothing is written if *bad > nq / 4.
+hipError_t launch_bits_sweep(const void *PA, int nq, const void *P, int n, int d, const float *A,
+                             const float *B, const int *bad, unsigned *bits, hipStream_t s);
+// Columns of the set bits: count[q] of them, the first BITS_KEEP in cols[q * BITS_KEEP].
+hipError_t launch_bits_columns(const unsigned *bits, int nq, int n, const int *bad, int *count,
+                               int *cols, hipStream_t s);
+template <typename T>
+hipError_t launch_bits_merge(const int *count, const int *cols, int nq, const int *bad, const T *Q,
+                             const T *Y, int d, int k, const double *lim, const WideScale *sc,
+                             int post, int q0, T *out_dist, int *out_idx, int *fb_count,
+                             int *fb_list, hipStream_t s);
 // ---- IVF-Flat search on the matrix cores (operands knn_wide.hip, search ivf_mfma.hip) ----
 // Largest row width, neighbours and probes of that path.
 constexpr int IVF_TILE_D = 128, IVF_TILE_K = 128, IVF_TILE_PROBE = 1024;

@@ -17,6 +17,7 @@ struct SearchParams {
     int variant = -1; // fused tile kernel variant (-1: tuning table)
     int kc_min = 0;   // minimum candidates kept per (query, split) on the fused tile
     bool automatic = false; // operand form and tile options as the library chooses
+    bool bits = false; // the search by hit bits may be used
     bool seed = false; // seed the fused tile's thresholds (group minima over a row sample)
     // Candidate-list length of the fused tile for k neighbours.
     int tile_kc(int k) const;
@@ -42,6 +43,9 @@ struct SearchContext {
     SearchParams last_params;
     std::unique_ptr<SearchContext> retry;
     bool second_pass = false;
+    // The last launch searched by hit bits; its workspaces.
+    bool by_bits = false;
+    DeviceBuffer bits_q, bits_nrm, bits_a, bits_lim, bits_mins, bits_count, bits_cols, bits;
     ~SearchContext();
 };
 
@@ -131,6 +135,14 @@ template <typename T> class NNHandle : public AlgHandle {
     da_status prepare_wide();
     da_status search_wide(SearchContext &ctx, const T *dQ, da_int nq, da_int k,
                           bool return_distance, da_int *d_ind, T *d_dist);
+    // Searches by hit bits (knn_bits.hip): the operands are laid out at the first search that uses
+    // them.
+    bool bits_eligible(const SearchParams &p, da_int nq, da_int k) const;
+    da_status prepare_bits();
+    da_status search_bits(SearchContext &ctx, const T *dQ, da_int nq, da_int k,
+                          bool return_distance, da_int *d_ind, T *d_dist);
+    int bits_state_ = 0, bits_sample_ = 0; // state as wide_state_; rows of the sample
+    DeviceBuffer bits_op_, bits_b_, bits_mu_, bits_sc_, bits_sop_, bits_sh_, bits_smap_;
     int wide_state_ = 0; // 0: not laid out, 1: ready, 2: the data need the general path
     int wide_cos_ = -1;  // metric of the layout: cosine or euclidean
     DeviceBuffer wide_op_, wide_h_, wide_mu_, wide_sc_;

@@ -1,0 +1,120 @@
+"""kNN by hit bits (large searches of up to 128 features, squared-euclidean metrics): bit for bit the
+neighbours of the fused tile (which serves a handle with a tile option set), and of the oracle."""
+import ctypes as C
+
+import numpy as np
+import pytest
+
+import aoclda
+from aoclda import _lib as L
+
+pytestmark = pytest.mark.gpu
+
+KEEP = 2048  # hits per query; reported as the candidates of such a search
+
+
+def _stats(nn):
+    nfb, ncand = L.da_int(), L.da_int()
+    L.check(L.lib.da_nn_last_query_stats(nn.handle.h, C.byref(nfb), C.byref(ncand)))
+    return nfb.value, ncand.value
+
+
+def _compare(X, Q, k, most_listed=None, **opts):
+    nn = aoclda.neighbors.nearest_neighbors(**opts).fit(X)
+    dist, ind = nn.kneighbors(Q, n_neighbors=k)
+    nfb, ncand = _stats(nn)
+    assert ncand == KEEP
+    if most_listed is not None:
+        assert nfb <= most_listed
+    tile = aoclda.neighbors.nearest_neighbors(seed_thresholds=False, **opts).fit(X)
+    de, ie = tile.kneighbors(Q, n_neighbors=k)
+    assert _stats(tile)[1] != KEEP
+    np.testing.assert_array_equal(ind, ie)
+    np.testing.assert_array_equal(dist, de)
+    return nfb
+
+
+def _mixture(rng, n, d, dtype, means):
+    return (means[rng.integers(0, len(means), n)] + rng.standard_normal((n, d))).astype(dtype)
+
+
+def _queries(n, d):
+    """Enough for the products from which searches take the hit bits, and ragged."""
+    return int(np.ceil(2**32 / (n * (d + 16)))) + 37
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+@pytest.mark.parametrize("d", [3, 31, 32, 33, 64, 65, 96, 97, 127, 128])
+def test_widths(dtype, d):
+    """One to four k steps and their edges; rows of whole 16-byte pieces and others."""
+    rng = np.random.default_rng(d)
+    means = rng.uniform(-10, 10, (16, d))
+    X = _mixture(rng, 20011, d, dtype, means)
+    Q = _mixture(rng, _queries(20011, d), d, dtype, means)
+    # fewer than one query in ten is left to the tile, except in the few dimensions where a
+    # cluster is dense against fp16's steps
+    _compare(X, Q, 10, most_listed=len(Q) // 10 if d >= 31 else None)
+
+
+@pytest.mark.parametrize("k", [1, 2, 20, 100, 128])
+@pytest.mark.parametrize("n", [16384, 16385, 65537, 140000])
+def test_sizes(n, k):
+    rng = np.random.default_rng(n + k)
+    means = rng.uniform(-10, 10, (8, 24))
+    X = _mixture(rng, n, 24, np.float32, means)
+    Q = _mixture(rng, _queries(n, 24), 24, np.float32, means)
+    _compare(X, Q, k)
+
+
+@pytest.mark.parametrize("precision", ["fp16", "fp16c", "bf16", "fp16x3"])
+@pytest.mark.parametrize("metric", ["euclidean", "sqeuclidean", "euclidean_gemm", "sqeuclidean_gemm"])
+def test_forms(precision, metric):
+    rng = np.random.default_rng(3)
+    means = rng.uniform(-10, 10, (8, 40))
+    X = _mixture(rng, 30000, 40, np.float32, means)
+    Q = _mixture(rng, 2600, 40, np.float32, means)
+    _compare(X, Q, 12, precision=precision, metric=metric)
+
+
+def test_difficult_queries():
+    """Duplicates (ties by index), queries equal to rows, far queries, a value outside fp16's range,
+    more equal rows than the merge holds."""
+    rng = np.random.default_rng(7)
+    means = rng.uniform(-10, 10, (8, 32))
+    X = _mixture(rng, 40000, 32, np.float32, means)
+    X[20000:20400] = X[:400]
+    X[30000:33000] = X[5]
+    Q = _mixture(rng, _queries(40000, 32), 32, np.float32, means)
+    Q[:500] = X[:500]
+    Q[600:620] *= 50
+    Q[700] = 1e6  # beyond fp16 at the data's scale, its keys still distinct in double
+    Q[701] = 0
+    assert _compare(X, Q, 9) > 0
+
+
+@pytest.mark.parametrize("scale,shift", [(1e-12, 0), (1e12, 0), (1e-3, 1e4)])
+def test_ranges_and_tight_clusters(scale, shift):
+    """Any magnitude; clusters so tight against their spread that fp16 cannot tell their rows apart
+    (the sample shows it and the tile serves the search)."""
+    rng = np.random.default_rng(11)
+    means = rng.uniform(-10, 10, (8, 20))
+    X = _mixture(rng, 30000, 20, np.float64, means) * scale + shift
+    Q = _mixture(rng, 4100, 20, np.float64, means) * scale + shift
+    _compare(X, Q, 5)
+    X = means[rng.integers(0, 8, 30000)] + 1e-4 * rng.standard_normal((30000, 20))
+    Q = means[rng.integers(0, 8, 4100)] + 1e-4 * rng.standard_normal((4100, 20))
+    assert _compare(X, Q, 5) == len(Q)
+
+
+def test_not_finite_rows():
+    """Rows that are not finite keep the search on the tile's path."""
+    rng = np.random.default_rng(13)
+    X = rng.standard_normal((20000, 20)).astype(np.float32)
+    X[77, 3] = 1e38
+    Q = rng.standard_normal((6100, 20)).astype(np.float32)
+    nn = aoclda.neighbors.nearest_neighbors().fit(X)
+    dist, ind = nn.kneighbors(Q, n_neighbors=5)
+    tile = aoclda.neighbors.nearest_neighbors(seed_thresholds=False).fit(X)
+    de, ie = tile.kneighbors(Q, n_neighbors=5)
+    np.testing.assert_array_equal(ind, ie)
+    np.testing.assert_array_equal(dist, de)
