@@ -16,19 +16,23 @@
 // too (euclidean_gemm_distance.cpp:59-230, cosine_distance.cpp:66-161,
 // inner_product_distance.cpp) and are stored as computed.
 //
-// Work decomposition: a 256-thread workgroup owns a 64 x 64 output tile, stages 16-deep k
-// slices of X and Y in LDS as double (transposed, as the direct tile does), and each wave
-// accumulates a 32 x 32 quarter as 2 x 2 blocks of 16 x 16 on the matrix cores. Operand
+// Work decomposition: a 256-thread workgroup owns a TB x TB output tile (TB = 128, or 64 where
+// fewer than 1,024 tiles of 128 would leave CUs idle), and each wave accumulates a quarter of it in
+// 16 x 16 blocks on the matrix cores. 16-deep k slices of X and Y lie in LDS in the input type
+// (widened when read) in two buffers: the next slice is loaded to registers before the products
+// of this one and stored after them, with one barrier a slice. Bound by the matrix cores (a product
+// occupies its SIMD for 64 cycles). 8,192 x 8,192 x 256 fp32: 675 us; with one buffer, a tile of
+// 64 and loads waited for between barriers 920. Operand
 // layout of v_mfma_f64_16x16x4f64 for lane l: A[l % 16][l / 16], B[l / 16][l % 16]; the
 // accumulator's register r holds C[4 r + l / 16][l % 16].
 #include "launch.hpp"
+#include <cstdint>
 #include <hip/hip_runtime.h>
 
 namespace dagpu {
 
 namespace {
 
-constexpr int TB = 64; // output tile edge
 constexpr int KC = 16; // k slice staged in LDS
 
 typedef double v4d __attribute__((ext_vector_type(4)));
@@ -43,71 +47,104 @@ __device__ double direct_sqdist(const T *__restrict__ x, const TY *__restrict__ 
     return acc;
 }
 
-template <typename T, typename TY, typename U, int METRIC>
-__global__ __launch_bounds__(256) void pairwise_mfma_kernel(
+// A thread's part of a TB x KC slice: VE consecutive k of TB * KC / (256 VE) rows. VE > 1 needs rows
+// of whole 16-byte pieces.
+template <typename T, int TB, int VE> struct Slice {
+    static constexpr int PER = KC / VE, ROWS = 256 / PER, N = TB / ROWS;
+    T v[N][VE];
+    __device__ __forceinline__ void load(const T *__restrict__ X, int i0, int m, int k, int k0,
+                                         int tid) {
+        const int kk = k0 + (tid % PER) * VE, row = tid / PER;
+#pragma unroll
+        for (int s = 0; s < N; s++) {
+            const int gi = i0 + row + s * ROWS;
+            const bool in = kk < k && gi < m;
+            if constexpr (VE > 1) {
+                uint4 u = make_uint4(0, 0, 0, 0);
+                if (in)
+                    u = *reinterpret_cast<const uint4 *>(X + (int64_t)gi * k + kk);
+                __builtin_memcpy(v[s], &u, 16);
+            } else {
+                v[s][0] = in ? X[(int64_t)gi * k + kk] : (T)0;
+            }
+        }
+    }
+    __device__ __forceinline__ void store(T (*S)[TB + 4], int tid) const {
+        const int kk = (tid % PER) * VE, row = tid / PER;
+#pragma unroll
+        for (int s = 0; s < N; s++)
+#pragma unroll
+            for (int e = 0; e < VE; e++)
+                S[kk + e][row + s * ROWS] = v[s][e];
+    }
+};
+
+template <typename T, typename TY, typename U, int METRIC, int TB, bool VEC>
+__global__ __launch_bounds__(256)
+__attribute__((amdgpu_waves_per_eu(2))) void pairwise_mfma_kernel(
     const T *__restrict__ X, const TY *__restrict__ Y, int m, int n, int k, U *__restrict__ D,
     int64_t ldd, const double *__restrict__ nx, const double *__restrict__ ny, int zero_diag,
     int diag_offset, double gam, double inv_rtol) {
-    __shared__ double Xs[KC][TB + 1];
-    __shared__ double Ys[KC][TB + 1];
+    constexpr int RB = TB / 32; // blocks of 16 per wave and side
+    __shared__ T Xs[2][KC][TB + 4];
+    __shared__ TY Ys[2][KC][TB + 4];
     const int tid = threadIdx.x;
     const int lane = tid & 63, w = tid >> 6;
     const int wr = w >> 1, wc = w & 1;
     const int i0 = blockIdx.y * TB, j0 = blockIdx.x * TB;
 
-    v4d acc[2][2];
+    v4d acc[RB][RB];
 #pragma unroll
-    for (int a = 0; a < 2; a++)
+    for (int a = 0; a < RB; a++)
 #pragma unroll
-        for (int b = 0; b < 2; b++)
+        for (int b = 0; b < RB; b++)
             acc[a][b] = (v4d){0.0, 0.0, 0.0, 0.0};
 
-    // Loader mapping: 16 consecutive k per row, 16 rows per pass, 4 passes.
-    const int lk = tid & 15, lr = tid >> 4;
     const int kq = lane >> 4, col = lane & 15;
-    for (int k0 = 0; k0 < k; k0 += KC) {
-        const int kk = k0 + lk;
-#pragma unroll
-        for (int s = 0; s < 4; s++) {
-            const int row = lr + 16 * s;
-            const int gi = i0 + row, gj = j0 + row;
-            double xv = 0.0, yv = 0.0;
-            if (kk < k) {
-                if (gi < m)
-                    xv = (double)X[(int64_t)gi * k + kk];
-                if (gj < n)
-                    yv = (double)Y[(int64_t)gj * k + kk];
-            }
-            Xs[lk][row] = xv;
-            Ys[lk][row] = yv;
-        }
+    Slice<T, TB, VEC ? 16 / (int)sizeof(T) : 1> xs;
+    Slice<TY, TB, VEC ? 16 / (int)sizeof(TY) : 1> ys;
+    xs.load(X, i0, m, k, 0, tid);
+    ys.load(Y, j0, n, k, 0, tid);
+    xs.store(Xs[0], tid);
+    ys.store(Ys[0], tid);
+    int cur = 0;
+    for (int k0 = 0; k0 < k; k0 += KC, cur ^= 1) {
         __syncthreads();
+        const bool more = k0 + KC < k;
+        if (more) {
+            xs.load(X, i0, m, k, k0 + KC, tid);
+            ys.load(Y, j0, n, k, k0 + KC, tid);
+        }
 #pragma unroll
         for (int q = 0; q < KC; q += 4) {
-            double a[2], b[2];
+            double a[RB], b[RB];
 #pragma unroll
-            for (int t = 0; t < 2; t++) {
-                a[t] = Xs[q + kq][wr * 32 + t * 16 + col];
-                b[t] = Ys[q + kq][wc * 32 + t * 16 + col];
+            for (int t = 0; t < RB; t++) {
+                a[t] = (double)Xs[cur][q + kq][wr * (TB / 2) + t * 16 + col];
+                b[t] = (double)Ys[cur][q + kq][wc * (TB / 2) + t * 16 + col];
             }
 #pragma unroll
-            for (int ra = 0; ra < 2; ra++)
+            for (int ra = 0; ra < RB; ra++)
 #pragma unroll
-                for (int cb = 0; cb < 2; cb++)
+                for (int cb = 0; cb < RB; cb++)
                     acc[ra][cb] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[ra], b[cb], acc[ra][cb],
                                                                         0, 0, 0);
         }
-        __syncthreads();
+        // The other buffer was last read before this slice's barrier.
+        if (more) {
+            xs.store(Xs[cur ^ 1], tid);
+            ys.store(Ys[cur ^ 1], tid);
+        }
     }
 
 #pragma unroll
-    for (int ra = 0; ra < 2; ra++) {
+    for (int ra = 0; ra < RB; ra++) {
 #pragma unroll
-        for (int cb = 0; cb < 2; cb++) {
+        for (int cb = 0; cb < RB; cb++) {
 #pragma unroll
             for (int r = 0; r < 4; r++) {
-                const int i = i0 + wr * 32 + ra * 16 + 4 * r + kq;
-                const int j = j0 + wc * 32 + cb * 16 + col;
+                const int i = i0 + wr * (TB / 2) + ra * 16 + 4 * r + kq;
+                const int j = j0 + wc * (TB / 2) + cb * 16 + col;
                 if (i >= m || j >= n)
                     continue;
                 const double g = acc[ra][cb][r];
@@ -138,6 +175,28 @@ __global__ __launch_bounds__(256) void pairwise_mfma_kernel(
     }
 }
 
+// Tile edge and load width of a call.
+template <typename T, typename TY, typename U, int METRIC>
+void pairwise_mfma_run(const T *X, const TY *Y, int m, int n, int k, U *D, int64_t ldd,
+                       const double *nx, const double *ny, int zero_diag, int diag_offset,
+                       double gam, double inv_rtol, hipStream_t s) {
+    auto run = [&](auto kern, int tb) {
+        hipLaunchKernelGGL(kern, dim3((n + tb - 1) / tb, (m + tb - 1) / tb), dim3(256), 0, s, X, Y,
+                           m, n, k, D, ldd, nx, ny, zero_diag, diag_offset, gam, inv_rtol);
+    };
+    auto aligned = [&](const void *p, size_t size) {
+        return ((uintptr_t)p & 15) == 0 && k * size % 16 == 0;
+    };
+    const bool vec = aligned(X, sizeof(T)) && aligned(Y, sizeof(TY));
+    const bool large = (int64_t)((m + 127) / 128) * ((n + 127) / 128) >= 1024;
+    if (large)
+        run(vec ? pairwise_mfma_kernel<T, TY, U, METRIC, 128, true>
+                : pairwise_mfma_kernel<T, TY, U, METRIC, 128, false>, 128);
+    else
+        run(vec ? pairwise_mfma_kernel<T, TY, U, METRIC, 64, true>
+                : pairwise_mfma_kernel<T, TY, U, METRIC, 64, false>, 64);
+}
+
 } // namespace
 
 bool pairwise_mfma_metric(int metric) {
@@ -153,15 +212,14 @@ hipError_t launch_pairwise_mfma(int metric, const T *X, const T *Y, int m, int n
         return hipErrorInvalidValue;
     if (m <= 0 || n <= 0)
         return hipSuccess;
-    dim3 grid((n + TB - 1) / TB, (m + TB - 1) / TB);
     const double u = 1.0 / 9007199254740992.0; // 2^-53
     const double nk = (double)(k + 2);
     const double gam = nk * u / (1.0 - nk * u);
     const double inv_rtol = sizeof(U) == 8 ? 2e12 : 2e6;
 #define DA_PWM_CASE(M)                                                                       \
     case M:                                                                                  \
-        hipLaunchKernelGGL((pairwise_mfma_kernel<T, T, U, M>), grid, dim3(256), 0, s, X, Y, m, n, \
-                           k, D, ldd, nx, ny, zero_diag, diag_offset, gam, inv_rtol);         \
+        pairwise_mfma_run<T, T, U, M>(X, Y, m, n, k, D, ldd, nx, ny, zero_diag, diag_offset,  \
+                                      gam, inv_rtol, s);                                      \
         break;
     switch (metric) {
         DA_PWM_CASE(KM_SQEUCLIDEAN)
@@ -183,13 +241,12 @@ hipError_t launch_inner_mfma(const TX *X, const TY *Y, int m, int n, int k, floa
     if (m <= 0 || n <= 0)
         return hipSuccess;
     // At most 65,535 row tiles per launch (the grid's y extent).
-    const int chunk = 65535 * TB;
+    const int chunk = 65535 * 64;
     for (int i0 = 0; i0 < m; i0 += chunk) {
         const int mm = m - i0 < chunk ? m - i0 : chunk;
-        dim3 grid((n + TB - 1) / TB, (mm + TB - 1) / TB);
-        hipLaunchKernelGGL((pairwise_mfma_kernel<TX, TY, float, KM_INNER>), grid, dim3(256), 0,
-                           s, X + (int64_t)i0 * k, Y, mm, n, k, D + (int64_t)i0 * ldd, ldd,
-                           nullptr, nullptr, 0, 0, 0.0, 0.0);
+        pairwise_mfma_run<TX, TY, float, KM_INNER>(X + (int64_t)i0 * k, Y, mm, n, k,
+                                                   D + (int64_t)i0 * ldd, ldd, nullptr, nullptr, 0,
+                                                   0, 0.0, 0.0, s);
         const hipError_t e = hipGetLastError();
         if (e != hipSuccess)
             return e;

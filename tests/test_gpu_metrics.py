@@ -154,3 +154,26 @@ def test_gemm_form_tile_edges(oracle, dtype, metric):
             E = np.nan_to_num(E, nan=0.0)
         scale = 1.0 if metric in ("euclidean", "sqeuclidean", "cosine") else max(1.0, np.abs(E).max())
         close(D, E, dtype, scale)
+
+
+@pytest.mark.parametrize("dtype", [np.float64, np.float32])
+@pytest.mark.parametrize("m,n,k", [(4097, 4095, 17), (8193, 2049, 16), (4096, 4224, 32), (4100, 4200, 3),
+                                   (127, 129, 64), (65, 63, 1)])
+def test_gemm_tiles(dtype, m, n, k):
+    """Both tile sizes of the GEMM-form kernel (128 from 1,024 tiles on) at their edges, rows of
+    whole 16-byte pieces and others, one to a few k slices. Every element against the direct
+    differences in double; the kernel recomputes what the GEMM form does not hold to 5e-13 (5e-7)."""
+    rng = np.random.default_rng(m + k)
+    X = rng.standard_normal((m, k)).astype(dtype)
+    Y = rng.standard_normal((n, k)).astype(dtype)
+    Y[:5] = X[:5]
+    D = aoclda.metrics.pairwise_distances(X, Y, metric="sqeuclidean")
+    A, B = X.astype(np.float64), Y.astype(np.float64)
+    E = np.zeros((m, n))
+    for l in range(k):
+        E += (A[:, l, None] - B[None, :, l]) ** 2
+    # 1e-12 relative covers 5e-13 and the reference's own k + 1 roundings for fp64, 6e-7 the
+    # output's rounding beside 5e-7 for fp32.
+    np.testing.assert_allclose(D, E, rtol=1e-12 if dtype == np.float64 else 6e-7, atol=0)
+    G = aoclda.metrics.pairwise_distances(X, Y, metric="inner_product")
+    np.testing.assert_allclose(G, A @ B.T, rtol=RTOL[dtype], atol=RTOL[dtype] * k)
