@@ -292,11 +292,8 @@ da_status ApproxNNHandle<T>::add(da_int n_add, da_int n_features, const T *X, da
             DA_HIP(err, (launch_pack_rows<T, T>(added, d, n_add, d, as_x_.as<T>(), kp, n_add, st)));
             DA_HIP(err, launch_centre_prep<T>(cdouble_d_.as<double>(), n_list_, d, kp,
                                               as_c_.as<T>(), as_h_.as<T>(), cmax2, st, sph));
-            double hc = 0;
-            DA_HIP(err, hipMemcpyAsync(&hc, cmax2, sizeof(double), hipMemcpyDeviceToHost, st));
-            DA_HIP(err, hipStreamSynchronize(st));
             DA_HIP(err, launch_kmeans_assign_mfma<T>(as_x_.as<T>(), n_add, kp, as_c_.as<T>(),
-                                                     as_h_.as<T>(), n_list_, std::sqrt(hc),
+                                                     as_h_.as<T>(), n_list_, cmax2,
                                                      lab_d_.as<int>(), nullptr, cnt, cnt + 1,
                                                      as_list_.as<int>(), st));
             DA_HIP(err, launch_kmeans_recheck<T>(added, d, d, cdouble_d_.as<double>(), n_list_,

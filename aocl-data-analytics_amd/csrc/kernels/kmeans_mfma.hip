@@ -114,7 +114,8 @@ template <typename E, int KCH, int PTT>
 __global__ __launch_bounds__(256)
 __attribute__((amdgpu_waves_per_eu(2))) void kmeans_assign_mfma_kernel(
     const E *__restrict__ X, int n, int Kp, const E *__restrict__ CP,
-    const E *__restrict__ chalf, int k, int kch, double cmax, int *__restrict__ labels,
+    const E *__restrict__ chalf, int k, int kch, const double *__restrict__ cmax2,
+    int *__restrict__ labels,
     const int *__restrict__ prev, int *__restrict__ changed, int *__restrict__ list_count,
     int *__restrict__ list) {
     using Op = AssignOp<E>;
@@ -219,6 +220,7 @@ __attribute__((amdgpu_waves_per_eu(2))) void kmeans_assign_mfma_kernel(
                 const double unit = Op::unit;
                 const double xnorm = sqrt((double)xs) * (1.0 + 4.0 * unit);
                 const double gam = (Kp + 2) * unit / (1.0 - (Kp + 2) * unit);
+                const double cmax = sqrt(*cmax2);
                 const double e = (gam + 2.0 * unit) * (xnorm * cmax + 0.5 * cmax * cmax);
                 const bool near_tie = (double)best1[pt] - (double)best2[pt] <= 2.0 * e;
                 const int lab = bidx[pt] < k ? bidx[pt] : 0;
@@ -255,7 +257,8 @@ template <int KCH>
 __global__ __launch_bounds__(256)
 __attribute__((amdgpu_waves_per_eu(2))) void kmeans_assign_bf16_kernel(
     const __bf16 *__restrict__ X, int n, int Kp, const __bf16 *__restrict__ C16,
-    const float *__restrict__ chalf, int k, double cmax, int *__restrict__ labels,
+    const float *__restrict__ chalf, int k, const double *__restrict__ cmax2,
+    int *__restrict__ labels,
     const int *__restrict__ prev, int *__restrict__ changed, int *__restrict__ list_count,
     int *__restrict__ list) {
     constexpr int NF = KCH / 8;
@@ -358,6 +361,7 @@ __attribute__((amdgpu_waves_per_eu(2))) void kmeans_assign_bf16_kernel(
                 // fp32 accumulation gamma_{Kp+2} over |x~| |c~| + cmax^2/2, the rounded -|c|^2/2.
                 const double xnorm = sqrt((double)xs) / (1.0 - u) * (1.0 + 1e-6);
                 const double gam = (Kp + 2) * u32 / (1.0 - (Kp + 2) * u32);
+                const double cmax = sqrt(*cmax2);
                 const double S = xnorm * cmax;
                 const double e = (2.0 * u + u * u) * S + gam * (S * (1.0 + u) * (1.0 + u) + 0.5 * cmax * cmax) +
                                  u32 * 0.5 * cmax * cmax;
@@ -524,7 +528,7 @@ size_t kmeans_assign_bf16_lds(int k, int Kp) {
 }
 
 hipError_t launch_kmeans_assign_bf16(const void *X, int n, int Kp, const void *C16,
-                                     const float *chalf, int k, double cmax, int *labels,
+                                     const float *chalf, int k, const double *cmax2, int *labels,
                                      const int *prev, int *changed, int *list_count, int *list,
                                      hipStream_t s, int wg_per_cu) {
     const size_t lds = kmeans_assign_bf16_lds(k, Kp);
@@ -539,7 +543,7 @@ hipError_t launch_kmeans_assign_bf16(const void *X, int n, int Kp, const void *C
         if (lds > 65536)                                                                         \
             (void)hipFuncSetAttribute((const void *)kern,                                        \
                                       hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);     \
-        hipLaunchKernelGGL(kern, grid, block, lds, s, x, n, Kp, c, chalf, k, cmax, labels, prev, \
+        hipLaunchKernelGGL(kern, grid, block, lds, s, x, n, Kp, c, chalf, k, cmax2, labels, prev, \
                            changed, list_count, list);                                           \
     }
     switch (Kp / 4) {
@@ -568,7 +572,7 @@ template hipError_t launch_centre_prep<double>(const double *, int, int, int, do
 
 template <typename E>
 hipError_t launch_kmeans_assign_mfma(const E *X, int n, int Kp, const E *CP, const E *chalf,
-                                     int k, double cmax, int *labels, const int *prev,
+                                     int k, const double *cmax2, int *labels, const int *prev,
                                      int *changed, int *list_count, int *list, hipStream_t s,
                                      int wg_per_cu) {
     if (Kp % 16 != 0 || Kp > 128 || k < 1)
@@ -584,7 +588,7 @@ hipError_t launch_kmeans_assign_mfma(const E *X, int n, int Kp, const E *CP, con
         if (lds > 65536)                                                                         \
             (void)hipFuncSetAttribute((const void *)kern,                                        \
                                       hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);     \
-        hipLaunchKernelGGL(kern, grid, block, lds, s, X, n, Kp, CP, chalf, k, kch, cmax, labels, \
+        hipLaunchKernelGGL(kern, grid, block, lds, s, X, n, Kp, CP, chalf, k, kch, cmax2, labels, \
                            prev, changed, list_count, list);                                     \
     }
     switch (Kp / 4) {
@@ -611,11 +615,11 @@ hipError_t launch_kmeans_assign_mfma(const E *X, int n, int Kp, const E *CP, con
     return hipGetLastError();
 }
 template hipError_t launch_kmeans_assign_mfma<float>(const float *, int, int, const float *,
-                                                     const float *, int, double, int *,
+                                                     const float *, int, const double *, int *,
                                                      const int *, int *, int *, int *,
                                                      hipStream_t, int);
 template hipError_t launch_kmeans_assign_mfma<double>(const double *, int, int, const double *,
-                                                      const double *, int, double, int *,
+                                                      const double *, int, const double *, int *,
                                                       const int *, int *, int *, int *,
                                                       hipStream_t, int);
 

@@ -617,14 +617,14 @@ hipError_t launch_centre_prep(const double *C, int k, int d, int Kp, E *CP, E *c
 // workgroups per CU, each taking every gridDim.x-th block of samples.
 template <typename E>
 hipError_t launch_kmeans_assign_mfma(const E *X, int n, int Kp, const E *CP, const E *chalf,
-                                     int k, double cmax, int *labels, const int *prev,
+                                     int k, const double *cmax2, int *labels, const int *prev,
                                      int *changed, int *list_count, int *list, hipStream_t s,
                                      int wg_per_cu = 0);
 // bf16 cross-term form of the same assignment: X and C16 are bf16 rows padded to Kp (a
 // multiple of 32, at most 128) features; C16 has (k+15)/16*16 rows.
 size_t kmeans_assign_bf16_lds(int k, int Kp);
 hipError_t launch_kmeans_assign_bf16(const void *X, int n, int Kp, const void *C16,
-                                     const float *chalf, int k, double cmax, int *labels,
+                                     const float *chalf, int k, const double *cmax2, int *labels,
                                      const int *prev, int *changed, int *list_count, int *list,
                                      hipStream_t s, int wg_per_cu = 0);
 hipError_t launch_centre_prep_bf16(const double *C, int k, int d, int Kp, void *C16,

@@ -284,7 +284,8 @@ da_status KMeansHandle<T>::lloyd_step(const U *dX, const double *Cin, double *Co
     hipStream_t st = gpu->stream();
     const int n = n_samples_, d = n_features_, k = n_clusters_;
     int *dchanged = reinterpret_cast<int *>(small_.as<double>() + 4);
-    DA_HIP(err, hipMemsetAsync(dchanged, 0, 2 * sizeof(int), st));
+    double *cmax2 = small_.as<double>() + 6;
+    DA_HIP(err, hipMemsetAsync(dchanged, 0, 3 * sizeof(double), st)); // the counters and *cmax2
     const bool on_data = std::is_same_v<U, T> && (const void *)dX == (const void *)X_.ptr();
     const bool use_bf16 = on_data && std::is_same_v<U, float> && bf16_ok_ &&
                           opts.skey("cross term precision") == 1 &&
@@ -293,7 +294,6 @@ da_status KMeansHandle<T>::lloyd_step(const U *dX, const double *Cin, double *Co
     if (use_bf16) {
         // bf16 cross term on MFMA, exact re-check of near ties (kmeans_mfma.hip).
         int *dlist_count = dchanged + 1;
-        double *cmax2 = small_.as<double>() + 6;
         DA_HIP(err, xb_.reserve((size_t)n * kp16_ * 2));
         if (!xb_ready_) {
             DA_HIP(err, launch_rows_to_bf16(reinterpret_cast<const float *>(X_.ptr()), n, d, d,
@@ -303,16 +303,12 @@ da_status KMeansHandle<T>::lloyd_step(const U *dX, const double *Cin, double *Co
         DA_HIP(err, c16_.reserve((size_t)(k + 16) * kp16_ * 2));
         DA_HIP(err, chalf_.reserve((size_t)(k + 16) * sizeof(float)));
         DA_HIP(err, list_.reserve((size_t)n * sizeof(int)));
-        DA_HIP(err, hipMemsetAsync(cmax2, 0, sizeof(double), st));
         DA_HIP(err, launch_centre_prep_bf16(Cin, k, d, kp16_, c16_.ptr(), chalf_.as<float>(),
                                             cmax2, st, sph_));
-        double hc = 0;
-        DA_HIP(err, hipMemcpyAsync(&hc, cmax2, sizeof(double), hipMemcpyDeviceToHost, st));
-        DA_HIP(err, hipStreamSynchronize(st));
         {
             KernelScope ks(*gpu, "kmeans_assign");
             DA_HIP(err, launch_kmeans_assign_bf16(xb_.ptr(), n, kp16_, c16_.ptr(),
-                                                  chalf_.as<float>(), k, std::sqrt(hc), lab_new,
+                                                  chalf_.as<float>(), k, cmax2, lab_new,
                                                   lab_old, dchanged, dlist_count, list_.as<int>(),
                                                   st, (int)opts.ival("assignment workgroups per cu")));
         }
@@ -327,17 +323,12 @@ da_status KMeansHandle<T>::lloyd_step(const U *dX, const double *Cin, double *Co
         // Cross term on the fp32 or fp64 matrix cores, exact re-check of near ties
         // (kmeans_mfma.hip).
         int *dlist_count = dchanged + 1;
-        double *cmax2 = small_.as<double>() + 6;
-        DA_HIP(err, hipMemsetAsync(cmax2, 0, sizeof(double), st));
         DA_HIP(err, launch_centre_prep<T>(Cin, k, d, kp_, c32_.as<T>(), chalf_.as<T>(), cmax2,
                                           st, sph_));
-        double hc = 0;
-        DA_HIP(err, hipMemcpyAsync(&hc, cmax2, sizeof(double), hipMemcpyDeviceToHost, st));
-        DA_HIP(err, hipStreamSynchronize(st));
         {
             KernelScope ks(*gpu, "kmeans_assign");
             DA_HIP(err, launch_kmeans_assign_mfma<T>(xpad_.as<T>(), n, kp_, c32_.as<T>(),
-                                                     chalf_.as<T>(), k, std::sqrt(hc), lab_new,
+                                                     chalf_.as<T>(), k, cmax2, lab_new,
                                                   lab_old, dchanged, dlist_count, list_.as<int>(), st,
                                                   (int)opts.ival("assignment workgroups per cu")));
         }
