@@ -92,3 +92,29 @@ def test_dbscan_metrics(oracle, metric, d):
     labels, core, _ = oracle.dbscan(X, eps, 5, metric, single=True)
     np.testing.assert_array_equal(db.labels, labels)
     np.testing.assert_array_equal(db.core_sample_indices, np.flatnonzero(core))
+
+
+def test_dbscan_several_blocks():
+    """More rows than one block of bits holds (2 GiB: 131,072): core samples and clusters against a
+    k-d tree."""
+    from scipy.sparse import coo_matrix
+    from scipy.sparse.csgraph import connected_components
+    from scipy.spatial import cKDTree
+    rng = np.random.default_rng(23)
+    means = rng.uniform(-50, 50, (300, 3))
+    X = means[rng.integers(0, 300, 140001)] + rng.standard_normal((140001, 3))
+    eps, min_samples = 0.3, 8
+    db = aoclda.clustering.DBSCAN(eps=eps, min_samples=min_samples).fit(X)
+    tree = cKDTree(X)
+    pairs = tree.query_pairs(eps, output_type="ndarray")
+    deg = np.bincount(pairs.ravel(), minlength=len(X)) + 1
+    core = deg >= min_samples
+    np.testing.assert_array_equal(np.sort(np.asarray(db.core_sample_indices)), np.flatnonzero(core))
+    cc = pairs[core[pairs[:, 0]] & core[pairs[:, 1]]]
+    g = coo_matrix((np.ones(len(cc)), (cc[:, 0], cc[:, 1])), shape=(len(X), len(X)))
+    _, comp = connected_components(g, directed=False)
+    lab = np.asarray(db.labels)
+    first = {}
+    for c, l in zip(comp[core], lab[core]):
+        assert first.setdefault(c, l) == l
+    assert len(set(first.values())) == len(first) == db.n_clusters
