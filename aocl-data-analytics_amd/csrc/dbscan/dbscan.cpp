@@ -109,11 +109,11 @@ da_status DBSCANHandle<T>::reserve_edges(long long total, long long used) {
     return da_status_success;
 }
 
-// Hit bits (radius_mfma.hip) for row blocks of up to 2 GiB of bits, counts, offsets and a fill of the
-// set bits. Each block costs two host round trips and a tail of every kernel, more than the last
-// level cache gives to small blocks: 100,000 x 16 fp32 take 6.3 ms in blocks of 128 MiB, 5.6 of 512
-// MiB, 4.9 in one block of 1.25 GB (33.5 by the key tiles of the general path, 40 GB of keys written
-// and read).
+// Hit bits (radius_mfma.hip) for row blocks of up to 256 MiB of bits, counts, offsets and a fill of
+// the set bits. A block costs two host round trips and a tail of every kernel, a larger buffer its
+// allocation by each new handle: 100,000 x 16 fp32 take 6.2 ms in blocks of 128 MiB (the first time
+// 6.3), 5.9 of 256 MiB (6.0), 5.6 of 512 MiB (10.7), and 33 by the key tiles of the general path (40
+// GB of keys written and read).
 template <typename T>
 da_status DBSCANHandle<T>::neighbour_graph_bits(int km, T thr, const double *nrm, bool &done) {
     done = false;
@@ -132,7 +132,7 @@ da_status DBSCANHandle<T>::neighbour_graph_bits(int km, T thr, const double *nrm
     const T *X = X_.as<T>();
     const double thr2 = km == KM_EUCLIDEAN ? (double)thr * (double)thr : (double)thr;
     const int chunk = (int)std::max<size_t>(
-        512, std::min<size_t>((size_t)n_pad, ((size_t)1 << 31) / ((size_t)n_pad / 8) / 512 * 512));
+        512, std::min<size_t>((size_t)n_pad, ((size_t)256 << 20) / ((size_t)n_pad / 8) / 512 * 512));
     DA_HIP(err, rbits_.reserve((size_t)chunk * n_pad / 8));
     DA_HIP(err, cnt_.reserve((size_t)n_pad * sizeof(int)));
     DA_HIP(err, offs_.reserve((size_t)(n + 1) * sizeof(long long)));

@@ -95,8 +95,7 @@ def test_dbscan_metrics(oracle, metric, d):
 
 
 def test_dbscan_several_blocks():
-    """More rows than one block of bits holds (2 GiB: 131,072): core samples and clusters against a
-    k-d tree."""
+    """Several blocks of bits and a ragged last one: core samples and clusters against a k-d tree."""
     from scipy.sparse import coo_matrix
     from scipy.sparse.csgraph import connected_components
     from scipy.spatial import cKDTree
