@@ -144,7 +144,8 @@ def run_form(L, aoclda, Xt, dq, nq, d, k, precision, steps, warmup, variant=-1, 
     L.check(L.lib.da_amd_synchronize(h.h))
     kern = {}
     for name in ("knn_seed", "knn_query_centre", "knn_tile", "knn_merge", "knn_retry_tile",
-                 "knn_retry_merge", "pairwise_direct", "row_topk"):
+                 "knn_retry_merge", "knn_sample", "knn_sweep", "knn_wide_scores",
+                 "pairwise_direct", "row_topk"):
         ms, cnt = C.c_double(), L.da_int()
         L.check(L.lib.da_amd_profile_get(h.h, name.encode(), C.byref(ms), C.byref(cnt)))
         if cnt.value:
@@ -490,7 +491,7 @@ def dbscan_bench(args, L, aoclda):
         t0 = time.perf_counter()
         h.call("da_dbscan_compute")
         times.append(time.perf_counter() - t0)
-    names = ("pairwise_direct", "radius_segsum", "radius_fill", "dbscan_union", "dbscan_label")
+    names = ("radius_sweep", "radius_verify", "pairwise_direct", "radius_segsum", "radius_fill", "dbscan_union", "dbscan_label")
     kern = {}
     for nm in names:
         ms_, cnt = C.c_double(), L.da_int()
@@ -502,13 +503,20 @@ def dbscan_bench(args, L, aoclda):
     h.call("da_handle_get_result", L.RINFO, C.byref(dim), L.ptr(r))
     step = float(np.median(times))
     log(f"dbscan: {n}x{d}, step {step * 1e3:.2f} ms, clusters {int(r[8])}, core {int(r[7])}")
-    # Dominant kernel: the exact key tile (3d fp64 operations per pair, the tile written once).
+    # Dominant kernel: the sweep of the hit bits (fp16 matrix cores, three products per term), or
+    # the exact key tile (3d fp64 operations per pair, the tile written once).
+    sw_s = kern.get("radius_sweep", {"total_ms": 0.0})["total_ms"] / args.steps * 1e-3
     pd = kern.get("pairwise_direct", {"total_ms": 0.0, "launches": 1})
     pd_s = pd["total_ms"] / args.steps * 1e-3
     flops = 3.0 * n * n * d
     byts = 4.0 * n * n + 4.0 * n * d
     t_f, t_b = flops / 78.6e12, byts / 8e12
-    if t_b >= t_f:
+    if sw_s:
+        tf = 2.0 * n * n * d / sw_s / 1e12
+        roof = {"kernel": "radius_sweep", "bound": "mfma", "achieved": tf, "peak": 2500.0,
+                "unit": "TFLOP/s", "frac": tf / 2500.0, "traffic": None,
+                "issued_mfma_tflops": tf * 3 * ((d + 31) // 32 * 32) / d}
+    elif t_b >= t_f:
         roof = {"kernel": "pairwise_direct", "bound": "hbm", "achieved": byts / pd_s / 1e9,
                 "peak": 8000.0, "unit": "GB/s", "frac": byts / pd_s / 8e12, "traffic": None}
     else:
@@ -665,7 +673,7 @@ def ivf_bench(args, L, aoclda):
             _, ind = ann.kneighbors(Q, n_neighbors=k)
             ts.append(time.perf_counter() - t0)
         kern = {}
-        for nm in ("ivf_coarse", "ivf_scan", "ivf_select"):
+        for nm in ("ivf_coarse", "ivf_tile_scores", "ivf_tile_select", "ivf_scan", "ivf_select"):
             ms_, cnt = C.c_double(), L.da_int()
             L.check(L.lib.da_amd_profile_get(ann._h.h, nm.encode(), C.byref(ms_), C.byref(cnt)))
             if cnt.value:
@@ -688,6 +696,13 @@ def ivf_bench(args, L, aoclda):
     roof = {"kernel": "ivf_scan", "bound": "hbm", "achieved": byts / scan_s / 1e9 if scan_s else None,
             "peak": 8000.0, "unit": "GB/s", "frac": byts / scan_s / 8e12 if scan_s else None,
             "traffic": None, "candidates_per_step": cand, "fp64_tflops": 3 * d * cand / scan_s / 1e12 if scan_s else None}
+    ts_ = H["kernels_ms"].get("ivf_tile_scores")
+    if ts_:
+        # List by list on the matrix cores: a score written (4 bytes) per query and candidate.
+        t = ts_["total_ms"] / args.steps * 1e-3
+        roof = {"kernel": "ivf_tile_scores", "bound": "hbm", "achieved": 4 * cand / t / 1e9,
+                "peak": 8000.0, "unit": "GB/s", "frac": 4 * cand / t / 8e12, "traffic": None,
+                "candidates_per_step": cand, "mfma_tflops": 2 * d * cand / t / 1e12}
     print(json.dumps({
         "metric": IVF_METRIC, "value": H["qps"], "unit": "queries/s", "n_gpus": 1,
         "steps": args.steps, "warmup": args.warmup, "ms_per_step": H["ms_per_step"],
@@ -833,7 +848,19 @@ def main():
     H = results[head]
     flops = 2.0 * nq * args.n_train * d
     roofline = None
-    if "knn_tile" in H["kernels"]:
+    swept = "knn_sweep" in H["kernels"]
+    if swept:
+        # The sweep multiplies the rows' fp16 parts once per pair, whatever the form; the blocks
+        # of a step together cover the batch.
+        tot_ms, cnt = H["kernels"]["knn_sweep"]
+        per_step = tot_ms / args.steps * 1e-3
+        achieved = flops / per_step
+        roofline = {"kernel": "knn_sweep", "bound": "mfma", "achieved": achieved / 1e12,
+                    "peak": PEAK["fp16"] / 1e12, "unit": "TFLOP/s",
+                    "frac": achieved / PEAK["fp16"], "traffic": None,
+                    "avg_launch_ms": tot_ms / cnt, "algorithmic_flops_per_launch": flops * args.steps / cnt,
+                    "issued_mfma_tflops": achieved / 1e12 * ((d + 31) // 32 * 32) / d}
+    elif "knn_tile" in H["kernels"]:
         tot_ms, cnt = H["kernels"]["knn_tile"]
         per_launch = tot_ms / cnt * 1e-3
         achieved = flops / per_launch  # one tile launch per step covers the whole batch
@@ -856,7 +883,7 @@ def main():
         "metric": METRIC, "value": H["qps"], "unit": "queries/s", "n_gpus": 1,
         "steps": args.steps, "warmup": args.warmup, "ms_per_step": H["ms_per_step"],
         "higher_is_better": True, "scaling": "weak", "vs_baseline": None,
-        "dtype": DTYPE_NAME.get(split_form(head)[0], head),
+        "dtype": "f16" if swept else DTYPE_NAME.get(split_form(head)[0], head),
         "data": "synthetic: 64-component isotropic Gaussian mixture (means U[-10,10]^128, "
                 "sigma 1), numpy default_rng(0)",
         "config": {"workload": f"brute-force kNN, train {args.n_train}x{d} fp32, {nq} queries, "
