@@ -113,7 +113,7 @@ da_status build(BatchRun &r, da_int n_inst, const da_int *n, const da_int *d, co
     // wide instance ends last. At least 16 k samples, so that a chunk's partial sums (16 k d
     // bytes written, then read) stay below a quarter of its rows; at most 16,384 (the sorted
     // sample list in LDS). With 16,384-sample chunks throughout, 256 instances of 1,000-50,000
-    // samples gave some 400 workgroups and 18.6 ms a run; now 2,000 and 5.5 ms.
+    // samples gave some 400 workgroups and 18.6-22 ms a run; now 2,000 and 7.2 ms.
     int dev = 0, cus = 0;
     if (hipGetDevice(&dev) != hipSuccess ||
         hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
