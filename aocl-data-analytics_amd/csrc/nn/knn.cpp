@@ -665,6 +665,7 @@ da_status NNHandle<T>::search_launch(SearchContext &ctx, const SearchParams &sp,
     if (fused && sp.automatic && !ctx.second_pass && tiles_faster(nq)) {
         fused = false;
         ctx.last_candidates = n_samples_; // every row has its exact key
+        return search_tiles(ctx, dQ, nq, k, return_distance, d_ind, d_dist, true);
     }
     if (!fused) {
         if (!ctx.second_pass && wide_eligible(nq, k)) {
@@ -1028,7 +1029,7 @@ da_status NNHandle<T>::search_finish(SearchContext &ctx, const T *dQ, da_int nq,
                                   ctx.fb_dist.as<T>(), fused2);
         } else {
             s = search_tiles(ctx, ctx.fb_q.as<T>(), nfb, k, true, ctx.fb_ind.as<da_int>(),
-                             ctx.fb_dist.as<T>());
+                             ctx.fb_dist.as<T>(), few);
         }
         if (s != da_status_success)
             return s;
@@ -1185,9 +1186,12 @@ da_status NNHandle<T>::search(const T *dQ, da_int nq, da_int k, bool return_dist
 // Generic path for every metric: key tiles (queries x training points, in double) followed
 // by the per-row selection, the structure of kneighbors_compute_brute_force
 // (nearest_neighbors.cpp:567-816) with the blocks sized for HBM instead of caches.
+// direct: in place of the fused tile or the hit bits, which order the *_gemm metrics by direct
+// differences too: |x|^2 + |y|^2 - 2 x.y would lose the digits that the norms have above the
+// distance (equal rows 1e-7 apart instead of 0), and the result would depend on the route.
 template <typename T>
 da_status NNHandle<T>::search_tiles(SearchContext &ctx, const T *dQ, da_int nq, da_int k,
-                                    bool return_distance, da_int *d_ind, T *d_dist) {
+                                    bool return_distance, da_int *d_ind, T *d_dist, bool direct) {
     hipStream_t st = ctx.gpu->stream();
     const da_int d = n_features_, n = n_samples_;
     if (k > 3840)
@@ -1206,13 +1210,13 @@ da_status NNHandle<T>::search_tiles(SearchContext &ctx, const T *dQ, da_int nq, 
         km = KM_SQEUCLIDEAN;
         break;
     case da_euclidean_gemm:
-        km = KM_SQEUCLIDEAN_GEMM;
+        km = direct ? KM_SQEUCLIDEAN : KM_SQEUCLIDEAN_GEMM;
         post = 1;
-        need_qsq = true;
+        need_qsq = !direct;
         break;
     case da_sqeuclidean_gemm:
-        km = KM_SQEUCLIDEAN_GEMM;
-        need_qsq = true;
+        km = direct ? KM_SQEUCLIDEAN : KM_SQEUCLIDEAN_GEMM;
+        need_qsq = !direct;
         break;
     case da_manhattan:
         km = KM_MANHATTAN;

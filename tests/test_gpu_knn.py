@@ -68,6 +68,29 @@ def test_vs_oracle_metrics(oracle, metric, dtype):
     np.testing.assert_array_equal(ind, ei)
 
 
+@pytest.mark.parametrize("metric", ["euclidean_gemm", "sqeuclidean_gemm"])
+@pytest.mark.parametrize("dtype", [np.float64, np.float32])
+@pytest.mark.parametrize("n,nq", [(500, 40), (3000, 500), (9000, 30), (40000, 500)])
+def test_gemm_metrics_order_by_direct_differences(oracle, metric, dtype, n, nq):
+    """The small-search route and the few queries that the hit bits leave (more equal rows than
+    they hold) order these metrics by direct differences, as the fused tile does: far from the
+    origin |x|^2 + |y|^2 - 2 x.y is off by 1e-16 of 2e7, and equal rows are not at distance 0."""
+    rng = np.random.default_rng(n)
+    Xt = (rng.standard_normal((n, 20)) + 1000).astype(dtype)
+    Xq = (rng.standard_normal((nq, 20)) + 1000).astype(dtype)
+    if n > 9000:
+        Xt[3000:6000] = Xt[5]
+    Xq[:9] = Xt[:9]
+    nn = aoclda.neighbors.nearest_neighbors(metric=metric).fit(Xt)
+    dist, ind = nn.kneighbors(Xq, 5)
+    om = "sqeuclidean" if metric == "sqeuclidean_gemm" else "euclidean"
+    ei, ed = oracle.knn(Xt.astype(np.float64), Xq.astype(np.float64), 5, om)
+    np.testing.assert_array_equal(ind, ei)
+    # 20 fused products and sums in the same order, a root and one rounding to the type
+    np.testing.assert_allclose(dist, ed, rtol=1e-14 if dtype == np.float64 else 1.2e-7, atol=0)
+    assert np.all(dist[:9, 0] == 0)
+
+
 @pytest.mark.parametrize("k", [1, 2, 64, 300])
 def test_k_edges(oracle, k):
     rng = np.random.default_rng(4)
