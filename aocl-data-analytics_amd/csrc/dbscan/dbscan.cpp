@@ -130,7 +130,7 @@ da_status DBSCANHandle<T>::neighbour_graph_bits(int km, T thr, const double *nrm
     unsigned long long *total = range + 2 * d + 1;
     float *A = rthr_.as<float>(), *B = A + n_pad;
     const T *X = X_.as<T>();
-    const double thr2 = km == KM_EUCLIDEAN ? (double)thr * (double)thr : (double)thr;
+    const double thr2 = radius_threshold2(km, thr);
     const int chunk = (int)std::max<size_t>(
         512, std::min<size_t>((size_t)n_pad, ((size_t)256 << 20) / ((size_t)n_pad / 8) / 512 * 512));
     DA_HIP(err, rbits_.reserve((size_t)chunk * n_pad / 8));

@@ -3,6 +3,7 @@
 #pragma once
 #include <cstdint>
 #include <hip/hip_runtime_api.h>
+#include <limits>
 
 namespace dagpu {
 
@@ -464,8 +465,15 @@ inline size_t radius_operand_elems(const RadiusPlan &p, int64_t rows_pad) {
 template <typename T>
 hipError_t launch_radius_scale(const T *X, int64_t nx, const T *Y, int64_t ny, int d, int metric,
                                unsigned long long *range, RadiusScale *sc, hipStream_t s);
+// The squared distance up to which a key rounded to T can be within thr. Keys below T's normal
+// range move by up to half its smallest number, whatever their size (for float, pairs of rows 1e-23
+// apart have the key 0); above it by a relative 2^-24, which the packed thresholds cover.
+template <typename T> inline double radius_threshold2(int metric, T thr) {
+    const double t = (double)thr + (double)std::numeric_limits<T>::denorm_min();
+    return metric == KM_EUCLIDEAN ? t * t : t;
+}
 // Operand rows P (rows_pad, a multiple of 16) and their thresholds: A for query rows, B for
-// training rows (either may be null). thr2: the threshold on the squared distance.
+// training rows (either may be null). thr2: radius_threshold2.
 template <typename T>
 hipError_t launch_radius_pack(const T *X, int rows, int rows_pad, int d, const RadiusPlan &p,
                               const RadiusScale *sc, double thr2, void *P, float *A, float *B,

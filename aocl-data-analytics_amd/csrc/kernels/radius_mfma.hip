@@ -19,7 +19,8 @@
 // 3 Kp products and the start value in fp32 carries gamma_{3 Kp + 8} (|x'||y'| + ...), the split
 // operands 2^-21 relative each and the dropped lo*lo 2^-22, and |x'||y'| <= (n(x') + n(y')) / 2;
 // the rounded thresholds add a few 2^-24. Together: ce (n(x') + n(y')) with ce = gamma + 2^-19,
-// plus a constant ca for values below fp16's normal range and the rounding of the centring.
+// plus a constant ca for values below fp16's normal range and the rounding of the centring. The
+// threshold itself is the largest squared distance whose rounded key passes (radius_threshold2).
 #include "launch.hpp"
 #include <algorithm>
 #include <hip/hip_runtime.h>
@@ -188,8 +189,10 @@ __global__ __launch_bounds__(256) void radius_pack_kernel(
     if (g == 0) {
         const float inf = __builtin_huge_valf();
         const bool in = row < rows;
+        // Not below -2^100: with -inf here a padding column (B = inf) would give NaN, not a miss.
         if (A)
-            A[row] = in ? (float)(0.5 * (nn * (1.0 - ce) - thr * s * s * (1.0 + 0x1p-20) - sc->ca))
+            A[row] = in ? (float)fmax(0.5 * (nn * (1.0 - ce) - thr * s * s * (1.0 + 0x1p-20) - sc->ca),
+                                      -0x1p100)
                         : inf;
         if (B)
             B[row] = in ? (float)(0.5 * nn * (1.0 - ce)) : inf;

@@ -1459,11 +1459,12 @@ da_status NNHandle<T>::radius_core(const T *dQ, da_int n_queries, T radius, bool
         set_total = range + range_words;
         A = rnn_thr_.as<float>();
         B = A + q_pad;
+        const double thr2 = radius_threshold2(km, thr);
         KernelScope ks(*gpu, "radius_pack");
         DA_HIP(err, launch_radius_scale<T>(train_.as<T>(), n, dQ, n_queries, d, km, range, rsc, st));
-        DA_HIP(err, launch_radius_pack<T>(train_.as<T>(), n, n_pad, d, plan, rsc, (double)thr,
+        DA_HIP(err, launch_radius_pack<T>(train_.as<T>(), n, n_pad, d, plan, rsc, thr2,
                                           rnn_op_.ptr(), nullptr, B, st));
-        DA_HIP(err, launch_radius_pack<T>(dQ, n_queries, q_pad, d, plan, rsc, (double)thr,
+        DA_HIP(err, launch_radius_pack<T>(dQ, n_queries, q_pad, d, plan, rsc, thr2,
                                           rnn_op_.as<char>() + opb, A, nullptr, st));
     }
     // Query blocks whose key tile stays within 256 MB (and 2^28 entries), or whose bits stay

@@ -117,3 +117,47 @@ def test_dbscan_several_blocks():
     for c, l in zip(comp[core], lab[core]):
         assert first.setdefault(c, l) == l
     assert len(set(first.values())) == len(first) == db.n_clusters
+
+
+def _sliced(nn, Q, step=60, **kw):
+    """The search a few queries at a time, which takes the key tiles of the general path."""
+    parts = [nn.radius_neighbors(Q[i:i + step], **kw) for i in range(0, len(Q), step)]
+    return [np.concatenate([np.concatenate([[], *v]) for v in p]) for p in
+            (zip(*parts) if isinstance(parts[0], tuple) else [parts])]
+
+
+# 1e-20 to 3e-22: squared distances about float's smallest normal number and below it; 1e-23: the
+# squared radius is 0 in float, and so is the key of every pair within a few of its units.
+SMALL = [1e-20, 1e-21, 3e-22, 1e-22, 5e-23, 1e-23, 1e-25]
+
+
+@pytest.mark.parametrize("scale", SMALL)
+@pytest.mark.parametrize("metric", ["euclidean", "sqeuclidean", "euclidean_gemm"])
+def test_radius_below_the_normal_range(oracle, scale, metric):
+    """Keys are rounded to float before they are compared; below its normal range by an absolute
+    amount that lets pairs beyond the radius in. Against key tiles, and for a few queries against
+    the oracle."""
+    X = (blobs(np.random.default_rng(31), 66000, 6, np.float64) * scale).astype(np.float32)
+    Q = (blobs(np.random.default_rng(31), 2050, 6, np.float64) * scale).astype(np.float32)
+    r = np.float32(0.5 * scale)
+    r = float(r * r if metric == "sqeuclidean" else r)
+    nn = aoclda.neighbors.nearest_neighbors(metric=metric, radius=r).fit(X)
+    ind = nn.radius_neighbors(Q, return_distance=False)
+    cnt, ei, _ = oracle.radius(X, Q[:60], r, metric, single=True)
+    np.testing.assert_array_equal([len(v) for v in ind[:60]], cnt)
+    np.testing.assert_array_equal(np.concatenate(list(ind[:60])), ei)
+    np.testing.assert_array_equal(np.concatenate(list(ind)),
+                                  _sliced(nn, Q, return_distance=False)[0])
+
+
+@pytest.mark.parametrize("scale", SMALL + [1e-30, 1e-43])
+@pytest.mark.parametrize("metric", ["euclidean", "l2", "sqeuclidean"])
+def test_dbscan_below_the_normal_range(oracle, scale, metric):
+    rng = np.random.default_rng(32)
+    X = (blobs(rng, 4200, 6, np.float64) * scale).astype(np.float32)
+    eps = np.float32(0.6 * scale)
+    eps = float(eps * eps if metric == "sqeuclidean" else eps)
+    db = aoclda.clustering.DBSCAN(eps=eps, min_samples=6, metric=metric, algorithm="brute").fit(X)
+    labels, core, _ = oracle.dbscan(X, eps, 6, metric, single=True)
+    np.testing.assert_array_equal(db.labels, labels)
+    np.testing.assert_array_equal(db.core_sample_indices, np.flatnonzero(core))
