@@ -1,6 +1,7 @@
 // Host-callable launchers of the HIP kernels. Every launcher enqueues on the given stream
 // and returns the launch status; none of them synchronizes.
 #pragma once
+#include <algorithm>
 #include <cstdint>
 #include <hip/hip_runtime_api.h>
 #include <limits>
@@ -365,6 +366,17 @@ hipError_t launch_wide_merge(const float *skey, const int *sidx, int nq, int kc,
 // ---- kNN by hit bits (operands knn_wide.hip, search knn_bits.hip) ----
 constexpr int BITS_D = 128, BITS_K = 128, BITS_KEEP = 2048;
 inline int bits_rows(int n) { return (n + 511) / 512 * 512; }
+// Bytes of a query's workspaces: bits, columns of its hits, sample minima, operand row, scalars.
+inline size_t bits_query_bytes(int n, int d) {
+    return (size_t)bits_rows(n) / 8 + BITS_KEEP * sizeof(int) + 256 * sizeof(float) +
+           (size_t)wide_ksteps(d) * 64 + 2 * sizeof(double) + 2 * sizeof(int);
+}
+// Queries of a block whose workspaces take up to max_bytes, whole groups of 256 (the sweep's row
+// block) and no more than nq needs; 0 if not even one group fits.
+inline int bits_block(int64_t nq, int n, int d, size_t max_bytes) {
+    const int64_t fit = (int64_t)(max_bytes / bits_query_bytes(n, d) / 256 * 256);
+    return (int)std::min<int64_t>(fit, (nq + 255) / 256 * 256);
+}
 // Relative part of the error bound of the sweep's products.
 double bits_relative_bound(int d);
 // Rank taken in the sample of ns of n rows for k neighbours.

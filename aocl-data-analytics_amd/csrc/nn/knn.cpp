@@ -659,8 +659,9 @@ da_status NNHandle<T>::search_launch(SearchContext &ctx, const SearchParams &sp,
         da_status s = prepare_bits();
         if (s != da_status_success)
             return s;
-        if (bits_state_ == 1)
-            return search_bits(ctx, dQ, nq, k, return_distance, d_ind, d_dist);
+        const int block = bits_state_ == 1 ? bits_workspaces(ctx, nq) : 0;
+        if (block > 0)
+            return search_bits(ctx, dQ, nq, k, block, return_distance, d_ind, d_dist);
     }
     if (fused && sp.automatic && !ctx.second_pass && tiles_faster(nq)) {
         fused = false;
@@ -822,7 +823,11 @@ template <typename T> da_status NNHandle<T>::prepare_bits() {
     if (bits_op_.reserve((size_t)bits_rows(n) * ks * 64) != hipSuccess ||
         bits_b_.reserve((size_t)bits_rows(n) * sizeof(float)) != hipSuccess ||
         bits_sop_.reserve((size_t)ns * ks * 64) != hipSuccess) {
-        (void)hipGetLastError(); // without the memory the fused tile serves the search
+        // Without the memory the fused tile serves the searches of this training set.
+        bits_op_.release();
+        bits_b_.release();
+        bits_sop_.release();
+        bits_state_ = 2;
         return da_status_success;
     }
     DA_HIP(err, bits_sh_.reserve((size_t)ns * sizeof(float)));
@@ -849,33 +854,46 @@ template <typename T> da_status NNHandle<T>::prepare_bits() {
     return da_status_success;
 }
 
-// Query blocks of up to 512 MB of bits.
+// Blocks of up to 1 GiB of workspaces (20,000 queries of 200,000 rows in one: 690 MB; 128 MB of
+// columns alone for 16,384 queries, however few the rows) or of one group of queries, fewer queries
+// at a time where the memory runs out. A limit of the context's own is kept to.
+template <typename T> int NNHandle<T>::bits_workspaces(SearchContext &ctx, da_int nq) {
+    const int n = n_samples_, d = n_features_;
+    const size_t own = std::max<size_t>((size_t)1 << 30, 256 * bits_query_bytes(n, d));
+    const size_t most = ctx.max_bytes ? std::min(ctx.max_bytes, own) : own;
+    for (int block = bits_block(nq, n, d, most); block > 0; block = block / 2 / 256 * 256) {
+        if (ctx.bits_q.reserve((size_t)block * wide_ksteps(d) * 64) == hipSuccess &&
+            ctx.bits_nrm.reserve((size_t)block * sizeof(double)) == hipSuccess &&
+            ctx.bits_a.reserve((size_t)block * sizeof(float)) == hipSuccess &&
+            ctx.bits_lim.reserve((size_t)block * sizeof(double)) == hipSuccess &&
+            ctx.bits_mins.reserve((size_t)block * 256 * sizeof(float)) == hipSuccess &&
+            ctx.bits_count.reserve((size_t)block * sizeof(int)) == hipSuccess &&
+            ctx.bits_cols.reserve((size_t)block * BITS_KEEP * sizeof(int)) == hipSuccess &&
+            ctx.bits.reserve((size_t)block * (bits_rows(n) / 8)) == hipSuccess)
+            return block;
+        for (DeviceBuffer *b : {&ctx.bits_q, &ctx.bits_nrm, &ctx.bits_a, &ctx.bits_lim,
+                                &ctx.bits_mins, &ctx.bits_count, &ctx.bits_cols, &ctx.bits})
+            b->release();
+    }
+    return 0;
+}
+
 template <typename T>
-da_status NNHandle<T>::search_bits(SearchContext &ctx, const T *dQ, da_int nq, da_int k,
+da_status NNHandle<T>::search_bits(SearchContext &ctx, const T *dQ, da_int nq, da_int k, int block,
                                    bool return_distance, da_int *d_ind, T *d_dist) {
     hipStream_t st = ctx.gpu->stream();
     const int n = n_samples_, d = n_features_, ns = bits_sample_;
     const int post = metric_ == da_sqeuclidean || metric_ == da_sqeuclidean_gemm ? 0 : 1;
     if (!ctx.h_fb)
         DA_HIP(err, hipHostMalloc((void **)&ctx.h_fb, sizeof(int)));
-    const int64_t most = ((int64_t)1 << 32) / bits_rows(n);
-    const int chunk = (int)std::max<int64_t>(
-        256, std::min<int64_t>((nq + 255) / 256 * 256, most / 256 * 256));
-    DA_HIP(err, ctx.bits_q.reserve((size_t)chunk * wide_ksteps(d) * 64));
-    DA_HIP(err, ctx.bits_nrm.reserve((size_t)chunk * sizeof(double)));
-    DA_HIP(err, ctx.bits_a.reserve((size_t)chunk * sizeof(float)));
-    DA_HIP(err, ctx.bits_lim.reserve((size_t)chunk * sizeof(double)));
-    DA_HIP(err, ctx.bits_mins.reserve((size_t)chunk * 256 * sizeof(float)));
-    DA_HIP(err, ctx.bits_count.reserve((size_t)chunk * sizeof(int)));
-    DA_HIP(err, ctx.bits_cols.reserve((size_t)chunk * BITS_KEEP * sizeof(int)));
-    DA_HIP(err, ctx.bits.reserve((size_t)chunk * (bits_rows(n) / 8)));
     DA_HIP(err, ctx.fb.reserve((size_t)(nq + 2) * sizeof(int)));
     int *fbc = ctx.fb.as<int>(), *bad = fbc + nq + 1;
     DA_HIP(err, hipMemsetAsync(fbc, 0, sizeof(int), st));
     const WideScale *sc = bits_sc_.as<WideScale>();
     const double ce = bits_relative_bound(d);
-    for (da_int q0 = 0; q0 < nq; q0 += chunk) {
-        const int rows = (int)std::min<da_int>(chunk, nq - q0);
+    for (int64_t at = 0; at < nq; at += block) {
+        const da_int q0 = (da_int)at;
+        const int rows = (int)std::min<da_int>(block, nq - q0);
         const T *q = dQ + (size_t)q0 * d;
         DA_HIP(err, hipMemsetAsync(bad, 0, sizeof(int), st));
         {
@@ -1012,6 +1030,7 @@ da_status NNHandle<T>::search_finish(SearchContext &ctx, const T *dQ, da_int nq,
             SearchContext &rc = *ctx.retry;
             rc.gpu = ctx.gpu;
             rc.tuning = ctx.tuning ? ctx.tuning : &ctx;
+            rc.max_bytes = ctx.max_bytes;
             // Queries the hit bits could not settle take the fused tile's passes from the first.
             rc.second_pass = !ctx.by_bits;
             SearchParams sp2 = ctx.last_params;
@@ -1255,9 +1274,17 @@ da_status NNHandle<T>::search_tiles(SearchContext &ctx, const T *dQ, da_int nq, 
         }
         nq_norm = ctx.q_norm.as<double>();
     }
-    const size_t max_keys = (size_t)64 << 20; // 512 MB of double keys per chunk
+    // 512 MB of double keys per chunk, less where the memory or the context's limit asks for it.
+    size_t max_keys = (size_t)64 << 20;
+    if (ctx.max_bytes)
+        max_keys = std::min(max_keys, ctx.max_bytes / sizeof(double));
     da_int chunk = (da_int)std::max<size_t>(1, std::min<size_t>(nq, max_keys / (size_t)n));
-    DA_HIP(err, ctx.keys.reserve((size_t)chunk * n * sizeof(double)));
+    hipError_t room = ctx.keys.reserve((size_t)chunk * n * sizeof(double));
+    while (room != hipSuccess && chunk > 1) {
+        chunk = (chunk + 1) / 2;
+        room = ctx.keys.reserve((size_t)chunk * n * sizeof(double));
+    }
+    DA_HIP(err, room);
     DA_HIP(err, ctx.sel_key.reserve((size_t)chunk * k * sizeof(double)));
     DA_HIP(err, ctx.sel_idx.reserve((size_t)chunk * k * sizeof(int)));
     double *seg_key = nullptr;

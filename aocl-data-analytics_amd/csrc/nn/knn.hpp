@@ -43,6 +43,9 @@ struct SearchContext {
     SearchParams last_params;
     std::unique_ptr<SearchContext> retry;
     bool second_pass = false;
+    // Most bytes that a launch may take for the workspaces of a query block (hit bits, keys or
+    // scores); 0: the search's own limit.
+    size_t max_bytes = 0;
     // The last launch searched by hit bits; its workspaces.
     bool by_bits = false;
     DeviceBuffer bits_q, bits_nrm, bits_a, bits_lim, bits_mins, bits_count, bits_cols, bits;
@@ -139,7 +142,9 @@ template <typename T> class NNHandle : public AlgHandle {
     // them.
     bool bits_eligible(const SearchParams &p, da_int nq, da_int k) const;
     da_status prepare_bits();
-    da_status search_bits(SearchContext &ctx, const T *dQ, da_int nq, da_int k,
+    // Queries per block of a search of nq, its workspaces reserved; 0 if they cannot be had.
+    int bits_workspaces(SearchContext &ctx, da_int nq);
+    da_status search_bits(SearchContext &ctx, const T *dQ, da_int nq, da_int k, int block,
                           bool return_distance, da_int *d_ind, T *d_dist);
     int bits_state_ = 0, bits_sample_ = 0; // state as wide_state_; rows of the sample
     DeviceBuffer bits_op_, bits_b_, bits_mu_, bits_sc_, bits_sop_, bits_sh_, bits_smap_;

@@ -118,3 +118,37 @@ def test_not_finite_rows():
     de, ie = tile.kneighbors(Q, n_neighbors=5)
     np.testing.assert_array_equal(ind, ie)
     np.testing.assert_array_equal(dist, de)
+
+
+def _free_bytes():
+    free, total = C.c_size_t(), C.c_size_t()
+    assert L.lib.hipMemGetInfo(C.byref(free), C.byref(total)) == 0
+    return free.value
+
+
+def test_blocks_and_workspaces(oracle):
+    """Several query blocks and a ragged last one, with queries left to the tile in each: the
+    results are those of the queries in slices of one block, and of the oracle. Few rows and many
+    queries: the columns of the hits, 8 KB a query, are what fills a block's 1 GiB."""
+    rng = np.random.default_rng(17)
+    means = rng.uniform(-10, 10, (16, 16))
+    X = _mixture(rng, 8192, 16, np.float32, means)
+    Q = _mixture(rng, 300007, 16, np.float32, means)
+    odd = [5, 120000, 239999, 300006]
+    Q[odd] *= 500  # beyond fp16's range at the data's scale
+    nn = aoclda.neighbors.nearest_neighbors().fit(X)
+    nn.kneighbors(Q[:8192], n_neighbors=7)
+    free = _free_bytes()
+    dist, ind = nn.kneighbors(Q, n_neighbors=7)
+    # workspaces, and the queries (19 MB) and results (17 MB) of a search on host arrays
+    assert free - _free_bytes() < (1 << 30) + (64 << 20)
+    nfb, ncand = _stats(nn)
+    assert ncand == KEEP and len(odd) <= nfb < 30000
+    for i in range(0, len(Q), 90000):
+        de, ie = nn.kneighbors(Q[i:i + 90000], n_neighbors=7)
+        np.testing.assert_array_equal(ind[i:i + 90000], ie)
+        np.testing.assert_array_equal(dist[i:i + 90000], de)
+    pick = np.concatenate([odd, rng.integers(0, len(Q), 500)])
+    ei, ed = oracle.knn(X.astype(np.float64), Q[pick].astype(np.float64), 7)
+    np.testing.assert_array_equal(ind[pick], ei)
+    np.testing.assert_allclose(dist[pick], ed, rtol=1.2e-7)  # one rounding to float
