@@ -495,6 +495,16 @@ template <typename T> da_status NNHandle<T>::prepare_search(const SearchParams &
     return da_status_success;
 }
 
+template <typename T>
+da_status NNHandle<T>::prepare_batches(const SearchParams &p, da_int nq) {
+    da_status s = prepare_search(p);
+    if (s == da_status_success && fused_eligible(1) && bits_eligible(p, nq, 1))
+        s = prepare_bits();
+    if (s == da_status_success && wide_eligible(nq, 1))
+        s = prepare_wide();
+    return s;
+}
+
 SearchContext::~SearchContext() {
     if (h_fb)
         (void)hipHostFree(h_fb);
@@ -859,23 +869,12 @@ template <typename T> da_status NNHandle<T>::prepare_bits() {
 // at a time where the memory runs out. A limit of the context's own is kept to.
 template <typename T> int NNHandle<T>::bits_workspaces(SearchContext &ctx, da_int nq) {
     const int n = n_samples_, d = n_features_;
-    const size_t own = std::max<size_t>((size_t)1 << 30, 256 * bits_query_bytes(n, d));
+    const size_t each = bits_query_bytes(n, d), own = std::max<size_t>((size_t)1 << 30, 256 * each);
     const size_t most = ctx.max_bytes ? std::min(ctx.max_bytes, own) : own;
-    for (int block = bits_block(nq, n, d, most); block > 0; block = block / 2 / 256 * 256) {
-        if (ctx.bits_q.reserve((size_t)block * wide_ksteps(d) * 64) == hipSuccess &&
-            ctx.bits_nrm.reserve((size_t)block * sizeof(double)) == hipSuccess &&
-            ctx.bits_a.reserve((size_t)block * sizeof(float)) == hipSuccess &&
-            ctx.bits_lim.reserve((size_t)block * sizeof(double)) == hipSuccess &&
-            ctx.bits_mins.reserve((size_t)block * 256 * sizeof(float)) == hipSuccess &&
-            ctx.bits_count.reserve((size_t)block * sizeof(int)) == hipSuccess &&
-            ctx.bits_cols.reserve((size_t)block * BITS_KEEP * sizeof(int)) == hipSuccess &&
-            ctx.bits.reserve((size_t)block * (bits_rows(n) / 8)) == hipSuccess)
-            return block;
-        for (DeviceBuffer *b : {&ctx.bits_q, &ctx.bits_nrm, &ctx.bits_a, &ctx.bits_lim,
-                                &ctx.bits_mins, &ctx.bits_count, &ctx.bits_cols, &ctx.bits})
-            b->release();
-    }
-    return 0;
+    int block = bits_block(nq, n, d, most);
+    while (block > 0 && ctx.block.reserve(block * each) != hipSuccess)
+        block = block / 2 / 256 * 256;
+    return block;
 }
 
 template <typename T>
@@ -889,6 +888,21 @@ da_status NNHandle<T>::search_bits(SearchContext &ctx, const T *dQ, da_int nq, d
     DA_HIP(err, ctx.fb.reserve((size_t)(nq + 2) * sizeof(int)));
     int *fbc = ctx.fb.as<int>(), *bad = fbc + nq + 1;
     DA_HIP(err, hipMemsetAsync(fbc, 0, sizeof(int), st));
+    // The block's workspaces one after another (block is a multiple of 256, so all are aligned).
+    char *at_byte = ctx.block.as<char>();
+    auto take = [&](size_t bytes) {
+        char *p = at_byte;
+        at_byte += (size_t)block * bytes;
+        return static_cast<void *>(p);
+    };
+    unsigned *bits = static_cast<unsigned *>(take(bits_rows(n) / 8));
+    int *cols = static_cast<int *>(take(BITS_KEEP * sizeof(int)));
+    float *mins = static_cast<float *>(take(256 * sizeof(float)));
+    void *qop = take((size_t)wide_ksteps(d) * 64);
+    double *nrm = static_cast<double *>(take(sizeof(double)));
+    double *lim = static_cast<double *>(take(sizeof(double)));
+    float *A = static_cast<float *>(take(sizeof(float)));
+    int *count = static_cast<int *>(take(sizeof(int)));
     const WideScale *sc = bits_sc_.as<WideScale>();
     const double ce = bits_relative_bound(d);
     for (int64_t at = 0; at < nq; at += block) {
@@ -899,27 +913,21 @@ da_status NNHandle<T>::search_bits(SearchContext &ctx, const T *dQ, da_int nq, d
         {
             KernelScope ks(*ctx.gpu, "knn_sample");
             DA_HIP(err, launch_bits_queries<T>(q, rows, d, bits_mu_.as<double>(),
-                                               bits_sc_.as<WideScale>(), ctx.bits_q.ptr(),
-                                               ctx.bits_nrm.as<double>(), st));
-            DA_HIP(err, launch_bits_sample(ctx.bits_q.ptr(), rows, bits_sop_.ptr(),
-                                           bits_sh_.as<float>(), ns, d, ctx.bits_mins.as<float>(),
-                                           st));
-            DA_HIP(err, launch_bits_guess(ctx.bits_mins.as<float>(), rows, ns, n, d,
-                                          bits_rank((int)k, n, ns), ce, ctx.bits_nrm.as<double>(),
-                                          sc, ctx.bits_a.as<float>(), ctx.bits_lim.as<double>(),
-                                          bad, ctx.bits_count.as<int>(), st));
+                                               bits_sc_.as<WideScale>(), qop, nrm, st));
+            DA_HIP(err, launch_bits_sample(qop, rows, bits_sop_.ptr(), bits_sh_.as<float>(), ns, d,
+                                           mins, st));
+            DA_HIP(err, launch_bits_guess(mins, rows, ns, n, d, bits_rank((int)k, n, ns), ce, nrm,
+                                          sc, A, lim, bad, count, st));
         }
         {
             KernelScope ks(*ctx.gpu, "knn_sweep");
-            DA_HIP(err, launch_bits_sweep(ctx.bits_q.ptr(), rows, bits_op_.ptr(), n, d,
-                                          ctx.bits_a.as<float>(), bits_b_.as<float>(), bad,
-                                          ctx.bits.as<unsigned>(), st));
+            DA_HIP(err, launch_bits_sweep(qop, rows, bits_op_.ptr(), n, d, A, bits_b_.as<float>(),
+                                          bad, bits, st));
         }
         KernelScope ks(*ctx.gpu, "knn_merge");
-        DA_HIP(err, launch_bits_columns(ctx.bits.as<unsigned>(), rows, n, bad,
-                                        ctx.bits_count.as<int>(), ctx.bits_cols.as<int>(), st));
-        DA_HIP(err, launch_bits_merge<T>(ctx.bits_count.as<int>(), ctx.bits_cols.as<int>(), rows,
-                                         bad, q, train_.as<T>(), d, k, ctx.bits_lim.as<double>(), sc, post, q0,
+        DA_HIP(err, launch_bits_columns(bits, rows, n, bad, count, cols, st));
+        DA_HIP(err, launch_bits_merge<T>(count, cols, rows, bad, q, train_.as<T>(), d, k, lim, sc,
+                                         post, q0,
                                          return_distance ? d_dist + (size_t)q0 * k : nullptr,
                                          d_ind + (size_t)q0 * k, fbc, fbc + 1, st));
     }
@@ -954,7 +962,7 @@ da_status NNHandle<T>::search_wide(SearchContext &ctx, const T *dQ, da_int nq, d
         128, std::min<int64_t>(wide_rows(nq), ((int64_t)64 << 20) / ld / 128 * 128));
     DA_HIP(err, ctx.wide_q.reserve(wide_operand_bytes(chunk, d)));
     DA_HIP(err, ctx.wide_err.reserve((size_t)chunk * sizeof(float)));
-    DA_HIP(err, ctx.keys.reserve((size_t)chunk * ld * sizeof(float)));
+    DA_HIP(err, ctx.block.reserve((size_t)chunk * ld * sizeof(float)));
     DA_HIP(err, ctx.sel_key.reserve((size_t)chunk * kc * sizeof(float)));
     DA_HIP(err, ctx.sel_idx.reserve((size_t)chunk * kc * sizeof(int)));
     DA_HIP(err, ctx.seg_key.reserve((size_t)1024 * kc * sizeof(double)));
@@ -973,11 +981,11 @@ da_status NNHandle<T>::search_wide(SearchContext &ctx, const T *dQ, da_int nq, d
                                                wide_mu_.as<double>(), sc, ctx.wide_q.ptr(),
                                                ctx.wide_err.as<float>(), st));
             DA_HIP(err, launch_wide_scores(ctx.wide_q.ptr(), rows, wide_op_.ptr(), n, d,
-                                           wide_h_.as<float>(), ctx.keys.as<float>(), st));
+                                           wide_h_.as<float>(), ctx.block.as<float>(), st));
         }
         {
             KernelScope ks(*ctx.gpu, "row_topk");
-            DA_HIP(err, launch_row_topk<float>(ctx.keys.as<float>(), ld, rows, n, kc, 0,
+            DA_HIP(err, launch_row_topk<float>(ctx.block.as<float>(), ld, rows, n, kc, 0,
                                                ctx.sel_key.as<float>(), ctx.sel_idx.as<int>(), st,
                                                ctx.seg_key.as<float>(), ctx.seg_idx.as<int>()));
         }
@@ -1031,6 +1039,7 @@ da_status NNHandle<T>::search_finish(SearchContext &ctx, const T *dQ, da_int nq,
             rc.gpu = ctx.gpu;
             rc.tuning = ctx.tuning ? ctx.tuning : &ctx;
             rc.max_bytes = ctx.max_bytes;
+            rc.block.swap(ctx.block); // this search is through with it
             // Queries the hit bits could not settle take the fused tile's passes from the first.
             rc.second_pass = !ctx.by_bits;
             SearchParams sp2 = ctx.last_params;
@@ -1046,6 +1055,7 @@ da_status NNHandle<T>::search_finish(SearchContext &ctx, const T *dQ, da_int nq,
             if (s == da_status_success)
                 s = search_finish(rc, ctx.fb_q.as<T>(), nfb, k, true, ctx.fb_ind.as<da_int>(),
                                   ctx.fb_dist.as<T>(), fused2);
+            rc.block.swap(ctx.block);
         } else {
             s = search_tiles(ctx, ctx.fb_q.as<T>(), nfb, k, true, ctx.fb_ind.as<da_int>(),
                              ctx.fb_dist.as<T>(), few);
@@ -1279,12 +1289,13 @@ da_status NNHandle<T>::search_tiles(SearchContext &ctx, const T *dQ, da_int nq, 
     if (ctx.max_bytes)
         max_keys = std::min(max_keys, ctx.max_bytes / sizeof(double));
     da_int chunk = (da_int)std::max<size_t>(1, std::min<size_t>(nq, max_keys / (size_t)n));
-    hipError_t room = ctx.keys.reserve((size_t)chunk * n * sizeof(double));
+    hipError_t room = ctx.block.reserve((size_t)chunk * n * sizeof(double));
     while (room != hipSuccess && chunk > 1) {
         chunk = (chunk + 1) / 2;
-        room = ctx.keys.reserve((size_t)chunk * n * sizeof(double));
+        room = ctx.block.reserve((size_t)chunk * n * sizeof(double));
     }
     DA_HIP(err, room);
+    double *keys = ctx.block.as<double>();
     DA_HIP(err, ctx.sel_key.reserve((size_t)chunk * k * sizeof(double)));
     DA_HIP(err, ctx.sel_idx.reserve((size_t)chunk * k * sizeof(int)));
     double *seg_key = nullptr;
@@ -1302,12 +1313,12 @@ da_status NNHandle<T>::search_tiles(SearchContext &ctx, const T *dQ, da_int nq, 
             KernelScope ks(*ctx.gpu, "pairwise_direct");
             DA_HIP(err, (launch_pairwise_direct<T, double>(
                             km, dQ + (size_t)q0 * d, train_.as<T>(), rows, n, d,
-                            ctx.keys.as<double>(), n, nq_norm ? nq_norm + q0 : nullptr, nt_norm, p,
+                            keys, n, nq_norm ? nq_norm + q0 : nullptr, nt_norm, p,
                             0, 0, st)));
         }
         {
             KernelScope ks(*ctx.gpu, "row_topk");
-            DA_HIP(err, launch_row_topk<double>(ctx.keys.as<double>(), n, rows, n, k, largest,
+            DA_HIP(err, launch_row_topk<double>(keys, n, rows, n, k, largest,
                                                 ctx.sel_key.as<double>(), ctx.sel_idx.as<int>(), st,
                                                 seg_key, seg_idx));
         }

@@ -33,7 +33,7 @@ struct SearchContext {
     // When set, the tuned maps above are read and written in this context instead: contexts
     // that search the same handle from one thread share their tuning.
     SearchContext *tuning = nullptr;
-    DeviceBuffer q_norm, keys, sel_key, sel_idx, seg_key, seg_idx, wide_q, wide_err, qpad, part_key, part_idx, part_tau, fb, fb_q,
+    DeviceBuffer q_norm, sel_key, sel_idx, seg_key, seg_idx, wide_q, wide_err, qpad, part_key, part_idx, part_tau, fb, fb_q,
         fb_ind, fb_dist, fb_bound, tau0, qc;
     // Pinned host word receiving the fallback count of the last fused launch.
     int *h_fb = nullptr;
@@ -43,12 +43,12 @@ struct SearchContext {
     SearchParams last_params;
     std::unique_ptr<SearchContext> retry;
     bool second_pass = false;
-    // Most bytes that a launch may take for the workspaces of a query block (hit bits, keys or
-    // scores); 0: the search's own limit.
+    // Workspaces of a query block: hit bits and what goes with them, keys or scores; most bytes
+    // that it may take (0: the search's own limit).
+    DeviceBuffer block;
     size_t max_bytes = 0;
-    // The last launch searched by hit bits; its workspaces.
+    // The last launch searched by hit bits.
     bool by_bits = false;
-    DeviceBuffer bits_q, bits_nrm, bits_a, bits_lim, bits_mins, bits_count, bits_cols, bits;
     ~SearchContext();
 };
 
@@ -93,6 +93,8 @@ template <typename T> class NNHandle : public AlgHandle {
     // threshold seeds of the fused tile (in place of the sample seeds).
     SearchParams params() const;
     da_status prepare_search(const SearchParams &p);
+    // Lays out what batches of up to nq queries will search, ahead of the first of them.
+    da_status prepare_batches(const SearchParams &p, da_int nq);
     da_status search_launch(SearchContext &ctx, const SearchParams &p, const T *dQ, da_int nq,
                             da_int k, bool return_distance, da_int *d_ind, T *d_dist,
                             bool &fused, const float *seed_in = nullptr);

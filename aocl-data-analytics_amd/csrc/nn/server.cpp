@@ -70,23 +70,29 @@ template <typename T> class Server : public ServerBase {
     da_status start() {
         ErrorStack *err = nn_->errors();
         params_ = nn_->params();
-        da_status s = nn_->prepare_search(params_);
-        if (s != da_status_success)
-            return s;
+        da_status s = da_status_success;
         d_ = nn_->n_features();
-        // Device bytes per batched query: the query, its padded operand rows (up to three
-        // copies of the row for the split forms), the per-split candidates (at most
-        // knn_merge_max_candidates() (key, index) pairs, 9 bytes each with the split
-        // thresholds), the fallback slots and the results.
+        // A slot has half of the bytes. Up to half of those are for what grows with the batch, per
+        // query: the query, its padded operand rows (up to three copies of the row for the split
+        // forms), the per-split candidates (at most knn_merge_max_candidates() (key, index) pairs,
+        // 9 bytes each with the split thresholds), the fallback slots and the results. The rest is
+        // for the workspaces that searches take block by block (hit bits, keys or scores).
         per_query_bytes_ = (size_t)d_ * sizeof(T) * 4 + (size_t)knn_merge_max_candidates() * 9 +
                            64 + (size_t)kmax_ * 16;
-        const size_t cap = std::max<size_t>(1, max_bytes_ / 2 / per_query_bytes_);
+        const size_t cap = std::max<size_t>(1, max_bytes_ / 4 / per_query_bytes_);
         batch_cap_ = (int)std::min<size_t>(max_batch_, cap);
+        const size_t lists = (size_t)batch_cap_ * per_query_bytes_;
+        const size_t block_bytes = std::max<size_t>(lists + 1, max_bytes_ / 2) - lists;
+        // The training operands are laid out here, not by the first request.
+        s = nn_->prepare_batches(params_, batch_cap_);
+        if (s != da_status_success)
+            return s;
         for (auto &sl : slots_) {
             s = sl.gpu.init(err);
             if (s != da_status_success)
                 return s;
             sl.ctx.gpu = &sl.gpu;
+            sl.ctx.max_bytes = block_bytes;
             DA_HIP(err, sl.dq.reserve((size_t)batch_cap_ * d_ * sizeof(T)));
             DA_HIP(err, hipHostMalloc((void **)&sl.hq, (size_t)batch_cap_ * d_ * sizeof(T)));
         }

@@ -117,3 +117,37 @@ def test_second_wait_on_a_request_is_refused():
     assert sorted(results) == [L.CODE["success"], L.CODE["invalid_input"]]
     srv._k.pop(rid)
     srv.close()
+
+
+@pytest.mark.parametrize("max_bytes", [64 << 20, 256 << 20])
+def test_device_bytes_stay_within_the_limit(max_bytes):
+    """Batches of 1,000,000 rows, hit bits of 134 KB a query: with 256 MB a slot searches them in
+    blocks, with 64 MB not even one group of 256 queries fits and the fused tile serves. The
+    training operand (64 MB) is laid out when the server is created."""
+    rng = np.random.default_rng(36)
+    means = rng.uniform(-10, 10, (32, 16))
+    Xt = (means[rng.integers(0, 32, 1000000)] +
+          rng.standard_normal((1000000, 16))).astype(np.float32)
+    Q = (means[rng.integers(0, 32, 9000)] + rng.standard_normal((9000, 16))).astype(np.float32)
+    nn = aoclda.neighbors.nearest_neighbors().fit(Xt)
+
+    def free():
+        a, b = C.c_size_t(), C.c_size_t()
+        assert L.lib.hipMemGetInfo(C.byref(a), C.byref(b)) == 0
+        return a.value
+
+    srv = nn_server(nn, max_batch_queries=4096, max_device_bytes=max_bytes)
+    before = free()
+    cuts = [0, 1, 700, 4796, 9000]
+    ks = [10, 1, 100, 16]
+    got = []
+    for _ in range(2):
+        ids = [srv.submit(Q[a:b], k) for a, b, k in zip(cuts, cuts[1:], ks)]
+        got = [srv.wait(r) for r in ids]
+    # 24 MB: allocations are rounded up to 2 MB, and the selection's own scratch
+    assert before - free() < max_bytes + (24 << 20)
+    srv.close()
+    for (dist, ind, _), a, b, k in zip(got, cuts, cuts[1:], ks):
+        de, ie = nn.kneighbors(Q[a:b], n_neighbors=k)
+        np.testing.assert_array_equal(ind, ie)
+        np.testing.assert_array_equal(dist, de)
