@@ -161,7 +161,8 @@ __global__ __launch_bounds__(1024) void wide_pack_kernel(
     const double s = sc->scale;
     const double inv = (cosn && src >= 0) ? 1.0 / cosn[src] : 1.0;
     double nn = 0.0, big = 0.0, top = 0.0;
-    bool nf = false;
+    // A norm that overflowed makes a row of zeros here and keys of 1 or NaN there.
+    bool nf = inv == 0.0;
     for (int ks = w; ks < KS; ks += nw) {
         v8h hi, lo;
 #pragma unroll

@@ -121,3 +121,29 @@ def test_data(oracle, case):
     nfb = search(oracle, X, Q, 5, "euclidean", wide)
     if expect_fallback:
         assert nfb > 0
+
+
+@pytest.mark.parametrize("where", ["rows", "queries"])
+@pytest.mark.parametrize("d", [16, 160])
+def test_cosine_norms_that_overflow(oracle, d, where):
+    """Rows of 1e200 have infinite norms: products with ordinary rows give the key 1, with large
+    ones infinity over infinity, which comes last. Key tiles in slices that are too small for the
+    approximate scores are the answer."""
+    rng = np.random.default_rng(d)
+    n, nq, k = 40000 if d == 16 else 5000, 3600 if d == 16 else 2800, 90
+    X, Q = rng.standard_normal((n, d)), rng.standard_normal((nq, d))
+    X[:, 0] -= 50  # most rows point away from the queries
+    Q[:, 0] += 50
+    X[::n // 9, 0] += 100
+    if where == "rows":
+        X[5::n // 30] *= 1e200
+        Q *= 1e150
+    else:
+        Q[::7] *= 1e200
+    nn = aoclda.neighbors.nearest_neighbors(metric="cosine", algorithm="brute").fit(X)
+    dist, ind = nn.kneighbors(Q, n_neighbors=k)
+    for i in range(0, nq, 400):
+        de, ie = nn.kneighbors(Q[i:i + 400], n_neighbors=k)
+        assert stats(nn)[1] == 0  # the general path
+        np.testing.assert_array_equal(ind[i:i + 400], ie)
+        np.testing.assert_array_equal(dist[i:i + 400], de)
