@@ -352,23 +352,23 @@ __attribute__((amdgpu_waves_per_eu(2))) void wide_scores_kernel(
 }
 
 // One wave per query: the kc selected scores (ascending, by (score, row)) -> exact keys of those
-// within 2 E of the k-th, ordered by (key, row). all: every training row was selected.
+// within 2 E of the k-th, ordered by (key, row).
 template <typename T, bool COS>
 __global__ __launch_bounds__(64) void wide_merge_kernel(
-    const float *__restrict__ skey, const int *__restrict__ sidx, int kc, int k, int all,
+    const float *__restrict__ skey, const int *__restrict__ sidx, int kc, int k,
     const T *__restrict__ Q, const T *__restrict__ Y, int d, const float *__restrict__ err,
     const double *__restrict__ qcos, const double *__restrict__ ycos, int post, int q0,
     T *__restrict__ out_dist, int *__restrict__ out_idx, int *__restrict__ fb_count,
     int *__restrict__ fb_list) {
     extern __shared__ double qrow[];
-    __shared__ double xk[128];
-    __shared__ int xi[128];
+    __shared__ double xk[WIDE_KEEP];
+    __shared__ int xi[WIDE_KEEP];
     const int q = blockIdx.x, lane = threadIdx.x;
     const float *kk = skey + (int64_t)q * kc;
     const int *ki = sidx + (int64_t)q * kc;
     const double E = (double)err[q];
     const double lim = (double)kk[k - 1] + 2.0 * E;
-    const bool certified = E < __builtin_huge_val() && (all || (double)kk[kc - 1] > lim);
+    const bool certified = E < __builtin_huge_val() && (double)kk[kc - 1] > lim;
     if (!certified) {
         if (lane == 0)
             fb_list[atomicAdd(fb_count, 1)] = q0 + q;
@@ -535,14 +535,14 @@ hipError_t launch_wide_scores(const void *PA, int nq, const void *PB, int n, int
 }
 
 template <typename T>
-hipError_t launch_wide_merge(const float *skey, const int *sidx, int nq, int kc, int k, int all,
-                             const T *Q, const T *Y, int d, const float *err, const double *qcos,
+hipError_t launch_wide_merge(const float *skey, const int *sidx, int nq, int kc, int k, const T *Q,
+                             const T *Y, int d, const float *err, const double *qcos,
                              const double *ycos, int post, int q0, T *out_dist, int *out_idx,
                              int *fb_count, int *fb_list, hipStream_t s) {
-    if (kc > 128 || k > kc || nq < 1 || (size_t)d * sizeof(double) > 60 * 1024)
+    if (kc > WIDE_KEEP || k > kc || nq < 1 || (size_t)d * sizeof(double) > 60 * 1024)
         return hipErrorInvalidValue;
     auto kern = qcos ? wide_merge_kernel<T, true> : wide_merge_kernel<T, false>;
-    hipLaunchKernelGGL(kern, dim3(nq), dim3(64), d * sizeof(double), s, skey, sidx, kc, k, all, Q,
+    hipLaunchKernelGGL(kern, dim3(nq), dim3(64), d * sizeof(double), s, skey, sidx, kc, k, Q,
                        Y, d, err, qcos, ycos, post, q0, out_dist, out_idx, fb_count, fb_list);
     return hipGetLastError();
 }
@@ -564,7 +564,7 @@ hipError_t launch_wide_merge(const float *skey, const int *sidx, int nq, int kc,
                                             float *, hipStream_t);                               \
     template hipError_t launch_ivf_queries<T>(const T *, int, int, int, const double *,          \
                                               WideScale *, void *, float *, hipStream_t);        \
-    template hipError_t launch_wide_merge<T>(const float *, const int *, int, int, int, int,     \
+    template hipError_t launch_wide_merge<T>(const float *, const int *, int, int, int,          \
                                              const T *, const T *, int, const float *,           \
                                              const double *, const double *, int, int, T *,      \
                                              int *, int *, int *, hipStream_t);

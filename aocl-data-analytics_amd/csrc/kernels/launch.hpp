@@ -356,11 +356,12 @@ hipError_t launch_wide_queries(const T *Q, int nq, int d, const double *qcos, co
 // out[q * wide_rows(n) + j] = score of the pair, all wide_rows(nq) rows written.
 hipError_t launch_wide_scores(const void *PA, int nq, const void *PB, int n, int d, const float *h,
                               float *out, hipStream_t s);
-// Exact keys of the selected rows (kc <= 128 per query, ascending by (score, row)) within twice
-// the bound of the k-th; queries that cannot be certified are appended to fb_list (as q0 + q).
+// Exact keys of the selected rows (kc <= WIDE_KEEP per query, fewer than there are rows, ascending
+// by (score, row)) within twice the bound of the k-th; queries that cannot be certified are appended
+// to fb_list (as q0 + q).
+constexpr int WIDE_KEEP = 128;
 template <typename T>
-hipError_t launch_wide_merge(const float *skey, const int *sidx, int nq, int kc, int k, int all,
-                             const T *Q, const T *Y, int d, const float *err, const double *qcos,
+hipError_t launch_wide_merge(const float *skey, const int *sidx, int nq, int kc, int k, const T *Q, const T *Y, int d, const float *err, const double *qcos,
                              const double *ycos, int post, int q0, T *out_dist, int *out_idx,
                              int *fb_count, int *fb_list, hipStream_t s);
 // ---- kNN by hit bits (operands knn_wide.hip, search knn_bits.hip) ----

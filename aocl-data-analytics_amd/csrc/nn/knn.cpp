@@ -683,9 +683,10 @@ da_status NNHandle<T>::search_launch(SearchContext &ctx, const SearchParams &sp,
             da_status s = prepare_wide();
             if (s != da_status_success)
                 return s;
-            if (wide_state_ == 1) {
+            const int block = wide_state_ == 1 ? wide_workspaces(ctx, nq) : 0;
+            if (block > 0) {
                 fused = true;
-                return search_wide(ctx, dQ, nq, k, return_distance, d_ind, d_dist);
+                return search_wide(ctx, dQ, nq, k, block, return_distance, d_ind, d_dist);
             }
         }
         return search_tiles(ctx, dQ, nq, k, return_distance, d_ind, d_dist);
@@ -793,8 +794,15 @@ template <typename T> da_status NNHandle<T>::prepare_wide() {
         return da_status_success;
     hipStream_t st = gpu->stream();
     const int n = n_samples_, d = n_features_;
-    DA_HIP(err, wide_op_.reserve(wide_operand_bytes(n, d)));
-    DA_HIP(err, wide_h_.reserve((size_t)wide_rows(n) * sizeof(float)));
+    wide_cos_ = cos;
+    if (wide_op_.reserve(wide_operand_bytes(n, d)) != hipSuccess ||
+        wide_h_.reserve((size_t)wide_rows(n) * sizeof(float)) != hipSuccess) {
+        // Without the memory the key tiles serve the searches of this training set.
+        wide_op_.release();
+        wide_h_.release();
+        wide_state_ = 2;
+        return da_status_success;
+    }
     DA_HIP(err, wide_mu_.reserve((size_t)3 * d * sizeof(double)));
     DA_HIP(err, wide_sc_.reserve(sizeof(WideScale)));
     WideScale *sc = wide_sc_.as<WideScale>();
@@ -806,7 +814,6 @@ template <typename T> da_status NNHandle<T>::prepare_wide() {
     DA_HIP(err, hipMemcpyAsync(&bad, &sc->bad, sizeof(int), hipMemcpyDeviceToHost, st));
     DA_HIP(err, hipStreamSynchronize(st));
     wide_state_ = bad ? 2 : 1;
-    wide_cos_ = cos;
     return da_status_success;
 }
 
@@ -937,15 +944,40 @@ da_status NNHandle<T>::search_bits(SearchContext &ctx, const T *dQ, da_int nq, d
     return da_status_success;
 }
 
-// Query blocks of up to 256 MB of scores. The selection keeps 64 candidates for k <= 32 and 128
-// beyond: the margin between the k-th and the last of them certifies a query.
+// Query blocks of up to 256 MB of scores or of one tile of 128 queries, fewer tiles at a time where
+// the memory runs out; with a limit of the context's own, operand rows, bounds and selections
+// count too.
+template <typename T> int NNHandle<T>::wide_workspaces(SearchContext &ctx, da_int nq) {
+    const int64_t d = n_features_, ld = wide_rows(n_samples_);
+    int64_t fit = std::max<int64_t>(128, ((int64_t)64 << 20) / ld / 128 * 128);
+    if (ctx.max_bytes) {
+        const int64_t each = ld * (int64_t)sizeof(float) + wide_ksteps(d) * 128 +
+                             (int64_t)sizeof(float) + WIDE_KEEP * 8;
+        fit = std::min<int64_t>(fit, (int64_t)ctx.max_bytes / each / 128 * 128);
+    }
+    int64_t block = std::min<int64_t>(fit, ((int64_t)nq + 127) / 128 * 128);
+    while (block > 0 &&
+           (ctx.block.reserve((size_t)block * ld * sizeof(float)) != hipSuccess ||
+            ctx.wide_q.reserve(wide_operand_bytes((int)block, (int)d)) != hipSuccess ||
+            ctx.wide_err.reserve((size_t)block * sizeof(float)) != hipSuccess ||
+            ctx.sel_key.reserve((size_t)block * WIDE_KEEP * sizeof(float)) != hipSuccess ||
+            ctx.sel_idx.reserve((size_t)block * WIDE_KEEP * sizeof(int)) != hipSuccess)) {
+        ctx.block.release();
+        ctx.wide_q.release();
+        block = block / 2 / 128 * 128;
+    }
+    return (int)block;
+}
+
+// The selection keeps 64 candidates for k <= 32 and 128 beyond: the margin between the k-th and the
+// last of them certifies a query.
 template <typename T>
-da_status NNHandle<T>::search_wide(SearchContext &ctx, const T *dQ, da_int nq, da_int k,
+da_status NNHandle<T>::search_wide(SearchContext &ctx, const T *dQ, da_int nq, da_int k, int block,
                                    bool return_distance, da_int *d_ind, T *d_dist) {
     hipStream_t st = ctx.gpu->stream();
     const int n = n_samples_, d = n_features_;
     const bool cos = metric_ == da_cosine;
-    const int kc = std::min(n, k <= 32 ? 64 : 128);
+    const int kc = k <= 32 ? WIDE_KEEP / 2 : WIDE_KEEP;
     const int post = cos || metric_ == da_sqeuclidean ? 0 : 1;
     if (!ctx.h_fb)
         DA_HIP(err, hipHostMalloc((void **)&ctx.h_fb, sizeof(int)));
@@ -958,13 +990,6 @@ da_status NNHandle<T>::search_wide(SearchContext &ctx, const T *dQ, da_int nq, d
         qcos = ctx.q_norm.as<double>();
     }
     const int64_t ld = wide_rows(n);
-    const int chunk = (int)std::max<int64_t>(
-        128, std::min<int64_t>(wide_rows(nq), ((int64_t)64 << 20) / ld / 128 * 128));
-    DA_HIP(err, ctx.wide_q.reserve(wide_operand_bytes(chunk, d)));
-    DA_HIP(err, ctx.wide_err.reserve((size_t)chunk * sizeof(float)));
-    DA_HIP(err, ctx.block.reserve((size_t)chunk * ld * sizeof(float)));
-    DA_HIP(err, ctx.sel_key.reserve((size_t)chunk * kc * sizeof(float)));
-    DA_HIP(err, ctx.sel_idx.reserve((size_t)chunk * kc * sizeof(int)));
     DA_HIP(err, ctx.seg_key.reserve((size_t)1024 * kc * sizeof(double)));
     DA_HIP(err, ctx.seg_idx.reserve((size_t)1024 * kc * sizeof(int)));
     DA_HIP(err, ctx.fb.reserve((size_t)(nq + 1) * sizeof(int)));
@@ -972,8 +997,8 @@ da_status NNHandle<T>::search_wide(SearchContext &ctx, const T *dQ, da_int nq, d
     int *fbc = ctx.fb.as<int>();
     DA_HIP(err, hipMemsetAsync(fbc, 0, sizeof(int), st));
     WideScale *sc = wide_sc_.as<WideScale>();
-    for (da_int q0 = 0; q0 < nq; q0 += chunk) {
-        const da_int rows = std::min<da_int>(chunk, nq - q0);
+    for (int64_t at = 0; at < nq; at += block) {
+        const da_int q0 = (da_int)at, rows = std::min<da_int>(block, nq - q0);
         const T *q = dQ + (size_t)q0 * d;
         {
             KernelScope ks(*ctx.gpu, "knn_wide_scores");
@@ -991,7 +1016,7 @@ da_status NNHandle<T>::search_wide(SearchContext &ctx, const T *dQ, da_int nq, d
         }
         KernelScope ks(*ctx.gpu, "knn_merge");
         DA_HIP(err, launch_wide_merge<T>(
-                        ctx.sel_key.as<float>(), ctx.sel_idx.as<int>(), rows, kc, k, kc == n, q,
+                        ctx.sel_key.as<float>(), ctx.sel_idx.as<int>(), rows, kc, k, q,
                         train_.as<T>(), d, ctx.wide_err.as<float>(), qcos ? qcos + q0 : nullptr,
                         cos ? train_cos_.as<double>() : nullptr, post, q0,
                         return_distance ? d_dist + (size_t)q0 * k : nullptr,

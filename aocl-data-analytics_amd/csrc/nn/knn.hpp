@@ -138,7 +138,9 @@ template <typename T> class NNHandle : public AlgHandle {
     // first search that uses it.
     bool wide_eligible(da_int nq, da_int k) const;
     da_status prepare_wide();
-    da_status search_wide(SearchContext &ctx, const T *dQ, da_int nq, da_int k,
+    // Queries per block of a search of nq, its workspaces reserved; 0 if they cannot be had.
+    int wide_workspaces(SearchContext &ctx, da_int nq);
+    da_status search_wide(SearchContext &ctx, const T *dQ, da_int nq, da_int k, int block,
                           bool return_distance, da_int *d_ind, T *d_dist);
     // Searches by hit bits (knn_bits.hip): the operands are laid out at the first search that uses
     // them.

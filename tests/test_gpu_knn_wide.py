@@ -147,3 +147,23 @@ def test_cosine_norms_that_overflow(oracle, d, where):
         assert stats(nn)[1] == 0  # the general path
         np.testing.assert_array_equal(ind[i:i + 400], ie)
         np.testing.assert_array_equal(dist[i:i + 400], de)
+
+
+@pytest.mark.parametrize("metric,d,nq", [("cosine", 16, 389), ("euclidean", 160, 389)])
+def test_several_blocks(metric, d, nq):
+    """Blocks of 128 queries and a ragged last one, some queries of each block beyond fp16's range;
+    slices too small for the approximate scores are the answer."""
+    rng = np.random.default_rng(d)
+    n = 400000 if d == 16 else 300000
+    X, Q = mixture(rng, n, d, np.float32), mixture(rng, nq, d, np.float32)
+    Q[[3, 130, 300, 388]] *= 3000
+    step = 250 if d == 16 else 40
+    nn = aoclda.neighbors.nearest_neighbors(metric=metric, algorithm="brute").fit(X)
+    dist, ind = nn.kneighbors(Q, n_neighbors=6)
+    nfb, ncand = stats(nn)
+    assert ncand > 0 and nfb < nq // 10
+    for i in range(0, nq, step):
+        de, ie = nn.kneighbors(Q[i:i + step], n_neighbors=6)
+        assert stats(nn)[1] == 0
+        np.testing.assert_array_equal(ind[i:i + step], ie)
+        np.testing.assert_array_equal(dist[i:i + step], de)

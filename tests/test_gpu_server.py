@@ -151,3 +151,32 @@ def test_device_bytes_stay_within_the_limit(max_bytes):
         de, ie = nn.kneighbors(Q[a:b], n_neighbors=k)
         np.testing.assert_array_equal(ind, ie)
         np.testing.assert_array_equal(dist, de)
+
+
+@pytest.mark.parametrize("max_bytes", [64 << 20, 256 << 20])
+@pytest.mark.parametrize("metric", ["euclidean", "cosine"])
+def test_device_bytes_of_wide_rows(metric, max_bytes):
+    """150,000 rows of 200 features: approximate scores in blocks of 128 queries (77 MB) with 256 MB,
+    key tiles a few queries at a time with 64 MB; clusters so tight that every query is searched
+    again."""
+    rng = np.random.default_rng(37)
+    means = rng.uniform(-10, 10, (32, 200))
+    lab, qlab = rng.integers(0, 32, 150000), rng.integers(0, 32, 700)
+    for sigma in (1.0, 1e-3):
+        Xt = (means[lab] + sigma * rng.standard_normal((150000, 200))).astype(np.float32)
+        Q = (means[qlab] + sigma * rng.standard_normal((700, 200))).astype(np.float32)
+        nn = aoclda.neighbors.nearest_neighbors(metric=metric, algorithm="brute").fit(Xt)
+
+        def free():
+            a, b = C.c_size_t(), C.c_size_t()
+            assert L.lib.hipMemGetInfo(C.byref(a), C.byref(b)) == 0
+            return a.value
+
+        srv = nn_server(nn, max_batch_queries=1024, max_device_bytes=max_bytes)
+        before = free()
+        dist, ind, _ = srv.wait(srv.submit(Q, 10))
+        assert before - free() < max_bytes + (24 << 20)
+        srv.close()
+        de, ie = nn.kneighbors(Q, n_neighbors=10)
+        np.testing.assert_array_equal(ind, ie)
+        np.testing.assert_array_equal(dist, de)
