@@ -8,9 +8,6 @@
 
 namespace dagpu {
 
-// Smallest set served by hit bits: below it the general path's few launches are as fast.
-constexpr int BITS_MIN_ROWS = 2048;
-
 // Algorithm codes of the "algorithm" option (da_neighbors_types::nn_algorithm).
 enum { DB_BRUTE = 0, DB_KD_TREE = 1, DB_BALL_TREE = 2, DB_AUTO = 3 };
 
@@ -113,7 +110,7 @@ da_status DBSCANHandle<T>::reserve_edges(long long total, long long used) {
 // the set bits. A block costs two host round trips and a tail of every kernel, a larger buffer its
 // allocation by each new handle: 100,000 x 16 fp32 take 6.2 ms in blocks of 128 MiB (the first time
 // 6.3), 5.9 of 256 MiB (6.0), 5.6 of 512 MiB (10.7), and 33 by the key tiles of the general path (40
-// GB of keys written and read).
+// GB of keys written and read). Without the memory, or with too many hits, the general path serves.
 template <typename T>
 da_status DBSCANHandle<T>::neighbour_graph_bits(int km, T thr, const double *nrm, bool &done) {
     done = false;
@@ -123,17 +120,21 @@ da_status DBSCANHandle<T>::neighbour_graph_bits(int km, T thr, const double *nrm
     const int n_pad = (n + 511) / 512 * 512;
     const size_t range_bytes = (size_t)(2 * d + 1) * sizeof(unsigned long long);
     DA_HIP(err, rsc_.reserve(sizeof(RadiusScale) + range_bytes + sizeof(unsigned long long)));
-    DA_HIP(err, rop_.reserve(radius_operand_elems(plan, n_pad) * 2));
-    DA_HIP(err, rthr_.reserve((size_t)2 * n_pad * sizeof(float)));
+    const int chunk = (int)std::max<size_t>(
+        512, std::min<size_t>((size_t)n_pad, ((size_t)256 << 20) / ((size_t)n_pad / 8) / 512 * 512));
+    if (rop_.reserve(radius_operand_elems(plan, n_pad) * 2) != hipSuccess ||
+        rthr_.reserve((size_t)2 * n_pad * sizeof(float)) != hipSuccess ||
+        rbits_.reserve((size_t)chunk * n_pad / 8) != hipSuccess) {
+        rop_.release();
+        rthr_.release();
+        return da_status_success;
+    }
     RadiusScale *sc = rsc_.as<RadiusScale>();
     unsigned long long *range = reinterpret_cast<unsigned long long *>(sc + 1);
     unsigned long long *total = range + 2 * d + 1;
     float *A = rthr_.as<float>(), *B = A + n_pad;
     const T *X = X_.as<T>();
     const double thr2 = radius_threshold2(km, thr);
-    const int chunk = (int)std::max<size_t>(
-        512, std::min<size_t>((size_t)n_pad, ((size_t)256 << 20) / ((size_t)n_pad / 8) / 512 * 512));
-    DA_HIP(err, rbits_.reserve((size_t)chunk * n_pad / 8));
     DA_HIP(err, cnt_.reserve((size_t)n_pad * sizeof(int)));
     DA_HIP(err, offs_.reserve((size_t)(n + 1) * sizeof(long long)));
     size_t scan_bytes = 0;
@@ -146,6 +147,19 @@ da_status DBSCANHandle<T>::neighbour_graph_bits(int km, T thr, const double *nrm
         DA_HIP(err, launch_radius_scale<T>(X, n, (const T *)nullptr, 0, d, km, range, sc, st));
         DA_HIP(err, launch_radius_pack<T>(X, n, n_pad, d, plan, sc, thr2, rop_.ptr(), A, B, st));
     }
+    unsigned long long set = 0, seen = 0;
+    int bad = 0;
+    {
+        KernelScope ks(*gpu, "radius_probe");
+        DA_HIP(err, hipMemsetAsync(total, 0, sizeof(*total), st));
+        DA_HIP(err, launch_radius_probe(plan, rop_.ptr(), n, rop_.ptr(), n_pad, A, B,
+                                        rbits_.as<unsigned>(), total, st));
+    }
+    DA_HIP(err, hipMemcpyAsync(&set, total, sizeof(set), hipMemcpyDeviceToHost, st));
+    DA_HIP(err, hipMemcpyAsync(&bad, &sc->bad, sizeof(int), hipMemcpyDeviceToHost, st));
+    DA_HIP(err, hipStreamSynchronize(st));
+    if (bad || !dbscan_bits_sparse(set, (int64_t)radius_probe_rows(plan) * n, d))
+        return da_status_success;
     for (int r0 = 0; r0 < n; r0 += chunk) {
         const int rows = std::min(chunk, n - r0);
         const int rows_pad = (rows + plan.row_block - 1) / plan.row_block * plan.row_block;
@@ -157,15 +171,10 @@ da_status DBSCANHandle<T>::neighbour_graph_bits(int km, T thr, const double *nrm
             DA_HIP(err, launch_radius_sweep(plan, rop_.as<char>() + radius_operand_elems(plan, r0) * 2,
                                             rows_pad, rop_.ptr(), n_pad, A + r0, B, bits, total, st));
         }
-        struct {
-            unsigned long long set;
-            int bad;
-        } h = {0, 0};
-        DA_HIP(err, hipMemcpyAsync(&h.set, total, sizeof(h.set), hipMemcpyDeviceToHost, st));
-        if (r0 == 0)
-            DA_HIP(err, hipMemcpyAsync(&h.bad, &sc->bad, sizeof(int), hipMemcpyDeviceToHost, st));
+        DA_HIP(err, hipMemcpyAsync(&set, total, sizeof(set), hipMemcpyDeviceToHost, st));
         DA_HIP(err, hipStreamSynchronize(st));
-        if (h.bad || !radius_bits_sparse(h.set, rows, n))
+        seen += set;
+        if (!dbscan_bits_sparse(seen / 2, (int64_t)n * n, d))
             return da_status_success;
         {
             KernelScope ks(*gpu, "radius_verify");
@@ -174,7 +183,7 @@ da_status DBSCANHandle<T>::neighbour_graph_bits(int km, T thr, const double *nrm
                                                 cnt, st));
         }
         // Room for every bit of the sweep; the verified ones are at most as many.
-        da_status s = reserve_edges(E + (long long)h.set, E);
+        da_status s = reserve_edges(E + (long long)set, E);
         if (s != da_status_success)
             return s;
         KernelScope ks(*gpu, "radius_fill");
@@ -212,7 +221,7 @@ template <typename T> da_status DBSCANHandle<T>::neighbour_graph(int km, T thr) 
                                         st));
         nrm = norms_.as<double>();
     }
-    if (radius_bits_metric(km) && d <= 128 && n >= BITS_MIN_ROWS && thr >= (T)0) {
+    if (radius_bits_metric(km) && d <= 128 && n >= DBSCAN_BITS_ROWS && thr >= (T)0) {
         if (km == KM_SQEUCLIDEAN_GEMM) {
             DA_HIP(err, norms_.reserve((size_t)n * sizeof(double)));
             DA_HIP(err, launch_row_sqnorms<T>(X_.as<T>(), d, n, d, norms_.as<double>(), st));

@@ -507,11 +507,35 @@ hipError_t launch_radius_verify(int metric, const T *X, const T *Y, int rows, in
 template <typename O>
 hipError_t launch_radius_bits_fill(const unsigned *bits, int rows, int n_pad, const O *offs,
                                    const int *cnt, int *ind, hipStream_t s);
-// Whether `set` of rows x n pairs are few enough to be verified one by one: up to one in 32. A
-// pair verified costs a gather of its row, some ten times a pair of the general path's tiles.
-inline bool radius_bits_sparse(unsigned long long set, int64_t rows, int64_t n) {
-    return set <= (unsigned long long)(rows * n / 32 + 65536);
+// Where the hit bits serve. Against the key tiles of the general path, over 3-128 features,
+// 2,048-1,000,000 rows, 4-8,192 queries and 0.05-10% of the pairs within the radius:
+// - A row's hits are verified by one wave, so few queries leave the chip idle (1,000,000 x 128, 32
+//   queries, 3%: 37 ms against 1.3), and packing, sweep and two answers to the host cost some 70 us
+//   whatever the size: searches win from 2,048 queries and 2^27 pairs on (131,072 x 16, 2,048
+//   queries, 0.04%: 0.41 ms against 1.17; 32,768 rows, 1%: 0.77 against 0.70).
+// - DBSCAN wins from 4,096 rows (x 64, 0.2%: 0.53 ms against 0.83; 3,000 rows: 0.49 against 0.44).
+// - A verified pair costs a gather of its row, twice where the distances are wanted, some ten to
+//   a hundred times a pair of the key tiles: with distances the two are equal at 0.5% of the pairs
+//   for 128 features, 0.7% for 64, 1.3% for 16 and more below, with 2,048 queries at half of that
+//   (131,072 x 64, 0.8%: 4.0 ms against 2.8); DBSCAN's at 2.5% for 128 features.
+//   So the share is measured on a sample of the rows before the sweep; the whole sweep may find twice
+//   as much.
+inline bool radius_bits_size(int64_t rows, int64_t n) {
+    return rows >= 2048 && n >= 2048 && rows * n >= ((int64_t)1 << 27);
 }
+constexpr int DBSCAN_BITS_ROWS = 4096;
+inline bool radius_bits_sparse(unsigned long long set, int64_t pairs, int d, int64_t queries) {
+    return set <= (unsigned long long)(pairs / ((64 + d) * (queries < 8192 ? 2 : 1)));
+}
+inline bool dbscan_bits_sparse(unsigned long long set, int64_t pairs, int d) {
+    return set <= (unsigned long long)(pairs / std::max(32, d / 3));
+}
+// The sweep over four row blocks spread over `rows` (at least 4 row blocks) rows: *total counts
+// their bits, bits (row_block rows) is scratch. The rows swept.
+inline int radius_probe_rows(const RadiusPlan &p) { return 4 * p.row_block; }
+hipError_t launch_radius_probe(const RadiusPlan &p, const void *PA, int rows, const void *PB,
+                               int n_pad, const float *A, const float *B, unsigned *bits,
+                               unsigned long long *total, hipStream_t s);
 // key[p] for the listed neighbours p in [offs[row], offs[row + 1]) of each row.
 template <typename T>
 hipError_t launch_radius_hit_keys(int metric, const T *X, const T *Y, int rows, int d,

@@ -11,9 +11,9 @@
 // that miss, so the bits that remain are those of the general path. The rows are centred (the
 // middle of each column's range) and scaled by a power of two to fp16's range first: distances
 // do not change with the centre, and the bound shrinks with the norms. Values that are not
-// finite, and searches that leave too many pairs set (a radius that holds a good part of the
+// finite, and searches that leave too many pairs set (a radius that holds some percent of the
 // rows, or rows with outliers many orders of magnitude beyond it), are reported to the caller,
-// which then takes the general path.
+// which then takes the general path (radius_bits_sparse).
 //
 // Bound: with the scaled rows x', y', n(.) the squared norm and Kp the padded width, the sum of
 // 3 Kp products and the start value in fp32 carries gamma_{3 Kp + 8} (|x'||y'| + ...), the split
@@ -609,6 +609,22 @@ hipError_t launch_radius_sweep(const RadiusPlan &p, const void *PA, int rows_pad
     }
 #undef DA_SWEEP
     return hipGetLastError();
+}
+
+hipError_t launch_radius_probe(const RadiusPlan &p, const void *PA, int rows, const void *PB,
+                               int n_pad, const float *A, const float *B, unsigned *bits,
+                               unsigned long long *total, hipStream_t s) {
+    if (rows < radius_probe_rows(p))
+        return hipErrorInvalidValue;
+    for (int q = 0; q < 4; q++) {
+        const int r0 = (int)((int64_t)q * rows / 4) / p.row_block * p.row_block;
+        const hipError_t e = launch_radius_sweep(
+            p, static_cast<const _Float16 *>(PA) + radius_operand_elems(p, r0), p.row_block, PB,
+            n_pad, A + r0, B, bits, total, s);
+        if (e != hipSuccess)
+            return e;
+    }
+    return hipSuccess;
 }
 
 template <typename T>

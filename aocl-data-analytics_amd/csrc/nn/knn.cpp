@@ -1499,11 +1499,11 @@ da_status NNHandle<T>::radius_core(const T *dQ, da_int n_queries, T radius, bool
         nq_norm = main_ctx.q_norm.as<double>();
     }
     // Hit bits from the matrix cores (radius_mfma.hip) where the metric is a function of the
-    // squared distance and the search is large enough for their preparation (2^22 pairs: below
-    // it the general path's few launches are as fast); the general path takes over for values
-    // that are not finite and for radii that hold too many rows to verify one by one.
-    bool use_bits = radius_bits_metric(km) && d <= 128 && n >= 2048 && n <= (1 << 23) &&
-                    (int64_t)n_queries * n >= ((int64_t)1 << 22) && thr >= (T)0;
+    // squared distance and the search is large enough (radius_bits_size); the general path takes
+    // over for values that are not finite, for radii that hold too many rows to verify one by one
+    // and where the memory does not suffice.
+    bool use_bits = radius_bits_metric(km) && d <= 128 && n <= (1 << 23) &&
+                    radius_bits_size(n_queries, n) && thr >= (T)0;
     const RadiusPlan plan = radius_plan(std::min<int>(d, 128));
     const int nw = (n + 63) / 64;
     const int n_pad = (n + 511) / 512 * 512, q_pad = (n_queries + 511) / 512 * 512;
@@ -1511,33 +1511,55 @@ da_status NNHandle<T>::radius_core(const T *dQ, da_int n_queries, T radius, bool
     unsigned long long *set_total = nullptr;
     float *A = nullptr, *B = nullptr;
     const size_t opb = use_bits ? radius_operand_elems(plan, n_pad) * 2 : 0;
+    const da_int bits_chunk = (da_int)std::max<int64_t>(
+        256, std::min<int64_t>({(int64_t)q_pad, ((int64_t)128 << 20) / (n_pad / 8) / 256 * 256,
+                                (int64_t)std::numeric_limits<int>::max() / n / 256 * 256}));
+    if (use_bits &&
+        (rnn_op_.reserve(opb + radius_operand_elems(plan, q_pad) * 2) != hipSuccess ||
+         rnn_thr_.reserve(((size_t)q_pad + n_pad) * sizeof(float)) != hipSuccess ||
+         rnn_bits_.reserve((size_t)bits_chunk * n_pad / 8) != hipSuccess)) {
+        rnn_op_.release();
+        rnn_thr_.release();
+        use_bits = false;
+    }
+    unsigned long long set = 0, seen = 0;
     if (use_bits) {
         const size_t range_words = (size_t)2 * d + 1;
         DA_HIP(err, rnn_scale_.reserve(sizeof(RadiusScale) +
                                        (range_words + 1) * sizeof(unsigned long long)));
-        DA_HIP(err, rnn_op_.reserve(opb + radius_operand_elems(plan, q_pad) * 2));
-        DA_HIP(err, rnn_thr_.reserve(((size_t)q_pad + n_pad) * sizeof(float)));
         rsc = rnn_scale_.as<RadiusScale>();
         unsigned long long *range = reinterpret_cast<unsigned long long *>(rsc + 1);
         set_total = range + range_words;
         A = rnn_thr_.as<float>();
         B = A + q_pad;
         const double thr2 = radius_threshold2(km, thr);
-        KernelScope ks(*gpu, "radius_pack");
-        DA_HIP(err, launch_radius_scale<T>(train_.as<T>(), n, dQ, n_queries, d, km, range, rsc, st));
-        DA_HIP(err, launch_radius_pack<T>(train_.as<T>(), n, n_pad, d, plan, rsc, thr2,
-                                          rnn_op_.ptr(), nullptr, B, st));
-        DA_HIP(err, launch_radius_pack<T>(dQ, n_queries, q_pad, d, plan, rsc, thr2,
-                                          rnn_op_.as<char>() + opb, A, nullptr, st));
+        {
+            KernelScope ks(*gpu, "radius_pack");
+            DA_HIP(err, launch_radius_scale<T>(train_.as<T>(), n, dQ, n_queries, d, km, range, rsc,
+                                               st));
+            DA_HIP(err, launch_radius_pack<T>(train_.as<T>(), n, n_pad, d, plan, rsc, thr2,
+                                              rnn_op_.ptr(), nullptr, B, st));
+            DA_HIP(err, launch_radius_pack<T>(dQ, n_queries, q_pad, d, plan, rsc, thr2,
+                                              rnn_op_.as<char>() + opb, A, nullptr, st));
+        }
+        int bad = 0;
+        {
+            KernelScope ks(*gpu, "radius_probe");
+            DA_HIP(err, hipMemsetAsync(set_total, 0, sizeof(*set_total), st));
+            DA_HIP(err, launch_radius_probe(plan, rnn_op_.as<char>() + opb, n_queries, rnn_op_.ptr(),
+                                            n_pad, A, B, rnn_bits_.as<unsigned>(), set_total, st));
+        }
+        DA_HIP(err, hipMemcpyAsync(&set, set_total, sizeof(set), hipMemcpyDeviceToHost, st));
+        DA_HIP(err, hipMemcpyAsync(&bad, &rsc->bad, sizeof(int), hipMemcpyDeviceToHost, st));
+        DA_HIP(err, hipStreamSynchronize(st));
+        use_bits = !bad && radius_bits_sparse(
+                              set, (int64_t)radius_probe_rows(plan) * n, d, n_queries);
     }
     // Query blocks whose key tile stays within 256 MB (and 2^28 entries), or whose bits stay
     // within 128 MiB and whose neighbours fit 32-bit offsets.
     const size_t max_keys = ((size_t)256 << 20) / sizeof(T);
     const da_int tile_chunk = (da_int)std::max<size_t>(
         1, std::min<size_t>(n_queries, std::min<size_t>(max_keys, (size_t)1 << 28) / (size_t)n));
-    const da_int bits_chunk = (da_int)std::max<int64_t>(
-        256, std::min<int64_t>({(int64_t)q_pad, ((int64_t)128 << 20) / (n_pad / 8) / 256 * 256,
-                                (int64_t)std::numeric_limits<int>::max() / n / 256 * 256}));
     const int seg = radius_segment_len(n), nseg = (n + seg - 1) / seg;
     std::vector<int> scnt, soff, off(std::max(tile_chunk, use_bits ? bits_chunk : 0) + 1);
     for (da_int q0 = 0; q0 < n_queries;) {
@@ -1546,11 +1568,8 @@ da_status NNHandle<T>::radius_core(const T *dQ, da_int n_queries, T radius, bool
         off[0] = 0;
         if (use_bits) {
             const int rows_pad = (rows + plan.row_block - 1) / plan.row_block * plan.row_block;
-            DA_HIP(err, rnn_bits_.reserve((size_t)rows_pad * n_pad / 8));
             DA_HIP(err, rnn_cnt_.reserve((size_t)rows_pad * sizeof(int)));
             unsigned *bits = rnn_bits_.as<unsigned>();
-            unsigned long long set = 0;
-            int bad = 0;
             scnt.resize(rows);
             {
                 KernelScope ks(*gpu, "radius_sweep");
@@ -1561,10 +1580,9 @@ da_status NNHandle<T>::radius_core(const T *dQ, da_int n_queries, T radius, bool
                                 rows_pad, rnn_op_.ptr(), n_pad, A + q0, B, bits, set_total, st));
             }
             DA_HIP(err, hipMemcpyAsync(&set, set_total, sizeof(set), hipMemcpyDeviceToHost, st));
-            if (q0 == 0)
-                DA_HIP(err, hipMemcpyAsync(&bad, &rsc->bad, sizeof(int), hipMemcpyDeviceToHost, st));
             DA_HIP(err, hipStreamSynchronize(st));
-            if (bad || !radius_bits_sparse(set, rows, n)) {
+            seen += set;
+            if (!radius_bits_sparse(seen / 2, (int64_t)n_queries * n, d, n_queries)) {
                 use_bits = false; // this block and the rest through the key tiles
                 continue;
             }
