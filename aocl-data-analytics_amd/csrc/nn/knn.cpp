@@ -237,11 +237,13 @@ template <typename T> int NNHandle<T>::split_cap(int kc) const {
 // (about 300 us, with few workgroups). Measured over 5-128 features, 500-30,000 rows, 100-10,000
 // queries, k = 5 and 50, in fp64, fp32 and fp16c: the tiles win by 1.1x to 15x wherever
 // queries x rows x (features + 16) is at most 2^30 (2,068 x 2,125 x 20: 62 against 362 us), and
-// lose from about 3e9 on. Training sets beyond 65,536 rows keep the fused tile (a row of keys is
-// selected from by one workgroup), and so do searches that choose an operand form or set one of
-// the tile's options.
+// lose from about 3e9 on. A row of keys takes a workgroup 8 ns, however short; the fused tile 4 ns a
+// query beside its start, which grows with the rows of a split: the two meet at 13,000 queries for
+// 16 rows (131,072: 1,040 against 600 us), 33,000 for 200 and 50,000 for 500. Training sets beyond
+// 65,536 rows keep the fused tile (a row of keys is selected from by one workgroup), and so do
+// searches that choose an operand form or set one of the tile's options.
 template <typename T> bool NNHandle<T>::tiles_faster(da_int nq) const {
-    return n_samples_ <= 65536 &&
+    return n_samples_ <= 65536 && nq <= 8192 + 64 * (int64_t)n_samples_ &&
            (double)nq * n_samples_ * (n_features_ + 16) <= (double)((int64_t)1 << 30);
 }
 

@@ -91,6 +91,24 @@ def test_gemm_metrics_order_by_direct_differences(oracle, metric, dtype, n, nq):
     assert np.all(dist[:9, 0] == 0)
 
 
+@pytest.mark.parametrize("n,nq,tiles", [(16, 9000, True), (16, 9300, False), (200, 20000, True),
+                                        (200, 22000, False), (1000, 30000, True)])
+def test_small_searches_with_many_queries(oracle, n, nq, tiles):
+    """Key tiles up to 8,192 + 64 n queries, the fused tile beyond; the same neighbours either
+    way."""
+    rng = np.random.default_rng(nq)
+    Xt, Xq = rng.standard_normal((n, 4)), rng.standard_normal((nq, 4))
+    nn = aoclda.neighbors.nearest_neighbors().fit(Xt)
+    L.check(L.lib.da_amd_profile_enable(nn.handle.h, 1))
+    dist, ind = nn.kneighbors(Xq, n_neighbors=3)
+    ms, cnt = C.c_double(), L.da_int()
+    st = L.lib.da_amd_profile_get(nn.handle.h, b"pairwise_direct", C.byref(ms), C.byref(cnt))
+    assert (st == 0 and cnt.value > 0) == tiles
+    ei, ed = oracle.knn(Xt, Xq, 3)
+    np.testing.assert_array_equal(ind, ei)
+    np.testing.assert_allclose(dist, ed, rtol=1e-14)
+
+
 @pytest.mark.parametrize("k", [1, 2, 64, 300])
 def test_k_edges(oracle, k):
     rng = np.random.default_rng(4)
