@@ -220,6 +220,7 @@ da_status NNHandle<T>::set_data(da_int n_samples, da_int n_features, const T *X,
     ypad_prec_ = -1;
     wide_state_ = 0;
     bits_state_ = 0;
+    bits_backoff_ = wide_backoff_ = {};
     return prepare_fused(tile_prec());
 }
 
@@ -666,8 +667,8 @@ da_status NNHandle<T>::search_launch(SearchContext &ctx, const SearchParams &sp,
     ctx.last_fallback = 0;
     ctx.last_candidates = 0;
     ctx.last_params = sp;
-    ctx.by_bits = false;
-    if (fused && !ctx.second_pass && bits_eligible(sp, nq, k)) {
+    ctx.by_bits = ctx.by_wide = false;
+    if (fused && !ctx.second_pass && bits_eligible(sp, nq, k) && !bits_backoff_.skipped()) {
         da_status s = prepare_bits();
         if (s != da_status_success)
             return s;
@@ -681,7 +682,7 @@ da_status NNHandle<T>::search_launch(SearchContext &ctx, const SearchParams &sp,
         return search_tiles(ctx, dQ, nq, k, return_distance, d_ind, d_dist, true);
     }
     if (!fused) {
-        if (!ctx.second_pass && wide_eligible(nq, k)) {
+        if (!ctx.second_pass && wide_eligible(nq, k) && !wide_backoff_.skipped()) {
             da_status s = prepare_wide();
             if (s != da_status_success)
                 return s;
@@ -1025,6 +1026,7 @@ da_status NNHandle<T>::search_wide(SearchContext &ctx, const T *dQ, da_int nq, d
                         d_ind + (size_t)q0 * k, fbc, fbc + 1, st));
     }
     DA_HIP(err, hipMemcpyAsync(ctx.h_fb, fbc, sizeof(int), hipMemcpyDeviceToHost, st));
+    ctx.by_wide = true;
     ctx.last_candidates = kc;
     return da_status_success;
 }
@@ -1033,13 +1035,17 @@ template <typename T>
 da_status NNHandle<T>::search_finish(SearchContext &ctx, const T *dQ, da_int nq, da_int k,
                                      bool return_distance, da_int *d_ind, T *d_dist,
                                      bool fused) {
-    (void)nq;
     if (!fused)
         return da_status_success;
     hipStream_t st = ctx.gpu->stream();
     DA_HIP(err, hipStreamSynchronize(st));
     const int nfb = *ctx.h_fb;
     ctx.last_fallback = nfb;
+    // More than half searched again: the other path alone is faster.
+    if (ctx.by_bits)
+        bits_backoff_.report(nfb > nq / 2);
+    if (ctx.by_wide)
+        wide_backoff_.report(nfb > nq / 2);
     if (nfb > 0) {
         // The uncertified queries (listed by the merge kernel): gather their rows, search
         // them again, scatter the results back. The first pass is followed by a second

@@ -5,6 +5,7 @@
 #include "../core/handle.hpp"
 #include "../kernels/launch.hpp"
 #include <functional>
+#include <algorithm>
 #include <map>
 #include <memory>
 #include <vector>
@@ -47,9 +48,21 @@ struct SearchContext {
     // that it may take (0: the search's own limit).
     DeviceBuffer block;
     size_t max_bytes = 0;
-    // The last launch searched by hit bits.
-    bool by_bits = false;
+    // The last launch searched by hit bits, by approximate scores.
+    bool by_bits = false, by_wide = false;
     ~SearchContext();
+};
+
+// Keeps a search that turned out to be of no use for the data (most queries had to be searched
+// again) from being tried every time: 1, 2, 4, ... up to 16 searches go straight to the other path
+// before the next trial. The results are the same either way.
+struct SearchBackoff {
+    int skip = 0, next = 1;
+    bool skipped() { return skip > 0 && skip-- > 0; }
+    void report(bool useless) {
+        skip = useless ? next : 0;
+        next = useless ? std::min(16, 2 * next) : 1;
+    }
 };
 
 template <typename T> class NNHandle : public AlgHandle {
@@ -153,6 +166,7 @@ template <typename T> class NNHandle : public AlgHandle {
     int bits_state_ = 0, bits_sample_ = 0; // state as wide_state_; rows of the sample
     DeviceBuffer bits_op_, bits_b_, bits_mu_, bits_sc_, bits_sop_, bits_sh_, bits_smap_;
     int wide_state_ = 0; // 0: not laid out, 1: ready, 2: the data need the general path
+    SearchBackoff bits_backoff_, wide_backoff_;
     int wide_cos_ = -1;  // metric of the layout: cosine or euclidean
     DeviceBuffer wide_op_, wide_h_, wide_mu_, wide_sc_;
 

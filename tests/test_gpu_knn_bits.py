@@ -152,3 +152,32 @@ def test_blocks_and_workspaces(oracle):
     ei, ed = oracle.knn(X.astype(np.float64), Q[pick].astype(np.float64), 7)
     np.testing.assert_array_equal(ind[pick], ei)
     np.testing.assert_allclose(dist[pick], ed, rtol=1.2e-7)  # one rounding to float
+
+
+@pytest.mark.parametrize("n", [8192, 20000, 30000])
+def test_tight_clusters_are_not_tried_every_time(n):
+    """Clusters that fp16 cannot resolve hold thousands of hits a query: the sample shows it at
+    any number of rows (every query is listed before the sweep), and of the searches that follow
+    1, 2, 4, ... go straight to the fused tile before the bits are tried again."""
+    rng = np.random.default_rng(n)
+    means = rng.uniform(-10, 10, (2, 20))
+    X = means[rng.integers(0, 2, n)] + 1e-4 * rng.standard_normal((n, 20))
+    Q = means[rng.integers(0, 2, 6000)] + 1e-4 * rng.standard_normal((6000, 20))
+    nn = aoclda.neighbors.nearest_neighbors().fit(X)
+    tile = aoclda.neighbors.nearest_neighbors(seed_thresholds=False).fit(X)
+    de, ie = tile.kneighbors(Q, n_neighbors=5)
+    tried = []
+    for _ in range(6):
+        dist, ind = nn.kneighbors(Q, n_neighbors=5)
+        np.testing.assert_array_equal(ind, ie)
+        np.testing.assert_array_equal(dist, de)
+        nfb, ncand = _stats(nn)
+        tried.append(ncand == KEEP)
+        assert not tried[-1] or nfb == len(Q)
+    assert tried == [True, False, True, False, False, True]
+    # new training rows are tried at once, and stay with the bits
+    X = rng.uniform(-10, 10, (n, 20))
+    nn.fit(X)
+    for _ in range(3):
+        nn.kneighbors(X[:6000], n_neighbors=5)
+        assert _stats(nn)[1] == KEEP and _stats(nn)[0] < 600

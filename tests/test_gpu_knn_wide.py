@@ -167,3 +167,20 @@ def test_several_blocks(metric, d, nq):
         assert stats(nn)[1] == 0
         np.testing.assert_array_equal(ind[i:i + step], ie)
         np.testing.assert_array_equal(dist[i:i + step], de)
+
+
+def test_tight_clusters_are_not_tried_every_time():
+    """Where most queries are searched again, the next searches take the key tiles at once."""
+    rng = np.random.default_rng(4)
+    means = rng.uniform(-10, 10, (8, 200))
+    X = (means[rng.integers(0, 8, 9000)] + 1e-3 * rng.standard_normal((9000, 200))).astype(np.float32)
+    Q = (means[rng.integers(0, 8, 1300)] + 1e-3 * rng.standard_normal((1300, 200))).astype(np.float32)
+    nn = aoclda.neighbors.nearest_neighbors(algorithm="brute").fit(X)
+    got = []
+    for _ in range(4):
+        got.append(nn.kneighbors(Q, n_neighbors=5) + stats(nn))
+    assert [g[3] > 0 for g in got] == [True, False, True, False]
+    assert got[0][2] > len(Q) // 2
+    for g in got[1:]:
+        np.testing.assert_array_equal(g[1], got[0][1])
+        np.testing.assert_array_equal(g[0], got[0][0])
