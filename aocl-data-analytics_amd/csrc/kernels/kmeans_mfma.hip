@@ -431,6 +431,9 @@ __global__ __launch_bounds__(256) void kmeans_recheck_kernel(
                 bl = oi;
             }
         }
+        // A sample that is not finite, or whose distances overflow, is nearer to no centre: the
+        // first, as in the exact assignment.
+        bl = bl < k ? bl : 0;
         if (lane == 0) {
             labels[i] = bl;
             if (prev && prev[i] != bl)

@@ -261,3 +261,20 @@ def test_batch_argument_errors():
                                        [np.zeros((2, 65), dtype=np.float32)])
     with pytest.raises(KeyError):
         aoclda.clustering.kmeans_batch([X], [X[:2].copy()], precision="fp8")
+
+
+@pytest.mark.parametrize("dtype,precision", [(np.float32, "working"), (np.float32, "bf16"),
+                                             (np.float64, "working")])
+def test_samples_that_are_not_finite(dtype, precision):
+    """Samples with NaN or infinities belong to the first centre, the others to theirs."""
+    rng = np.random.default_rng(12)
+    means = np.array([[-9.0] * 20, [9.0] * 20, [30.0] * 20])
+    lab = rng.integers(0, 3, 5000)
+    X = (means[lab] + rng.standard_normal((5000, 20))).astype(dtype)
+    odd = [7, 100, 4999]
+    X[7, 3], X[100, 0], X[4999, 19] = np.nan, np.inf, -np.inf
+    km = aoclda.clustering.kmeans(n_clusters=3, C=means.astype(dtype), max_iter=1, tol=0.0,
+                                  precision=precision).fit(X)
+    lab[odd] = 0
+    np.testing.assert_array_equal(km.labels, lab)
+    np.testing.assert_array_equal(km.predict(X), lab)
