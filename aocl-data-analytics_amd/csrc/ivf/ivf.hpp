@@ -58,9 +58,11 @@ template <typename T> class ApproxNNHandle : public AlgHandle {
     // Buffers of the MFMA assignment of added vectors: padded rows, padded centroids and
     // their -|c|^2/2, counters, the re-check list and the transposed centroids.
     DeviceBuffer as_x_, as_c_, as_h_, as_small_, as_list_, as_ct_;
-    // Matrix-core search: operand rows of the lists, rebuilt by the first search after a change of
-    // the index (0 none, 1 usable, 2 the data do not fit), and the workspaces of a query block.
+    // Matrix-core search: operand rows of the lists, rebuilt after a change of the index by its
+    // first large or its second search (0 none, 1 usable, 2 the data do not fit or the memory does
+    // not suffice), and the workspaces of a query block.
     int tiles_state_ = 0;
+    bool searched_ = false; // since the last change
     std::vector<int> tile_off_;
     DeviceBuffer tile_off_d_, tile_map_, tile_op_, tile_h_, tile_mu_, tile_sc_, tile_q_, tile_err_,
         tile_scores_, tile_work_, fb_, fb_q_, fb_ind_, fb_dist_;
