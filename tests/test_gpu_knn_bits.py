@@ -1,5 +1,6 @@
 """kNN by hit bits (large searches of up to 128 features, squared-euclidean metrics): bit for bit the
-neighbours of the fused tile (which serves a handle with a tile option set), and of the oracle."""
+neighbours of the fused tile (which serves a handle with a tile option set), and of the oracle. The
+fused tile also serves the queries that the bits list, so tests on ordinary data bound their number."""
 import ctypes as C
 
 import numpy as np
@@ -107,7 +108,7 @@ def test_ranges_and_tight_clusters(scale, shift):
 
 
 def test_not_finite_rows():
-    """Rows that are not finite keep the search on the tile's path."""
+    """A row so large that fp16 cannot hold the others beside it: the bits list every query."""
     rng = np.random.default_rng(13)
     X = rng.standard_normal((20000, 20)).astype(np.float32)
     X[77, 3] = 1e38
@@ -181,3 +182,43 @@ def test_tight_clusters_are_not_tried_every_time(n):
     for _ in range(3):
         nn.kneighbors(X[:6000], n_neighbors=5)
         assert _stats(nn)[1] == KEEP and _stats(nn)[0] < 600
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+def test_nan_and_infinity(dtype):
+    """Training rows that are not finite keep the search on the tile's path; queries that are not
+    finite are listed and come out as the tile's, the others untouched by them."""
+    rng = np.random.default_rng(14)
+    X = rng.standard_normal((20000, 20)).astype(dtype)
+    Q = rng.standard_normal((6100, 20)).astype(dtype)
+    odd = [3, 4, 5, 6099]
+    Q[3, 1], Q[4, 0], Q[5, 19], Q[6099] = np.nan, np.inf, -np.inf, np.nan
+    nfb = _compare(X, Q, 5, most_listed=600)
+    assert nfb >= len(odd)
+    X[77, 3], X[78, 0], X[19999, 19] = np.nan, np.inf, -np.inf
+    nn = aoclda.neighbors.nearest_neighbors().fit(X)
+    tile = aoclda.neighbors.nearest_neighbors(seed_thresholds=False).fit(X)
+    for part in (Q, np.delete(Q, odd, axis=0)):
+        dist, ind = nn.kneighbors(part, n_neighbors=5)
+        assert _stats(nn)[1] != KEEP
+        de, ie = tile.kneighbors(part, n_neighbors=5)
+        np.testing.assert_array_equal(ind, ie)
+        np.testing.assert_array_equal(dist, de)
+    assert not np.isin(ind, [77, 78, 19999]).any()
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+@pytest.mark.parametrize("n,d,k", [(20011, 20, 10), (16385, 64, 100), (66000, 100, 1),
+                                   (140000, 16, 20), (8192, 128, 128)])
+def test_ordinary_data_against_the_oracle(oracle, dtype, n, d, k):
+    """Fewer than one query in ten is left to the tile, and none comes out differently: all by the
+    tile, and the first 150 by the oracle."""
+    rng = np.random.default_rng(n + d)
+    means = rng.uniform(-10, 10, (16, d))
+    X = _mixture(rng, n, d, dtype, means)
+    Q = _mixture(rng, _queries(n, d), d, dtype, means)
+    _compare(X, Q, k, most_listed=len(Q) // 10)
+    dist, ind = aoclda.neighbors.nearest_neighbors().fit(X).kneighbors(Q, n_neighbors=k)
+    ei, ed = oracle.knn(X.astype(np.float64), Q[:150].astype(np.float64), k)
+    np.testing.assert_array_equal(ind[:150], ei)
+    np.testing.assert_allclose(dist[:150], ed, rtol=1e-14 if dtype == np.float64 else 1.2e-7)
