@@ -16,16 +16,16 @@
 // too (euclidean_gemm_distance.cpp:59-230, cosine_distance.cpp:66-161,
 // inner_product_distance.cpp) and are stored as computed.
 //
-// Work decomposition: a 256-thread workgroup owns a TB x TB output tile (TB = 128, or 64 where
-// fewer than 1,024 tiles of 128 would leave CUs idle), and each wave accumulates a quarter of it in
-// 16 x 16 blocks on the matrix cores. 16-deep k slices of X and Y lie in LDS in the input type
-// (widened when read) in two buffers: the next slice is loaded to registers before the products
-// of this one and stored after them, with one barrier a slice. Bound by the matrix cores (a product
-// occupies its SIMD for 64 cycles). 8,192 x 8,192 x 256 fp32: 675 us; with one buffer, a tile of
-// 64 and loads waited for between barriers 920. Operand
+// Work decomposition: a 256-thread workgroup owns a TB x TB output tile, and each wave accumulates a
+// quarter of it in 16 x 16 blocks on the matrix cores. 16-deep k slices of X and Y lie in LDS in the
+// input type (widened when read) in two buffers: the next slice is loaded to registers before the
+// products of this one and stored after them, with one barrier a slice. Bound by the matrix cores (a
+// product occupies its SIMD for 64 cycles) and, for few features, by the epilogue. 8,192 x 8,192 x
+// 256 fp32: 626 us; with one buffer and loads waited for between barriers 920. Operand
 // layout of v_mfma_f64_16x16x4f64 for lane l: A[l % 16][l / 16], B[l / 16][l % 16]; the
 // accumulator's register r holds C[4 r + l / 16][l % 16].
 #include "launch.hpp"
+#include <algorithm>
 #include <cstdint>
 #include <hip/hip_runtime.h>
 
@@ -175,20 +175,29 @@ __attribute__((amdgpu_waves_per_eu(2))) void pairwise_mfma_kernel(
     }
 }
 
-// Tile edge and load width of a call.
+// Tile edge and load width of a call. Tiles of 128 halve the operand reads but leave fewer
+// workgroups on a CU, so that epilogues overlap less with products: 8,192 x 8,192 fp32 euclidean
+// by tiles of 64 and 128: 148 and 204 us with 3 features, 238 and 292 with 64, 626 and 676 with 256,
+// equal with 512; inner products 1,205 and 1,169 with 512, 4,096 x 4,096 fp64 699 and 646 with 1,024.
 template <typename T, typename TY, typename U, int METRIC>
 void pairwise_mfma_run(const T *X, const TY *Y, int m, int n, int k, U *D, int64_t ldd,
                        const double *nx, const double *ny, int zero_diag, int diag_offset,
                        double gam, double inv_rtol, hipStream_t s) {
     auto run = [&](auto kern, int tb) {
-        hipLaunchKernelGGL(kern, dim3((n + tb - 1) / tb, (m + tb - 1) / tb), dim3(256), 0, s, X, Y,
-                           m, n, k, D, ldd, nx, ny, zero_diag, diag_offset, gam, inv_rtol);
+        // At most 65,535 row tiles per launch (the grid's y extent).
+        const int64_t step = (int64_t)65535 * tb;
+        for (int64_t i0 = 0; i0 < m; i0 += step) {
+            const int mm = (int)std::min<int64_t>(step, m - i0);
+            hipLaunchKernelGGL(kern, dim3((n + tb - 1) / tb, (mm + tb - 1) / tb), dim3(256), 0, s,
+                               X + i0 * k, Y, mm, n, k, D + i0 * ldd, ldd, nx ? nx + i0 : nx, ny,
+                               zero_diag, diag_offset + (int)i0, gam, inv_rtol);
+        }
     };
     auto aligned = [&](const void *p, size_t size) {
         return ((uintptr_t)p & 15) == 0 && k * size % 16 == 0;
     };
     const bool vec = aligned(X, sizeof(T)) && aligned(Y, sizeof(TY));
-    const bool large = (int64_t)((m + 127) / 128) * ((n + 127) / 128) >= 1024;
+    const bool large = k >= 512 && (int64_t)((m + 127) / 128) * ((n + 127) / 128) >= 1024;
     if (large)
         run(vec ? pairwise_mfma_kernel<T, TY, U, METRIC, 128, true>
                 : pairwise_mfma_kernel<T, TY, U, METRIC, 128, false>, 128);
@@ -240,18 +249,9 @@ hipError_t launch_inner_mfma(const TX *X, const TY *Y, int m, int n, int k, floa
                              int64_t ldd, hipStream_t s) {
     if (m <= 0 || n <= 0)
         return hipSuccess;
-    // At most 65,535 row tiles per launch (the grid's y extent).
-    const int chunk = 65535 * 64;
-    for (int i0 = 0; i0 < m; i0 += chunk) {
-        const int mm = m - i0 < chunk ? m - i0 : chunk;
-        pairwise_mfma_run<TX, TY, float, KM_INNER>(X + (int64_t)i0 * k, Y, mm, n, k,
-                                                   D + (int64_t)i0 * ldd, ldd, nullptr, nullptr, 0,
-                                                   0, 0.0, 0.0, s);
-        const hipError_t e = hipGetLastError();
-        if (e != hipSuccess)
-            return e;
-    }
-    return hipSuccess;
+    pairwise_mfma_run<TX, TY, float, KM_INNER>(X, Y, m, n, k, D, ldd, nullptr, nullptr, 0, 0, 0.0,
+                                               0.0, s);
+    return hipGetLastError();
 }
 template hipError_t launch_inner_mfma<double, float>(const double *, const float *, int, int,
                                                      int, float *, int64_t, hipStream_t);

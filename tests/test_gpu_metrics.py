@@ -177,3 +177,29 @@ def test_gemm_tiles(dtype, m, n, k):
     np.testing.assert_allclose(D, E, rtol=1e-12 if dtype == np.float64 else 6e-7, atol=0)
     G = aoclda.metrics.pairwise_distances(X, Y, metric="inner_product")
     np.testing.assert_allclose(G, A @ B.T, rtol=RTOL[dtype], atol=RTOL[dtype] * k)
+
+
+@pytest.mark.parametrize("dtype", [np.float64, np.float32])
+@pytest.mark.parametrize("m,n,k", [(4097, 4095, 513), (4100, 4224, 512), (3969, 4300, 520),
+                                   (4096, 4096, 511), (65535 * 64 + 70, 3, 2)])
+def test_gemm_tiles_of_many_features(dtype, m, n, k):
+    """Tiles of 128 (from 512 features and 1,024 tiles on) at their edges, tiles of 64 just below,
+    and more row tiles than one launch takes."""
+    rng = np.random.default_rng(m + k)
+    X = rng.standard_normal((m, k)).astype(dtype)
+    Y = rng.standard_normal((n, k)).astype(dtype)
+    A, B = X.astype(np.float64), Y.astype(np.float64)
+    G = A @ B.T
+    nx, ny = (A * A).sum(1), (B * B).sum(1)
+    D = aoclda.metrics.pairwise_distances(X, Y, metric="inner_product")
+    # k + 2 roundings of sums of at most |x||y|, in double on both sides; one to the type
+    scale = np.sqrt(nx)[:, None] * np.sqrt(ny)[None]
+    tol = 2 * (k + 2) * 2.0 ** -53 + (2.0 ** -24 if dtype == np.float32 else 0)
+    assert np.all(np.abs(D - G) <= tol * scale)
+    if k > 2:
+        D = aoclda.metrics.pairwise_distances(X, Y, metric="cosine")
+        assert np.all(np.abs(D - (1 - G / scale)) <= 2 * tol)
+    else:
+        D = aoclda.metrics.pairwise_distances(X, Y, metric="sqeuclidean")
+        E = sum((A[:, l, None] - B[None, :, l]) ** 2 for l in range(k))
+        np.testing.assert_allclose(D, E, rtol=1e-12 if dtype == np.float64 else 6e-7, atol=0)
