@@ -510,9 +510,11 @@ hipError_t launch_radius_bits_fill(const unsigned *bits, int rows, int n_pad, co
 // Where the hit bits serve. Against the key tiles of the general path, over 3-128 features,
 // 2,048-1,000,000 rows, 4-8,192 queries and 0.05-10% of the pairs within the radius:
 // - A row's hits are verified by one wave, so few queries leave the chip idle (1,000,000 x 128, 32
-//   queries, 3%: 37 ms against 1.3), and packing, sweep and two answers to the host cost some 70 us
-//   whatever the size: searches win from 2,048 queries and 2^27 pairs on (131,072 x 16, 2,048
-//   queries, 0.04%: 0.41 ms against 1.17; 32,768 rows, 1%: 0.77 against 0.70).
+//   queries, 3%: 37 ms against 1.3), and packing, sample, sweep and three answers to the host cost
+//   some 150 us whatever the size: searches win from 2,048 queries and 2^28 pairs on (131,072 x 16,
+//   2,048 queries, 0.05%: 0.52 ms against 1.14; 2%, where the sample sends them to the key tiles:
+//   3.7 against 3.5). With 2^27 pairs 65,536 x 32 take 0.48 against 0.74 ms, but with 0.8% 1.39
+//   against 1.20.
 // - DBSCAN wins from 4,096 rows (x 64, 0.2%: 0.53 ms against 0.83; 3,000 rows: 0.49 against 0.44).
 // - A verified pair costs a gather of its row, twice where the distances are wanted, some ten to
 //   a hundred times a pair of the key tiles: with distances the two are equal at 0.5% of the pairs
@@ -521,7 +523,7 @@ hipError_t launch_radius_bits_fill(const unsigned *bits, int rows, int n_pad, co
 //   So the share is measured on a sample of the rows before the sweep; the whole sweep may find twice
 //   as much.
 inline bool radius_bits_size(int64_t rows, int64_t n) {
-    return rows >= 2048 && n >= 2048 && rows * n >= ((int64_t)1 << 27);
+    return rows >= 2048 && n >= 2048 && rows * n >= ((int64_t)1 << 28);
 }
 constexpr int DBSCAN_BITS_ROWS = 4096;
 inline bool radius_bits_sparse(unsigned long long set, int64_t pairs, int d, int64_t queries) {

@@ -1,5 +1,5 @@
 """Radius search and DBSCAN of the squared-euclidean metrics, up to 128 features: small searches,
-which take key tiles, against the oracle; large ones (2,048 queries and 2^27 pairs, DBSCAN of 4,096
+which take key tiles, against the oracle; large ones (2,048 queries and 2^28 pairs, DBSCAN of 4,096
 rows), which go through the matrix-core hit bits, against the oracle and against key tiles: tile
 edges, padded widths, rows that need the exact re-check, and the data that send the search to the
 general path."""
@@ -165,9 +165,9 @@ def _same(nn, Q, profiled, step, served=True, **kw):
 
 # Every k-step count and the smallest width; edges of 512-row blocks and of 128- and 256-row blocks.
 @pytest.mark.parametrize("dtype", [np.float32, np.float64])
-@pytest.mark.parametrize("n,nq,d", [(65536, 2048, 1), (65537, 2050, 3), (65111, 2300, 16),
-                                    (64513, 2111, 32), (66000, 2049, 33), (65600, 2200, 65),
-                                    (60001, 2400, 97), (65024, 2304, 128)])
+@pytest.mark.parametrize("n,nq,d", [(65536, 4096, 1), (65537, 4098, 3), (66111, 4300, 16),
+                                    (65600, 4223, 32), (66000, 4097, 33), (131073, 2048, 65),
+                                    (65537, 4400, 97), (66048, 4352, 128)])
 @pytest.mark.parametrize("metric", ["euclidean", "sqeuclidean", "euclidean_gemm"])
 def test_radius_hit_bits(profiled, dtype, n, nq, d, metric):
     rng = np.random.default_rng(n + d)
@@ -201,7 +201,7 @@ def test_radius_general_path(profiled, case):
     """Large searches whose data the bits cannot separate, hold values that are not finite, or
     whose radius holds too many rows."""
     rng = np.random.default_rng(9)
-    X, Q = blobs(rng, 65536, 6, np.float32), blobs(rng, 2100, 6, np.float32)
+    X, Q = blobs(rng, 65536, 6, np.float32), blobs(rng, 4100, 6, np.float32)
     r = radius_of(X, Q, 0.05 if case == "dense" else 0.002)
     if case == "outlier":
         X[17] = 1e9
@@ -275,7 +275,7 @@ def test_radius_below_the_normal_range(oracle, scale, metric):
     amount that lets pairs beyond the radius in. Against key tiles, and for a few queries against
     the oracle."""
     X = (blobs(np.random.default_rng(31), 66000, 6, np.float64) * scale).astype(np.float32)
-    Q = (blobs(np.random.default_rng(31), 2050, 6, np.float64) * scale).astype(np.float32)
+    Q = (blobs(np.random.default_rng(31), 4100, 6, np.float64) * scale).astype(np.float32)
     r = np.float32(0.5 * scale)
     r = float(r * r if metric == "sqeuclidean" else r)
     nn = aoclda.neighbors.nearest_neighbors(metric=metric, radius=r).fit(X)
