@@ -119,7 +119,7 @@ da_status DBSCANHandle<T>::neighbour_graph_bits(int km, T thr, const double *nrm
     const RadiusPlan plan = radius_plan(d);
     const int n_pad = (n + 511) / 512 * 512;
     const size_t range_bytes = (size_t)(2 * d + 1) * sizeof(unsigned long long);
-    DA_HIP(err, rsc_.reserve(sizeof(RadiusScale) + range_bytes + sizeof(unsigned long long)));
+    DA_HIP(err, rsc_.reserve(sizeof(RadiusScale) + range_bytes));
     const int chunk = (int)std::max<size_t>(
         512, std::min<size_t>((size_t)n_pad, ((size_t)256 << 20) / ((size_t)n_pad / 8) / 512 * 512));
     if (rop_.reserve(radius_operand_elems(plan, n_pad) * 2) != hipSuccess ||
@@ -131,7 +131,6 @@ da_status DBSCANHandle<T>::neighbour_graph_bits(int km, T thr, const double *nrm
     }
     RadiusScale *sc = rsc_.as<RadiusScale>();
     unsigned long long *range = reinterpret_cast<unsigned long long *>(sc + 1);
-    unsigned long long *total = range + 2 * d + 1;
     float *A = rthr_.as<float>(), *B = A + n_pad;
     const T *X = X_.as<T>();
     const double thr2 = radius_threshold2(km, thr);
@@ -147,34 +146,32 @@ da_status DBSCANHandle<T>::neighbour_graph_bits(int km, T thr, const double *nrm
         DA_HIP(err, launch_radius_scale<T>(X, n, (const T *)nullptr, 0, d, km, range, sc, st));
         DA_HIP(err, launch_radius_pack<T>(X, n, n_pad, d, plan, sc, thr2, rop_.ptr(), A, B, st));
     }
-    unsigned long long set = 0, seen = 0;
-    int bad = 0;
+    const unsigned long long most = dbscan_bits_most((int64_t)n * n, d);
+    const unsigned long long probe_most =
+        dbscan_bits_most((int64_t)radius_probe_rows(plan) * n, d);
+    unsigned long long seen = 0;
+    RadiusCounts h;
     {
         KernelScope ks(*gpu, "radius_probe");
-        DA_HIP(err, hipMemsetAsync(total, 0, sizeof(*total), st));
-        DA_HIP(err, launch_radius_probe(plan, rop_.ptr(), n, rop_.ptr(), n_pad, A, B,
-                                        rbits_.as<unsigned>(), total, st));
+        DA_HIP(err, launch_radius_probe(plan, rop_.ptr(), n, rop_.ptr(), n_pad, A, B, sc, st));
     }
-    DA_HIP(err, hipMemcpyAsync(&set, total, sizeof(set), hipMemcpyDeviceToHost, st));
-    DA_HIP(err, hipMemcpyAsync(&bad, &sc->bad, sizeof(int), hipMemcpyDeviceToHost, st));
-    DA_HIP(err, hipStreamSynchronize(st));
-    if (bad || !dbscan_bits_sparse(set, (int64_t)radius_probe_rows(plan) * n, d))
-        return da_status_success;
     for (int r0 = 0; r0 < n; r0 += chunk) {
         const int rows = std::min(chunk, n - r0);
         const int rows_pad = (rows + plan.row_block - 1) / plan.row_block * plan.row_block;
         int *cnt = cnt_.as<int>() + r0;
         unsigned *bits = rbits_.as<unsigned>();
-        DA_HIP(err, hipMemsetAsync(total, 0, sizeof(*total), st));
+        if (r0 > 0)
+            DA_HIP(err, hipMemsetAsync(&sc->total, 0, sizeof(sc->total), st));
         {
             KernelScope ks(*gpu, "radius_sweep");
             DA_HIP(err, launch_radius_sweep(plan, rop_.as<char>() + radius_operand_elems(plan, r0) * 2,
-                                            rows_pad, rop_.ptr(), n_pad, A + r0, B, bits, total, st));
+                                            rows_pad, rop_.ptr(), n_pad, A + r0, B, bits, sc,
+                                            probe_most, st));
         }
-        DA_HIP(err, hipMemcpyAsync(&set, total, sizeof(set), hipMemcpyDeviceToHost, st));
+        DA_HIP(err, hipMemcpyAsync(&h, &sc->bad, sizeof(h), hipMemcpyDeviceToHost, st));
         DA_HIP(err, hipStreamSynchronize(st));
-        seen += set;
-        if (!dbscan_bits_sparse(seen / 2, (int64_t)n * n, d))
+        seen += h.total;
+        if (h.bad || h.probe > probe_most || seen / 2 > most)
             return da_status_success;
         {
             KernelScope ks(*gpu, "radius_verify");
@@ -183,7 +180,7 @@ da_status DBSCANHandle<T>::neighbour_graph_bits(int km, T thr, const double *nrm
                                                 cnt, st));
         }
         // Room for every bit of the sweep; the verified ones are at most as many.
-        da_status s = reserve_edges(E + (long long)set, E);
+        da_status s = reserve_edges(E + (long long)h.total, E);
         if (s != da_status_success)
             return s;
         KernelScope ks(*gpu, "radius_fill");

@@ -459,8 +459,17 @@ bool radius_bits_metric(int metric);
 struct RadiusScale {
     double scale, ca;
     double mu[128];
-    int bad;
+    int bad, unused;
+    // Bits set by the sample of the rows and by the sweep (both zeroed with the scale).
+    unsigned long long probe, total;
 };
+// The last three, as they are read back.
+struct RadiusCounts {
+    int bad, unused;
+    unsigned long long probe, total;
+};
+static_assert(sizeof(RadiusScale) == 130 * sizeof(double) + sizeof(RadiusCounts),
+              "the counts are the end of the scale");
 // Operand shape for d <= 128 features: ks steps of 32; row_block query rows per workgroup (the
 // query operand is padded to a multiple of it, the training operand to a multiple of 512 rows);
 // ce: the relative part of the error bound.
@@ -492,10 +501,11 @@ hipError_t launch_radius_pack(const T *X, int rows, int rows_pad, int d, const R
                               const RadiusScale *sc, double thr2, void *P, float *A, float *B,
                               hipStream_t s);
 // bits: n_pad bits per row (all written; in the order of radius_mfma.hip), set where the pair may
-// be within the threshold; *total (zeroed before) counts them. n_pad: a multiple of 512.
+// be within the threshold; sc->total counts them. n_pad: a multiple of 512. Nothing is done if
+// sc->probe > most.
 hipError_t launch_radius_sweep(const RadiusPlan &p, const void *PA, int rows_pad, const void *PB,
                                int n_pad, const float *A, const float *B, unsigned *bits,
-                               unsigned long long *total, hipStream_t s);
+                               RadiusScale *sc, unsigned long long most, hipStream_t s);
 // Clears the bits of pairs whose key (double, features in order, rounded to T) is above thr, and
 // of column self0 + row when self0 >= 0; cnt[row]: the bits left. nx, ny: squared norms
 // (KM_SQEUCLIDEAN_GEMM).
@@ -520,24 +530,24 @@ hipError_t launch_radius_bits_fill(const unsigned *bits, int rows, int n_pad, co
 //   a hundred times a pair of the key tiles: with distances the two are equal at 0.5% of the pairs
 //   for 128 features, 0.7% for 64, 1.3% for 16 and more below, with 2,048 queries at half of that
 //   (131,072 x 64, 0.8%: 4.0 ms against 2.8); DBSCAN's at 2.5% for 128 features.
-//   So the share is measured on a sample of the rows before the sweep; the whole sweep may find twice
-//   as much.
+//   So the share is measured on a sample of the rows before the sweep, which ends at once if it is
+//   more; the whole sweep may find twice as much.
 inline bool radius_bits_size(int64_t rows, int64_t n) {
     return rows >= 2048 && n >= 2048 && rows * n >= ((int64_t)1 << 28);
 }
 constexpr int DBSCAN_BITS_ROWS = 4096;
-inline bool radius_bits_sparse(unsigned long long set, int64_t pairs, int d, int64_t queries) {
-    return set <= (unsigned long long)(pairs / ((64 + d) * (queries < 8192 ? 2 : 1)));
+inline unsigned long long radius_bits_most(int64_t pairs, int d, int64_t queries) {
+    return (unsigned long long)(pairs / ((64 + d) * (queries < 8192 ? 2 : 1)));
 }
-inline bool dbscan_bits_sparse(unsigned long long set, int64_t pairs, int d) {
-    return set <= (unsigned long long)(pairs / std::max(32, d / 3));
+inline unsigned long long dbscan_bits_most(int64_t pairs, int d) {
+    return (unsigned long long)(pairs / std::max(32, d / 3));
 }
-// The sweep over four row blocks spread over `rows` (at least 4 row blocks) rows: *total counts
-// their bits, bits (row_block rows) is scratch. The rows swept.
+// The sweep over four row blocks spread over `rows` (at least radius_probe_rows) rows: sc->probe
+// counts their bits.
 inline int radius_probe_rows(const RadiusPlan &p) { return 4 * p.row_block; }
 hipError_t launch_radius_probe(const RadiusPlan &p, const void *PA, int rows, const void *PB,
-                               int n_pad, const float *A, const float *B, unsigned *bits,
-                               unsigned long long *total, hipStream_t s);
+                               int n_pad, const float *A, const float *B, RadiusScale *sc,
+                               hipStream_t s);
 // key[p] for the listed neighbours p in [offs[row], offs[row + 1]) of each row.
 template <typename T>
 hipError_t launch_radius_hit_keys(int metric, const T *X, const T *Y, int rows, int d,

@@ -13,7 +13,7 @@
 // do not change with the centre, and the bound shrinks with the norms. Values that are not
 // finite, and searches that leave too many pairs set (a radius that holds some percent of the
 // rows, or rows with outliers many orders of magnitude beyond it), are reported to the caller,
-// which then takes the general path (radius_bits_sparse).
+// which then takes the general path (radius_bits_most).
 //
 // Bound: with the scaled rows x', y', n(.) the squared norm and Kp the padded width, the sum of
 // 3 Kp products and the start value in fp32 carries gamma_{3 Kp + 8} (|x'||y'| + ...), the split
@@ -148,6 +148,7 @@ __global__ __launch_bounds__(128) void radius_scale_kernel(const unsigned long l
         out->scale = s;
         out->ca = ca;
         out->bad = range[2 * d] != 0 || !(big[0] < 1e300) ? 1 : 0;
+        out->probe = out->total = 0;
     }
 }
 
@@ -219,22 +220,27 @@ constexpr int rt_of(int ks) { return ks <= 2 ? 4 : 2; }
 //
 // Bit order: a lane (r, g) sees columns 16 k + r of a row, so word [row][j / 512][j % 16] holds
 // column j at bit 31 - (j % 512) / 16.
+// Row block rb starts at row rb * rstep. Without bits only their number is left; with a probe above
+// `most` nothing is done.
 // Two waves per SIMD are asked for explicitly: with the whole register file to itself the
 // compiler keeps the accumulators in accumulation registers and copies every element in and out.
 template <int KS, int RT>
 __global__ __launch_bounds__(256)
 __attribute__((amdgpu_waves_per_eu(2))) void radius_sweep_kernel(
     const _Float16 *__restrict__ PA, const _Float16 *__restrict__ PB,
-    const float *__restrict__ A, const float *__restrict__ B, int nrb, int nblk, int segblk,
-    unsigned *__restrict__ bits, unsigned long long *__restrict__ total) {
+    const float *__restrict__ A, const float *__restrict__ B, int nrb, int rstep, int nblk,
+    int segblk, unsigned *__restrict__ bits, unsigned long long *total,
+    const unsigned long long *probe, unsigned long long most) {
     constexpr int STAGE = CTS * KS * 1024; // fp16 elements of 16 CTS training rows
     __shared__ __attribute__((aligned(16))) _Float16 s0[STAGE];
     __shared__ __attribute__((aligned(16))) _Float16 s1[STAGE];
+    if (probe && *probe > most)
+        return;
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
     const int r = lane & 15, g = lane >> 4;
     // All row blocks of one segment first, so that the workgroups running at a time share it.
     const int segi = (int)blockIdx.x / nrb, rb = (int)blockIdx.x - segi * nrb;
-    const int row0 = (rb * 4 + w) * RT * 16;
+    const int row0 = rb * rstep + w * RT * 16;
     const int b0 = segi * segblk, b1 = min(nblk, b0 + segblk);
     if (b0 >= b1)
         return;
@@ -329,7 +335,8 @@ __attribute__((amdgpu_waves_per_eu(2))) void radius_sweep_kernel(
 #pragma unroll
             for (int i = 0; i < 4; i++) {
                 const unsigned v = ~word[rt][i];
-                bits[((int64_t)(row0 + rt * 16 + 4 * g + i) * nblk + blk) * 16 + r] = v;
+                if (bits)
+                    bits[((int64_t)(row0 + rt * 16 + 4 * g + i) * nblk + blk) * 16 + r] = v;
                 set += __popc(v);
             }
     }
@@ -580,24 +587,18 @@ hipError_t launch_radius_pack(const T *X, int rows, int rows_pad, int d, const R
     return hipGetLastError();
 }
 
-hipError_t launch_radius_sweep(const RadiusPlan &p, const void *PA, int rows_pad, const void *PB,
-                               int n_pad, const float *A, const float *B, unsigned *bits,
-                               unsigned long long *total, hipStream_t s) {
-    if (rows_pad % p.row_block != 0 || n_pad % 512 != 0)
-        return hipErrorInvalidValue;
-    const int nblk = n_pad / 512;
-    const int nrb = rows_pad / p.row_block;
-    // Column segments: about 1,024 workgroups (two run on a CU at a time), each of at least 1,024
-    // training rows: a workgroup's start (its query rows) and end cost a few steps. 10,000 x
-    // 100,000 pairs of 16 features: 222 us with 4,096 workgroups, 177 us with 512 to 2,048.
-    int nseg = std::max(1, std::min((nblk + 1) / 2, (1024 + nrb - 1) / nrb));
-    const int segblk = (nblk + nseg - 1) / nseg;
-    nseg = (nblk + segblk - 1) / segblk;
+static hipError_t radius_sweep(const RadiusPlan &p, const void *PA, int nrb, int rstep,
+                               const void *PB, int n_pad, int segblk, const float *A,
+                               const float *B, unsigned *bits, unsigned long long *total,
+                               const unsigned long long *probe, unsigned long long most,
+                               hipStream_t s) {
+    const int nblk = n_pad / 512, nseg = (nblk + segblk - 1) / segblk;
     const _Float16 *pa = static_cast<const _Float16 *>(PA), *pb = static_cast<const _Float16 *>(PB);
 #define DA_SWEEP(K)                                                                              \
     case K:                                                                                      \
         hipLaunchKernelGGL((radius_sweep_kernel<K, rt_of(K)>), dim3((unsigned)nrb * nseg),       \
-                           dim3(256), 0, s, pa, pb, A, B, nrb, nblk, segblk, bits, total);       \
+                           dim3(256), 0, s, pa, pb, A, B, nrb, rstep, nblk, segblk, bits,        \
+                           total, probe, most);                                                  \
         break;
     switch (p.ks) {
         DA_SWEEP(1)
@@ -611,20 +612,30 @@ hipError_t launch_radius_sweep(const RadiusPlan &p, const void *PA, int rows_pad
     return hipGetLastError();
 }
 
-hipError_t launch_radius_probe(const RadiusPlan &p, const void *PA, int rows, const void *PB,
+hipError_t launch_radius_sweep(const RadiusPlan &p, const void *PA, int rows_pad, const void *PB,
                                int n_pad, const float *A, const float *B, unsigned *bits,
-                               unsigned long long *total, hipStream_t s) {
-    if (rows < radius_probe_rows(p))
+                               RadiusScale *sc, unsigned long long most, hipStream_t s) {
+    if (rows_pad % p.row_block != 0 || n_pad % 512 != 0 || !bits)
         return hipErrorInvalidValue;
-    for (int q = 0; q < 4; q++) {
-        const int r0 = (int)((int64_t)q * rows / 4) / p.row_block * p.row_block;
-        const hipError_t e = launch_radius_sweep(
-            p, static_cast<const _Float16 *>(PA) + radius_operand_elems(p, r0), p.row_block, PB,
-            n_pad, A + r0, B, bits, total, s);
-        if (e != hipSuccess)
-            return e;
-    }
-    return hipSuccess;
+    const int nblk = n_pad / 512;
+    const int nrb = rows_pad / p.row_block;
+    // Column segments: about 1,024 workgroups (two run on a CU at a time), each of at least 1,024
+    // training rows: a workgroup's start (its query rows) and end cost a few steps. 10,000 x
+    // 100,000 pairs of 16 features: 222 us with 4,096 workgroups, 177 us with 512 to 2,048.
+    const int nseg = std::max(1, std::min((nblk + 1) / 2, (1024 + nrb - 1) / nrb));
+    return radius_sweep(p, PA, nrb, p.row_block, PB, n_pad, (nblk + nseg - 1) / nseg, A, B, bits,
+                        &sc->total, &sc->probe, most, s);
+}
+
+// Four row blocks alone leave most CUs idle, so here the segments are short.
+hipError_t launch_radius_probe(const RadiusPlan &p, const void *PA, int rows, const void *PB,
+                               int n_pad, const float *A, const float *B, RadiusScale *sc,
+                               hipStream_t s) {
+    if (rows < radius_probe_rows(p) || n_pad % 512 != 0)
+        return hipErrorInvalidValue;
+    const int segblk = std::max(1, n_pad / 512 / 256);
+    return radius_sweep(p, PA, 4, rows / 4 / p.row_block * p.row_block, PB, n_pad, segblk, A, B,
+                        nullptr, &sc->probe, nullptr, 0, s);
 }
 
 template <typename T>

@@ -1516,7 +1516,6 @@ da_status NNHandle<T>::radius_core(const T *dQ, da_int n_queries, T radius, bool
     const int nw = (n + 63) / 64;
     const int n_pad = (n + 511) / 512 * 512, q_pad = (n_queries + 511) / 512 * 512;
     RadiusScale *rsc = nullptr;
-    unsigned long long *set_total = nullptr;
     float *A = nullptr, *B = nullptr;
     const size_t opb = use_bits ? radius_operand_elems(plan, n_pad) * 2 : 0;
     const da_int bits_chunk = (da_int)std::max<int64_t>(
@@ -1530,14 +1529,16 @@ da_status NNHandle<T>::radius_core(const T *dQ, da_int n_queries, T radius, bool
         rnn_thr_.release();
         use_bits = false;
     }
-    unsigned long long set = 0, seen = 0;
+    const unsigned long long most = radius_bits_most((int64_t)n_queries * n, d, n_queries);
+    const unsigned long long probe_most =
+        radius_bits_most((int64_t)radius_probe_rows(plan) * n, d, n_queries);
+    unsigned long long seen = 0;
     if (use_bits) {
         const size_t range_words = (size_t)2 * d + 1;
         DA_HIP(err, rnn_scale_.reserve(sizeof(RadiusScale) +
-                                       (range_words + 1) * sizeof(unsigned long long)));
+                                       range_words * sizeof(unsigned long long)));
         rsc = rnn_scale_.as<RadiusScale>();
         unsigned long long *range = reinterpret_cast<unsigned long long *>(rsc + 1);
-        set_total = range + range_words;
         A = rnn_thr_.as<float>();
         B = A + q_pad;
         const double thr2 = radius_threshold2(km, thr);
@@ -1550,18 +1551,9 @@ da_status NNHandle<T>::radius_core(const T *dQ, da_int n_queries, T radius, bool
             DA_HIP(err, launch_radius_pack<T>(dQ, n_queries, q_pad, d, plan, rsc, thr2,
                                               rnn_op_.as<char>() + opb, A, nullptr, st));
         }
-        int bad = 0;
-        {
-            KernelScope ks(*gpu, "radius_probe");
-            DA_HIP(err, hipMemsetAsync(set_total, 0, sizeof(*set_total), st));
-            DA_HIP(err, launch_radius_probe(plan, rnn_op_.as<char>() + opb, n_queries, rnn_op_.ptr(),
-                                            n_pad, A, B, rnn_bits_.as<unsigned>(), set_total, st));
-        }
-        DA_HIP(err, hipMemcpyAsync(&set, set_total, sizeof(set), hipMemcpyDeviceToHost, st));
-        DA_HIP(err, hipMemcpyAsync(&bad, &rsc->bad, sizeof(int), hipMemcpyDeviceToHost, st));
-        DA_HIP(err, hipStreamSynchronize(st));
-        use_bits = !bad && radius_bits_sparse(
-                              set, (int64_t)radius_probe_rows(plan) * n, d, n_queries);
+        KernelScope ks(*gpu, "radius_probe");
+        DA_HIP(err, launch_radius_probe(plan, rnn_op_.as<char>() + opb, n_queries, rnn_op_.ptr(),
+                                        n_pad, A, B, rsc, st));
     }
     // Query blocks whose key tile stays within 256 MB (and 2^28 entries), or whose bits stay
     // within 128 MiB and whose neighbours fit 32-bit offsets.
@@ -1581,16 +1573,19 @@ da_status NNHandle<T>::radius_core(const T *dQ, da_int n_queries, T radius, bool
             scnt.resize(rows);
             {
                 KernelScope ks(*gpu, "radius_sweep");
-                DA_HIP(err, hipMemsetAsync(set_total, 0, sizeof(*set_total), st));
+                if (q0 > 0)
+                    DA_HIP(err, hipMemsetAsync(&rsc->total, 0, sizeof(rsc->total), st));
                 DA_HIP(err, launch_radius_sweep(
                                 plan,
                                 rnn_op_.as<char>() + opb + radius_operand_elems(plan, q0) * 2,
-                                rows_pad, rnn_op_.ptr(), n_pad, A + q0, B, bits, set_total, st));
+                                rows_pad, rnn_op_.ptr(), n_pad, A + q0, B, bits, rsc, probe_most,
+                                st));
             }
-            DA_HIP(err, hipMemcpyAsync(&set, set_total, sizeof(set), hipMemcpyDeviceToHost, st));
+            RadiusCounts h;
+            DA_HIP(err, hipMemcpyAsync(&h, &rsc->bad, sizeof(h), hipMemcpyDeviceToHost, st));
             DA_HIP(err, hipStreamSynchronize(st));
-            seen += set;
-            if (!radius_bits_sparse(seen / 2, (int64_t)n_queries * n, d, n_queries)) {
+            seen += h.total;
+            if (h.bad || h.probe > probe_most || seen / 2 > most) {
                 use_bits = false; // this block and the rest through the key tiles
                 continue;
             }
