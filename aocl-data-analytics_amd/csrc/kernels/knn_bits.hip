@@ -39,7 +39,7 @@ typedef unsigned v4u __attribute__((ext_vector_type(4)));
 // One wave per query: the rank-th smallest of its 256 minima (at least the rank-th smallest score,
 // and with rank well below 256 close to it).
 __global__ __launch_bounds__(256) void bits_guess_kernel(
-    const float *__restrict__ mins, int nq, int ns, double n, int d, int rank, double ce,
+    const float *__restrict__ mins, int nq, int most_within, int d, int rank, double ce,
     const double *__restrict__ nrm, const WideScale *__restrict__ sc, float *__restrict__ A,
     double *__restrict__ lim, int *bad, int *__restrict__ count) {
     const int q = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
@@ -65,11 +65,7 @@ __global__ __launch_bounds__(256) void bits_guess_kernel(
     for (int u = 0; u < 4; u++)
         within += __popcll(__builtin_amdgcn_ballot_w64((double)m[u] <= 0.5 * (L - nn) + ce * nn));
     if (lane == 0) {
-        // Hits to expect: with a share f of the rows hit, a group of g sample rows holds none with
-        // probability (1 - f)^g. (The number of groups itself stops at 256, too few to tell below
-        // 24,577 rows, where a group stands for 96 rows or less.)
-        const double empty = fmax(256.0 - within, 0.5) / 256.0;
-        const bool hopeless = n * (1.0 - pow(empty, 256.0 / ns)) > 0.75 * BITS_KEEP;
+        const bool hopeless = within > most_within;
         const double s = sc->scale, y2 = __longlong_as_double((long long)sc->ymax2);
         // A query that fits stays within 60,000 / s of the centre.
         const double alpha = 0x1p-24 + 0x1p-51 * (60000.0 + 2.0 * s * sc->big);
@@ -529,8 +525,13 @@ hipError_t launch_bits_guess(const float *mins, int nq, int ns, int64_t n, int d
                              double *lim, int *bad, int *count, hipStream_t s) {
     if (rank < 1 || rank > 256)
         return hipErrorInvalidValue;
-    hipLaunchKernelGGL(bits_guess_kernel, dim3((nq + 255) / 256 * 64), dim3(256), 0, s, mins, nq, ns,
-                       (double)n, d, rank, ce, nrm, sc, A, lim, bad, count);
+    // Hits to expect: with a share f of the rows hit, a group of g sample rows holds none with
+    // probability (1 - f)^g. (The number of groups with one, times the rows a group stands for, ends
+    // at 256 groups, too few to tell below 24,577 rows.)
+    const double f = 0.75 * BITS_KEEP / (double)n;
+    const int most_within = (int)(256.0 * (1.0 - std::pow(1.0 - f, ns / 256.0)));
+    hipLaunchKernelGGL(bits_guess_kernel, dim3((nq + 255) / 256 * 64), dim3(256), 0, s, mins, nq,
+                       most_within, d, rank, ce, nrm, sc, A, lim, bad, count);
     return hipGetLastError();
 }
 
