@@ -13,10 +13,11 @@ class nearest_neighbors:
                  metric="euclidean", p=2.0, radius=1.0, outlier_handling=None,
                  check_data=False, precision="working", tile_variant=-1,
                  candidates_per_split=0, seed_thresholds=None):
-        # precision: operand precision of the MFMA distance tiles ("working", "fp32",
+        # precision: operand precision of the fused MFMA distance tile ("working", "fp32",
         # "fp16", "bf16", "fp16x3", "bf16x3", "fp16c": fp16 rows stored about k-means group
-        # centres); results are re-ranked exactly whatever the
-        # choice. candidates_per_split: candidate-list length per query and split of
+        # centres); results are re-ranked exactly whatever the choice, and large searches go by
+        # hit bits, whose operands are the same in every form, unless one of the next three is
+        # set. candidates_per_split: candidate-list length per query and split of
         # the fused tile (0 = from k; shorter than k is allowed and stays exact).
         # seed_thresholds: bound the tile's thresholds (k <= 16) by the group
         # minima over a row sample first (None: the library's choice, which seeds the

@@ -6,11 +6,12 @@
 
 A step is one da_nn_kneighbors_device_s call over the whole 20,000-query batch, with the
 training set resident in GPU memory (da_nn_set_data_s) and the queries already in GPU
-memory when the timed region starts. Each precision form of the distance tiles is timed:
-"working" (fp32 MFMA, the plain path) and the low-precision forms (fp16 / bf16 MFMA with
-fp32 accumulation); all of them re-rank candidates with exact double distances. The
-headline value is the fastest form whose recall@10 against the fp64 oracle is 1.0 on the
-checked sample. Prints one JSON line.
+memory when the timed region starts. Timed are the library's own choice ("working": hit bits
+from one fp16 product per pair, exact double keys of the hits) and the fused tile in its operand
+forms ("working+tile": fp32 MFMA, the plain path; fp16 / bf16 MFMA with fp32 accumulation); all
+of them order by exact double distances. The headline value is the fastest form whose recall@10
+against the fp64 oracle is 1.0 on the checked sample, the low-precision speed-up its ratio to
+"working+tile". Prints one JSON line.
 """
 import argparse
 import ctypes as C
@@ -40,14 +41,18 @@ FORM_KEY = {"working": "fp32", "fp32": "fp32"}
 
 def split_form(form):
     """A form is a precision, optionally followed by /N: the minimum candidate-list length
-    per query and split of the fused tile (e.g. fp16/32)."""
+    per query and split of the fused tile (e.g. fp16/32), and by +tile: the fused tile in place
+    of the hit bits (as it serves with a length, a variant or a choice of seeds set). Returns the
+    precision, the length and whether the tile is asked for."""
+    form, _, tile = form.partition("+")
     prec, _, kc = form.partition("/")
-    return prec, int(kc) if kc else 0
+    return prec, int(kc) if kc else 0, tile == "tile"
 
 
 def measured_traffic(form):
     """HBM bytes per knn_tile launch of this form from the committed rocprofv3 counter
     summary (two counter passes calibrated with a copy of known size), or None."""
+    form = form.partition("+")[0]
     key = FORM_KEY.get(form, form)
     try:
         with open(TRAFFIC_FILE) as f:
@@ -109,7 +114,9 @@ def cpu_baseline(Xt, Xq, k, ei, args):
 
 
 def run_form(L, aoclda, Xt, dq, nq, d, k, precision, steps, warmup, variant=-1, seed=None):
-    prec, kc_min = split_form(precision)
+    prec, kc_min, tile = split_form(precision)
+    if tile and seed is None:
+        seed = prec not in ("working", "fp32")  # the 16-bit forms' default
     nn = aoclda.neighbors.nearest_neighbors(n_neighbors=k, precision=prec, tile_variant=variant,
                                             candidates_per_split=kc_min,
                                             seed_thresholds=seed).fit(Xt)
@@ -491,7 +498,7 @@ def dbscan_bench(args, L, aoclda):
         t0 = time.perf_counter()
         h.call("da_dbscan_compute")
         times.append(time.perf_counter() - t0)
-    names = ("radius_sweep", "radius_verify", "pairwise_direct", "radius_segsum", "radius_fill", "dbscan_union", "dbscan_label")
+    names = ("radius_probe", "radius_sweep", "radius_verify", "pairwise_direct", "radius_segsum", "radius_fill", "dbscan_union", "dbscan_label")
     kern = {}
     for nm in names:
         ms_, cnt = C.c_double(), L.da_int()
@@ -724,7 +731,8 @@ def main():
     ap.add_argument("--n-query", type=int, default=20_000)
     ap.add_argument("--dim", type=int, default=128)
     ap.add_argument("--k", type=int, default=10)
-    ap.add_argument("--forms", default="working,fp16x3,bf16x3,fp16c")
+    ap.add_argument("--forms",
+                    default="working,working+tile,fp16x3+tile,bf16x3+tile,fp16c+tile")
     ap.add_argument("--kb-forms", default="working,bf16x3,bf16",
                     help="cross-term forms of the batched k-means mode")
     ap.add_argument("--tile-variant", type=int, default=-1,
@@ -764,7 +772,7 @@ def main():
     ap.add_argument("--serving", action="store_true",
                     help="run the continuous-batching serving benchmark instead")
     ap.add_argument("--serve-rows", type=int, default=2_000_000)
-    ap.add_argument("--serve-forms", default="fp16,fp16x3")
+    ap.add_argument("--serve-forms", default="working")
     ap.add_argument("--serve-batch", type=int, default=4096)
     ap.add_argument("--serve-bytes", type=int, default=1 << 30)
     ap.add_argument("--serve-closed", type=int, default=200)
@@ -842,7 +850,7 @@ def main():
             r["max_rel_dist_err"] = float(rel.max())
             r["mean_rel_dist_err"] = float(rel.mean())
 
-    plain = results.get("working")
+    plain = results.get("working+tile")
     ok = [f for f in results if results[f].get("recall_at_10", 1.0) == 1.0]
     head = max(ok, key=lambda f: results[f]["qps"]) if ok else "working"
     H = results[head]
@@ -891,7 +899,7 @@ def main():
                    "dim": d, "k": k, "precision_form": head},
         "p50_ms": H["p50_ms"], "p99_ms": H["p99_ms"],
         "recall_at_10": H.get("recall_at_10"),
-        "lowp_speedup": (H["qps"] / plain["qps"]) if plain and head != "working" else None,
+        "lowp_speedup": (H["qps"] / plain["qps"]) if plain and head != "working+tile" else None,
         "plain_fp32_qps": plain["qps"] if plain else None,
         "host_buffers_qps": H["host_buffers_qps"],
         "forms": forms, "roofline": roofline, "cpu_baseline": cpu,

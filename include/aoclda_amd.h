@@ -84,11 +84,11 @@ da_status da_amd_pairwise_profile_reset(void);
 da_status da_amd_pairwise_profile_get(const char *kernel, double *total_ms, da_int *count);
 
 /*
- * Diagnostics of the last k-NN query of the handle: number of queries whose candidate
- * set from the first pass of the fused tile could not be certified exact (they are searched
- * again: a second seeded pass, then the exact fallback for any still uncertified), and the
- * candidates kept per query by that first pass (a small search without a chosen operand form
- * is served by exact keys of every row: n_samples).
+ * Diagnostics of the last k-NN query of the handle: the number of queries that the search's first
+ * pass could not settle (they are searched again, exactly), and the candidates that pass kept per
+ * query: by hit bits (large squared-euclidean searches) 2,048, the most hits that are looked at; by
+ * the fused tile its lists; by approximate scores (wide rows, cosine) 64 or 128; n_samples for a
+ * small search, served by exact keys of every row; 0 for the general path.
  */
 da_status da_nn_last_query_stats(da_handle handle, da_int *n_fallback, da_int *n_candidates);
 
@@ -107,7 +107,8 @@ da_status da_kmeans_last_compute_stats(da_handle handle, da_int *n_rechecked);
  * queued by da_nn_server_submit_? (the queries are copied, the call does not block) and
  * served by a worker thread that coalesces queued requests into batches of at most
  * max_batch_queries queries whose device buffers fit in max_device_bytes (admission by
- * memory; a request larger than a batch is served in slices). Two batches are in flight on
+ * memory; a request larger than a batch is served in slices; the training operands, laid out
+ * by da_nn_server_create, are not counted). Two batches are in flight on
  * two HIP streams, so a batch is prepared and admitted while the previous one runs.
  * Every query's result is the exact k nearest neighbours, identical whether the request is
  * served alone or together with others. da_nn_server_wait_? blocks until a request is
