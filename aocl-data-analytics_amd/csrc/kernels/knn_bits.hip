@@ -14,7 +14,7 @@
 // Queries with fewer than k rows within lim, more than BITS_KEEP hits or values beyond fp16's range
 // are listed for the fused tile. When the error bound is wide against the distances (tight clusters
 // far apart), the sample shows it: such queries are counted, and if they are more than a quarter the
-// sweep does not run at all. (Sample and second search still cost 0.2 of 0.7 ms at 16,384 x 20 with
+// sweep does not run at all. (Sample and second search still cost 0.2 of 0.8 ms at 16,384 x 20 with
 // 6,000 queries, so after a search that listed most of its queries the caller leaves some to the tile.)
 //
 // Bound: rows are centred and scaled by a power of two (knn_wide.hip); hi = x' (1 + 2^-11), so
