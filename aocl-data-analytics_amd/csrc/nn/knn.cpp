@@ -680,7 +680,7 @@ da_status NNHandle<T>::search_launch(SearchContext &ctx, const SearchParams &sp,
     if (fused && sp.automatic && !ctx.second_pass && tiles_faster(nq)) {
         fused = false;
         ctx.last_candidates = n_samples_; // every row has its exact key
-        return search_tiles(ctx, dQ, nq, k, return_distance, d_ind, d_dist, true);
+        return search_tiles(ctx, dQ, nq, k, return_distance, d_ind, d_dist);
     }
     if (!fused) {
         if (!ctx.second_pass && wide_eligible(nq, k) && !wide_backoff_.skipped()) {
@@ -1093,7 +1093,7 @@ da_status NNHandle<T>::search_finish(SearchContext &ctx, const T *dQ, da_int nq,
             rc.block.swap(ctx.block);
         } else {
             s = search_tiles(ctx, ctx.fb_q.as<T>(), nfb, k, true, ctx.fb_ind.as<da_int>(),
-                             ctx.fb_dist.as<T>(), few);
+                             ctx.fb_dist.as<T>());
         }
         if (s != da_status_success)
             return s;
@@ -1250,17 +1250,19 @@ da_status NNHandle<T>::search(const T *dQ, da_int nq, da_int k, bool return_dist
 // Generic path for every metric: key tiles (queries x training points, in double) followed
 // by the per-row selection, the structure of kneighbors_compute_brute_force
 // (nearest_neighbors.cpp:567-816) with the blocks sized for HBM instead of caches.
-// direct: in place of the fused tile or the hit bits, which order the *_gemm metrics by direct
-// differences too: |x|^2 + |y|^2 - 2 x.y would lose the digits that the norms have above the
-// distance (equal rows 1e-7 apart instead of 0), and the result would depend on the route.
+// What the fused tile or the hit bits could serve is ordered by direct differences here too, also
+// for the *_gemm metrics: |x|^2 + |y|^2 - 2 x.y would lose the digits that the norms have above
+// the distance (equal rows 1e-7 apart instead of 0), and the result would depend on the route,
+// which follows what earlier searches met.
 template <typename T>
 da_status NNHandle<T>::search_tiles(SearchContext &ctx, const T *dQ, da_int nq, da_int k,
-                                    bool return_distance, da_int *d_ind, T *d_dist, bool direct) {
+                                    bool return_distance, da_int *d_ind, T *d_dist) {
     hipStream_t st = ctx.gpu->stream();
     const da_int d = n_features_, n = n_samples_;
     if (k > 3840)
         return err->error(da_status_not_implemented,
                           "k > 3840 neighbours is not supported by the GPU selection kernel.");
+    const bool direct = fused_eligible(k);
     int km, post = 0, largest = 0;
     const double *nq_norm = nullptr, *nt_norm = nullptr;
     double p = p_;

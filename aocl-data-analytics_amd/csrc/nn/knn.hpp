@@ -139,7 +139,7 @@ template <typename T> class NNHandle : public AlgHandle {
     da_status search(const T *dQ, da_int nq, da_int k, bool return_distance, da_int *d_ind,
                      T *d_dist);
     da_status search_tiles(SearchContext &ctx, const T *dQ, da_int nq, da_int k,
-                           bool return_distance, da_int *d_ind, T *d_dist, bool direct = false);
+                           bool return_distance, da_int *d_ind, T *d_dist);
     bool fused_eligible(da_int k) const;
     bool tiles_faster(da_int nq) const;
     int split_cap(int kc) const;

@@ -91,6 +91,28 @@ def test_gemm_metrics_order_by_direct_differences(oracle, metric, dtype, n, nq):
     assert np.all(dist[:9, 0] == 0)
 
 
+@pytest.mark.parametrize("dtype", [np.float64, np.float32])
+@pytest.mark.parametrize("n,d,nq,k", [(70000, 6, 200, 3), (20000, 64, 300, 40), (1500, 80, 10000, 20),
+                                      (2000, 128, 6000, 100)])
+def test_gemm_metrics_do_not_depend_on_the_route(dtype, n, d, nq, k):
+    """Data that neither the hit bits nor the fused tile resolve: a search takes one or the other
+    by what the searches before it met, and ends in key tiles. Every call gives the bits of the
+    euclidean metric, which is ordered by direct differences throughout."""
+    rng = np.random.default_rng(n)
+    means = rng.uniform(-10, 10, (16, d))
+    Xt = (means[rng.integers(0, 16, n)] + 1e-3 * rng.standard_normal((n, d))).astype(dtype)
+    Xq = (means[rng.integers(0, 16, nq)] + 1e-3 * rng.standard_normal((nq, d))).astype(dtype)
+    Xq[::9] = Xt[: len(Xq[::9])]
+    nn = aoclda.neighbors.nearest_neighbors(metric="euclidean").fit(Xt)
+    dist, ind = nn.kneighbors(Xq, k)
+    assert np.all(dist[::9, 0] == 0)
+    gemm = aoclda.neighbors.nearest_neighbors(metric="euclidean_gemm").fit(Xt)
+    for _ in range(4):
+        gd, gi = gemm.kneighbors(Xq, k)
+        np.testing.assert_array_equal(gi, ind)
+        np.testing.assert_array_equal(gd, dist)
+
+
 @pytest.mark.parametrize("n,nq,tiles", [(16, 9000, True), (16, 9300, False), (200, 20000, True),
                                         (200, 22000, False), (1000, 30000, True)])
 def test_small_searches_with_many_queries(oracle, n, nq, tiles):
