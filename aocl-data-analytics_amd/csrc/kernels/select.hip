@@ -130,7 +130,8 @@ namespace {
 // average (5 for k = 5, 127 for k = 100), and one sort of those ends the row: two barriers-free
 // sweeps instead of two barriers per 256 elements and a 512-entry sort whenever the buffer fills.
 // Rows with more than SEL_CAP elements at or below the bound (ties) are left to the general
-// kernel: their out_idx[0] is set to -2.
+// kernel: their out_idx[0] is set to -2. Rows of up to SEL_CAP elements never are, so that
+// launch is left out for them (5 us of a small search).
 constexpr int SEL_CAP = 1024;
 template <typename K>
 __global__ __launch_bounds__(256) void row_topk_bound_kernel(const K *__restrict__ keys,
@@ -266,6 +267,8 @@ static hipError_t topk_level(const K *keys, int64_t ld, int rows, int n, int k, 
     if (k <= 128)
         hipLaunchKernelGGL(row_topk_bound_kernel<K>, grid, block, 0, s, keys, ld, n, k, largest,
                            out_key, out_idx, seg);
+    if (k <= 128 && std::min(n, seg) <= SEL_CAP)
+        return hipGetLastError();
     auto kern = k + 256 <= 512    ? row_topk_kernel<K, 512>
                 : k + 256 <= 1024 ? row_topk_kernel<K, 1024>
                 : k + 256 <= 2048 ? row_topk_kernel<K, 2048>

@@ -113,6 +113,22 @@ def test_gemm_metrics_do_not_depend_on_the_route(dtype, n, d, nq, k):
         np.testing.assert_array_equal(gd, dist)
 
 
+@pytest.mark.parametrize("n", [1, 255, 257, 1023, 1024, 1025, 2049])
+@pytest.mark.parametrize("equal", [True, False])
+def test_selection_of_short_and_tied_rows(oracle, n, equal):
+    """Rows of up to 1,024 keys end with the bounded selection, longer ones with more ties than it
+    holds with the general one; equal keys by index."""
+    rng = np.random.default_rng(n)
+    Xt = np.ones((n, 3)) if equal else rng.integers(0, 4, (n, 3)).astype(np.float64)
+    Xq = rng.integers(0, 4, (50, 3)).astype(np.float64)
+    nn = aoclda.neighbors.nearest_neighbors(metric="manhattan").fit(Xt)
+    for k in sorted({1, min(n, 100), min(n, 128), min(n, 129)}):
+        dist, ind = nn.kneighbors(Xq, k)
+        ei, ed = oracle.knn(Xt, Xq, k, "manhattan")
+        np.testing.assert_array_equal(ind, ei)
+        np.testing.assert_array_equal(dist, ed)
+
+
 @pytest.mark.parametrize("n,nq,tiles", [(16, 9000, True), (16, 9300, False), (200, 20000, True),
                                         (200, 22000, False), (1000, 30000, True)])
 def test_small_searches_with_many_queries(oracle, n, nq, tiles):
