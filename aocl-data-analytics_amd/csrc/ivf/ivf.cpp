@@ -616,14 +616,24 @@ da_status ApproxNNHandle<T>::kneighbors(da_int n_queries, da_int n_features, con
         ld += longest[p];
     bool tiles = d <= IVF_TILE_D && k <= IVF_TILE_K && n_probe <= IVF_TILE_PROBE &&
                  ld <= ((int64_t)1 << 26);
-    // The first search after a change of the index lays out its lists (1,000,000 x 96: 1.0-1.4 ms
-    // with the search) only if it scans some eight times the index: 256 queries of 16 of 1,024 lists
-    // (four times) take 1.24 ms by scans, 1,000 (sixteen times) 3.4; and if it scans some 2^20 vectors
-    // (20,000 x 32, 256 queries of 4 of 64 lists: 0.17 ms by scans, 0.24 with the layout). A second
-    // search lays them out whatever its size (0.2 ms against 1.0 for every one that follows).
-    const double lists = (double)n_queries * n_probe;
-    if (tiles_state_ == 0 && !searched_ &&
-        (lists < 8.0 * n_list_ || lists * n_index_ < (double)(1 << 20) * n_list_))
+    // Small searches stay with the scans, whose launches and wait take 20 us less than those of the
+    // list-major search. What they take beyond that, in us: a workgroup's walk through a list, a
+    // query's selection, the probed lists of all queries on the host and on the device (fitted over
+    // 500-400,000 vectors of 8-120 features, 1-1,000 queries, k = 1-100, both types; k adds 0.1 us
+    // to the list-major merge: 1 query, 1 of 64 lists of 2,000 x 8: 99 us by scans, 131 list-major;
+    // 64 queries, 4 of 64 lists of 10,000 x 120: 266 against 177).
+    const double lists = (double)n_queries * n_probe, mean = (double)n_index_ / n_list_;
+    const double scan_us =
+        0.004 * mean * d + 0.008 * mean * n_probe + lists * (0.012 + 1e-6 * mean * d);
+    const bool small = scan_us < 20 + 0.1 * k;
+    // Beyond those, the first search after a change of the index lays out its lists (1,000,000 x 96:
+    // 1.0-1.4 ms with the search) only if it scans some eight times the index: 256 queries of 16 of
+    // 1,024 lists (four times) take 1.24 ms by scans, 1,000 (sixteen times) 3.4; and if it scans some
+    // 2^20 vectors (20,000 x 32, 256 queries of 4 of 64 lists: 0.17 ms by scans, 0.24 with the
+    // layout). A second search lays them out whatever its size (0.2 ms against 1.0 for every one that
+    // follows).
+    if (small || (tiles_state_ == 0 && !searched_ &&
+                  (lists < 8.0 * n_list_ || lists * n_index_ < (double)(1 << 20) * n_list_)))
         tiles = false;
     searched_ = true;
     if (tiles) {

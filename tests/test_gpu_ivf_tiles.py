@@ -146,6 +146,28 @@ def test_layout_after_a_change():
     assert search(80) == (1, 0)
 
 
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+@pytest.mark.parametrize("n,d,n_list,n_probe,nq,k,small", [
+    (2000, 8, 64, 1, 1, 10, True), (2000, 8, 64, 1, 1000, 10, True), (2000, 8, 64, 4, 1000, 10, False),
+    (1200, 32, 26, 20, 7, 88, True), (4096, 20, 1, 1, 1, 1, False), (600, 80, 98, 44, 1, 2, True),
+    (10000, 120, 64, 4, 64, 10, False), (12, 3, 1, 1, 1, 1, True)])
+def test_small_searches(dtype, n, d, n_list, n_probe, nq, k, small):
+    """Small searches are scanned however often they are made, and leave no layout behind; the same
+    answers on either side of the line."""
+    rng = np.random.default_rng(n)
+    X, Q = rng.standard_normal((n, d)).astype(dtype), rng.standard_normal((nq, d)).astype(dtype)
+    ann = aoclda.neighbors.approximate_neighbors(n_list=n_list, n_probe=n_probe, kmeans_iter=2,
+                                                 seed=1).train_and_add(X)
+    L.check(L.lib.da_amd_profile_enable(ann._h.h, 1))
+    for i in range(3):
+        dist, ind = ann.kneighbors(Q, n_neighbors=k)
+    assert _launches(ann)[0] == (0 if small else 2)
+    if n > 129:
+        de, ie = ann.kneighbors(Q, n_neighbors=129)
+        np.testing.assert_array_equal(ind, ie[:, :k])
+        np.testing.assert_array_equal(dist, de[:, :k])
+
+
 @pytest.mark.parametrize("metric", ["sqeuclidean", "inner product", "cosine"])
 @pytest.mark.parametrize("where", ["rows", "queries"])
 def test_not_finite(metric, where):
