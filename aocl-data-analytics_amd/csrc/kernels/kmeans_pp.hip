@@ -151,17 +151,29 @@ __global__ __launch_bounds__(KPP_ROWS) void kpp_cost_kernel(
             }
         } else {
             wi = (!first && tid < m) ? w[i] : 0.0;
+            // The next FB features are read while these are computed: with few rows nothing else
+            // hides the memory's latency (1,828 x 281 fp64, 8 workgroups: 118 -> 47 us).
             const int lc = tid % FB, lr = tid / FB;
+            T next[FB];
+            auto load = [&](int l0) {
+#pragma unroll
+                for (int u = 0; u < FB; u++) {
+                    const int r = lr + u * (KPP_ROWS / FB);
+                    next[u] = r < m && l0 + lc < d ? X[(i0 + r) * d + l0 + lc] : T(0);
+                }
+            };
+            load(0);
             for (int l0 = 0; l0 < d; l0 += FB) {
                 const int fl = d - l0 < FB ? d - l0 : FB;
                 __syncthreads();
-#pragma unroll 8
-                for (int r = lr; r < KPP_ROWS; r += KPP_ROWS / FB)
-                    if (r < m && lc < fl)
-                        tile[r * (FB + 1) + lc] = X[(i0 + r) * d + l0 + lc];
+#pragma unroll
+                for (int u = 0; u < FB; u++)
+                    tile[(lr + u * (KPP_ROWS / FB)) * (FB + 1) + lc] = next[u];
                 __syncthreads();
+                if (l0 + FB < d)
+                    load(l0 + FB);
                 if (tid < m) {
-#pragma unroll 4
+#pragma unroll 8
                     for (int l = 0; l < fl; l++)
                         take((double)tile[tid * (FB + 1) + l], crow + (int64_t)(l0 + l) * NT);
                 }

@@ -32,6 +32,14 @@ def test_row_widths(oracle, dtype, d):
     _check(oracle, _blobs(d, 1037, d, 9, dtype), 9, dtype)
 
 
+@pytest.mark.parametrize("dtype", [np.float64, np.float32])
+@pytest.mark.parametrize("d", [79, 80, 81, 96, 97, 127, 128, 129, 600])
+def test_wide_rows(oracle, dtype, d):
+    """Rows staged 16 or 32 features at a time, the next ones read ahead: whole and partial stages,
+    a last step of a few rows."""
+    _check(oracle, _blobs(d, 773, d, 5, dtype), 5, dtype, max_iter=2)
+
+
 @pytest.mark.parametrize("n", [2, 255, 256, 257, 2048, 2049, 20001])
 def test_row_counts(oracle, n):
     k = 2 if n == 2 else 6
