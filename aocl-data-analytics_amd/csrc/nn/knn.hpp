@@ -142,6 +142,7 @@ template <typename T> class NNHandle : public AlgHandle {
                            bool return_distance, da_int *d_ind, T *d_dist);
     bool fused_eligible(da_int k) const;
     bool tiles_faster(da_int nq) const;
+    bool few_chunks(const SearchContext &ctx, da_int nq) const;
     int split_cap(int kc) const;
     int tile_splits(SearchContext &ctx, int prec, int kc, int variant, da_int nq,
                     const void *qpad, const float *seed, hipStream_t st,

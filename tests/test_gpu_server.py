@@ -180,3 +180,23 @@ def test_device_bytes_of_wide_rows(metric, max_bytes):
         de, ie = nn.kneighbors(Q, n_neighbors=10)
         np.testing.assert_array_equal(ind, ie)
         np.testing.assert_array_equal(dist, de)
+
+
+@pytest.mark.parametrize("n,d", [(47000, 8), (31531, 1), (3000, 5)])
+def test_few_bytes_and_queries_the_hit_bits_leave(n, d):
+    """Key tiles of a few rows at a time or, beyond eight of those, the fused tile: the results of
+    the handle's own search."""
+    rng = np.random.default_rng(d)
+    means = rng.uniform(-10, 10, (16, d))
+    X = (means[rng.integers(0, 16, n)] + 0.1 * rng.standard_normal((n, d))).astype(np.float32)
+    nn = aoclda.neighbors.nearest_neighbors(metric="euclidean").fit(X)
+    qs = [(means[rng.integers(0, 16, q)] + 0.1 * rng.standard_normal((q, d))).astype(np.float32)
+          for q in (1, 40, 130, 300, 2200)]
+    want = [nn.kneighbors(q, n_neighbors=9) for q in qs]
+    srv = nn_server(nn, max_batch_queries=4096, max_device_bytes=64 << 20)
+    for _ in range(2):
+        for (wd, wi), rid in zip(want, [srv.submit(q, 9) for q in qs]):
+            dist, ind, _ = srv.wait(rid)
+            np.testing.assert_array_equal(ind, wi)
+            np.testing.assert_array_equal(dist, wd)
+    srv.close()
