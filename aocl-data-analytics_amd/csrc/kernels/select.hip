@@ -44,24 +44,14 @@ __device__ void block_bitonic_sort(K *bkey, int *bidx) {
     }
 }
 
+// The k smallest of rk[0..n), by (key, column), to out_key / out_idx (columns from c0 on).
+// bkey, bidx: CAP entries of LDS. All threads of the block must call.
 template <typename K, int CAP>
-__global__ __launch_bounds__(256) void row_topk_kernel(const K *__restrict__ keys, int64_t ld,
-                                                       int rows, int n, int k, int largest,
-                                                       K *__restrict__ out_key,
-                                                       int *__restrict__ out_idx, int listed,
-                                                       int seg) {
-    __shared__ K bkey[CAP];
-    __shared__ int bidx[CAP];
+__device__ void row_select(const K *__restrict__ rk, int n, int k, int largest, int c0, K *bkey,
+                           int *bidx, K *__restrict__ out_key, int *__restrict__ out_idx) {
     __shared__ int count;
     __shared__ K thr_k;
     __shared__ int thr_i;
-    // Segment blockIdx.y of `seg` columns (the whole row when there is one); the results of
-    // (row, segment) pairs lie one after another.
-    const int64_t o = ((int64_t)blockIdx.x * gridDim.y + blockIdx.y) * k;
-    const int c0 = (int)blockIdx.y * seg;
-    // listed: only those that the bounded selection has left (marked -2).
-    if ((int)blockIdx.x >= rows || (listed && out_idx[o] != -2))
-        return;
     const K inf = (K)__builtin_huge_val();
     if (threadIdx.x == 0) {
         count = 0;
@@ -69,8 +59,6 @@ __global__ __launch_bounds__(256) void row_topk_kernel(const K *__restrict__ key
         thr_i = INT_MAX;
     }
     __syncthreads();
-    const K *rk = keys + (int64_t)blockIdx.x * ld + c0;
-    n = n - c0 < seg ? n - c0 : seg;
     for (int base = 0; base < n; base += 256) {
         const int j = base + threadIdx.x;
         if (j < n) {
@@ -115,9 +103,21 @@ __global__ __launch_bounds__(256) void row_topk_kernel(const K *__restrict__ key
     block_bitonic_sort<K, CAP>(bkey, bidx);
     for (int t = threadIdx.x; t < k; t += blockDim.x) {
         K v = bkey[t];
-        out_key[o + t] = largest ? -v : v;
-        out_idx[o + t] = bidx[t] == INT_MAX ? INT_MAX : c0 + bidx[t];
+        out_key[t] = largest ? -v : v;
+        out_idx[t] = bidx[t] == INT_MAX ? INT_MAX : c0 + bidx[t];
     }
+}
+
+template <typename K, int CAP>
+__global__ __launch_bounds__(256) void row_topk_kernel(const K *__restrict__ keys, int64_t ld,
+                                                       int n, int k, int largest,
+                                                       K *__restrict__ out_key,
+                                                       int *__restrict__ out_idx) {
+    __shared__ K bkey[CAP];
+    __shared__ int bidx[CAP];
+    const int64_t row = blockIdx.x;
+    row_select<K, CAP>(keys + row * ld, n, k, largest, 0, bkey, bidx, out_key + row * k,
+                       out_idx + row * k);
 }
 
 } // namespace
@@ -129,9 +129,10 @@ namespace {
 // key from above. A second pass collects the elements at or below it, -256 ln(1 - k / 256) on
 // average (5 for k = 5, 127 for k = 100), and one sort of those ends the row: two barriers-free
 // sweeps instead of two barriers per 256 elements and a 512-entry sort whenever the buffer fills.
-// Rows with more than SEL_CAP elements at or below the bound (ties) are left to the general
-// kernel: their out_idx[0] is set to -2. Rows of up to SEL_CAP elements never are, so that
-// launch is left out for them (5 us of a small search).
+// Rows with more than SEL_CAP elements at or below the bound (ties) are selected from by the
+// general way, in the same launch (a launch of its own behind this one: 5 us of a small search).
+// Segment blockIdx.y of `seg` columns (the whole row when there is one); the results of
+// (row, segment) pairs lie one after another.
 constexpr int SEL_CAP = 1024;
 template <typename K>
 __global__ __launch_bounds__(256) void row_topk_bound_kernel(const K *__restrict__ keys,
@@ -209,8 +210,7 @@ __global__ __launch_bounds__(256) void row_topk_bound_kernel(const K *__restrict
     __syncthreads();
     const int c = count;
     if (c > SEL_CAP) {
-        if (tid == 0)
-            out_idx[o] = -2;
+        row_select<K, 512>(rk, n, k, largest, c0, bkey, bidx, out_key + o, out_idx + o);
         return;
     }
     int cap = 2;
@@ -259,22 +259,21 @@ __global__ void row_topk_map_kernel(int *__restrict__ idx, const int *__restrict
 
 } // namespace
 
-// The selection over (row, segment) pairs: rows x nseg results of k.
+// The selection over (row, segment) pairs: rows x nseg results of k (segments only for k <= 128).
 template <typename K>
 static hipError_t topk_level(const K *keys, int64_t ld, int rows, int n, int k, int largest,
                              K *out_key, int *out_idx, int seg, int nseg, hipStream_t s) {
     dim3 grid(rows, nseg), block(256);
-    if (k <= 128)
+    if (k <= 128) {
         hipLaunchKernelGGL(row_topk_bound_kernel<K>, grid, block, 0, s, keys, ld, n, k, largest,
                            out_key, out_idx, seg);
-    if (k <= 128 && std::min(n, seg) <= SEL_CAP)
         return hipGetLastError();
+    }
     auto kern = k + 256 <= 512    ? row_topk_kernel<K, 512>
                 : k + 256 <= 1024 ? row_topk_kernel<K, 1024>
                 : k + 256 <= 2048 ? row_topk_kernel<K, 2048>
                                   : row_topk_kernel<K, 4096>;
-    hipLaunchKernelGGL(kern, grid, block, 0, s, keys, ld, rows, n, k, largest, out_key, out_idx,
-                       k <= 128 ? 1 : 0, seg);
+    hipLaunchKernelGGL(kern, dim3(rows), block, 0, s, keys, ld, n, k, largest, out_key, out_idx);
     return hipGetLastError();
 }
 
